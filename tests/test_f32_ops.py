@@ -333,3 +333,39 @@ def test_rms_norm_device_and_extremes(hip_ctx):
     assert np.all(same[:hd]) and np.all(np.isfinite(y[hd:]))
     for p in (dx, dg, dw, dy):
         hip_ctx.device_free(p)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("rows,cols", [
+    (1024, 260), (1025, 260),      # two waves a row, one (2048 waves are the line)
+    (512, 1028), (256, 2052),      # four and eight waves a row
+    (128, 4100), (129, 4097),      # sixteen; eight, in single floats
+    (5, 64 * 16 * 8 * 4 + 4),      # a second pass of eight loads, one unit long
+])
+def test_f32_matvec_wave_splits(hip_ctx, rows, cols):
+    rng = np.random.default_rng(rows * 7 + cols)
+    w = rng.standard_normal((rows, cols)).astype(np.float32)
+    x = rng.standard_normal(cols).astype(np.float32)
+    exact = w.astype(np.float64) @ x.astype(np.float64)
+    absdot = np.abs(w).astype(np.float64) @ np.abs(x).astype(np.float64)
+    y = hip_ctx.f32_matvec(w, rows, cols, x)
+    assert np.all(np.abs(y - exact) <= DOT_TOL * absdot)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("hd", [1023, 1025, 2049, 4096, 4097, 4100, 8192, 8196, 16384, 16388])
+@pytest.mark.parametrize("mode,heads", [(0, 1), (1, 2), (2, 3)])
+def test_rms_norm_register_passes(hip_ctx, mode, heads, hd):
+    """Head lengths on both sides of what one pass holds (1, 2 and 4 units a thread, floats and
+    float4s), and heads of more than one pass."""
+    rng = np.random.default_rng(mode * 100 + hd)
+    x = rng.standard_normal(heads * hd).astype(np.float32)
+    w = (rng.standard_normal(hd) * 0.5).astype(np.float32)
+    g = (rng.standard_normal(heads * hd) * 3).astype(np.float32)
+    if mode == 0:
+        y = hip_ctx.rms_norm(x, w, 1e-6)
+    elif mode == 1:
+        y = hip_ctx.rms_norm_heads(x, w, heads, hd, 1e-6)
+    else:
+        y = hip_ctx.rms_norm_gated(x, g, w, heads, hd, 1e-6)
+    assert_rms_close(y, f64_rms(mode, x, w, heads, hd, 1e-6, g), f"mode {mode}")
