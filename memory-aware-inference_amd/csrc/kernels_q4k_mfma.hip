@@ -54,7 +54,6 @@
 // counts nor orders buffer->LDS copies, and a fence would drain them.
 #include "mfma_common.h"
 #include "si_hip_tuned.h"
-#include "tokens_common.h"
 
 namespace sihip {
 namespace {
@@ -942,898 +941,6 @@ __global__ __launch_bounds__(WAVES * 64) void q4k_matvec_mfma(const uint8_t* __r
   if (fail != 0u) report_device_error(wsp, fail);
 }
 
-// ---- Several activation vectors in the MFMA rows --------------------------
-//
-// For a pass over the weights with 2..4 activation vectors (matmul-many,
-// replacing si_q4_k_matmul_many, metal.rs:1052-1262) the vectors share the A
-// operand of v_mfma_i32_16x16x32_i8, whose K = 32 is exactly one unit:
-//
-//  * A row 4 t + d holds digit d of vector t over the unit's 32 activations
-//    (lane 16 g + m supplies activations 8 g .. 8 g + 7 of row m); vectors
-//    past the pass's count are zero.
-//  * B lane (g, n) holds weights 8 g .. 8 g + 7 of the unit for tile row n:
-//    the low (unit 2 j) or high (unit 2 j + 1) nibbles of qs bytes
-//    32 j + 8 g .. 32 j + 8 g + 7.
-//  * Result lane (g, n) holds the four digit sums of vector g and row n, so
-//    T_d = sum_u sc_u C_u[d] over the block's eight units and the row's dot
-//    stay in that lane: y_g[n] += d * (sum_d T_d 256^d) * 2^(e_gb - 30) -
-//    dmin * sum_u m_u X_gu, with X_gu the f32 sum of vector g's unit u.
-//
-// Group images (4 KB per block, in the place of the four vectors' copies):
-// block b at img + 4096 b, unit pair p at + 1024 p, lane l at + 16 l, units
-// 2 p and 2 p + 1 in its two 8-byte halves.
-//
-// K slices.  Four vectors' images of a whole row (4 KB per block) would
-// crowd the stage buffers out of LDS, and with them the bytes in flight.  So
-// a launch with S > 1 cuts K into its S stages: GS workgroups per stage,
-// workgroup g works on stage k = g / GS for tiles g % GS, g % GS + GS, ...,
-// and keeps the images of that stage only.  Each pair is then its
-// workgroup's whole share of a tile: the wave stores each vector's and row's
-// sum over the stage in the scratch (part_out[(k * 4 NG + v) * rows + row],
-// or kPartRedo for a stage left to the exact path), and tok_reduce adds the
-// S sums in stage order (deterministic).  With S == 1 a workgroup keeps the
-// whole row's images and sums a tile's stages in its LDS slot ring.
-
-// Headers and the lane's four 8-byte qs slices of the four blocks of a stage
-// buffer: header of block b at hb + 2304 b, slice j at qb + 2304 b + 512 j.
-__device__ __forceinline__ void lds_read_weights_tok4(uint32_t hb, uint32_t qb, u32x4 (&h)[4],
-                                                      u32x2 (&q)[16]) {
-  asm volatile(
-      "ds_read_b128 %0, %20\n"
-      "ds_read_b64 %4, %21\n"
-      "ds_read_b64 %5, %21 offset:512\n"
-      "ds_read_b64 %6, %21 offset:1024\n"
-      "ds_read_b64 %7, %21 offset:1536\n"
-      "ds_read_b128 %1, %20 offset:2304\n"
-      "ds_read_b64 %8, %21 offset:2304\n"
-      "ds_read_b64 %9, %21 offset:2816\n"
-      "ds_read_b64 %10, %21 offset:3328\n"
-      "ds_read_b64 %11, %21 offset:3840\n"
-      "ds_read_b128 %2, %20 offset:4608\n"
-      "ds_read_b64 %12, %21 offset:4608\n"
-      "ds_read_b64 %13, %21 offset:5120\n"
-      "ds_read_b64 %14, %21 offset:5632\n"
-      "ds_read_b64 %15, %21 offset:6144\n"
-      "ds_read_b128 %3, %20 offset:6912\n"
-      "ds_read_b64 %16, %21 offset:6912\n"
-      "ds_read_b64 %17, %21 offset:7424\n"
-      "ds_read_b64 %18, %21 offset:7936\n"
-      "ds_read_b64 %19, %21 offset:8448\n"
-      "s_waitcnt lgkmcnt(0)"
-      : "=&v"(h[0]), "=&v"(h[1]), "=&v"(h[2]), "=&v"(h[3]), "=&v"(q[0]), "=&v"(q[1]),
-        "=&v"(q[2]), "=&v"(q[3]), "=&v"(q[4]), "=&v"(q[5]), "=&v"(q[6]), "=&v"(q[7]),
-        "=&v"(q[8]), "=&v"(q[9]), "=&v"(q[10]), "=&v"(q[11]), "=&v"(q[12]), "=&v"(q[13]),
-        "=&v"(q[14]), "=&v"(q[15])
-      : "v"(hb), "v"(qb)
-      : "memory");
-}
-
-// Q5_K (176-byte blocks: header, qh at +16, qs at +48): the same for a stage
-// buffer of Q5_K blocks -- header of block b at hb + 2816 b, qs slice j at
-// qb + 2816 b + 512 j -- and the lane's 8-byte qh slice of each block (the qh
-// bytes of its elements 8 g .. 8 g + 7, bit u for unit u) at qhb + 2816 b.
-__device__ __forceinline__ void lds_read_weights_tok5(uint32_t hb, uint32_t qb, uint32_t qhb,
-                                                      u32x4 (&h)[4], u32x2 (&q)[16],
-                                                      u32x2 (&qh)[4]) {
-  asm volatile(
-      "ds_read_b128 %0, %24\n"
-      "ds_read_b64 %4, %25\n"
-      "ds_read_b64 %5, %25 offset:512\n"
-      "ds_read_b64 %6, %25 offset:1024\n"
-      "ds_read_b64 %7, %25 offset:1536\n"
-      "ds_read_b64 %20, %26\n"
-      "ds_read_b128 %1, %24 offset:2816\n"
-      "ds_read_b64 %8, %25 offset:2816\n"
-      "ds_read_b64 %9, %25 offset:3328\n"
-      "ds_read_b64 %10, %25 offset:3840\n"
-      "ds_read_b64 %11, %25 offset:4352\n"
-      "ds_read_b64 %21, %26 offset:2816\n"
-      "ds_read_b128 %2, %24 offset:5632\n"
-      "ds_read_b64 %12, %25 offset:5632\n"
-      "ds_read_b64 %13, %25 offset:6144\n"
-      "ds_read_b64 %14, %25 offset:6656\n"
-      "ds_read_b64 %15, %25 offset:7168\n"
-      "ds_read_b64 %22, %26 offset:5632\n"
-      "ds_read_b128 %3, %24 offset:8448\n"
-      "ds_read_b64 %16, %25 offset:8448\n"
-      "ds_read_b64 %17, %25 offset:8960\n"
-      "ds_read_b64 %18, %25 offset:9472\n"
-      "ds_read_b64 %19, %25 offset:9984\n"
-      "ds_read_b64 %23, %26 offset:8448\n"
-      "s_waitcnt lgkmcnt(0)"
-      : "=&v"(h[0]), "=&v"(h[1]), "=&v"(h[2]), "=&v"(h[3]), "=&v"(q[0]), "=&v"(q[1]),
-        "=&v"(q[2]), "=&v"(q[3]), "=&v"(q[4]), "=&v"(q[5]), "=&v"(q[6]), "=&v"(q[7]),
-        "=&v"(q[8]), "=&v"(q[9]), "=&v"(q[10]), "=&v"(q[11]), "=&v"(q[12]), "=&v"(q[13]),
-        "=&v"(q[14]), "=&v"(q[15]), "=&v"(qh[0]), "=&v"(qh[1]), "=&v"(qh[2]), "=&v"(qh[3])
-      : "v"(hb), "v"(qb), "v"(qhb)
-      : "memory");
-}
-
-// The stage of a vectors-in-rows pass in registers: per block its header,
-// the lane's four 8-byte qs slices and (Q5_K) its qh slice.
-template <int QB>
-struct TokStage {
-  u32x4 h[4];
-  u32x2 q[16];
-  u32x2 qh[QB == 5 ? 4 : 1];
-};
-// The lane's stage addresses: header (hb0), qs slices (qb0) and qh slice
-// (qhb0, Q5_K) of the stage's first block.
-struct TokAddr {
-  uint32_t hb0, qb0, qhb0;
-};
-template <int QB>
-__device__ __forceinline__ void lds_read_weights_tok(const TokAddr& a, TokStage<QB>& st) {
-  if constexpr (QB == 5)
-    lds_read_weights_tok5(a.hb0, a.qb0, a.qhb0, st.h, st.q, st.qh);
-  else
-    lds_read_weights_tok4(a.hb0, a.qb0, st.h, st.q);
-}
-
-// The lane's group-image quarters of one block (unit pairs 0..3) and its
-// vector's eight unit sums.
-__device__ __forceinline__ void lds_read_group_block(uint32_t ia, uint32_t xa, u32x4 (&a)[4],
-                                                     u32x4 (&xs)[2]) {
-  asm volatile(
-      "ds_read_b128 %0, %6\n"
-      "ds_read_b128 %1, %6 offset:1024\n"
-      "ds_read_b128 %2, %6 offset:2048\n"
-      "ds_read_b128 %3, %6 offset:3072\n"
-      "ds_read_b128 %4, %7\n"
-      "ds_read_b128 %5, %7 offset:16\n"
-      "s_waitcnt lgkmcnt(0)"
-      : "=&v"(a[0]), "=&v"(a[1]), "=&v"(a[2]), "=&v"(a[3]), "=&v"(xs[0]), "=&v"(xs[1])
-      : "v"(ia), "v"(xa)
-      : "memory");
-}
-
-// The eight MFMAs of one block of row n against the lane's vector: c[u] the
-// four digit sums of unit u.  Q5_K: bit u of each qh byte is the weight's
-// fifth bit (rotated to bit 4: v_alignbit of a word with itself).
-template <int QB>
-__device__ __forceinline__ void block_mfma_tok(const TokStage<QB>& st, int b,
-                                               const u32x4 (&a)[4], i32x4 (&c)[8]) {
-  const i32x4 zero = {0, 0, 0, 0};
-#pragma unroll
-  for (int j = 0; j < 4; ++j) {
-    const u32x2 w = st.q[4 * b + j];
-    uint32_t lo0 = w[0] & 0x0f0f0f0fu, lo1 = w[1] & 0x0f0f0f0fu;
-    uint32_t hi0 = (w[0] >> 4) & 0x0f0f0f0fu, hi1 = (w[1] >> 4) & 0x0f0f0f0fu;
-    if constexpr (QB == 5) {
-      const u32x2 qh = st.qh[b];
-      const uint32_t rl = (2u * j + 28u) & 31u, rh = (2u * j + 29u) & 31u;  // bit u -> bit 4
-      lo0 |= __builtin_amdgcn_alignbit(qh[0], qh[0], rl) & 0x10101010u;
-      lo1 |= __builtin_amdgcn_alignbit(qh[1], qh[1], rl) & 0x10101010u;
-      hi0 |= __builtin_amdgcn_alignbit(qh[0], qh[0], rh) & 0x10101010u;
-      hi1 |= __builtin_amdgcn_alignbit(qh[1], qh[1], rh) & 0x10101010u;
-    }
-    c[2 * j] = __builtin_amdgcn_mfma_i32_16x16x32_i8(as_i64(a[j][0], a[j][1]), as_i64(lo0, lo1),
-                                                     zero, 0, 0, 0);
-    c[2 * j + 1] = __builtin_amdgcn_mfma_i32_16x16x32_i8(as_i64(a[j][2], a[j][3]),
-                                                         as_i64(hi0, hi1), zero, 0, 0, 0);
-  }
-}
-
-// One block of row n against vector g (the lane's), fast path: eight MFMAs,
-// the integer scale combine and the f32 digit and min terms over the
-// fixed-point unit sums xs; `err` gets the bound on its f32 rounding.  The
-// eight-term um is summed in pairs (within 5 * 2^-24 sum_u m_u |X_u| with the
-// sums' own rounding), so as in block_dot 2^-21 of the two terms' magnitudes
-// covers the whole.
-template <int QB>
-__device__ __forceinline__ float block_dot_tok(const TokStage<QB>& st, int b,
-                                               const u32x4 (&a)[4], const u32x4 (&xs)[2], int eb,
-                                               float& err) {
-  const u32x4 h = st.h[b];
-  const uint32_t sc03 = h[1] & 0x3f3f3f3fu;
-  const uint32_t mn03 = h[2] & 0x3f3f3f3fu;
-  const uint32_t sc47 = (h[3] & 0x0f0f0f0fu) | ((h[1] >> 2) & 0x30303030u);
-  const uint32_t mn47 = ((h[3] >> 4) & 0x0f0f0f0fu) | ((h[2] >> 2) & 0x30303030u);
-  i32x4 c[8];
-  block_mfma_tok<QB>(st, b, a, c);
-  int t[4] = {0, 0, 0, 0};
-#pragma unroll
-  for (int u = 0; u < 8; ++u) {
-    const int s = (int)(((u < 4 ? sc03 : sc47) >> (8 * (u & 3))) & 0xffu);
-#pragma unroll
-    for (int d = 0; d < 4; ++d) t[d] = mad_i24(s, c[u][d], t[d]);
-  }
-  const float tc =
-      fmaf(fmaf(fmaf((float)t[3], 256.0f, (float)t[2]), 256.0f, (float)t[1]), 256.0f, (float)t[0]);
-  float pr[4], ua = 0.0f;
-#pragma unroll
-  for (int k = 0; k < 4; ++k) {
-    const int u = 2 * k;
-    const float m0 = (float)(((u < 4 ? mn03 : mn47) >> (8 * (u & 3))) & 0xffu);
-    const float m1 = (float)(((u < 4 ? mn03 : mn47) >> (8 * ((u + 1) & 3))) & 0xffu);
-    const float s0 = __uint_as_float(xs[u >> 2][u & 3]);
-    const float s1 = __uint_as_float(xs[u >> 2][(u + 1) & 3]);
-    pr[k] = fmaf(m1, s1, m0 * s0);
-    ua = fmaf(m1, fabsf(s1), fmaf(m0, fabsf(s0), ua));
-  }
-  const float um = (pr[0] + pr[1]) + (pr[2] + pr[3]);
-  const float d = half_bits_to_float(h[0] & 0xffffu);
-  const float dmin = half_bits_to_float(h[0] >> 16);
-  const float dt = d * tc;
-  err = __builtin_amdgcn_ldexpf(fmaf(fabsf(dmin), ua, fabsf(dt)), eb - 21);
-  return __builtin_amdgcn_ldexpf(fmaf(-dmin, um, dt), eb);
-}
-
-// block_dot_tok's second try for a lane whose stage failed its check: the
-// same eight MFMAs and the same int32 digit sums T_d = sum_u sc_u C_u[d], then
-// sum_d 256^d T_d (< 2^50) formed exactly in f64 and the min term's products
-// (exact in f64) summed in f64.  What rounding is
-// left is that of the f32 unit sums xs (2^-24 each) and the f64 steps, so
-// err = 2^(eb-24) 1.01 |dmin| sum_u m_u |xs_u| + 2^(eb-48) of the two terms,
-// about an eighth of the fast path's bound.
-template <int QB>
-__device__ __forceinline__ double block_dot_tok_f64(const TokStage<QB>& st, int b,
-                                                    const u32x4 (&a)[4], const u32x4 (&xs)[2],
-                                                    int eb, float& err) {
-  const u32x4 h = st.h[b];
-  const uint32_t sc03 = h[1] & 0x3f3f3f3fu;
-  const uint32_t mn03 = h[2] & 0x3f3f3f3fu;
-  const uint32_t sc47 = (h[3] & 0x0f0f0f0fu) | ((h[1] >> 2) & 0x30303030u);
-  const uint32_t mn47 = ((h[3] >> 4) & 0x0f0f0f0fu) | ((h[2] >> 2) & 0x30303030u);
-  i32x4 c[8];
-  block_mfma_tok<QB>(st, b, a, c);
-  int t[4] = {0, 0, 0, 0};
-#pragma unroll
-  for (int u = 0; u < 8; ++u) {
-    const int s = (int)(((u < 4 ? sc03 : sc47) >> (8 * (u & 3))) & 0xffu);
-#pragma unroll
-    for (int d = 0; d < 4; ++d) t[d] = mad_i24(s, c[u][d], t[d]);
-  }
-  const double tc =
-      fma(fma(fma((double)t[3], 256.0, (double)t[2]), 256.0, (double)t[1]), 256.0, (double)t[0]);
-  double um = 0.0, ua = 0.0;
-#pragma unroll
-  for (int u = 0; u < 8; ++u) {
-    const double mn = (double)((((u < 4 ? mn03 : mn47) >> (8 * (u & 3))) & 0xffu));
-    const double xu = (double)__uint_as_float(xs[u >> 2][u & 3]);
-    um = fma(mn, xu, um);
-    ua = fma(mn, fabs(xu), ua);
-  }
-  const double d = (double)half_bits_to_float(h[0] & 0xffffu);
-  const double dmin = (double)half_bits_to_float(h[0] >> 16);
-  const double dt = d * tc;
-  const double mt = fabs(dmin) * ua;
-  err = (float)ldexp(fma(0x1.02p-24, mt, 0x1p-48 * (fabs(dt) + mt)), eb);
-  return ldexp(fma(-dmin, um, dt), eb);
-}
-
-// Exact per-weight path of one block of row n against 256 activations: the
-// block's 144 (Q4_K) or 176 (Q5_K) bytes at byte `off` of the buffer `wr`
-// (read from memory: by then the stage buffer may hold the next stage; bytes
-// past the buffer's end, those of rows past the matrix, read as zero).
-__device__ __forceinline__ float block_exact_row5(__amdgpu_buffer_rsrc_t wr, uint32_t off,
-                                                  const float* __restrict__ xs);
-template <int QB>
-__device__ __forceinline__ float block_exact_row(__amdgpu_buffer_rsrc_t wr, uint32_t off,
-                                                 const float* __restrict__ xs) {
-  if constexpr (QB == 5) return block_exact_row5(wr, off, xs);
-  auto ld = [&](uint32_t o) {
-    return __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(wr, off + o, 0, 0));
-  };
-  const u32x4 h = ld(0u);
-  u32x4 qa[4], qb[4];
-#pragma unroll
-  for (int k = 0; k < 4; ++k) {
-    qa[k] = ld(16u + 16u * k);
-    qb[k] = ld(80u + 16u * k);
-  }
-  const uint32_t sc03 = h[1] & 0x3f3f3f3fu;
-  const uint32_t mn03 = h[2] & 0x3f3f3f3fu;
-  const uint32_t sc47 = (h[3] & 0x0f0f0f0fu) | ((h[1] >> 2) & 0x30303030u);
-  const uint32_t mn47 = ((h[3] >> 4) & 0x0f0f0f0fu) | ((h[2] >> 2) & 0x30303030u);
-  const float d = half_bits_to_float(h[0] & 0xffffu);
-  const float dmin = half_bits_to_float(h[0] >> 16);
-  float acc = 0.0f;
-#pragma unroll
-  for (int u = 0; u < 8; ++u) {
-    // unit u: the low (even u) or high nibbles of qs pieces u & ~1, (u & ~1) + 1
-    const uint32_t sc = ((u < 4 ? sc03 : sc47) >> (8 * (u & 3))) & 0xffu;
-    const uint32_t mn = ((u < 4 ? mn03 : mn47) >> (8 * (u & 3))) & 0xffu;
-    const float d1 = __fmul_rn(d, (float)sc), m1 = __fmul_rn(dmin, (float)mn);
-    const int shift = 4 * (u & 1);
-    const int k = u & ~1;
-    acc = exact_dot16(k < 4 ? qa[k] : qb[k - 4], shift, d1, m1, xs + 32 * u, acc);
-    acc = exact_dot16(k < 4 ? qa[k + 1] : qb[k - 3], shift, d1, m1, xs + 32 * u + 16, acc);
-  }
-  return acc;
-}
-
-// Q5_K: unit u of the block is the low (even u) or high nibbles of qs bytes
-// 32 (u / 2) .. + 31 (at 48) with bit u of qh bytes 0 .. 31 (at 16) as the
-// fifth bit (quant.rs:67-125); the same order as the Q4_K form.
-__device__ __forceinline__ float block_exact_row5(__amdgpu_buffer_rsrc_t wr, uint32_t off,
-                                                  const float* __restrict__ xs) {
-  auto ld = [&](uint32_t o) {
-    return __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(wr, off + o, 0, 0));
-  };
-  const u32x4 h = ld(0u);
-  const u32x4 qh[2] = {ld(16u), ld(32u)};
-  u32x4 qs[8];
-#pragma unroll
-  for (int k = 0; k < 8; ++k) qs[k] = ld(48u + 16u * k);
-  const uint32_t sc03 = h[1] & 0x3f3f3f3fu;
-  const uint32_t mn03 = h[2] & 0x3f3f3f3fu;
-  const uint32_t sc47 = (h[3] & 0x0f0f0f0fu) | ((h[1] >> 2) & 0x30303030u);
-  const uint32_t mn47 = ((h[3] >> 4) & 0x0f0f0f0fu) | ((h[2] >> 2) & 0x30303030u);
-  const float d = half_bits_to_float(h[0] & 0xffffu);
-  const float dmin = half_bits_to_float(h[0] >> 16);
-  float acc = 0.0f;
-#pragma unroll
-  for (int u = 0; u < 8; ++u) {
-    const uint32_t sc = ((u < 4 ? sc03 : sc47) >> (8 * (u & 3))) & 0xffu;
-    const uint32_t mn = ((u < 4 ? mn03 : mn47) >> (8 * (u & 3))) & 0xffu;
-    const float d1 = __fmul_rn(d, (float)sc), m1 = __fmul_rn(dmin, (float)mn);
-    const int shift = 4 * (u & 1);
-    const int k = u & ~1;
-#pragma unroll
-    for (int half = 0; half < 2; ++half) {
-      const u32x4 q = qs[k + half], hbits = qh[half];
-#pragma unroll
-      for (int j = 0; j < 16; ++j) {
-        const uint32_t wq = ((q[j >> 2] >> (8 * (j & 3) + shift)) & 0x0fu) |
-                            (((hbits[j >> 2] >> (8 * (j & 3) + u)) & 1u) << 4);
-        acc = fmaf(k4_value_exact(d1, m1, wq), xs[32 * u + 16 * half + j], acc);
-      }
-    }
-  }
-  return acc;
-}
-
-// Launch constants: the slice count S (1: whole rows), GS workgroups per
-// slice (all of them when S == 1), the ring's slot count, and the division
-// constants of GS, of the stages per tile and of the slot count.
-struct TokArgs {
-  uint32_t slices, groups_per_slice, m_gps, m_parts;
-  uint32_t slots, m_slots;
-  void* wsp;  // the workspace, for failure reports
-};
-
-// LDS map: per-wave stage buffers; the images of ng groups of nbl blocks
-// (4 ng vectors), their unit sums and exponents; the slot ring (unused with
-// K slices).
-template <int QB>
-__host__ __device__ constexpr Layout tok_layout(uint32_t waves, uint32_t nbl, uint32_t ng,
-                                                uint32_t slots) {
-  return make_layout(stage_bytes(QB), 4u, 32u, waves, 1u, nbl, slots, 1u, 4u * ng);
-}
-
-// One vector group's sum over the live blocks of a stage (the weights in h,
-// q) on the fast path; blocks of the lane's vector that must take the exact
-// path count zero here.  iabase/xabase/eabase: the group's images, the
-// vector's unit sums and exponents at the stage's first block.  abs_part and
-// err get the lane's sum of |block dot| and the bound on their rounding.
-template <int QB>
-__device__ __forceinline__ float tok_group_stage(const TokStage<QB>& st, uint32_t nlive,
-                                                 uint32_t iabase, uint32_t xabase,
-                                                 uint32_t eabase, float& abs_part, float& err) {
-  i32x4 ex;
-  asm volatile("ds_read_b128 %0, %1\ns_waitcnt lgkmcnt(0)" : "=&v"(ex) : "v"(eabase) : "memory");
-  float part = 0.0f;
-  abs_part = 0.0f;
-  err = 0.0f;
-#pragma unroll
-  for (int b = 0; b < 4; ++b) {
-    if ((uint32_t)b < nlive) {
-      u32x4 a[4], xs[2];
-      lds_read_group_block(iabase + 4096u * b, xabase + 32u * b, a, xs);
-      float e;
-      const float v = block_dot_tok<QB>(st, b, a, xs, ex[b], e);
-      const bool fast = ex[b] != kBadBlock;
-      const float c = fast ? v : 0.0f;
-      part += c;
-      abs_part += fabsf(c);
-      err += fast ? e : 0.0f;
-    }
-  }
-  return part;
-}
-
-// tok_group_stage with block_dot_tok_f64: the sum in f64, with abs_part and
-// err (the bound on its rounding) as there.  Not inlined, and reading the
-// stage again from its LDS buffer (ta: the lane's addresses there), so that
-// its registers are taken on this rare path only.
-struct StageF64 {
-  double part;
-  float abs_part, err;
-};
-template <int QB>
-__device__ __noinline__ StageF64 tok_group_stage_f64(TokAddr ta, uint32_t nlive, uint32_t iabase,
-                                                     uint32_t xabase, uint32_t eabase) {
-  TokStage<QB> st;
-  lds_read_weights_tok<QB>(ta, st);
-  float abs_part, err;
-  i32x4 ex;
-  asm volatile("ds_read_b128 %0, %1\ns_waitcnt lgkmcnt(0)" : "=&v"(ex) : "v"(eabase) : "memory");
-  double part = 0.0;
-  abs_part = 0.0f;
-  err = 0.0f;
-#pragma unroll
-  for (int b = 0; b < 4; ++b) {
-    if ((uint32_t)b < nlive) {
-      u32x4 a[4], xs[2];
-      lds_read_group_block(iabase + 4096u * b, xabase + 32u * b, a, xs);
-      float e;
-      const double v = block_dot_tok_f64<QB>(st, b, a, xs, ex[b], e);
-      const bool fast = ex[b] != kBadBlock;
-      const double c = fast ? v : 0.0;
-      part += c;
-      abs_part += (float)fabs(c);
-      err += fast ? e : 0.0f;
-    }
-  }
-  return StageF64{part, abs_part, err};
-}
-
-// Side elements of a stage for the four vectors of one group (lane group r
-// accumulates vector r of the group, row n).  list0 / cnt0: side lists and
-// counts of the group's first vector at the stage's first block; the other
-// vectors follow at side_stride).  For an entry (i, x_i) of
-// vector r's block b, the lanes of group (i & 31) / 8 hold the qs byte of
-// element i for their rows (slice (i / 32) / 2 of the block; Q5_K: and the
-// qh byte of element i % 32 in their qh slice qh); lane group r takes w_i
-// from them and adds w_i x_i.
-template <int B, int QB>
-__device__ __forceinline__ float tok_side_block(u32x4 h, u32x2 s0, u32x2 s1, u32x2 s2, u32x2 s3,
-                                                u32x2 qh, uint32_t list, uint32_t counts,
-                                                uint32_t r, uint32_t lane, float part) {
-  const uint32_t grp = lane >> 4, n = lane & 15u;
-  uint32_t c = (counts >> (8 * B)) & 0xffu;
-  if (c == kSideRounded) c = 0u;
-  for (uint32_t k = 0; k < c; ++k) {
-    const u32x2 ent = lds_read_b64(list + kSideBytes * B + kSideEntryBytes * k);
-    const uint32_t i = ent[0];  // the same in every lane
-    const float xi = __uint_as_float(ent[1]);
-    const uint32_t u = i >> 5, l = i & 31u, j = u >> 1;
-    const u32x2 sl = j == 0u ? s0 : j == 1u ? s1 : j == 2u ? s2 : s3;
-    const uint32_t byte = (((l & 4u) ? sl[1] : sl[0]) >> (8u * (l & 3u))) & 0xffu;
-    uint32_t qv = (byte >> (4u * (u & 1u))) & 0x0fu;
-    if constexpr (QB == 5) {
-      const uint32_t hb = (((l & 4u) ? qh[1] : qh[0]) >> (8u * (l & 3u))) & 0xffu;
-      qv |= ((hb >> u) & 1u) << 4;
-    }
-    const float wv = k4_weight(h, u, qv);
-    const float wr = __int_as_float(
-        __builtin_amdgcn_ds_bpermute((int)(4u * (16u * (l >> 3) + n)), __float_as_int(wv)));
-    if (grp == r) part = fmaf(wr, xi, part);
-  }
-  return part;
-}
-// Largest |w| of a Q4_K (QMAX 15) or Q5_K (QMAX 31) block (all eight units)
-// from its header.
-template <int QMAX>
-__device__ __forceinline__ float k4_block_bound(const u32x4& h) {
-  const uint32_t sc03 = h[1] & 0x3f3f3f3fu;
-  const uint32_t mn03 = h[2] & 0x3f3f3f3fu;
-  const uint32_t sc47 = (h[3] & 0x0f0f0f0fu) | ((h[1] >> 2) & 0x30303030u);
-  const uint32_t mn47 = ((h[3] >> 4) & 0x0f0f0f0fu) | ((h[2] >> 2) & 0x30303030u);
-  const float ad = fabsf(half_bits_to_float(h[0] & 0xffffu));
-  const float am = fabsf(half_bits_to_float(h[0] >> 16));
-  float mx = 0.0f;
-#pragma unroll
-  for (int u = 0; u < 8; ++u) {
-    const uint32_t sc = ((u < 4 ? sc03 : sc47) >> (8 * (u & 3))) & 0xffu;
-    const uint32_t mn = ((u < 4 ? mn03 : mn47) >> (8 * (u & 3))) & 0xffu;
-    mx = fmaxf(mx, fmaf(ad, (float)((uint32_t)QMAX * sc), am * (float)mn));
-  }
-  return mx;
-}
-
-// Listed side elements of a stage for the four vectors of one group: lane
-// (r, n) gets vector r's sum of w_i x_i over them for row n.  list0 / cnt0:
-// side areas and counts of the group's first vector at the stage's first
-// block (the other vectors at side_stride); `mine`: the lane's
-// vector's counts.
-template <int QB>
-__device__ __forceinline__ float tok_listed(const TokStage<QB>& st, uint32_t list0, uint32_t mine,
-                                            uint32_t side_stride, uint32_t lane) {
-  const u32x4(&h)[4] = st.h;
-  const u32x2(&q)[16] = st.q;
-  auto qh = [&](int b) { return QB == 5 ? st.qh[QB == 5 ? b : 0] : u32x2{0u, 0u}; };
-  float part = 0.0f;
-  if (__builtin_amdgcn_ballot_w64((mine & ~(rounded_mask(mine) * 0xffu)) != 0u) == 0u)
-    return part;
-#pragma unroll 1
-  for (uint32_t r = 0; r < 4u; ++r) {
-    const uint32_t counts = __builtin_amdgcn_readlane(mine, 16 * r);
-    if (counts == 0u) continue;
-    const uint32_t list = list0 + r * side_stride;
-    part = tok_side_block<0, QB>(h[0], q[0], q[1], q[2], q[3], qh(0), list, counts, r, lane,
-                                 part);
-    part = tok_side_block<1, QB>(h[1], q[4], q[5], q[6], q[7], qh(1), list, counts, r, lane,
-                                 part);
-    part = tok_side_block<2, QB>(h[2], q[8], q[9], q[10], q[11], qh(2), list, counts, r, lane,
-                                 part);
-    part = tok_side_block<3, QB>(h[3], q[12], q[13], q[14], q[15], qh(3), list, counts, r, lane,
-                                 part);
-  }
-  return part;
-}
-
-// The lane's (vector r of the group, row n) error bound from its vector's
-// rounded blocks of the stage: the largest |w| of each such block (from its
-// header in h) times the block's error sum.
-template <int QB>
-__device__ __forceinline__ float tok_rounded_bound(uint32_t mine, uint32_t mylist,
-                                                   const u32x4 (&h)[4]) {
-  const uint32_t rmask = rounded_mask(mine);
-  float err = 0.0f;
-  if (__builtin_amdgcn_ballot_w64(rmask != 0u) == 0u) return err;
-#pragma unroll
-  for (int b = 0; b < 4; ++b)
-    if ((rmask >> b) & 1u)
-      err = fmaf(k4_block_bound<QB == 5 ? 31 : 15>(h[b]), rounded_err_all(mylist + kSideBytes * b),
-                 err);
-  return err;
-}
-
-template <int WAVES, int NG, int QB>
-__global__ __launch_bounds__(WAVES * 64) void q4k_tokens_mfma(const uint8_t* __restrict__ w,
-                                                              const float* __restrict__ x,
-                                                              float* __restrict__ y, uint32_t rows,
-                                                              uint32_t nb, uint32_t ntok,
-                                                              float* __restrict__ part_out,
-                                                              TokArgs ta) {
-  extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
-  constexpr uint32_t kPieces = block_pieces(QB);
-  constexpr uint32_t kStage = stage_bytes(QB);
-  constexpr uint32_t kBytes = QB == 5 ? kQ5Bytes : kQ4Bytes;
-  const uint32_t wave = uniform(threadIdx.x >> 6);
-  const uint32_t lane = threadIdx.x & 63u;
-  const uint32_t grp = lane >> 4, n = lane & 15u;
-  const uint32_t row_bytes = nb * kBytes;
-  const uint32_t ntiles = (rows + 15u) / 16u;
-  const uint32_t nstages = (nb + 3u) / 4u;
-  const uint32_t sbase = (uint32_t)(uintptr_t)smem;
-  uint8_t* const wstage = smem + wave * kStage;
-  const bool sliced = ta.slices > 1u;
-  const uint32_t ng = (ntok + 3u) / 4u;  // groups that hold vectors (<= NG)
-
-  // this workgroup's slice k (stages [s0, s0 + spt)) and its tiles tg,
-  // tg + GS, ...
-  const FastDiv by_gps{ta.groups_per_slice, ta.m_gps};
-  const uint32_t k = quo(blockIdx.x, by_gps);
-  const uint32_t tg = blockIdx.x - k * ta.groups_per_slice;
-  const uint32_t tstep = ta.groups_per_slice;
-  const uint32_t s0 = sliced ? k : 0u, spt = sliced ? 1u : nstages;
-  const uint32_t blk0 = 4u * s0, nbl = min(4u * spt, nb - blk0);
-  const Layout L = tok_layout<QB>(WAVES, nbl, NG, ta.slots);
-  const uint32_t ntw = tg < ntiles ? quo(ntiles - 1u - tg, by_gps) + 1u : 0u;
-  const uint32_t npairs = ntw * spt;
-  const FastDiv by_parts{spt, sliced ? 0u : ta.m_parts};
-
-  // 1. the vectors' blocks of the range into the image area
-  copy_x_group<WAVES>(smem, L.img, x, nb, blk0, nbl, ng, ntok, wave, lane);
-
-  // 2. this wave's pairs p = wave, wave + WAVES, ...: local tile p / spt,
-  //    stage s0 + p % spt; the first stage's copy goes out now
-  const uint32_t my_pairs = wave < npairs ? (npairs - 1u - wave) / WAVES + 1u : 0u;
-  const uint32_t voff = n * row_bytes + 16u * grp;
-  auto pair_of = [&](uint32_t p) {
-    Pair pr;
-    const uint32_t i = quo(p, by_parts);
-    pr.tile = tg + i * tstep;
-    pr.r = s0 + (p - i * spt);
-    pr.lt = i;
-    pr.lo = 0u;
-    pr.hi = spt;
-    return pr;
-  };
-  auto issue = [&](const Pair& pr) {
-    const uint32_t row0 = pr.tile * 16u;
-    const uint32_t nrows = min(16u, rows - row0);
-    const uint8_t* sb = w + (size_t)row0 * row_bytes + 4u * kBytes * pr.r;
-    const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc(
-        const_cast<uint8_t*>(sb), 0, (int)(nrows * row_bytes - 4u * kBytes * pr.r), kBufferWord3);
-#pragma unroll
-    for (int i = 0; i < (int)kPieces; ++i)
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, (lds_void*)(wstage + 1024 * i), 16,
-                                                voff + 64u * i, 0, 0, 0);
-  };
-  Pair pr_next = pair_of(wave);
-
-  // 3. ring slots and the builders' count, set before any wave goes on (the
-  //    waves start together, so this barrier costs little); every wave
-  //    issues its first copy, and the waves that copied x blocks (a wave
-  //    converts exactly the blocks it copied) build the group images once
-  //    they have landed and count themselves done.  A wave reads images only
-  //    once every builder has (wait_images), so no barrier makes a wave
-  //    whose stage has landed wait for the waves whose copies the memory
-  //    queue still holds back.  The first round of waves issues before the
-  //    barrier (the empty queue takes their copies at once), the rest after.
-  const bool first_round = wave < 4u;
-  if (first_round && my_pairs > 0u) issue(pr_next);
-  init_slots<WAVES>(sbase, L, ta.slots);
-  lds_wait();
-  __builtin_amdgcn_s_barrier();
-  if (!first_round && my_pairs > 0u) issue(pr_next);
-  const uint32_t builders = min((uint32_t)WAVES, ng * nbl);
-  if (wave < builders) {
-    if (my_pairs > 0u)
-      __builtin_amdgcn_s_waitcnt(waitcnt_vm(kPieces));
-    else
-      __builtin_amdgcn_s_waitcnt(waitcnt_vm(0));
-    build_group_images<WAVES, NG == 1>(sbase, L, nbl, ng, wave, lane);
-    lds_wait();
-    if (lane == 0u) (void)lds_add_rtn(sbase + L.ready, 1u);
-  }
-
-  // 4. the wave's pairs: lane (grp, n) accumulates, for each group g, vector
-  //    4 g + grp, row n
-  //    (the lane's 8-byte slices: qs bytes 32 j + 8 grp .. + 7 of unit pair j
-  //    and, Q5_K, qh bytes 8 grp .. + 7)
-  TokAddr sa;
-  sa.hb0 = sbase + wave * kStage + 16u * n;
-  sa.qhb0 = sa.hb0 + 256u * (1u + (grp >> 1)) + 8u * (grp & 1u);
-  sa.qb0 = QB == 5 ? sa.qhb0 + 512u : sa.qhb0;
-  uint32_t fail = 0u;  // a bounded wait that gave up (kDevErr*)
-  for (uint32_t j = 0; j < my_pairs; ++j) {
-    const Pair pr = pr_next;
-    const uint32_t s = pr.r, sl = s - s0;  // stage, and its place in the image range
-    __builtin_amdgcn_s_waitcnt(waitcnt_vm(0));
-    TokStage<QB> st;
-    lds_read_weights_tok<QB>(sa, st);
-    // the stage is in registers: the buffer takes the next stage's copy (the
-    // exact path reads its blocks from memory), issued once the stage's
-    // arithmetic is done: while the memory queue is full, issuing a copy
-    // holds the wave
-    auto issue_next = [&]() {
-      if (j + 1u < my_pairs) {
-        pr_next = pair_of(wave + (j + 1u) * WAVES);
-        issue(pr_next);
-      }
-    };
-    if (j == 0u) wait_images(sbase, L, builders, fail);
-    const uint32_t nlive = min(4u, nb - 4u * s);
-    bool any_bad = false;  // a block on the exact path
-    // the lane's vector's side counts of each group, kept for the groups'
-    // passes
-    uint32_t counts[NG];
-#pragma unroll
-    for (int g = 0; g < NG; ++g) counts[g] = 0u;
-    for (uint32_t g = 0; g < ng; ++g) {
-      i32x4 ex;
-      uint32_t cw;
-      asm volatile(
-          "ds_read_b128 %0, %2\n"
-          "ds_read_b32 %1, %2 offset:512\n"
-          "s_waitcnt lgkmcnt(0)"
-          : "=&v"(ex), "=&v"(cw)
-          : "v"(sbase + L.expo + (4u * g + grp) * L.expo_stride + 16u * sl)
-          : "memory");
-      cw = live_counts(cw, nlive);
-#pragma unroll
-      for (int gg = 0; gg < NG; ++gg)
-        if ((uint32_t)gg == g) counts[gg] = cw;
-      bool bad = false;
-#pragma unroll
-      for (int b = 0; b < 4; ++b) bad |= (uint32_t)b < nlive && ex[b] == kBadBlock;
-      any_bad |= __builtin_amdgcn_ballot_w64(bad) != 0u;
-    }
-    float part[NG];
-#pragma unroll
-    for (int g = 0; g < NG; ++g) part[g] = 0.0f;
-    uint32_t redo = 0u;  // bit g: the lane recomputes group g's stage exactly
-    float rbs[NG];  // (two or four groups: each group's rounded-block bound)
-    uint32_t redo_out = 0u;  // (K slices: bit g, tok_reduce recomputes it)
-    // (groups one after another: unrolled, their registers would add up)
-#pragma unroll 1
-    for (uint32_t g = 0; g < (NG == 1 ? 1u : ng); ++g) {
-      const uint32_t v = 4u * g + grp;
-      uint32_t mine = counts[0];
-#pragma unroll
-      for (int gg = 1; gg < NG; ++gg)
-        if ((uint32_t)gg == g) mine = counts[gg];
-      const bool any = __builtin_amdgcn_ballot_w64(mine != 0u) != 0u;
-      const uint32_t list0 =
-          sbase + L.expo + 4u * g * L.expo_stride + L.side_off + 4u * kSideBytes * sl;
-      // (listed side elements: one group only; with more, side elements make
-      // rounded blocks)
-      float side = 0.0f;
-      if constexpr (NG == 1)
-        side = any ? tok_listed<QB>(st, list0, mine, L.expo_stride, lane) : 0.0f;
-      float abs_pg, err;
-      const uint32_t iabase = sbase + L.img + 4096u * (g * nbl + 4u * sl) + 16u * lane;
-      const uint32_t xabase = sbase + L.xsum + v * L.xsum_stride + 128u * sl;
-      const uint32_t eabase = sbase + L.expo + v * L.expo_stride + 16u * sl;
-      float pg = side + tok_group_stage<QB>(st, nlive, iabase, xabase, eabase, abs_pg, err);
-      // the stage check of the lane's (vector, row): the fast path's rounding
-      // plus its rounded blocks against kStageTol of sum |partial|
-      const float rb = any ? tok_rounded_bound<QB>(mine, list0 + grp * L.expo_stride, st.h) : 0.0f;
-      err += rb;
-      const bool failed = !(err * 1.01f <= kStageTol * (abs_pg + fabsf(side) - err));
-      // One group (M <= 4): a lane that fails tries the stage again with the
-      // digit sums combined in f64 (a bound about eight times tighter; the
-      // stage is still in its LDS buffer, the images beside it) before it is
-      // left to the exact path, whose reads of weights from memory cost a
-      // launch 2.5 us of tail at about one failing lane in 2e4: M = 4 20.5 ->
-      // 18.6 us.  Made here, the call costs the two- and four-group kernels
-      // spills in their main loop (M = 8 31 -> 45 us); they make it after the
-      // groups' loop (below).
-      if (NG == 1 && __builtin_amdgcn_ballot_w64(failed) != 0u) {
-        const StageF64 sp = tok_group_stage_f64<QB>(sa, nlive, iabase, xabase, eabase);
-        const float err_p = sp.err + rb;
-        if (failed) {
-          if (err_p * 1.01f <= kStageTol * (sp.abs_part + fabsf(side) - err_p))
-            pg = side + (float)sp.part;
-          else
-            redo |= 1u << g;
-        }
-      } else if (NG > 1 && failed) {
-        redo |= 1u << g;
-      }
-#pragma unroll
-      for (int gg = 0; gg < NG; ++gg)
-        if ((uint32_t)gg == g) {
-          part[gg] = pg;
-          rbs[gg] = rb;
-        }
-    }
-    // Two or four groups: the lanes that failed try their groups' stages
-    // again in f64 once the groups' loop is done, one group at a time; what
-    // still fails goes to the exact path.  At M = 8 on Q4_K 17408x5120 about
-    // one stage lane in 2e4 fails the f32 check: left to tok_reduce, they
-    // gave 35 of its 544 workgroups an exact recompute (a second trip to
-    // memory) and the pass its tail.  Tried here, none is left: M = 8 / 16
-    // 28.5 / 42.6 -> 27.1 / 41.6 us, Q5_K 5120x5120 16.7 / 27.1 -> 15.3 /
-    // 25.1 us.
-    if constexpr (NG > 1) {
-      if (__builtin_amdgcn_ballot_w64(redo != 0u) != 0u) {
-#pragma unroll 1
-        for (uint32_t g = 0; g < ng; ++g) {
-          if (__builtin_amdgcn_ballot_w64((redo >> g) & 1u) == 0u) continue;
-          const uint32_t v = 4u * g + grp;
-          const StageF64 sp = tok_group_stage_f64<QB>(
-              sa, nlive, sbase + L.img + 4096u * (g * nbl + 4u * sl) + 16u * lane,
-              sbase + L.xsum + v * L.xsum_stride + 128u * sl,
-              sbase + L.expo + v * L.expo_stride + 16u * sl);
-          float rb = rbs[0];
-#pragma unroll
-          for (int gg = 1; gg < NG; ++gg)
-            if ((uint32_t)gg == g) rb = rbs[gg];
-          const float err_p = sp.err + rb;
-          if (((redo >> g) & 1u) && err_p * 1.01f <= kStageTol * (sp.abs_part - err_p)) {
-            redo &= ~(1u << g);
-#pragma unroll
-            for (int gg = 0; gg < NG; ++gg)
-              if ((uint32_t)gg == g) part[gg] = (float)sp.part;
-          }
-        }
-      }
-    }
-    // a K-sliced launch leaves the stages of lanes that failed the check to
-    // tok_reduce (kPartRedo below); the others take the exact path here
-    if (sliced) redo_out = redo;
-    const uint32_t redo_here = sliced ? 0u : redo;
-    if (any_bad || __builtin_amdgcn_ballot_w64(redo_here != 0u) != 0u) {
-      // the rare exact path: one loop over (group, block), weights read from
-      // memory, the rest addressed in LDS (no register array indexed at run
-      // time)
-      const uint32_t row0 = pr.tile * 16u;
-      const __amdgpu_buffer_rsrc_t wr = __builtin_amdgcn_make_buffer_rsrc(
-          const_cast<uint8_t*>(w + (size_t)row0 * row_bytes), 0,
-          (int)(min(16u, rows - row0) * row_bytes), kBufferWord3);
-#pragma unroll 1
-      for (uint32_t g = 0; g < ng; ++g) {
-        const uint32_t v = 4u * g + grp;
-        const float* const xv = x + (size_t)min(v, ntok - 1u) * nb * kBlockElems;
-        const bool whole = (redo_here >> g) & 1u;
-        float e = 0.0f;
-#pragma unroll 1
-        for (uint32_t b = 0; b < nlive; ++b) {
-          const uint32_t eb = lds_read_b32(sbase + L.expo + v * L.expo_stride + 4u * (4u * sl + b));
-          if ((int)eb == kBadBlock || whole)
-            e += block_exact_row<QB>(wr, n * row_bytes + kBytes * (4u * s + b),
-                                 xv + kBlockElems * (4u * s + b));
-        }
-#pragma unroll
-        for (int gg = 0; gg < NG; ++gg)
-          if ((uint32_t)gg == g) part[gg] = (whole ? 0.0f : part[gg]) + e;
-      }
-    }
-    issue_next();
-    if (!sliced) {
-      hand_off_lane_tokens(sbase, L, FastDiv{ta.slots, ta.m_slots}, pr, nstages, part[0], lane,
-                           rows, ntok, y, fail);
-      continue;
-    }
-    // the stage's partial sums of the tile's rows, for tok_reduce
-    const uint32_t row = pr.tile * 16u + n;
-    if (row < rows) {
-#pragma unroll
-      for (int g = 0; g < NG; ++g) {
-        const uint32_t v = 4u * g + grp;
-        if (v < ntok)
-          part_out[((size_t)s * 4u * NG + v) * rows + row] =
-              ((redo_out >> g) & 1u) ? __uint_as_float(kPartRedo) : part[g];
-      }
-    }
-  }
-  if (fail != 0u) report_device_error(ta.wsp, fail);
-}
-
-// Slice count of a launch: one per stage when the stages' partial sums of
-// nv vectors fit the workspace's scratch and every slice still has a
-// workgroup, else 1 (whole rows).
-inline uint32_t tok_slices(uint32_t rows, uint32_t nstages, uint32_t nv, size_t scratch_bytes) {
-  const uint32_t cus = (uint32_t)cu_count();
-  if (nstages < 2u || nstages > cus) return 1u;
-  if ((size_t)nstages * nv * rows * sizeof(float) > scratch_bytes) return 1u;
-  return nstages;
-}
-
-// ntok <= 4 NG vectors in one pass; false when the shape does not fit this
-// kernel (K slices need room in the scratch when NG > 1).
-template <int W, int NG, int QB = 4>
-bool launch_tokens_td(const uint8_t* w, const float* x, float* y, uint32_t rows, uint32_t nb,
-                      uint32_t ntok, const Workspace& ws, hipStream_t s, hipError_t* err) {
-  const uint32_t ntiles = (rows + 15u) / 16u;
-  const uint32_t nstages = (nb + 3u) / 4u;
-  TokArgs ta{};
-  uint32_t grid, lds;
-  ta.slices = tok_slices(rows, nstages, 4u * NG, ws.scratch_bytes);
-  if (ta.slices > 1u) {
-    ta.groups_per_slice = min((uint32_t)cu_count() / ta.slices, ntiles);
-    ta.slots = 1u;
-    grid = ta.groups_per_slice * ta.slices;
-    lds = tok_layout<QB>(W, min(4u, nb), NG, 1u).total;
-  } else {
-    if (NG > 1) return false;  // whole rows: one group's images already fill the LDS
-    ta.groups_per_slice = grid = min(ntiles, (uint32_t)cu_count());
-    const uint32_t tiles_per_group = (ntiles + grid - 1u) / grid;
-    ta.slots = ring_slots(W, 1, tiles_per_group, nstages);
-    ta.m_parts = div_magic(nstages);
-    lds = tok_layout<QB>(W, nb, NG, ta.slots).total;
-    // pair indices below tiles_per_group * nstages, divided by nstages
-    if ((uint64_t)tiles_per_group * nstages * nstages >= (1ull << 32)) return false;
-  }
-  ta.m_gps = div_magic(ta.groups_per_slice);
-  ta.m_slots = div_magic(ta.slots);
-  ta.wsp = ws.ptr;
-  // block and tile indices divided by GS
-  if ((uint64_t)(grid + ntiles) * ta.groups_per_slice >= (1ull << 32)) return false;
-  if (lds > kLdsBytes) return false;
-  static const hipError_t attr = hipFuncSetAttribute(
-      reinterpret_cast<const void*>(&q4k_tokens_mfma<W, NG, QB>),
-      hipFuncAttributeMaxDynamicSharedMemorySize, (int)kLdsBytes);
-  if (attr != hipSuccess) {
-    *err = attr;
-    return true;
-  }
-  hipLaunchKernelGGL((q4k_tokens_mfma<W, NG, QB>), dim3(grid), dim3(W * 64), lds, s, w, x, y, rows,
-                     nb, ntok, ws.scratch, ta);
-  *err = hipGetLastError();
-  if (*err == hipSuccess && ta.slices > 1u) {
-    launch_tok_reduce<QB == 5 ? kTypeQ5K : kTypeQ4K>(ws.scratch, y, rows, nstages, 4u * NG, ntok,
-                                                     w, x, nb, 4u, s);
-    *err = hipGetLastError();
-  }
-  return true;
-}
-
-// 3..16 vectors in one launch (with its reduce): the group count and wave
-// count that fit.
-template <int QB>
-bool launch_tokens_groups(const uint8_t* w, const float* x, float* y, uint32_t rows, uint32_t nb,
-                          uint32_t ntok, const Workspace& ws, hipStream_t s, hipError_t* err) {
-  if (ntok <= 4u) {
-    if constexpr (QB == 4) {
-      if (launch_tokens_td<12, 1, QB>(w, x, y, rows, nb, ntok, ws, s, err)) return true;
-    }
-    return launch_tokens_td<8, 1, QB>(w, x, y, rows, nb, ntok, ws, s, err) ||
-           launch_tokens_td<4, 1, QB>(w, x, y, rows, nb, ntok, ws, s, err);
-  }
-  // (the weights' decoded operands stay in registers across the groups: two
-  // waves per SIMD)
-  if (ntok <= 8u) return launch_tokens_td<8, 2, QB>(w, x, y, rows, nb, ntok, ws, s, err);
-  return launch_tokens_td<8, 4, QB>(w, x, y, rows, nb, ntok, ws, s, err) ||
-         launch_tokens_td<6, 4, QB>(w, x, y, rows, nb, ntok, ws, s, err);
-}
-
 template <int W, int D, int M, int NT = 1, int QB = 4, bool G = false, int SB = 4,
           bool LN = false>
 bool launch_wd(const uint8_t* w, const uint8_t* w2, const float* x, float* y, uint32_t rows,
@@ -2139,7 +1246,7 @@ bool matmul_passes(const uint8_t* w, const float* x, float* y, uint32_t rows, ui
       // up to sixteen vectors share the matrix-core rows in one pass (two
       // go faster one vector per MFMA)
       const uint32_t ng = batch - b >= 3u ? min(16u, batch - b) : nt;
-      if (ng >= 3u && launch_tokens_groups<QB>(w, xb, yb, rows, nb, ng, ws, s, err)) {
+      if (ng >= 3u && launch_q45_tokens(QB, w, xb, yb, rows, nb, ng, ws, s, err)) {
         if (*err != hipSuccess) return true;
         b += ng;
         continue;

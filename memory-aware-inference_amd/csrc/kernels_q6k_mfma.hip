@@ -1345,7 +1345,7 @@ bool launch_tok6(const uint8_t* w, const float* x, float* y, uint32_t rows, uint
                      ws.scratch, ta);
   *err = hipGetLastError();
   if (*err == hipSuccess) {
-    launch_tok_reduce<kTypeQ6K>(ws.scratch, y, rows, ta.slices, 4u * NG, ntok, w, x, nb, ta.nbs, s);
+    launch_tok_reduce<kTypeQ6K>(ws.scratch, y, rows, rows, ta.slices, 4u * NG, ntok, w, x, nb, ta.nbs, s);
     *err = hipGetLastError();
   }
   return true;

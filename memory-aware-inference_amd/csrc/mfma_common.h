@@ -1275,36 +1275,6 @@ __device__ __forceinline__ void hand_off_tokens(uint32_t sbase, const Layout& L,
   token_slot_done<NTOK>(sbase, L, by_slots, pr, tparts, lane, rows, y);
 }
 
-// hand_off_tokens for kernels that keep vector g's row sums in lane group g
-// (lane 16 g + n holds vector g, row n): every lane writes its own sum; the
-// finishing wave's lane group g stores vector g's rows (g < ntok).
-__device__ __forceinline__ void hand_off_lane_tokens(uint32_t sbase, const Layout& L,
-                                                     const FastDiv& by_slots, const Pair& pr,
-                                                     uint32_t tparts, float rowsum, uint32_t lane,
-                                                     uint32_t rows, uint32_t ntok,
-                                                     float* __restrict__ y, uint32_t& fail) {
-  const uint32_t grp = lane >> 4, n = lane & 15u;
-  const uint32_t slots = by_slots.d;
-  const uint32_t slot = pr.lt - quo(pr.lt, by_slots) * slots;
-  wait_slot(sbase + L.owner + 4u * slot, pr.lt, fail);
-  // the slot's partial r holds [vector][16 rows], 256 bytes
-  lds_write_b32(sbase + L.part + 256u * (slot * tparts + pr.r) + 4u * lane,
-                __float_as_uint(rowsum));
-  uint32_t old = 0u;
-  if (lane == 0u) old = lds_add_rtn(sbase + L.cnt + 4u * slot, 1u);
-  const uint32_t done = __builtin_amdgcn_readlane(old, 0);
-  if (done != tparts - 1u) return;
-  const uint32_t row = pr.tile * 16u + n;
-  float sum = 0.0f;
-  for (uint32_t st = 0; st < tparts; ++st)
-    sum += __uint_as_float(lds_read_b32(sbase + L.part + 256u * (slot * tparts + st) + 4u * lane));
-  if (grp < ntok && row < rows) y[(size_t)grp * rows + row] = sum;
-  if (lane == 0u) {
-    lds_write_b32(sbase + L.cnt + 4u * slot, 0u);
-    lds_write_b32(sbase + L.owner + 4u * slot, pr.lt + slots);
-  }
-}
-
 // The schedule constants of a launch, or false when a multiply-high quotient
 // of the schedule could be inexact (x * d >= 2^32 for some quotient taken) or
 // the counts do not fit their fields.
@@ -1332,6 +1302,13 @@ inline uint32_t ring_slots(uint32_t waves, uint32_t depth, uint32_t tiles_per_wg
   while (slots > 2u && slots * tparts * 64u > 8192u) --slots;
   return slots;
 }
+
+// kernels_q45_tokens.hip: Q4_K (qb 4) or Q5_K (qb 5), ntok = 2..16 vectors
+// (batch-major x and y) in one pass over the weights; false when the shape
+// does not fit.
+bool launch_q45_tokens(int qb, const uint8_t* w, const float* x, float* y, uint32_t rows,
+                       uint32_t nb, uint32_t ntok, const Workspace& ws, hipStream_t s,
+                       hipError_t* err);
 
 // kernels_q6k_mfma.hip: a group of Q6_K matrices (GroupArgs) in one launch.
 bool launch_q6k_matvec_group(const GroupArgs& ga, uint32_t total_rows, uint32_t cols,

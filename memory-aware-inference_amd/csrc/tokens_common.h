@@ -135,13 +135,178 @@ __device__ __forceinline__ void build_group_images(uint32_t sbase, const Layout&
 }
 
 
+// ---- Group images for v_mfma_i32_16x16x64_i8 -------------------------------
+//
+// The same four vectors of four digits per group in the 16 A rows, K = 64 (lane
+// 16 k + 4 t + d: digit d of vector t over the 16 elements that meet lane
+// group k's weights): a block is four MFMAs j, 1 KB each, chunk c (elements
+// 16 c .. 16 c + 15) at the offset a format's map gives, 1024 j + 256 k.
+
+// Plain LDS reads (the compiler places their waits, so that a block's reads
+// overlap).  Only between a wave's wait for its stage copy and its next copy:
+// with a buffer->LDS copy of its own in flight the compiler would wait for it
+// at the first such read.
+typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
+typedef _Float16 f16x4 __attribute__((ext_vector_type(4)));
+typedef uint16_t u16x2 __attribute__((ext_vector_type(2)));
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+__device__ __forceinline__ u32x4 lds_u32x4(const uint8_t* p) {
+  return *(const __attribute__((address_space(3))) u32x4*)p;
+}
+__device__ __forceinline__ uint32_t lds_u32(const uint8_t* p) {
+  return *(const __attribute__((address_space(3))) uint32_t*)p;
+}
+__device__ __forceinline__ void lds_write_b16(uint32_t addr, uint32_t v) {
+  asm volatile("ds_write_b16 %0, %1" : : "v"(addr), "v"(v) : "memory");
+}
+
+// The exponent slot of a block that takes the exact path: scaling by it gives
+// zero.
+constexpr int kBadTok = -(1 << 20);
+
+// LDS map of a launch whose workgroups keep nbl blocks of ng groups (group
+// g's block b is group-block gb = g nbl + b): the waves' stage buffers, then
+// the group images (4 KB per group-block); with `mins`, the unit sums
+// (256 bytes per group-block: lane group k's units 2 k and 2 k + 1 as two
+// halves at 64 k + 4 (4 t + p), piece p of vector t); with `dsum`, 128 times
+// each vector's digit sums (64 bytes per group-block, vector t's four at
+// 16 t); per vector v the exponents (16 bytes at 16 v; nbl <= 4 blocks, or
+// 4 nbl bytes) and the rounded blocks' error sums (0 for other blocks); the
+// count of builders done and the flag that some block is rounded or on the
+// exact path.
+struct TokLayout {
+  uint32_t img, usum, dsum, expo, rerr, ready, special, total;
+  uint32_t vec_stride;  // bytes per vector of exponents and of error sums
+};
+__host__ __device__ constexpr TokLayout tok64_layout(uint32_t stage_total, uint32_t nbl,
+                                                     uint32_t ng, bool mins, bool dsum) {
+  TokLayout l{};
+  l.vec_stride = 4u * ((nbl + 3u) & ~3u);
+  l.img = stage_total;
+  l.usum = l.img + 4096u * ng * nbl;
+  l.dsum = l.usum + (mins ? 256u * ng * nbl : 0u);
+  l.expo = l.dsum + (dsum ? 64u * ng * nbl : 0u);
+  l.rerr = l.expo + 4u * ng * l.vec_stride;
+  l.ready = l.rerr + 4u * ng * l.vec_stride;
+  l.special = l.ready + 4u;
+  l.total = l.ready + 16u;
+  return l;
+}
+
+// Waits until `builders` waves have counted themselves done at `ready`,
+// bounded like wait_slot.
+__device__ __forceinline__ void wait_count(uint32_t ready, uint32_t builders, uint32_t& fail) {
+  uint32_t spin = 0;
+  for (; lds_read_b32(ready) < builders && spin < (1u << 24); ++spin)
+    __builtin_amdgcn_s_sleep(1);
+  if (__builtin_amdgcn_readfirstlane(spin) == (1u << 24)) fail = kDevErrSlotWait;
+}
+
+// Inclusive sum over a DPP row's 16 lanes (valid in lane 15).
+__device__ __forceinline__ uint32_t row_sum_u(uint32_t v) {
+  v += dpp_u<kRowShr1>(v);
+  v += dpp_u<kRowShr2>(v);
+  v += dpp_u<kRowShr4>(v);
+  return v + dpp_u<kRowShr8>(v);
+}
+__device__ __forceinline__ float row_sum_f(float v) {
+  v += dpp<kRowShr1>(v);
+  v += dpp<kRowShr2>(v);
+  v += dpp<kRowShr4>(v);
+  return v + dpp<kRowShr8>(v);
+}
+
+// Turns the group-blocks copied by copy_x_group into images in place, with
+// what else the layout keeps of them; a wave converts exactly the group-blocks
+// it copied, lane (t, c) elements 16 c .. 16 c + 15 of vector 4 g + t.  Blocks
+// with side elements are rounded blocks (mfma_common.h), and a block with an
+// activation that is not finite or reaches 2^100 gets the exponent kBadTok.
+template <int WAVES, bool MINS, bool DSUM, typename ChunkSlot>
+__device__ __forceinline__ void build_group_images64(uint32_t sbase, const TokLayout& L,
+                                                     uint32_t nbl, uint32_t ng, uint32_t wave,
+                                                     uint32_t lane, ChunkSlot chunk_slot) {
+  const uint32_t t = lane >> 4, c = lane & 15u;
+  const uint32_t woff = chunk_slot(c) + 64u * t;
+  for_group_blocks<WAVES>(ng, nbl, wave, [&](uint32_t g, uint32_t b) {
+    const uint32_t gb = g * nbl + b;
+    const uint32_t blk = sbase + L.img + 4096u * gb;
+    const uint32_t vec = L.vec_stride * (4u * g + t) + 4u * b;
+    u32x4 xq[4];
+    lds_read4<16>(blk + 1024u * t + 64u * c, xq);
+    float xv[16];
+#pragma unroll
+    for (int k = 0; k < 4; ++k)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) xv[4 * k + i] = __uint_as_float(xq[k][i]);
+    const ChunkSplit cs = split_chunk(xv);
+    const uint64_t bad_any = __builtin_amdgcn_ballot_w64(cs.bad);
+    const uint64_t side_any = __builtin_amdgcn_ballot_w64(cs.smask != 0u);
+    const bool bad = ((bad_any >> (16u * t)) & 0xffffull) != 0u;
+    uint32_t uq[16];
+    biased_values(cs, false, uq);
+    uint32_t dg[4][4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k)
+      transpose_digits(uq[4 * k], uq[4 * k + 1], uq[4 * k + 2], uq[4 * k + 3], dg[k]);
+    // the wave has read the whole block (lds_read4 waits) before any write
+#pragma unroll
+    for (int d = 0; d < 4; ++d)
+      lds_write_b128(blk + woff + 16u * d, u32x4{dg[0][d], dg[1][d], dg[2][d], dg[3][d]});
+    if constexpr (MINS) {
+      // unit u = c / 2's sum (odd lanes hold both halves): |X_u| <= 2^35
+      uint32_t hi = 0u, lo = 0u;
+#pragma unroll
+      for (int k = 0; k < 16; ++k) {
+        const int32_t X = (int32_t)(uq[k] - 0x80808080u);
+        hi += (uint32_t)(X >> 15);
+        lo += (uint32_t)X & 0x7fffu;
+      }
+      hi += dpp_u<kRowShr1>(hi);
+      lo += dpp_u<kRowShr1>(lo);
+      int64_t v = (int64_t)(int32_t)hi * 32768 + (int64_t)lo;
+      const uint32_t at = sbase + L.usum + 256u * gb + 64u * (c >> 2) + 16u * t + (c & 2u);
+#pragma unroll
+      for (int p = 0; p < 3; ++p) {
+        // the low 12 bits, signed; the last piece is what is left (|.| <= 2048)
+        const int piece = p < 2 ? ((int)((uint32_t)v << 20) >> 20) : (int)v;
+        v = (v - piece) >> 12;
+        const _Float16 h = (_Float16)(float)piece;
+        if (c & 1u) lds_write_b16(at + 4u * p, __builtin_bit_cast(uint16_t, h));
+      }
+      if (c & 1u) lds_write_b16(at + 12u, 0u);
+    }
+    if constexpr (DSUM) {
+      uint32_t s[4];
+#pragma unroll
+      for (int d = 0; d < 4; ++d) {
+        int sum = 0;
+#pragma unroll
+        for (int k = 0; k < 4; ++k)
+          sum = __builtin_amdgcn_sdot4((int)dg[k][d], 0x01010101, sum, false);
+        s[d] = 128u * row_sum_u((uint32_t)sum);
+      }
+      if (c == 15u)
+        lds_write_b128(sbase + L.dsum + 64u * gb + 16u * t, u32x4{s[0], s[1], s[2], s[3]});
+    }
+    float err = 0.0f;
+    if ((bad_any | side_any) != 0u) {
+      err = row_sum_f(cs.err_side);
+      if (lane == 0u) lds_write_b32(sbase + L.special, 1u);
+    }
+    if (c == 15u) {
+      lds_write_b32(sbase + L.expo + vec, (uint32_t)(bad ? kBadTok : cs.e - kFixBits));
+      lds_write_b32(sbase + L.rerr + vec, bad ? 0u : __float_as_uint(err));
+    }
+  });
+}
+
 // Sum of all 16 chunk error sums of a rounded block's side area.
 __device__ __forceinline__ float rounded_err_all(uint32_t list) {
   return (rounded_err(list, 0u) + rounded_err(list, 1u)) +
          (rounded_err(list, 2u) + rounded_err(list, 3u));
 }
 
-// y[t * rows + row] = sum over the stages s of part[(s * nv + t) * rows + row],
+// y[t * yrows + row] = sum over the stages s of part[(s * nv + t) * rows + row],
 // in stage order (the sliced launch's second kernel; a "stage" here is the
 // first kernel's unit of partial sums, bps blocks).  A partial that holds
 // kPartRedo (its lane failed a check in the first kernel) is the stage's
@@ -156,7 +321,6 @@ __device__ __forceinline__ float rounded_err_all(uint32_t list) {
 // R rows per thread: 1, or 4 with 16-byte loads and stores (launch_tok_reduce
 // takes 4 when the rows, y and the grid allow it); each row's sum is the same.
 constexpr uint32_t kRedoQueue = 64;
-typedef float f32x4 __attribute__((ext_vector_type(4)));
 template <uint32_t T>
 __device__ __noinline__ float stage_exact(const uint8_t* __restrict__ w, uint32_t row,
                                           uint32_t nb, uint32_t b0, uint32_t b1,
@@ -179,7 +343,7 @@ __device__ __noinline__ float stage_exact(const uint8_t* __restrict__ w, uint32_
 template <uint32_t T, int R>
 __global__ __launch_bounds__(256) void tok_reduce(const float* __restrict__ part,
                                                   float* __restrict__ y, uint32_t rows,
-                                                  uint32_t nstages, uint32_t nv,
+                                                  uint32_t yrows, uint32_t nstages, uint32_t nv,
                                                   const uint8_t* __restrict__ w,
                                                   const float* __restrict__ x, uint32_t nb,
                                                   uint32_t bps) {
@@ -306,7 +470,7 @@ __global__ __launch_bounds__(256) void tok_reduce(const float* __restrict__ part
       }
     }
   }
-  float* const yo = y + (size_t)t * rows + row;
+  float* const yo = y + (size_t)t * yrows + row;
   if constexpr (R == 4) {
     *reinterpret_cast<f32x4*>(yo) = f32x4{sum[0], sum[1], sum[2], sum[3]};
   } else {
@@ -315,23 +479,23 @@ __global__ __launch_bounds__(256) void tok_reduce(const float* __restrict__ part
 }
 
 // The reduce of a sliced launch of ntok vectors: four rows a thread when the
-// row count is a multiple of 4, y is 16-byte aligned (the scratch always is)
-// and the grid still gives every CU two workgroups, else one.  The Q6_K head
+// row counts (of the launch, and yrows of a vector's outputs) are multiples
+// of 4, y is 16-byte aligned (the scratch always is) and the grid still gives every CU two workgroups, else one.  The Q6_K head
 // (151,936 rows) at M = 4 / 8 / 16: 144.6 / 180.1 / 321.5 -> 143.6 / 176.8 /
 // 317.4 us a call; Q4_K 17408 rows at M = 16 (one workgroup a CU) lost
 // 0.4 us, so it keeps one row a thread.
 template <uint32_t T>
-void launch_tok_reduce(const float* part, float* y, uint32_t rows, uint32_t nstages, uint32_t nv,
-                       uint32_t ntok, const uint8_t* w, const float* x, uint32_t nb, uint32_t bps,
-                       hipStream_t s) {
+void launch_tok_reduce(const float* part, float* y, uint32_t rows, uint32_t yrows,
+                       uint32_t nstages, uint32_t nv, uint32_t ntok, const uint8_t* w,
+                       const float* x, uint32_t nb, uint32_t bps, hipStream_t s) {
   const uint32_t g4 = (rows + 1023u) / 1024u;
-  if (rows % 4u == 0u && ((uintptr_t)y & 15u) == 0u &&
+  if (rows % 4u == 0u && yrows % 4u == 0u && ((uintptr_t)y & 15u) == 0u &&
       (uint64_t)g4 * ntok >= 2u * (uint64_t)cu_count())
-    hipLaunchKernelGGL((tok_reduce<T, 4>), dim3(g4, ntok), dim3(256), 0, s, part, y, rows, nstages,
-                       nv, w, x, nb, bps);
+    hipLaunchKernelGGL((tok_reduce<T, 4>), dim3(g4, ntok), dim3(256), 0, s, part, y, rows, yrows,
+                       nstages, nv, w, x, nb, bps);
   else
     hipLaunchKernelGGL((tok_reduce<T, 1>), dim3((rows + 255u) / 256u, ntok), dim3(256), 0, s, part,
-                       y, rows, nstages, nv, w, x, nb, bps);
+                       y, rows, yrows, nstages, nv, w, x, nb, bps);
 }
 
 }  // namespace
