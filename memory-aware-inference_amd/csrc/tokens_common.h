@@ -142,10 +142,9 @@ __device__ __forceinline__ void build_group_images(uint32_t sbase, const Layout&
 // group k's weights): a block is four MFMAs j, 1 KB each, chunk c (elements
 // 16 c .. 16 c + 15) at the offset a format's map gives, 1024 j + 256 k.
 
-// Plain LDS reads (the compiler places their waits, so that a block's reads
-// overlap).  Only between a wave's wait for its stage copy and its next copy:
-// with a buffer->LDS copy of its own in flight the compiler would wait for it
-// at the first such read.
+// Plain LDS reads: the compiler places their waits, so that a block's reads
+// overlap.  (For kernels without buffer->LDS copies, which the compiler would
+// wait for at the first such read.)
 typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
 typedef _Float16 f16x4 __attribute__((ext_vector_type(4)));
 typedef uint16_t u16x2 __attribute__((ext_vector_type(2)));
@@ -164,140 +163,173 @@ __device__ __forceinline__ void lds_write_b16(uint32_t addr, uint32_t v) {
 // zero.
 constexpr int kBadTok = -(1 << 20);
 
-// LDS map of a launch whose workgroups keep nbl blocks of ng groups (group
-// g's block b is group-block gb = g nbl + b): the waves' stage buffers, then
-// the group images (4 KB per group-block); with `mins`, the unit sums
-// (256 bytes per group-block: lane group k's units 2 k and 2 k + 1 as two
-// halves at 64 k + 4 (4 t + p), piece p of vector t); with `dsum`, 128 times
-// each vector's digit sums (64 bytes per group-block, vector t's four at
-// 16 t); per vector v the exponents (16 bytes at 16 v; nbl <= 4 blocks, or
-// 4 nbl bytes) and the rounded blocks' error sums (0 for other blocks); the
-// count of builders done and the flag that some block is rounded or on the
-// exact path.
+// LDS map of a launch whose workgroups keep up to stride = 4 blocks of ng
+// groups (group g's block b is group-block gb = stride g + b): the
+// group images (4 KB per group-block); with `mins`, the unit sums (256 bytes
+// per group-block: lane group k's units 2 k and 2 k + 1 as two halves at
+// 64 k + 4 (4 t + p), piece p of vector t); with `dsum`, 128 times each
+// vector's digit sums (64 bytes per group-block, vector t's four at 16 t); per
+// vector v, 4 stride bytes each, the exponents and the bounds on the side
+// elements' rounding (infinite for a block on the exact path).
 struct TokLayout {
-  uint32_t img, usum, dsum, expo, rerr, ready, special, total;
-  uint32_t vec_stride;  // bytes per vector of exponents and of error sums
+  uint32_t img, usum, dsum, expo, rerr, total;
+  uint32_t stride;
 };
-__host__ __device__ constexpr TokLayout tok64_layout(uint32_t stage_total, uint32_t nbl,
-                                                     uint32_t ng, bool mins, bool dsum) {
+__host__ __device__ constexpr TokLayout tok64_layout(uint32_t stride, uint32_t ng, bool mins,
+                                                     bool dsum) {
   TokLayout l{};
-  l.vec_stride = 4u * ((nbl + 3u) & ~3u);
-  l.img = stage_total;
-  l.usum = l.img + 4096u * ng * nbl;
-  l.dsum = l.usum + (mins ? 256u * ng * nbl : 0u);
-  l.expo = l.dsum + (dsum ? 64u * ng * nbl : 0u);
-  l.rerr = l.expo + 4u * ng * l.vec_stride;
-  l.ready = l.rerr + 4u * ng * l.vec_stride;
-  l.special = l.ready + 4u;
-  l.total = l.ready + 16u;
+  l.stride = stride;
+  l.img = 0u;
+  l.usum = l.img + 4096u * ng * stride;
+  l.dsum = l.usum + (mins ? 256u * ng * stride : 0u);
+  l.expo = l.dsum + (dsum ? 64u * ng * stride : 0u);
+  l.rerr = l.expo + 16u * ng * stride;
+  l.total = l.rerr + 16u * ng * stride;
   return l;
 }
 
-// Waits until `builders` waves have counted themselves done at `ready`,
-// bounded like wait_slot.
-__device__ __forceinline__ void wait_count(uint32_t ready, uint32_t builders, uint32_t& fail) {
-  uint32_t spin = 0;
-  for (; lds_read_b32(ready) < builders && spin < (1u << 24); ++spin)
-    __builtin_amdgcn_s_sleep(1);
-  if (__builtin_amdgcn_readfirstlane(spin) == (1u << 24)) fail = kDevErrSlotWait;
+// The wave's share of the image blocks: group-blocks q = wave + i WAVES, i <
+// SHARE, of the ng groups in order of group and of the blocks 0 .. stride - 1
+// (those past nbl hold nothing); lane (t, c) takes elements 16 c .. 16 c + 15 of
+// vector 4 g + t.  Vectors past ntok read as zero.
+template <int WAVES, int SHARE>
+__device__ __forceinline__ void load_group_x(u32x4 (&xq)[SHARE][4], const float* x, uint32_t nb,
+                                             uint32_t blk0, uint32_t nbl, uint32_t ng,
+                                             uint32_t ntok, uint32_t wave, uint32_t lane) {
+  const __amdgpu_buffer_rsrc_t xr = __builtin_amdgcn_make_buffer_rsrc(
+      const_cast<float*>(x), 0, (int)(ntok * nb * 1024u), kBufferWord3);
+#pragma unroll
+  for (int i = 0; i < SHARE; ++i) {
+    const uint32_t q = wave + (uint32_t)i * WAVES, g = q >> 2, b = q & 3u;
+    if (g < ng && b < nbl) {
+      const uint32_t off = ((4u * g + (lane >> 4)) * nb + blk0 + b) * 1024u + 64u * (lane & 15u);
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        xq[i][j] = __builtin_bit_cast(
+            u32x4, __builtin_amdgcn_raw_buffer_load_b128(xr, off + 16u * j, 0, 0));
+    }
+  }
 }
 
-// Inclusive sum over a DPP row's 16 lanes (valid in lane 15).
+// Sum over a DPP row's 16 lanes (valid in lane 15).
 __device__ __forceinline__ uint32_t row_sum_u(uint32_t v) {
   v += dpp_u<kRowShr1>(v);
   v += dpp_u<kRowShr2>(v);
   v += dpp_u<kRowShr4>(v);
   return v + dpp_u<kRowShr8>(v);
 }
-__device__ __forceinline__ float row_sum_f(float v) {
-  v += dpp<kRowShr1>(v);
-  v += dpp<kRowShr2>(v);
-  v += dpp<kRowShr4>(v);
-  return v + dpp<kRowShr8>(v);
-}
 
-// Turns the group-blocks copied by copy_x_group into images in place, with
-// what else the layout keeps of them; a wave converts exactly the group-blocks
-// it copied, lane (t, c) elements 16 c .. 16 c + 15 of vector 4 g + t.  Blocks
-// with side elements are rounded blocks (mfma_common.h), and a block with an
-// activation that is not finite or reaches 2^100 gets the exponent kBadTok.
-template <int WAVES, bool MINS, bool DSUM, typename ChunkSlot>
+// Turns the wave's share of activations (load_group_x) into images, with what
+// else the layout keeps of them: the fixed point of mfma_common.h.  Every
+// workgroup of a slice does this for itself, so it is written for few
+// instructions (about 270 a group-block; with the error sums and unit sums of
+// the one-vector kernels' build 540, a quarter of a sixteen-vector launch):
+// one pass over the shifted bits finds the block's largest |x| and whether
+// an element is not finite, the sums come from the digit bytes (v_dot4), and
+// a side element (0 < |x| < 2^(e - kSideShift)) is only counted, for the bound
+// of half a unit 2^(e - 30) each on its rounding.
+template <int WAVES, int SHARE, bool MINS, bool DSUM, typename ChunkSlot>
 __device__ __forceinline__ void build_group_images64(uint32_t sbase, const TokLayout& L,
-                                                     uint32_t nbl, uint32_t ng, uint32_t wave,
-                                                     uint32_t lane, ChunkSlot chunk_slot) {
+                                                     const u32x4 (&xr)[SHARE][4], uint32_t nbl,
+                                                     uint32_t ng, uint32_t wave, uint32_t lane,
+                                                     ChunkSlot chunk_slot) {
   const uint32_t t = lane >> 4, c = lane & 15u;
   const uint32_t woff = chunk_slot(c) + 64u * t;
-  for_group_blocks<WAVES>(ng, nbl, wave, [&](uint32_t g, uint32_t b) {
-    const uint32_t gb = g * nbl + b;
+#pragma unroll
+  for (int i = 0; i < SHARE; ++i) {
+    const uint32_t q = wave + (uint32_t)i * WAVES, g = q >> 2, b = q & 3u;
+    if (g >= ng || b >= nbl) continue;
+    const uint32_t gb = L.stride * g + b;
     const uint32_t blk = sbase + L.img + 4096u * gb;
-    const uint32_t vec = L.vec_stride * (4u * g + t) + 4u * b;
-    u32x4 xq[4];
-    lds_read4<16>(blk + 1024u * t + 64u * c, xq);
-    float xv[16];
+    const uint32_t vec = 4u * L.stride * (4u * g + t) + 4u * b;
+    auto bits = [&](int k) { return xr[i][k >> 2][k & 3]; };
+    uint32_t top = 0u;  // 2 |bits| of the largest |x|, of the chunk, then of the block
 #pragma unroll
-    for (int k = 0; k < 4; ++k)
-#pragma unroll
-      for (int i = 0; i < 4; ++i) xv[4 * k + i] = __uint_as_float(xq[k][i]);
-    const ChunkSplit cs = split_chunk(xv);
-    const uint64_t bad_any = __builtin_amdgcn_ballot_w64(cs.bad);
-    const uint64_t side_any = __builtin_amdgcn_ballot_w64(cs.smask != 0u);
-    const bool bad = ((bad_any >> (16u * t)) & 0xffffull) != 0u;
-    uint32_t uq[16];
-    biased_values(cs, false, uq);
+    for (int k = 0; k < 16; ++k) top = max(top, bits(k) << 1);
+    top = max(top, dpp_u<kRowShr1>(top));
+    top = max(top, dpp_u<kRowShr2>(top));
+    top = max(top, dpp_u<kRowShr4>(top));
+    top = max(top, dpp_u<kRowShr8>(top));
+    top = dpp_u<kRowBcast15>(top);
+    const bool bad = top >= 2u * 0x71800000u;  // 2^100 and above, infinities, NaN
+    const int e = __builtin_amdgcn_frexp_expf(__uint_as_float(top >> 1));
+    const uint32_t side = 2u * __float_as_uint(__builtin_amdgcn_ldexpf(1.0f, e - kSideShift)) - 2u;
+    uint32_t nside = 0u;
     uint32_t dg[4][4];
 #pragma unroll
-    for (int k = 0; k < 4; ++k)
-      transpose_digits(uq[4 * k], uq[4 * k + 1], uq[4 * k + 2], uq[4 * k + 3], dg[k]);
-    // the wave has read the whole block (lds_read4 waits) before any write
+    for (int k = 0; k < 4; ++k) {
+      uint32_t u[4];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const uint32_t v = bits(4 * k + j);
+        nside += (uint32_t)((v << 1) - 2u < side);
+        u[j] = (uint32_t)__float2int_rn(
+                   __builtin_amdgcn_ldexpf(__uint_as_float(v), kFixBits - e)) +
+               0x80808080u;
+      }
+      transpose_digits(u[0], u[1], u[2], u[3], dg[k]);
+    }
 #pragma unroll
     for (int d = 0; d < 4; ++d)
       lds_write_b128(blk + woff + 16u * d, u32x4{dg[0][d], dg[1][d], dg[2][d], dg[3][d]});
+    int sum[4];  // the chunk's digit sums, |.| <= 2^11
+#pragma unroll
+    for (int d = 0; d < 4; ++d) {
+      sum[d] = 0;
+      if constexpr (MINS || DSUM) {
+#pragma unroll
+        for (int k = 0; k < 4; ++k)
+          sum[d] = __builtin_amdgcn_sdot4((int)dg[k][d], 0x01010101, sum[d], false);
+      }
+    }
     if constexpr (MINS) {
-      // unit u = c / 2's sum (odd lanes hold both halves): |X_u| <= 2^35
-      uint32_t hi = 0u, lo = 0u;
-#pragma unroll
-      for (int k = 0; k < 16; ++k) {
-        const int32_t X = (int32_t)(uq[k] - 0x80808080u);
-        hi += (uint32_t)(X >> 15);
-        lo += (uint32_t)X & 0x7fffu;
+      // unit c / 2 (its two chunks meet in the odd lane): X_u = hi 2^16 + lo
+      // in 12-bit signed pieces, the last what is left (|X_u| <= 2^35, so at
+      // most 2^11, exact as a half)
+      int lo = sum[0] + 256 * sum[1], hi = sum[2] + 256 * sum[3];
+      lo += (int)dpp_u<kRowShr1>((uint32_t)lo);
+      hi += (int)dpp_u<kRowShr1>((uint32_t)hi);
+      const int p0 = (lo << 20) >> 20;
+      const int rest = 16 * hi + ((lo - p0) >> 12);
+      const int p1 = (rest << 20) >> 20;
+      const int p2 = (rest - p1) >> 12;
+      auto half = [](int p) {
+        return (uint32_t)__builtin_bit_cast(uint16_t, (_Float16)(float)p);
+      };
+      if (c & 1u) {
+        const uint32_t at = sbase + L.usum + 256u * gb + 64u * (c >> 2) + 16u * t + (c & 2u);
+        lds_write_b16(at, half(p0));
+        lds_write_b16(at + 4u, half(p1));
+        lds_write_b16(at + 8u, half(p2));
+        lds_write_b16(at + 12u, 0u);
       }
-      hi += dpp_u<kRowShr1>(hi);
-      lo += dpp_u<kRowShr1>(lo);
-      int64_t v = (int64_t)(int32_t)hi * 32768 + (int64_t)lo;
-      const uint32_t at = sbase + L.usum + 256u * gb + 64u * (c >> 2) + 16u * t + (c & 2u);
-#pragma unroll
-      for (int p = 0; p < 3; ++p) {
-        // the low 12 bits, signed; the last piece is what is left (|.| <= 2048)
-        const int piece = p < 2 ? ((int)((uint32_t)v << 20) >> 20) : (int)v;
-        v = (v - piece) >> 12;
-        const _Float16 h = (_Float16)(float)piece;
-        if (c & 1u) lds_write_b16(at + 4u * p, __builtin_bit_cast(uint16_t, h));
-      }
-      if (c & 1u) lds_write_b16(at + 12u, 0u);
     }
     if constexpr (DSUM) {
       uint32_t s[4];
 #pragma unroll
-      for (int d = 0; d < 4; ++d) {
-        int sum = 0;
-#pragma unroll
-        for (int k = 0; k < 4; ++k)
-          sum = __builtin_amdgcn_sdot4((int)dg[k][d], 0x01010101, sum, false);
-        s[d] = 128u * row_sum_u((uint32_t)sum);
-      }
+      for (int d = 0; d < 4; ++d) s[d] = 128u * row_sum_u((uint32_t)sum[d]);
       if (c == 15u)
         lds_write_b128(sbase + L.dsum + 64u * gb + 16u * t, u32x4{s[0], s[1], s[2], s[3]});
     }
-    float err = 0.0f;
-    if ((bad_any | side_any) != 0u) {
-      err = row_sum_f(cs.err_side);
-      if (lane == 0u) lds_write_b32(sbase + L.special, 1u);
-    }
+    nside = row_sum_u(nside);
     if (c == 15u) {
-      lds_write_b32(sbase + L.expo + vec, (uint32_t)(bad ? kBadTok : cs.e - kFixBits));
-      lds_write_b32(sbase + L.rerr + vec, bad ? 0u : __float_as_uint(err));
+      lds_write_b32(sbase + L.expo + vec, (uint32_t)(bad ? kBadTok : e - kFixBits));
+      lds_write_b32(sbase + L.rerr + vec,
+                    bad ? 0x7f800000u
+                        : __float_as_uint(__builtin_amdgcn_ldexpf((float)nside, e - kFixBits - 1)));
     }
-  });
+  }
+}
+
+// A vector's bound on the rounding of its side elements over the nbl blocks
+// of the slice (infinite when a block takes the exact path).
+__device__ __forceinline__ float slice_err(const uint8_t* rerr, uint32_t nbl) {
+  const u32x4 v = lds_u32x4(rerr);
+  float e = __uint_as_float(v[0]);
+#pragma unroll
+  for (uint32_t b = 1; b < 4u; ++b)
+    if (b < nbl) e += __uint_as_float(v[b]);
+  return e;
 }
 
 // Sum of all 16 chunk error sums of a rounded block's side area.
