@@ -45,9 +45,17 @@
 //
 // Weights go straight to registers: a block's pieces are loaded for the
 // wave's next tile as soon as the block is decoded, so a tile's worth of loads
-// is in flight through the arithmetic.  (Staged in LDS by buffer->LDS copies,
-// a wave's next copy went out after its arithmetic, and the waves of a SIMD
-// ended up waiting together.)
+// is in flight through the arithmetic, and the LDS holds images only.  (Staged
+// in LDS by buffer->LDS copies that went out after a stage's arithmetic:
+// 17408 x 5120 M = 4 / 16 19.2 / 33.4 us against 17.8 / 28.2, part of it the
+// shorter image build.  Reading each group's images one group ahead changed
+// nothing: 18.1 / 29.2.)
+//
+// Measured, 17408 x 5120 Q4_K M = 4 / 8 / 16 with the reduce (4.1-4.7 us of
+// it): 27.9 / 44.4 / 72.9 -> 17.8 / 21.2 / 28.2 us.  At M = 4 the launch is
+// bound by the weight stream behind its start (5 us until the first tile is in
+// and the images are built); at M = 16 VALU (about 180 instructions a tile and
+// block) and MFMA (36 of 16 cycles) add up to 13 of the kernel's 24 us.
 #include "mfma_common.h"
 #include "si_hip_tuned.h"
 #include "tokens_common.h"
@@ -320,9 +328,12 @@ bool launch_tok45(const uint8_t* w, const float* x, float* y, uint32_t rows, uin
 template <int QB>
 bool launch_tok45_any(const uint8_t* w, const float* x, float* y, uint32_t rows, uint32_t nb,
                       uint32_t ntok, const Workspace& ws, hipStream_t s, hipError_t* err) {
-  if (ntok <= 4u) return launch_tok45<12, 1, QB>(w, x, y, rows, nb, ntok, ws, s, err);
-  if (ntok <= 8u)
-    return launch_tok45<QB == 5 ? 10 : 12, 2, QB>(w, x, y, rows, nb, ntok, ws, s, err);
+  // Waves, measured (17408 x 5120, us, 12 / 8 waves): Q4_K M = 4 17.8 / 18.5,
+  // M = 8 21.2 / 21.3, M = 16 29.6 (spills) / 28.2; Q5_K, whose blocks take
+  // more registers, M = 4 21.7 / 21.0, M = 8 26.9 / 25.1.
+  constexpr int kWaves = QB == 5 ? 8 : 12;
+  if (ntok <= 4u) return launch_tok45<kWaves, 1, QB>(w, x, y, rows, nb, ntok, ws, s, err);
+  if (ntok <= 8u) return launch_tok45<kWaves, 2, QB>(w, x, y, rows, nb, ntok, ws, s, err);
   if (ntok <= 12u)
     return launch_tok45<QB == 5 ? 8 : 10, 3, QB>(w, x, y, rows, nb, ntok, ws, s, err);
   return launch_tok45<8, 4, QB>(w, x, y, rows, nb, ntok, ws, s, err);
