@@ -265,8 +265,7 @@ __global__ __launch_bounds__(WAVES * 64) void q45_tokens_mfma(const uint8_t* __r
         const double m = fma(fma((double)cm[2], 4096.0, (double)cm[1]), 4096.0, (double)cm[0]);
         t *= bd;
         const double p = fma(-bdmin, m, t);
-        // (not below 2^-30 of the first term, and no NaN)
-        redo[G] |= !(fma(fabs(p), 0x1p30, -fabs(t)) >= 0.0);
+        redo[G] |= cancels(p, t);
         const double v = __builtin_amdgcn_ldexp(p, e);  // 0 for kBadTok
         acc[G] += v;
         sum_abs[G] += fabs(v);

@@ -20,15 +20,14 @@
 //    lanes that hold that unit's scale and min.
 //
 // Per block and lane: C_e, C_o (4 digits each) from four MFMAs; T_d = sc_e *
-// C_e[d] + sc_o * C_o[d] in integers (|T_d| < 2^23, exact in f32); y +=
-// (d * (sum_d T_d * 256^d) - dmin * (m_e * X_e + m_o * X_o)) * 2^(e_b-30),
-// X_u the sum of unit u's fixed-point activations (exact, rounded once), so
-// both terms see the same rounded activations and, in exact arithmetic, the
-// pair is sum_i w_i X_i 2^(e_b-30) with w_i the weight of quant.rs.  Their
-// f32 rounding is bounded by 2^-21 (|d T| + |dmin| (m_e |X_e| + m_o |X_o|))
-// per block, which can exceed the bar where w_i cancels inside its own decode
-// (d sc q close to dmin m); every stage of a row checks that bound (stage_ok)
-// and a row that fails recomputes the stage on the exact per-weight path, so
+// C_e[d] + sc_o * C_o[d] in integers; y += (d * (sum_d T_d * 256^d) - dmin *
+// (m_e * X_e + m_o * X_o)) * 2^(e_b-30), X_u the exact sum of unit u's
+// fixed-point activations, so both terms see the same rounded activations
+// and the pair is sum_i w_i X_i 2^(e_b-30) with w_i the weight of quant.rs.
+// Both sums are exact integers below 2^53 and the terms are formed in f64
+// (block_dot), so their rounding shows only where every w_i of a lane's share
+// cancels inside its own decode (d sc q = dmin m); a lane that sees that
+// (cancels) recomputes its share of the stage on the exact per-weight path, so
 // the dot stays within 2e-5 * sum|w*x| on every input.  Blocks whose
 // activations are not finite or reach 2^100 take the exact per-weight f32
 // path instead, so NaN/Inf propagate as in the reference.
@@ -96,12 +95,12 @@ constexpr uint32_t kLineCopies = 10u;
 constexpr uint32_t kLineStage = 1024u * kLineCopies;  // 16 rows x 5 lines
 constexpr int kNontemporal = 2;                       // buffer cache policy: NT
 
-// LDS map (make_layout): SB-block stages, 32 bytes of unit sums per block.
+// LDS map (make_layout): SB-block stages, 64 bytes of unit sums per block.
 __host__ __device__ constexpr Layout layout(uint32_t waves, uint32_t depth, uint32_t nb,
-                                            uint32_t slots, uint32_t mats, uint32_t ntok = 1u,
-                                            int qb = 4, int sb = 4, bool lines = false) {
-  return make_layout(lines ? kLineStage : stage_bytes(qb, sb), (uint32_t)sb, 32u, waves, depth,
-                     nb, slots, mats, ntok);
+                                            uint32_t slots, uint32_t mats, int qb = 4, int sb = 4,
+                                            bool lines = false) {
+  return make_layout(lines ? kLineStage : stage_bytes(qb, sb), (uint32_t)sb, 64u, waves, depth,
+                     nb, slots, mats);
 }
 
 // The lane's header and two qs pieces of the four blocks of a full-line stage
@@ -167,17 +166,18 @@ __device__ __forceinline__ void lds_read_weights2(uint32_t hb, uint32_t qb, u32x
       : "memory");
 }
 
-// Unit sums of the lane's two units in the four blocks (xb + 32 b), the
+typedef double f64x2 __attribute__((ext_vector_type(2)));
+// Unit sums of the lane's two units in the four blocks (xb + 64 b), the
 // four block exponents (eb) and their four side counts (one byte each, at
 // eb + kCountOff).
-__device__ __forceinline__ void lds_read_sums(uint32_t xb, uint32_t eb, u32x2 (&xs)[4], i32x4& ex,
+__device__ __forceinline__ void lds_read_sums(uint32_t xb, uint32_t eb, f64x2 (&xs)[4], i32x4& ex,
                                               uint32_t& cnt) {
   static_assert(kCountOff == 512, "the offset below");
   asm volatile(
-      "ds_read_b64 %0, %6\n"
-      "ds_read_b64 %1, %6 offset:32\n"
-      "ds_read_b64 %2, %6 offset:64\n"
-      "ds_read_b64 %3, %6 offset:96\n"
+      "ds_read_b128 %0, %6\n"
+      "ds_read_b128 %1, %6 offset:64\n"
+      "ds_read_b128 %2, %6 offset:128\n"
+      "ds_read_b128 %3, %6 offset:192\n"
       "ds_read_b128 %4, %7\n"
       "ds_read_b32 %5, %7 offset:512\n"
       "s_waitcnt lgkmcnt(0)"
@@ -187,13 +187,13 @@ __device__ __forceinline__ void lds_read_sums(uint32_t xb, uint32_t eb, u32x2 (&
 }
 // The same for the two blocks of a two-block stage (exponents in ex[0..1],
 // the two side counts in the low 16 bits of cnt).
-__device__ __forceinline__ void lds_read_sums2(uint32_t xb, uint32_t eb, u32x2 (&xs)[2], i32x4& ex,
+__device__ __forceinline__ void lds_read_sums2(uint32_t xb, uint32_t eb, f64x2 (&xs)[2], i32x4& ex,
                                                uint32_t& cnt) {
   static_assert(kCountOff == 512, "the offset below");
   u32x2 e2;
   asm volatile(
-      "ds_read_b64 %0, %4\n"
-      "ds_read_b64 %1, %4 offset:32\n"
+      "ds_read_b128 %0, %4\n"
+      "ds_read_b128 %1, %4 offset:64\n"
       "ds_read_b64 %2, %5\n"
       "ds_read_u16 %3, %5 offset:512\n"
       "s_waitcnt lgkmcnt(0)"
@@ -291,16 +291,20 @@ __device__ __forceinline__ BlockQ4 decode_q4(const u32x4& h, const u32x4& qa, co
   return w;
 }
 
-// Fast-path dot of one decoded block with one activation vector's images
-// (xs: the fixed-point sums of the lane's two units); `err` gets the bound on
-// its f32 rounding.  tc below is the exact integer sum_d T_d 256^d to within
-// 5 * 2^-24 |tc| (a step of the fma chain rounds only when what is left of tc
-// is far larger than the terms still to come), um = m_e X_e + m_o X_o to
-// within 3 * 2^-24 (m_e |X_e| + m_o |X_o|), and the last fma rounds once:
-// 2^-21 of the two terms' magnitudes covers all of it.
-__device__ __forceinline__ float block_dot(const BlockQ4& w, const i32x4& a0, const i32x4& a1,
-                                           const i32x4& a2, const i32x4& a3, u32x2 xs, int eb,
-                                           float& err) {
+// Fast-path dot of one decoded block with the activations' images (xs: the
+// exact fixed-point sums of the lane's two units), in f64 from exact integers:
+// the digit sums T_d = sc_e C_e[d] + sc_o C_o[d] (|T_d| < 2^24), their total
+// sum_d 256^d T_d (< 2^50) and the mins' sum; only the two products with d and
+// dmin round, at 2^-53.  `redo` when the terms cancel so far that this could
+// show.  (In f32 the rounding was bounded by 2^-21 of the terms; weights
+// quantised from zero-mean data have d sc q and dmin m of one size, and one
+// row-stage in some thousand failed its check, a wave's whole stage then
+// waiting for the per-weight path.  On such weights, us: 17408 x 5120 12.2 ->
+// 11.5, 1024 x 5120 7.8 -> 6.3, the 6144 + 1024 + 1024 group 11.6 -> 8.7.)
+template <int QB>
+__device__ __forceinline__ double block_dot(const BlockQ4& w, const i32x4& a0, const i32x4& a1,
+                                            const i32x4& a2, const i32x4& a3, const f64x2& xs,
+                                            int eb, bool& redo) {
   const i32x4 zero = {0, 0, 0, 0};
   i32x4 ce = __builtin_amdgcn_mfma_i32_16x16x64_i8(a0, w.la, zero, 0, 0, 0);
   i32x4 co = __builtin_amdgcn_mfma_i32_16x16x64_i8(a2, w.ha, zero, 0, 0, 0);
@@ -310,14 +314,20 @@ __device__ __forceinline__ float block_dot(const BlockQ4& w, const i32x4& a0, co
   const int t1 = __mul24(w.sce, ce[1]) + __mul24(w.sco, co[1]);
   const int t2 = __mul24(w.sce, ce[2]) + __mul24(w.sco, co[2]);
   const int t3 = __mul24(w.sce, ce[3]) + __mul24(w.sco, co[3]);
-  const float tc =
-      fmaf(fmaf(fmaf((float)t3, 256.0f, (float)t2), 256.0f, (float)t1), 256.0f, (float)t0);
-  const float sxe = __uint_as_float(xs[0]), sxo = __uint_as_float(xs[1]);
-  const float dt = w.d * tc;
-  const float um = fmaf(w.mne, sxe, w.mno * sxo);
-  const float ua = fmaf(w.mne, fabsf(sxe), w.mno * fabsf(sxo));
-  err = __builtin_amdgcn_ldexpf(fmaf(fabsf(w.dmin), ua, fabsf(dt)), eb - 21);
-  return __builtin_amdgcn_ldexpf(fmaf(-w.dmin, um, dt), eb);
+  // |X| <= 2^30, so |D_3| <= 64: 256 T_3 + T_2 fits 32 bits for both formats
+  // (Q5_K: 31 63 64 64 256 + 2^24 < 2^31), 256 T_1 + T_0 for Q4_K
+  // (15 63 64 128 257 < 2^31)
+  const double hi = (double)(256 * t3 + t2);
+  double tc;
+  if constexpr (QB == 4)
+    tc = fma(hi, 65536.0, (double)(256 * t1 + t0));
+  else
+    tc = fma(hi, 65536.0, fma((double)t1, 256.0, (double)t0));
+  const double um = fma((double)w.mne, xs[0], (double)w.mno * xs[1]);
+  const double dt = (double)w.d * tc;
+  const double p = fma(-(double)w.dmin, um, dt);
+  redo |= cancels(p, dt);
+  return __builtin_amdgcn_ldexp(p, eb);
 }
 
 // Exact per-weight path of one block (activations not finite or >= 2^100).
@@ -453,18 +463,6 @@ __device__ __forceinline__ float block_exact5(const BlockQ4& w, const u32x4& h, 
   return exact_dot16_bytes(w.hb, d1o, m1o, xs + 48, acc);
 }
 
-// Exact per-weight path of one decoded block (the order of block_exact):
-// units 2 grp (la: elements 0..15, lb: 16..31 of the lane's 64) and
-// 2 grp + 1 (ha, hb), quant.rs rounding.
-__device__ __forceinline__ float block_exact_dec(const BlockQ4& w, const float* __restrict__ xs) {
-  const float d1e = __fmul_rn(w.d, (float)w.sce), m1e = __fmul_rn(w.dmin, w.mne);
-  const float d1o = __fmul_rn(w.d, (float)w.sco), m1o = __fmul_rn(w.dmin, w.mno);
-  float acc = exact_dot16_bytes(w.la, d1e, m1e, xs, 0.0f);
-  acc = exact_dot16_bytes(w.lb, d1e, m1e, xs + 16, acc);
-  acc = exact_dot16_bytes(w.ha, d1o, m1o, xs + 32, acc);
-  return exact_dot16_bytes(w.hb, d1o, m1o, xs + 48, acc);
-}
-
 // The weights of a stage of SB blocks in registers, per format: Q4_K keeps
 // (header, qs piece a, qs piece b) per block, Q5_K adds the two qh pieces.
 template <int QB, int SB = 4>
@@ -527,15 +525,16 @@ __device__ __forceinline__ float stage_rowsum(const StageRegs<QB, SB>& v, uint32
                                               uint32_t rot_lo, uint32_t rot_hi,
                                               const float* __restrict__ x) {
   static_assert(SB == 4 || SB == 2, "four- or two-block stages");
-  u32x2 xs[SB];
+  f64x2 xs[SB];
   i32x4 ex;
   uint32_t cnt;
   if constexpr (SB == 4)
-    lds_read_sums(sbase + L.xsum + 128u * ls + 8u * grp, sbase + L.expo + 16u * ls, xs, ex, cnt);
+    lds_read_sums(sbase + L.xsum + 256u * ls + 16u * grp, sbase + L.expo + 16u * ls, xs, ex, cnt);
   else
-    lds_read_sums2(sbase + L.xsum + 64u * ls + 8u * grp, sbase + L.expo + 8u * ls, xs, ex, cnt);
+    lds_read_sums2(sbase + L.xsum + 128u * ls + 16u * grp, sbase + L.expo + 8u * ls, xs, ex, cnt);
   float part[SB];
-  float err = 0.0f;  // bound on the error of the fast-path partials
+  double acc = 0.0;
+  bool redo = false;  // the lane's share takes the per-weight path
   bool bad_any = false;
 #pragma unroll
   for (int h = 0; h < SB / 2; ++h) {
@@ -544,44 +543,48 @@ __device__ __forceinline__ float stage_rowsum(const StageRegs<QB, SB>& v, uint32
     for (int b2 = 0; b2 < 2; ++b2) {
       const int b = 2 * h + b2;
       const int eb = __builtin_amdgcn_readfirstlane(ex[b]);
-      const bool use = (uint32_t)b < nlive;
+      const bool use = (uint32_t)b < nlive, fast = use && eb != kBadBlock;
       bad_any |= use && eb == kBadBlock;
-      float e;
-      const float c = block_dot(v.decode(b, hi_units, bsh, rot_lo, rot_hi), A[4 * b2],
-                                A[4 * b2 + 1], A[4 * b2 + 2], A[4 * b2 + 3], xs[b], eb, e);
-      const bool fast = use && eb != kBadBlock;
-      part[b] = fast ? c : 0.0f;
-      err += fast ? e : 0.0f;
+      bool r = false;
+      const double c =
+          block_dot<QB>(v.decode(b, hi_units, bsh, rot_lo, rot_hi), A[4 * b2], A[4 * b2 + 1],
+                        A[4 * b2 + 2], A[4 * b2 + 3], xs[b], eb, r);
+      redo |= fast && r;
+      acc += fast ? c : 0.0;
+      part[b] = fast ? (float)c : 0.0f;
     }
   }
-  // the stage check (the factored form's rounding plus the rounded blocks'
-  // bound); blocks on the exact path, and every live block of a row that
-  // fails the check, take the per-weight path
+  redo |= !(fabs(acc) < __builtin_huge_val());
+  // the rounded blocks' check; blocks on the exact path, and every live block
+  // of a lane that fails a check, take the per-weight path
   const uint32_t counts = live_counts(__builtin_amdgcn_readfirstlane(cnt), nlive);
   const uint32_t rmask = rounded_mask(counts);
   if (rmask != 0u) {
     const uint32_t list = sbase + L.expo + L.side_off + (uint32_t)SB * kSideBytes * ls;
-    err += rounded_bound<SB>(list, rmask, grp, [&](auto b) {
+    const float err = rounded_bound<SB>(list, rmask, grp, [&](auto b) {
       return k4_bound<QB == 5 ? 31 : 15>(
           v.decode(decltype(b)::value, hi_units, bsh, rot_lo, rot_hi));
     });
-  }
-  float apart = 0.0f;
+    float apart = 0.0f;
 #pragma unroll
-  for (int b = 0; b < SB; ++b) apart += fabsf(part[b]);
-  const uint32_t redo = stage_ok(err, apart) ? 0u : (1u << nlive) - 1u;
-  if (bad_any || redo != 0u) {
-#pragma unroll
-    for (int b = 0; b < SB; ++b)
-      if (((uint32_t)b < nlive && __builtin_amdgcn_readfirstlane(ex[b]) == kBadBlock) ||
-          ((redo >> b) & 1u))
-        part[b] = v.exact(b, hi_units, bsh, rot_lo, rot_hi,
-                          x + 256u * ((uint32_t)SB * s + b) + 64u * grp);
+    for (int b = 0; b < SB; ++b) apart += fabsf(part[b]);
+    redo |= !stage_ok(err, apart);
   }
-  if constexpr (SB == 4)
-    return sum_lane_groups((part[0] + part[1]) + (part[2] + part[3]));
-  else
-    return sum_lane_groups(part[0] + part[1]);
+  float sum = (float)acc;
+  if (bad_any || __builtin_amdgcn_ballot_w64(redo) != 0u) {
+    if (bad_any || redo) {
+      sum = 0.0f;
+#pragma unroll
+      for (int b = 0; b < SB; ++b) {
+        if ((uint32_t)b < nlive &&
+            (redo || __builtin_amdgcn_readfirstlane(ex[b]) == kBadBlock))
+          part[b] = v.exact(b, hi_units, bsh, rot_lo, rot_hi,
+                            x + 256u * ((uint32_t)SB * s + b) + 64u * grp);
+        sum += part[b];
+      }
+    }
+  }
+  return sum_lane_groups(sum);
 }
 
 // GROUPED: the rows are those of the group's matrices with one K, one after the
@@ -595,7 +598,7 @@ __device__ __forceinline__ float stage_rowsum(const StageRegs<QB, SB>& v, uint32
 // workgroups have few pairs per wave (finer pairs, a shorter last one).
 // LINES (Q4_K, one vector, four-block stages of whole rows, nb a multiple of
 // 4, every matrix 128-byte aligned): full-line copies (kLineCopies above).
-template <int WAVES, int DEPTH, int MATS, int NTOK, int QB, bool GROUPED, bool SLICED = false,
+template <int WAVES, int DEPTH, int MATS, int QB, bool GROUPED, bool SLICED = false,
           int SB = 4, bool LINES = false>
 __global__ __launch_bounds__(WAVES * 64) void q4k_matvec_mfma(const uint8_t* __restrict__ w,
                                                               const uint8_t* __restrict__ w2,
@@ -605,12 +608,11 @@ __global__ __launch_bounds__(WAVES * 64) void q4k_matvec_mfma(const uint8_t* __r
                                                               SchedArgs sa, GroupArgs ga,
                                                               SliceArgs sla) {
   extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
-  static_assert(NTOK == 1 || MATS == 1, "several activation vectors: one matrix");
   static_assert(QB == 4 || QB == 5, "Q4_K or Q5_K");
-  static_assert(!SLICED || (MATS == 1 && NTOK == 1 && !GROUPED), "slices of one matrix and vector");
-  static_assert(SB == 4 || (SB == 2 && MATS == 1 && NTOK == 1), "two-block stages: one vector");
-  static_assert(!LINES || (QB == 4 && SB == 4 && NTOK == 1 && !SLICED && DEPTH <= 2),
-                "full-line stages: Q4_K, four blocks, one vector, whole rows");
+  static_assert(!SLICED || (MATS == 1 && !GROUPED), "slices of one matrix");
+  static_assert(SB == 4 || (SB == 2 && MATS == 1), "two-block stages: one matrix");
+  static_assert(!LINES || (QB == 4 && SB == 4 && !SLICED && DEPTH <= 2),
+                "full-line stages: Q4_K, four blocks, whole rows");
   if constexpr (GROUPED) load_group_args_early(ga);
   const uint32_t slots = sa.packed & 0xffu;
   // copy instructions per stage
@@ -631,7 +633,7 @@ __global__ __launch_bounds__(WAVES * 64) void q4k_matvec_mfma(const uint8_t* __r
   const uint32_t st0 = SLICED ? ss.r_lo : 0u;
   const uint32_t nbl = SLICED ? min(SB * ss.ns, nb - SB * st0) : nb;
   const Layout L =
-      layout(WAVES, DEPTH, SLICED ? SB * ss.pstride : nb, slots, MATS, NTOK, QB, SB, LINES);
+      layout(WAVES, DEPTH, SLICED ? SB * ss.pstride : nb, slots, MATS, QB, SB, LINES);
   const SplitWs ws = split_ws(wsp);
   const uint32_t wave = uniform(threadIdx.x >> 6);
   const uint32_t lane = threadIdx.x & 63u;
@@ -640,13 +642,8 @@ __global__ __launch_bounds__(WAVES * 64) void q4k_matvec_mfma(const uint8_t* __r
   const uint32_t sbase = (uint32_t)(uintptr_t)smem;
   uint8_t* const wstage = smem + wave * DEPTH * kStage;
 
-  // 1. x into the image area, natural order (block b at img + 1024 b; vector
-  //    t of NTOK at img + t img_stride)
-#pragma unroll
-  for (int t = 0; t < NTOK; ++t)
-    copy_x<WAVES>(smem, L.img + t * L.img_stride,
-                  x + (size_t)t * nb * kBlockElems + (size_t)SB * st0 * kBlockElems, nbl, wave,
-                  lane);
+  // 1. x into the image area, natural order (block b at img + 1024 b)
+  copy_x<WAVES>(smem, L.img, x + (size_t)SB * st0 * kBlockElems, nbl, wave, lane);
 
   // 2. this wave's pairs k = wave, wave + WAVES, ... of the workgroup's pairs
   //    (pair_at: a tile and its partial r, r being stage r % nstages of
@@ -766,10 +763,8 @@ __global__ __launch_bounds__(WAVES * 64) void q4k_matvec_mfma(const uint8_t* __r
     else
       __builtin_amdgcn_s_waitcnt(waitcnt_vm(0));
     // chunk c = 4 p + t: units 2p, 2p + 1 of lane group p, MFMA t
-#pragma unroll
-    for (int t = 0; t < NTOK; ++t)
-      build_images<WAVES>(sbase, L, nbl, wave, grp, n,
-                          [](uint32_t c) { return 256u * (c & 3u) + 64u * (c >> 2); }, t);
+    build_images<WAVES>(sbase, L, nbl, wave, grp, n,
+                        [](uint32_t c) { return 256u * (c & 3u) + 64u * (c >> 2); });
     lds_wait();
     if (lane == 0u) (void)lds_add_rtn(sbase + L.ready, 1u);
   }
@@ -843,10 +838,9 @@ __global__ __launch_bounds__(WAVES * 64) void q4k_matvec_mfma(const uint8_t* __r
     } else {
       v.read(hb0 + buf, qb0 + buf);
     }
-    // The buffer just read is free again.  With one vector its next copy
-    // goes out after the stage's arithmetic: while the memory queue is full,
-    // issuing a copy holds the wave, and the stage in registers would wait
-    // for it.
+    // The buffer just read is free again.  Its next copy goes out after the
+    // stage's arithmetic: while the memory queue is full, issuing a copy holds
+    // the wave, and the stage in registers would wait for it.
     auto issue_next = [&]() {
       if (kClaimable && claims) {
         knext = lds_claim(sbase + L.ready + 4u);
@@ -861,70 +855,10 @@ __global__ __launch_bounds__(WAVES * 64) void q4k_matvec_mfma(const uint8_t* __r
         if (DEPTH == 1) pr_next = pn;
       }
     };
-    if (NTOK > 1) issue_next();
     const uint32_t nlive = min((uint32_t)SB, nb - SB * s);
     if (!images) {
       wait_images(sbase, L, builders, fail);
       images = true;
-    }
-    if constexpr (NTOK > 1) {
-      // the stage's weights are decoded once and meet every vector in turn
-      BlockQ4 bw[4];
-#pragma unroll
-      for (int b = 0; b < 4; ++b)
-        bw[b] = v.decode(b, hi_units, bsh, rot_lo, rot_hi);
-      float rs[NTOK];
-#pragma unroll
-      for (int t = 0; t < NTOK; ++t) {
-        u32x2 xs[4];
-        i32x4 ex;
-        uint32_t cnt;
-        lds_read_sums(sbase + L.xsum + t * L.xsum_stride + 128u * s + 8u * grp,
-                      sbase + L.expo + t * L.expo_stride + 16u * s, xs, ex, cnt);
-        float part[4];
-        float err = 0.0f;
-        bool bad_any = false;
-#pragma unroll
-        for (int h = 0; h < 2; ++h) {
-          lds_read_images8(sbase + L.img + t * L.img_stride + 4096u * s + 2048u * h + 16u * n,
-                           kActiveLanes, A);
-#pragma unroll
-          for (int b2 = 0; b2 < 2; ++b2) {
-            const int b = 2 * h + b2;
-            const int eb = __builtin_amdgcn_readfirstlane(ex[b]);
-            const bool use = (uint32_t)b < nlive;
-            bad_any |= use && eb == kBadBlock;
-            float e;
-            const float c = block_dot(bw[b], A[4 * b2], A[4 * b2 + 1], A[4 * b2 + 2],
-                                      A[4 * b2 + 3], xs[b], eb, e);
-            const bool fast = use && eb != kBadBlock;
-            part[b] = fast ? c : 0.0f;
-            err += fast ? e : 0.0f;
-          }
-        }
-        const uint32_t counts = live_counts(__builtin_amdgcn_readfirstlane(cnt), nlive);
-        const uint32_t rmask = rounded_mask(counts);
-        if (rmask != 0u) {
-          const uint32_t list =
-              sbase + L.expo + t * L.expo_stride + L.side_off + 4u * kSideBytes * s;
-          err += rounded_bound<4>(list, rmask, grp, [&](auto b) {
-            return k4_bound<QB == 5 ? 31 : 15>(bw[decltype(b)::value]);
-          });
-        }
-        const float apart = (fabsf(part[0]) + fabsf(part[1])) + (fabsf(part[2]) + fabsf(part[3]));
-        const uint32_t redo = stage_ok(err, apart) ? 0u : (1u << nlive) - 1u;
-        if (bad_any || redo != 0u) {
-#pragma unroll
-          for (int b = 0; b < 4; ++b)
-            if (((uint32_t)b < nlive && __builtin_amdgcn_readfirstlane(ex[b]) == kBadBlock) ||
-                ((redo >> b) & 1u))
-              part[b] = block_exact_dec(
-                  bw[b], x + (size_t)t * nb * kBlockElems + 256u * (4u * s + b) + 64u * grp);
-        }
-        rs[t] = sum_lane_groups((part[0] + part[1]) + (part[2] + part[3]));
-      }
-      hand_off_tokens<NTOK>(sbase, L, sc.by_slots, pr, tstages, rs, lane, rows, y, fail);
-      continue;
     }
     float rowsum = stage_rowsum(v, sbase, L, s - st0, s, nlive, grp, n, A, hi_units, bsh,
                                 rot_lo, rot_hi, x);
@@ -941,28 +875,26 @@ __global__ __launch_bounds__(WAVES * 64) void q4k_matvec_mfma(const uint8_t* __r
   if (fail != 0u) report_device_error(wsp, fail);
 }
 
-template <int W, int D, int M, int NT = 1, int QB = 4, bool G = false, int SB = 4,
-          bool LN = false>
+template <int W, int D, int M, int QB = 4, bool G = false, int SB = 4, bool LN = false>
 bool launch_wd(const uint8_t* w, const uint8_t* w2, const float* x, float* y, uint32_t rows,
                uint32_t nb, const Workspace& ws, hipStream_t s, hipError_t* err,
                const GroupArgs& ga = GroupArgs{}) {
   const uint32_t ntiles = (rows + 15u) / 16u;
   const uint32_t tstages = (nb + SB - 1u) / SB * M;
-  // several vectors: whole tiles only
-  const LaunchShape ls = launch_shape(ntiles, tstages, W, NT == 1 ? ws.bytes : 0u, M);
+  const LaunchShape ls = launch_shape(ntiles, tstages, W, ws.bytes, M);
   const uint32_t grid = ls.groups;
   const uint32_t slots = ring_slots(W, D, ls.tiles_per_group, tstages);
-  const uint32_t lds = layout(W, D, nb, slots, M, NT, QB, SB, LN).total;
+  const uint32_t lds = layout(W, D, nb, slots, M, QB, SB, LN).total;
   SchedArgs sa;
   if (lds > kLdsBytes || !make_sched_args(ntiles, tstages, slots, ls, &sa)) return false;
   static const hipError_t attr = hipFuncSetAttribute(
-      reinterpret_cast<const void*>(&q4k_matvec_mfma<W, D, M, NT, QB, G, false, SB, LN>),
+      reinterpret_cast<const void*>(&q4k_matvec_mfma<W, D, M, QB, G, false, SB, LN>),
       hipFuncAttributeMaxDynamicSharedMemorySize, (int)kLdsBytes);
   if (attr != hipSuccess) {
     *err = attr;
     return true;
   }
-  hipLaunchKernelGGL((q4k_matvec_mfma<W, D, M, NT, QB, G, false, SB, LN>), dim3(grid),
+  hipLaunchKernelGGL((q4k_matvec_mfma<W, D, M, QB, G, false, SB, LN>), dim3(grid),
                      dim3(W * 64), lds, s, w, w2, x, y, rows, nb, ws.ptr, sa, ga, SliceArgs{});
   *err = hipGetLastError();
   return true;
@@ -991,19 +923,19 @@ bool launch_sliced(const uint8_t* w, const float* x, float* y, uint32_t rows, ui
   if (!slice_shape(ntiles, nstages, S, (uint32_t)cu_count(), ws.bytes, &sh)) return false;
   if (SB * sh.ns_max > kMaxMetaBlocks) return false;
   const uint32_t slots = ring_slots(W, D, sh.tiles_per_group, sh.ns_max);
-  const uint32_t lds = layout(W, D, SB * sh.ns_max, slots, 1u, 1u, QB, SB).total;
+  const uint32_t lds = layout(W, D, SB * sh.ns_max, slots, 1u, QB, SB).total;
   if (lds > kLdsBytes || slots > 0xffu || sh.groups > 0xffffu) return false;
   SchedArgs sa{};
   sa.packed = (sh.groups << 16) | slots;
   sa.m_slots = div_magic(slots);
   static const hipError_t attr = hipFuncSetAttribute(
-      reinterpret_cast<const void*>(&q4k_matvec_mfma<W, D, 1, 1, QB, false, true, SB>),
+      reinterpret_cast<const void*>(&q4k_matvec_mfma<W, D, 1, QB, false, true, SB>),
       hipFuncAttributeMaxDynamicSharedMemorySize, (int)kLdsBytes);
   if (attr != hipSuccess) {
     *err = attr;
     return true;
   }
-  hipLaunchKernelGGL((q4k_matvec_mfma<W, D, 1, 1, QB, false, true, SB>), dim3(sh.groups),
+  hipLaunchKernelGGL((q4k_matvec_mfma<W, D, 1, QB, false, true, SB>), dim3(sh.groups),
                      dim3(W * 64), lds, s, w, nullptr, x, y, rows, nb, ws.ptr, sa, GroupArgs{},
                      sh.args);
   *err = hipGetLastError();
@@ -1049,7 +981,7 @@ bool unsliced_fits(uint32_t ntiles, uint32_t nb, uint32_t waves, int qb, int sb,
   const uint32_t tparts = (nb + sb - 1u) / sb;
   const LaunchShape ls = launch_shape(ntiles, tparts, waves, ws_bytes, 1u);
   const uint32_t slots = ring_slots(waves, 1u, ls.tiles_per_group, tparts);
-  return layout(waves, 1u, nb, slots, 1u, 1u, qb, sb).total <= kLdsBytes;
+  return layout(waves, 1u, nb, slots, 1u, qb, sb).total <= kLdsBytes;
 }
 
 struct SliceChoice {
@@ -1091,7 +1023,7 @@ SliceChoice q4_slices(uint32_t ntiles, uint32_t nb, size_t ws_bytes, int qb) {
     return c;
   };
   if (c.most0 <= 24u) return most(4u) < c.most0 || nb >= 64u ? pick(4u) : c;
-  if (layout(8u, 1u, nb, 2u, 1u, 1u, qb).total <= kLdsBytes) return c;
+  if (layout(8u, 1u, nb, 2u, 1u, qb).total <= kLdsBytes) return c;
   for (uint32_t S : {4u, 2u})
     if (most(S) <= c.most0) return pick(S);
   return c;
@@ -1184,7 +1116,7 @@ bool try_sliced(const uint8_t* w, const float* x, float* y, uint32_t rows, uint3
   const uint32_t ntiles = (rows + 15u) / 16u;
   const SliceChoice sc = q4_slices(ntiles, nb, ws.bytes, QB);
   if (shape_ok(rows, cols, 1u, QB, 2u) && two_block_stages(ntiles, nb, ws.bytes, QB, sc) &&
-      launch_wd<12, 1, 1, 1, QB, false, 2>(w, nullptr, x, y, rows, nb, ws, s, err))
+      launch_wd<12, 1, 1, QB, false, 2>(w, nullptr, x, y, rows, nb, ws, s, err))
     return true;
   const uint32_t S = sc.slices;
   if (S < 2u) return false;
@@ -1198,78 +1130,20 @@ bool try_sliced(const uint8_t* w, const float* x, float* y, uint32_t rows, uint3
          launch_sliced<4, 1, QB>(w, x, y, rows, nb, S, ws, s, err);
 }
 
-// NT activation vectors (batch-major x and y) in one pass over the weights.
-template <int NT, int QB>
-bool launch_tokens(const uint8_t* w, const float* x, float* y, uint32_t rows, uint32_t nb,
-                   const Workspace& ws, hipStream_t s, hipError_t* err) {
-  return launch_wd<8, 1, 1, NT, QB>(w, nullptr, x, y, rows, nb, ws, s, err) ||
-         launch_wd<6, 1, 1, NT, QB>(w, nullptr, x, y, rows, nb, ws, s, err) ||
-         launch_wd<4, 1, 1, NT, QB>(w, nullptr, x, y, rows, nb, ws, s, err);
-}
-
-
 // One vector, Q5_K in four-block stages (8 waves: their 20 weight pieces per
 // wave leave too few registers for 12).
 bool launch_q5k_one(const uint8_t* w, const float* x, float* y, uint32_t rows, uint32_t nb,
                     const Workspace& ws, hipStream_t s, hipError_t* err) {
   static const int cfg = env_int("SI_HIP_Q5K_MFMA_CFG", 0);
   switch (cfg) {
-    case 1: return launch_wd<8, 1, 1, 1, 5>(w, nullptr, x, y, rows, nb, ws, s, err);
+    case 1: return launch_wd<8, 1, 1, 5>(w, nullptr, x, y, rows, nb, ws, s, err);
     case 2:
       return shape_ok(rows, nb * kBlockElems, 1u, 5, 2u) &&
-             launch_wd<12, 1, 1, 1, 5, false, 2>(w, nullptr, x, y, rows, nb, ws, s, err);
+             launch_wd<12, 1, 1, 5, false, 2>(w, nullptr, x, y, rows, nb, ws, s, err);
     default: break;
   }
-  return launch_wd<8, 1, 1, 1, 5>(w, nullptr, x, y, rows, nb, ws, s, err) ||
-         launch_wd<4, 1, 1, 1, 5>(w, nullptr, x, y, rows, nb, ws, s, err);
-}
-
-// SI_HIP_TOKENS_TD=0 keeps the one-vector-per-MFMA kernel for batches
-inline bool td_policy() {
-  static const int v = env_int("SI_HIP_TOKENS_TD", 1);
-  return v != 0;
-}
-
-// batch >= 2 vectors: three to sixteen in one pass of the vectors-in-rows
-// kernel, two (or, under SI_HIP_TOKENS_TD=0, up to four) per pass of the
-// one-vector-per-MFMA kernel
-template <int QB>
-bool matmul_passes(const uint8_t* w, const float* x, float* y, uint32_t rows, uint32_t cols,
-                   uint32_t batch, const Workspace& ws, hipStream_t s, hipError_t* err) {
-  const uint32_t nb = cols / kBlockElems;
-  for (uint32_t b = 0; b < batch;) {
-    const uint32_t nt = min(4u, batch - b);
-    const float* xb = x + (size_t)b * cols;
-    float* yb = y + (size_t)b * rows;
-    bool ok;
-    if (nt >= 2 && td_policy()) {
-      // up to sixteen vectors share the matrix-core rows in one pass (two
-      // go faster one vector per MFMA)
-      const uint32_t ng = batch - b >= 3u ? min(16u, batch - b) : nt;
-      if (ng >= 3u && launch_q45_tokens(QB, w, xb, yb, rows, nb, ng, ws, s, err)) {
-        if (*err != hipSuccess) return true;
-        b += ng;
-        continue;
-      }
-    }
-    switch (nt) {
-      case 4: ok = launch_tokens<4, QB>(w, xb, yb, rows, nb, ws, s, err); break;
-      case 3: ok = launch_tokens<3, QB>(w, xb, yb, rows, nb, ws, s, err); break;
-      case 2: ok = launch_tokens<2, QB>(w, xb, yb, rows, nb, ws, s, err); break;
-      default:
-        ok = QB == 5 ? launch_q5k_matvec_mfma(w, xb, yb, rows, cols, ws, s, err)
-                     : launch_q4k_matvec_mfma(w, xb, yb, rows, cols, ws, s, err);
-        break;
-    }
-    if (!ok) {
-      if (b == 0) return false;
-      *err = hipErrorInvalidValue;
-      return true;
-    }
-    if (*err != hipSuccess) return true;
-    b += nt;
-  }
-  return true;
+  return launch_wd<8, 1, 1, 5>(w, nullptr, x, y, rows, nb, ws, s, err) ||
+         launch_wd<4, 1, 1, 5>(w, nullptr, x, y, rows, nb, ws, s, err);
 }
 
 }  // namespace
@@ -1283,20 +1157,20 @@ bool launch_q4k_matvec_mfma(const uint8_t* w, const float* x, float* y, uint32_t
   switch (cfg) {
     case 5:
       return shape_ok(rows, cols, 1u, 4, 2u) &&
-             launch_wd<12, 1, 1, 1, 4, false, 2>(w, nullptr, x, y, rows, nb, ws, s, err);
+             launch_wd<12, 1, 1, 4, false, 2>(w, nullptr, x, y, rows, nb, ws, s, err);
     case 1: return launch_wd<12, 1, 1>(w, nullptr, x, y, rows, nb, ws, s, err);
     case 2: return launch_wd<8, 1, 1>(w, nullptr, x, y, rows, nb, ws, s, err);
     case 3: return launch_wd<4, 3, 1>(w, nullptr, x, y, rows, nb, ws, s, err);
     case 4: return launch_wd<5, 3, 1>(w, nullptr, x, y, rows, nb, ws, s, err);
     case 6:
       return lines_fit(nb, w) &&
-             launch_wd<6, 2, 1, 1, 4, false, 4, true>(w, nullptr, x, y, rows, nb, ws, s, err);
+             launch_wd<6, 2, 1, 4, false, 4, true>(w, nullptr, x, y, rows, nb, ws, s, err);
     case 7:
       return lines_fit(nb, w) &&
-             launch_wd<12, 1, 1, 1, 4, false, 4, true>(w, nullptr, x, y, rows, nb, ws, s, err);
+             launch_wd<12, 1, 1, 4, false, 4, true>(w, nullptr, x, y, rows, nb, ws, s, err);
     case 8:
       return lines_fit(nb, w) &&
-             launch_wd<8, 1, 1, 1, 4, false, 4, true>(w, nullptr, x, y, rows, nb, ws, s, err);
+             launch_wd<8, 1, 1, 4, false, 4, true>(w, nullptr, x, y, rows, nb, ws, s, err);
     default: break;
   }
   // full-line copies where the shape allows them, measured on MI355X
@@ -1305,7 +1179,7 @@ bool launch_q4k_matvec_mfma(const uint8_t* w, const float* x, float* y, uint32_t
   // arithmetic needs three waves per SIMD to hide its latency); the
   // half-line copies at 12 waves 13.6
   if (lines_fit(nb, w) &&
-      launch_wd<12, 1, 1, 1, 4, false, 4, true>(w, nullptr, x, y, rows, nb, ws, s, err))
+      launch_wd<12, 1, 1, 4, false, 4, true>(w, nullptr, x, y, rows, nb, ws, s, err))
     return true;
   return launch_wd<12, 1, 1>(w, nullptr, x, y, rows, nb, ws, s, err) ||
          launch_wd<8, 1, 1>(w, nullptr, x, y, rows, nb, ws, s, err) ||
@@ -1336,21 +1210,21 @@ bool launch_matvec_group(uint32_t type, const uint8_t* const* w, const uint32_t*
   if (group_two_block != 0 && (type == kTypeQ4K || type == kTypeQ5K) && shape_ok(trows, cols, 1u, type == kTypeQ4K ? 4 : 5, 2u) &&
       two_block_stages((uint32_t)tiles, nb, ws.bytes, type == kTypeQ4K ? 4 : 5, SliceChoice{})) {
     if (type == kTypeQ4K &&
-        launch_wd<12, 1, 1, 1, 4, true, 2>(w[0], nullptr, x, y, trows, nb, ws, s, err, ga))
+        launch_wd<12, 1, 1, 4, true, 2>(w[0], nullptr, x, y, trows, nb, ws, s, err, ga))
       return true;
     if (type == kTypeQ5K &&
-        launch_wd<12, 1, 1, 1, 5, true, 2>(w[0], nullptr, x, y, trows, nb, ws, s, err, ga))
+        launch_wd<12, 1, 1, 5, true, 2>(w[0], nullptr, x, y, trows, nb, ws, s, err, ga))
       return true;
   }
   switch (type) {
     case kTypeQ4K:
       return shape_ok(trows, cols, 1u, 4) &&
-             (launch_wd<12, 1, 1, 1, 4, true>(w[0], nullptr, x, y, trows, nb, ws, s, err, ga) ||
-              launch_wd<8, 1, 1, 1, 4, true>(w[0], nullptr, x, y, trows, nb, ws, s, err, ga));
+             (launch_wd<12, 1, 1, 4, true>(w[0], nullptr, x, y, trows, nb, ws, s, err, ga) ||
+              launch_wd<8, 1, 1, 4, true>(w[0], nullptr, x, y, trows, nb, ws, s, err, ga));
     case kTypeQ5K:
       return shape_ok(trows, cols, 1u, 5) &&
-             (launch_wd<8, 1, 1, 1, 5, true>(w[0], nullptr, x, y, trows, nb, ws, s, err, ga) ||
-              launch_wd<4, 1, 1, 1, 5, true>(w[0], nullptr, x, y, trows, nb, ws, s, err, ga));
+             (launch_wd<8, 1, 1, 5, true>(w[0], nullptr, x, y, trows, nb, ws, s, err, ga) ||
+              launch_wd<4, 1, 1, 5, true>(w[0], nullptr, x, y, trows, nb, ws, s, err, ga));
     case kTypeQ6K:
       return launch_q6k_matvec_group(ga, trows, cols, x, y, ws, s, err);
     default:
@@ -1369,15 +1243,15 @@ bool launch_q5k_matvec_mfma(const uint8_t* w, const float* x, float* y, uint32_t
 bool launch_q4k_matmul_mfma(const uint8_t* w, const float* x, float* y, uint32_t rows,
                             uint32_t cols, uint32_t batch, const Workspace& ws, hipStream_t s,
                             hipError_t* err) {
-  if (batch < 2 || !shape_ok(rows, cols, 1u, 4)) return false;
-  return matmul_passes<4>(w, x, y, rows, cols, batch, ws, s, err);
+  if (batch < 2 || batch > 16 || !shape_ok(rows, cols, 1u, 4)) return false;
+  return launch_q45_tokens(4, w, x, y, rows, cols / kBlockElems, batch, ws, s, err);
 }
 
 bool launch_q5k_matmul_mfma(const uint8_t* w, const float* x, float* y, uint32_t rows,
                             uint32_t cols, uint32_t batch, const Workspace& ws, hipStream_t s,
                             hipError_t* err) {
-  if (batch < 2 || !shape_ok(rows, cols, 1u, 5)) return false;
-  return matmul_passes<5>(w, x, y, rows, cols, batch, ws, s, err);
+  if (batch < 2 || batch > 16 || !shape_ok(rows, cols, 1u, 5)) return false;
+  return launch_q45_tokens(5, w, x, y, rows, cols / kBlockElems, batch, ws, s, err);
 }
 
 bool launch_q4k_gate_up_mfma(const uint8_t* gate, const uint8_t* up, const float* x, float* h,
@@ -1392,16 +1266,16 @@ bool launch_q4k_gate_up_mfma(const uint8_t* gate, const uint8_t* up, const float
     case 3: return launch_wd<10, 1, 2>(gate, up, x, h, rows, nb, ws, s, err);
     case 4:
       return lines_fit(nb, gate, up) &&
-             launch_wd<6, 2, 2, 1, 4, false, 4, true>(gate, up, x, h, rows, nb, ws, s, err);
+             launch_wd<6, 2, 2, 4, false, 4, true>(gate, up, x, h, rows, nb, ws, s, err);
     case 5:
       return lines_fit(nb, gate, up) &&
-             launch_wd<12, 1, 2, 1, 4, false, 4, true>(gate, up, x, h, rows, nb, ws, s, err);
+             launch_wd<12, 1, 2, 4, false, 4, true>(gate, up, x, h, rows, nb, ws, s, err);
     default: break;
   }
   // full-line copies at 12 waves: 17408 x 5120 22.9 us against 23.5 (27.7
   // with 6 waves and two stages in flight)
   if (lines_fit(nb, gate, up) &&
-      launch_wd<12, 1, 2, 1, 4, false, 4, true>(gate, up, x, h, rows, nb, ws, s, err))
+      launch_wd<12, 1, 2, 4, false, 4, true>(gate, up, x, h, rows, nb, ws, s, err))
     return true;
   // 12 waves (161 VGPRs, no spills): measured on MI355X against 8, us:
   // 17408 x 5120 23.1 / 24.0, 14336 x 4096 15.5 / 16.6, 11008 x 4096

@@ -71,11 +71,11 @@ constexpr uint32_t kSideRounded = 0xffu;  // side count of a rounded block
 // A row's stage passes when (error bound) * 1.01 <= kRoundedTol *
 // (sum |partial| - error bound); 1.01 covers the f32 rounding of both sums.
 constexpr float kRoundedTol = 4e-6f;
-// The Q4_K / Q5_K kernels check every stage (stage_ok): the bound of the f32
-// rounding of their factored dots plus that of their rounded blocks against
-// kStageTol of the row's sum |partial|.  With the fixed point's 2^-17 on kept
-// elements and the f32 accumulation of the partials (under 3e-6) the dot stays
-// within 2e-5 * sum|w x|.
+// The Q4_K / Q5_K kernels form a block's terms in f64 from exact integers, so
+// their rounded blocks' bound has kStageTol of the row's sum |partial| to
+// itself.  With the fixed point's 2^-17 on kept elements and the f32
+// accumulation of the partials (under 3e-6) the dot stays within
+// 2e-5 * sum|w x|.
 constexpr float kStageTol = 8e-6f;
 // A stage partial the vectors-in-rows kernel leaves for its reduce kernel to
 // recompute exactly (its lane failed the stage check): a signalling-NaN
@@ -121,7 +121,7 @@ __host__ __device__ constexpr Layout make_layout(uint32_t stage_bytes, uint32_t 
   l.expo_stride = l.side_off + nb * kSideBytes;
   l.img = waves * depth * stage_bytes;
   l.xsum = l.img + ntok * l.img_stride + 4096u;
-  l.expo = l.xsum + (xsum_per_block ? ntok * l.xsum_stride + 128u : 0u);
+  l.expo = l.xsum + (xsum_per_block ? ntok * l.xsum_stride + 256u : 0u);
   l.part = l.expo + ntok * l.expo_stride + 16u;
   l.cnt = l.part + slots * partials * 64u * ntok;
   l.owner = l.cnt + slots * 4u;
@@ -401,9 +401,9 @@ __device__ __forceinline__ void biased_values(const ChunkSplit& cs, bool listed,
 // halves are held by this lane (biased digit words u = X + 0x80808080) and the
 // lane before it in its DPP row; the result is valid in the odd lanes.  The
 // sum is exact (X = hi 2^15 + lo with both parts summed as integers below
-// 2^20) and rounded to f32 once, so the min term d_min * m * sum X of a unit
-// sees the activations rounded exactly as the MFMA digit sums do.
-__device__ __forceinline__ float unit_fixed_sum(const uint32_t (&u)[16]) {
+// 2^20, |sum| <= 2^35), so the min term d_min * m * sum X of a unit sees the
+// activations rounded exactly as the MFMA digit sums do.
+__device__ __forceinline__ double unit_fixed_sum(const uint32_t (&u)[16]) {
   uint32_t hi = 0u, lo = 0u;
 #pragma unroll
   for (int k = 0; k < 16; ++k) {
@@ -413,7 +413,7 @@ __device__ __forceinline__ float unit_fixed_sum(const uint32_t (&u)[16]) {
   }
   hi += dpp_u<kRowShr1>(hi);
   lo += dpp_u<kRowShr1>(lo);
-  return fmaf((float)(int32_t)hi, 32768.0f, (float)lo);
+  return fma((double)(int32_t)hi, 32768.0, (double)lo);
 }
 
 // Turns the copied blocks of activation vector `tok` into digit images in
@@ -470,9 +470,10 @@ __device__ __forceinline__ void build_images(uint32_t sbase, const Layout& L, ui
                       __float_as_uint(cs.err_side));
     }
     if (want_sums) {
-      const float xsum = unit_fixed_sum(u);  // odd lanes: unit n / 2
+      const double xsum = unit_fixed_sum(u);  // odd lanes: unit n / 2
       if (store && (n & 1u))
-        lds_write_b32(sbase + xsb + 32u * pb + 4u * (n >> 1), __float_as_uint(xsum));
+        lds_write_b64(sbase + xsb + 64u * pb + 8u * (n >> 1),
+                      __builtin_bit_cast(u32x2, xsum));
     }
     if (store && n == 0u) {
       lds_write_b32(sbase + exb + 4u * pb, (uint32_t)(bad_blk ? kBadBlock : cs.e - kFixBits));
@@ -551,14 +552,20 @@ __device__ __forceinline__ float rounded_bound(uint32_t list, uint32_t rmask, ui
   return err;
 }
 
-// The stage check of the Q4_K / Q5_K kernels: whether the row of this lane
-// passes with `err`, the lane's bound on the error of its fast-path partials
-// (their f32 rounding plus its rounded blocks), and `abs_part`, its sum of
-// |partial| (both summed over the row's four lane groups here).  A row that
-// fails recomputes the stage on the exact per-weight path.
+// The rounded-block check of the Q4_K / Q5_K kernels: whether the row of this
+// lane passes with `err`, the lane's bound on the error of its rounded
+// blocks, and `abs_part`, its sum of |partial| (both summed over the row's
+// four lane groups here).  A row that fails recomputes the stage on the
+// exact per-weight path.
 __device__ __forceinline__ bool stage_ok(float err, float abs_part) {
   const float e = sum_lane_groups(err), a = sum_lane_groups(abs_part);
   return e * 1.01f <= kStageTol * (a - e);
+}
+// The f64 difference p of a block's two terms, the first of them `first`: whether
+// its rounding (2^-52 of the first term) can show, that is p below 2^-30 of
+// it -- weights that cancel inside their own decode -- or not a number.
+__device__ __forceinline__ bool cancels(double p, double first) {
+  return !(fma(fabs(p), 0x1p30, -fabs(first)) >= 0.0);
 }
 
 // Slot ring set-up: every slot empty and owned by local tile == its index;
@@ -1261,20 +1268,6 @@ __device__ __forceinline__ void token_slot_done(uint32_t sbase, const Layout& L,
     lds_write_b32(sbase + L.owner + 4u * slot, pr.lt + slots);
   }
 }
-template <int NTOK>
-__device__ __forceinline__ void hand_off_tokens(uint32_t sbase, const Layout& L,
-                                                const FastDiv& by_slots, const Pair& pr,
-                                                uint32_t tparts, const float (&rowsum)[NTOK],
-                                                uint32_t lane, uint32_t rows,
-                                                float* __restrict__ y, uint32_t& fail) {
-  const uint32_t base = token_slot(sbase, L, by_slots, pr, tparts, NTOK, lane, fail);
-  if ((lane >> 4) == 0u) {
-#pragma unroll
-    for (int t = 0; t < NTOK; ++t) lds_write_b32(base + 64u * t, __float_as_uint(rowsum[t]));
-  }
-  token_slot_done<NTOK>(sbase, L, by_slots, pr, tparts, lane, rows, y);
-}
-
 // The schedule constants of a launch, or false when a multiply-high quotient
 // of the schedule could be inexact (x * d >= 2^32 for some quotient taken) or
 // the counts do not fit their fields.

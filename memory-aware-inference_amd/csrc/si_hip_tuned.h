@@ -18,9 +18,8 @@ bool launch_matvec_tuned(uint32_t type, const uint8_t* w, const float* x, float*
 // slices of at most 8 stages still fit the LDS).
 bool launch_q4k_matvec_mfma(const uint8_t* w, const float* x, float* y, uint32_t rows,
                             uint32_t cols, const Workspace& ws, hipStream_t s, hipError_t* err);
-// Q4_K, batch >= 2 vectors (batch-major x and y): two in one pass of the
-// one-vector-per-MFMA kernel, three to sixteen in one pass of the
-// vectors-in-rows kernel (the weights decoded once per pass).
+// Q4_K, 2..16 vectors (batch-major x and y) in one pass of the vectors-in-rows
+// kernel (the weights decoded once per pass).
 bool launch_q4k_matmul_mfma(const uint8_t* w, const float* x, float* y, uint32_t rows,
                             uint32_t cols, uint32_t batch, const Workspace& ws, hipStream_t s,
                             hipError_t* err);
