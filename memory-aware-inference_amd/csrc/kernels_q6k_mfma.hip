@@ -58,35 +58,54 @@ __host__ __device__ constexpr Layout layout(uint32_t waves, uint32_t depth, uint
   return make_layout(kStageBytes, 2u, 0u, waves, depth, nb, slots, sums, ntok);
 }
 
-// The lane's 13 pieces of a stage buffer (piece q of row n at 256 q + 16 n;
+// The lane's 13 pieces of a stage buffer (piece q of row n at 432 n + 16 q;
 // qa = piece 4h + s, qh = piece 8 + 2h + s, sc = piece 12 of the lane's row):
 //   v0 ql chunk A, v1 ql chunk B (piece +2), v2 qh chunk, v3 scales,
 //   v4 piece 13 (d of block 0) -- block 0;
 //   v5,v6 / v7,v8 / v9,v10 the same chunks of block 1 (13 pieces later, two
 //   pieces each), v11 piece 25 (stage bytes 400..415), v12 piece 26 (bytes
 //   404..419) -- its scales and d, block 1.
+// (A row's 27 pieces, an odd count, so 16 lanes reading one piece of 16 rows
+// meet all bank groups alike.)
 __device__ __forceinline__ void lds_read_stage(uint32_t qa, uint32_t qh, uint32_t sc,
                                                u32x4 (&v)[13]) {
   asm volatile(
       "ds_read_b128 %0, %13\n"
-      "ds_read_b128 %1, %13 offset:512\n"
+      "ds_read_b128 %1, %13 offset:32\n"
       "ds_read_b128 %2, %14\n"
       "ds_read_b128 %3, %15\n"
-      "ds_read_b128 %4, %15 offset:256\n"
-      "ds_read_b128 %5, %13 offset:3328\n"
-      "ds_read_b128 %6, %13 offset:3584\n"
-      "ds_read_b128 %7, %13 offset:3840\n"
-      "ds_read_b128 %8, %13 offset:4096\n"
-      "ds_read_b128 %9, %14 offset:3328\n"
-      "ds_read_b128 %10, %14 offset:3584\n"
-      "ds_read_b128 %11, %15 offset:3328\n"
-      "ds_read_b128 %12, %15 offset:3584\n"
+      "ds_read_b128 %4, %15 offset:16\n"
+      "ds_read_b128 %5, %13 offset:208\n"
+      "ds_read_b128 %6, %13 offset:224\n"
+      "ds_read_b128 %7, %13 offset:240\n"
+      "ds_read_b128 %8, %13 offset:256\n"
+      "ds_read_b128 %9, %14 offset:208\n"
+      "ds_read_b128 %10, %14 offset:224\n"
+      "ds_read_b128 %11, %15 offset:208\n"
+      "ds_read_b128 %12, %15 offset:224\n"
       "s_waitcnt lgkmcnt(0)"
       : "=&v"(v[0]), "=&v"(v[1]), "=&v"(v[2]), "=&v"(v[3]), "=&v"(v[4]), "=&v"(v[5]),
         "=&v"(v[6]), "=&v"(v[7]), "=&v"(v[8]), "=&v"(v[9]), "=&v"(v[10]), "=&v"(v[11]),
         "=&v"(v[12])
       : "v"(qa), "v"(qh), "v"(sc)
       : "memory");
+}
+
+// The copies of a stage: copy i, lane l moves piece c % 27 of row c / 27, c =
+// 64 i + l, so that a row's 420 bytes are read by consecutive lanes; the lanes
+// of the last copy past the last piece re-read it.  vo[i]: the lane's offset
+// from the stage's first row.  (With sixteen rows' pieces side by side, lane l
+// taking row l % 16, each lane was a cache access of its own, 448 a stage
+// instead of about 130: the 151936 x 5120 head 125.8 -> 120.2 us, 5120 x 5120
+// 10.1 -> 9.0, 5120 x 17408 21.8 -> 21.2.)
+__device__ __forceinline__ void copy_offsets(uint32_t row_bytes, uint32_t lane,
+                                             uint32_t (&vo)[kCopies]) {
+#pragma unroll
+  for (uint32_t i = 0; i < kCopies; ++i) {
+    const uint32_t c = min(64u * i + lane, 16u * kRowPieces - 1u);
+    const uint32_t row = (c * 2428u) >> 16;  // c / 27 for c < 432
+    vo[i] = row * row_bytes + min(16u * (c - kRowPieces * row), kLastPiece);
+  }
 }
 
 // The 8 A images of a stage (block b, MFMA t at addr + 1024 b + 256 t), read
@@ -310,8 +329,8 @@ __global__ __launch_bounds__(WAVES * 64) void q6k_matvec_mfma(const uint8_t* __r
       return pair_at(sc, k, nstages);
   };
   const uint32_t npairs = SLICED ? ss.npairs : sc.npairs;
-  const uint32_t voff = n * row_bytes + 16u * grp;
-  const uint32_t voff_last = n * row_bytes + (grp < 2u ? 16u * (24u + grp) : kLastPiece);
+  uint32_t vo[kCopies];
+  copy_offsets(row_bytes, lane, vo);
   const uint32_t my_pairs = wave < npairs ? (npairs - 1u - wave) / WAVES + 1u : 0u;
   // the stage bytes of a pair's tile and the tile's row count
   auto tile_at = [&](const Pair& pr, uint32_t& nrows) -> const uint8_t* {
@@ -342,11 +361,9 @@ __global__ __launch_bounds__(WAVES * 64) void q6k_matvec_mfma(const uint8_t* __r
         kBufferWord3);
     uint8_t* dst = wstage + (j % DEPTH) * kStageBytes;
 #pragma unroll
-    for (int i = 0; i < (int)kCopies - 1; ++i)
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, (lds_void*)(dst + 1024 * i), 16,
-                                                voff + 64u * i, 0, 0, 0);
-    __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, (lds_void*)(dst + 1024 * (kCopies - 1)), 16,
-                                              voff_last, 0, 0, 0);
+    for (int i = 0; i < (int)kCopies; ++i)
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, (lds_void*)(dst + 1024 * i), 16, vo[i], 0, 0,
+                                                0);
   };
   // A long image build (48 blocks or more in the workgroup's range, every
   // wave a builder): the ring slots are set and a barrier passed first, so
@@ -417,10 +434,10 @@ __global__ __launch_bounds__(WAVES * 64) void q6k_matvec_mfma(const uint8_t* __r
 
   // 4. the wave's pairs
   const bool upper = half != 0u;  // lane groups 2, 3: scales 8..15
-  const uint32_t base = sbase + wave * DEPTH * kStageBytes + 16u * n;
-  const uint32_t qa0 = base + 256u * (4u * half + sub);
-  const uint32_t qh0 = base + 256u * (8u + 2u * half + sub);
-  const uint32_t sc0 = base + 256u * 12u;
+  const uint32_t base = sbase + wave * DEPTH * kStageBytes + 16u * kRowPieces * n;
+  const uint32_t qa0 = base + 16u * (4u * half + sub);
+  const uint32_t qh0 = base + 16u * (8u + 2u * half + sub);
+  const uint32_t sc0 = base + 16u * 12u;
   const uint32_t sb_lo = 8u * sub, sb_hi = 8u * sub + 16u;  // bit offsets of the lane's scales
   i32x4 A[8];
 #pragma unroll
