@@ -14,11 +14,8 @@
 // row's error from those blocks by (largest |w| the block header allows) x
 // (that sum), and compares it with the sum of |partial dot| over the row's
 // stage, which is at most sum|w x| over the stage.  A row whose bound exceeds
-// kRoundedTol of it recomputes its rounded blocks exactly.  (The
-// vectors-in-rows kernel, q4k_tokens_mfma, builds its own images and lists
-// up to kSideMax side elements of a block as (index, x) entries instead,
-// adding w_i * x_i for them with the exact per-weight decode: a rounded
-// block there holds back the next stage's copy until its rows are checked.)
+// kRoundedTol of it recomputes its rounded blocks exactly.  (The kernels of
+// several vectors build their own images, tokens_common.h.)
 //
 // A block with an activation that is not finite or reaches 2^100 takes the
 // exact per-weight path whole.  For every
@@ -58,15 +55,12 @@ constexpr int kBufferWord3 = 0x00020000;  // raw dword access (CDNA buffer descr
 constexpr int kFixBits = 30;
 constexpr uint32_t kLdsBytes = 163840u;
 constexpr int kBadBlock = 0x40000000;  // exponent slot of a block taking the exact path
-// Side elements: non-zero |x| below 2^(e_b - kSideShift).  Each block and
-// activation vector has kSideBytes of LDS: for a rounded block, 16 f32 error
-// sums, the one of chunk c at position 4 p + t for the chunk in MFMA t of
-// lane group p (the four of a lane group side by side); in q4k_tokens_mfma,
-// up to kSideMax 8-byte entries (element index, x bits) instead.
+// Side elements: non-zero |x| below 2^(e_b - kSideShift).  Each block has
+// kSideBytes of LDS: for a rounded block, 16 f32 error sums, the one of chunk c
+// at position 4 p + t for the chunk in MFMA t of lane group p (the four of a
+// lane group side by side).
 constexpr int kSideShift = 14;
-constexpr uint32_t kSideMax = 8;
-constexpr uint32_t kSideEntryBytes = 8;
-constexpr uint32_t kSideBytes = kSideMax * kSideEntryBytes;  // 64
+constexpr uint32_t kSideBytes = 64;
 constexpr uint32_t kSideRounded = 0xffu;  // side count of a rounded block
 // A row's stage passes when (error bound) * 1.01 <= kRoundedTol *
 // (sum |partial| - error bound); 1.01 covers the f32 rounding of both sums.
@@ -84,15 +78,14 @@ constexpr uint32_t kPartRedo = 0x7f8c0de5u;
 
 constexpr int waitcnt_vm(int n) { return (n & 0xf) | ((n >> 4) << 14) | (0x7 << 4) | (0xf << 8); }
 
-// LDS map of one workgroup (byte offsets): per-wave stage buffers; for each
-// of ntok activation vectors the digit images of all its blocks (a further
-// 4 KB after the last one, which dead blocks of a short last stage may
-// read), its unit sums [block][unit] (formats that need them) and its block
-// metadata; then a ring of `slots` tile slots: [slot][partial][token][16 rows]
-// f32 partials, and per slot a completion count and the tile index it
-// currently belongs to.
+// LDS map of one workgroup (byte offsets): per-wave stage buffers; the digit
+// images of all blocks of x (a further 4 KB after the last one, which dead
+// blocks of a short last stage may read), its unit sums [block][unit] (f64,
+// formats that need them) and its block metadata; then a ring of `slots` tile
+// slots: [slot][partial][16 rows] f32 partials, and per slot a completion
+// count and the tile index it currently belongs to.
 //
-// Block metadata of a vector (at expo + t expo_stride): the exponents
+// Block metadata (at expo): the exponents
 // [block] (4 bytes each, at most kMaxMetaBlocks blocks), at +kCountOff the
 // side counts, one byte per block, and at +side_off the side areas
 // [block][kSideBytes].  The counts of the bps blocks of a stage sit at
@@ -103,27 +96,24 @@ constexpr uint32_t kCountOff = 512;
 constexpr uint32_t kMaxMetaBlocks = kCountOff / 4u;
 struct Layout {
   uint32_t img, xsum, expo, part, cnt, owner, ready, total;
-  // per activation vector
-  uint32_t img_stride, xsum_stride, expo_stride;
   uint32_t side_off, bps;  // side areas in the metadata; blocks per stage
+  bool sums;               // unit sums are kept
 };
 __host__ __device__ constexpr Layout make_layout(uint32_t stage_bytes, uint32_t stage_blocks,
                                                  uint32_t xsum_per_block, uint32_t waves,
                                                  uint32_t depth, uint32_t nb, uint32_t slots,
-                                                 uint32_t mats, uint32_t ntok = 1u) {
+                                                 uint32_t mats) {
   Layout l{};
   const uint32_t nstages = (nb + stage_blocks - 1u) / stage_blocks;
   const uint32_t partials = nstages * mats;  // per tile
   l.bps = stage_blocks;
-  l.img_stride = nb * 1024u;
-  l.xsum_stride = nb * xsum_per_block;
+  l.sums = xsum_per_block != 0u;
   l.side_off = kCountOff + ((4u * stage_blocks * nstages + 15u) & ~15u);
-  l.expo_stride = l.side_off + nb * kSideBytes;
   l.img = waves * depth * stage_bytes;
-  l.xsum = l.img + ntok * l.img_stride + 4096u;
-  l.expo = l.xsum + (xsum_per_block ? ntok * l.xsum_stride + 256u : 0u);
-  l.part = l.expo + ntok * l.expo_stride + 16u;
-  l.cnt = l.part + slots * partials * 64u * ntok;
+  l.xsum = l.img + nb * 1024u + 4096u;
+  l.expo = l.xsum + (xsum_per_block ? nb * xsum_per_block + 256u : 0u);
+  l.part = l.expo + l.side_off + nb * kSideBytes + 16u;
+  l.cnt = l.part + slots * partials * 64u;
   l.owner = l.cnt + slots * 4u;
   l.ready = l.owner + slots * 4u;  // count of image builders done (16 bytes)
   l.total = l.ready + 16u;
@@ -298,14 +288,13 @@ __device__ __forceinline__ void copy_x(uint8_t* smem, uint32_t img, const float*
 // The fixed-point split of one lane's 16 activations (a 16-element chunk of a
 // block whose 16 lanes form one DPP row): the row's exponent e (largest |x|
 // below 2^e), the fixed-point values X (two's complement), the mask of side
-// elements, the f32 sum of all 16 and that of the side elements, the sum of
-// the side elements' rounding errors, and whether the chunk alone forces the
-// exact path.
+// elements, the f32 sum of all 16, the sum of the side elements' rounding
+// errors, and whether the chunk alone forces the exact path.
 struct ChunkSplit {
   int e;
   uint32_t fx[16];
   uint32_t smask;
-  float xsum, xsum_side, err_side;
+  float xsum, err_side;
   bool bad;
 };
 __device__ __forceinline__ ChunkSplit split_chunk(const float (&xv)[16]) {
@@ -332,7 +321,7 @@ __device__ __forceinline__ ChunkSplit split_chunk(const float (&xv)[16]) {
   for (int k = 0; k < 16; ++k)
     r.fx[k] = (uint32_t)__float2int_rn(__builtin_amdgcn_ldexpf(xv[k], kFixBits - r.e));
   r.smask = 0u;
-  r.xsum_side = r.err_side = 0.0f;
+  r.err_side = 0.0f;
   // (rare for dense activations: some |x| below the threshold, or a zero).
   // The empty asm keeps the compiler from hoisting this work above the
   // branch, into every block's build.
@@ -351,7 +340,6 @@ __device__ __forceinline__ ChunkSplit split_chunk(const float (&xv)[16]) {
     for (int k = 0; k < 16; ++k) {
       const bool side = ((__float_as_uint(xs[k]) & 0x7fffffffu) - 1u) < tb;
       r.smask |= (uint32_t)side << k;
-      r.xsum_side += side ? xs[k] : 0.0f;
       // |X| < 2^16 for a side element, so (float)X and the difference are exact
       const float err =
           fabsf(xs[k] - __builtin_amdgcn_ldexpf((float)(int)fs[k], r.e - kFixBits));
@@ -361,40 +349,10 @@ __device__ __forceinline__ ChunkSplit split_chunk(const float (&xv)[16]) {
   return r;
 }
 
-// Side list of one block from its 16 lanes (one DPP row, lane n holding
-// elements 16 n .. 16 n + 15 in `xv`): returns the block's side count (the
-// same in every lane of the row); when it is at most kSideMax and `write`,
-// the lanes store their entries (element index, x bits) in element order at
-// `list` (8 bytes each).
-__device__ __forceinline__ uint32_t side_list(const float (&xv)[16], uint32_t smask, uint32_t n,
-                                              uint32_t list, bool write) {
-  const uint32_t own = __builtin_popcount(smask);
-  uint32_t incl = own;  // inclusive prefix count over the row
-  incl += dpp_u<kRowShr1>(incl);
-  incl += dpp_u<kRowShr2>(incl);
-  incl += dpp_u<kRowShr4>(incl);
-  incl += dpp_u<kRowShr8>(incl);
-  const uint32_t total = dpp_u<kRowBcast15>(incl);
-  if (write && smask != 0u && total <= kSideMax) {
-    uint32_t pos = incl - own;
+// The biased digit words of a chunk: X + 0x80808080.
+__device__ __forceinline__ void biased_values(const ChunkSplit& cs, uint32_t (&u)[16]) {
 #pragma unroll
-    for (int k = 0; k < 16; ++k) {
-      if ((smask >> k) & 1u) {
-        lds_write_b64(list + kSideEntryBytes * pos, u32x2{16u * n + (uint32_t)k,
-                                                           __float_as_uint(xv[k])});
-        ++pos;
-      }
-    }
-  }
-  return total;
-}
-
-// The biased digit words of a chunk: X + 0x80808080, with X = 0 for side
-// elements that go to the block's side list (`listed`).
-__device__ __forceinline__ void biased_values(const ChunkSplit& cs, bool listed, uint32_t (&u)[16]) {
-#pragma unroll
-  for (int k = 0; k < 16; ++k)
-    u[k] = ((listed && ((cs.smask >> k) & 1u)) ? 0u : cs.fx[k]) + 0x80808080u;
+  for (int k = 0; k < 16; ++k) u[k] = cs.fx[k] + 0x80808080u;
 }
 
 // Sum of the fixed-point values X of a 32-element unit whose two 16-element
@@ -416,8 +374,7 @@ __device__ __forceinline__ double unit_fixed_sum(const uint32_t (&u)[16]) {
   return fma((double)(int32_t)hi, 32768.0, (double)lo);
 }
 
-// Turns the copied blocks of activation vector `tok` into digit images in
-// place, plus exponents, the error sums of rounded blocks, side counts
+// Turns the copied blocks of x into digit images in place, plus exponents, the error sums of rounded blocks, side counts
 // (kSideRounded or 0) and, when the layout keeps them, the sums of each
 // 32-element unit's fixed-point values (unit_fixed_sum, in units of
 // 2^(e_b - 30)).  The caller has waited for the copies.  CHUNK_SLOT(c)
@@ -428,12 +385,9 @@ __device__ __forceinline__ double unit_fixed_sum(const uint32_t (&u)[16]) {
 template <int WAVES, typename ChunkSlot>
 __device__ __forceinline__ void build_images(uint32_t sbase, const Layout& L, uint32_t nb,
                                              uint32_t wave, uint32_t grp, uint32_t n,
-                                             ChunkSlot chunk_slot, uint32_t tok = 0u) {
+                                             ChunkSlot chunk_slot) {
   const uint32_t npass = (nb + 4u * WAVES - 1u) / (4u * WAVES);
-  const bool want_sums = L.xsum_stride != 0u;
-  const uint32_t img = L.img + tok * L.img_stride;
-  const uint32_t xsb = L.xsum + tok * L.xsum_stride;
-  const uint32_t exb = L.expo + tok * L.expo_stride;
+  const uint32_t img = L.img, xsb = L.xsum, exb = L.expo;
   const uint32_t sdb = exb + L.side_off;
   for (uint32_t j = 0; j < npass; ++j) {
     if (4u * (wave + WAVES * j) >= nb) break;
@@ -454,7 +408,7 @@ __device__ __forceinline__ void build_images(uint32_t sbase, const Layout& L, ui
     const bool rounded =
         !bad_blk && ((__builtin_amdgcn_ballot_w64(cs.smask != 0u) >> (16u * grp)) & 0xffffull);
     uint32_t u[16];
-    biased_values(cs, false, u);
+    biased_values(cs, u);
     uint32_t dg[4][4];  // [element quad][digit]
 #pragma unroll
     for (int k = 0; k < 4; ++k) transpose_digits(u[4 * k], u[4 * k + 1], u[4 * k + 2], u[4 * k + 3], dg[k]);
@@ -469,7 +423,7 @@ __device__ __forceinline__ void build_images(uint32_t sbase, const Layout& L, ui
         lds_write_b32(list + 4u * (4u * ((slot >> 6) & 3u) + (slot >> 8)),
                       __float_as_uint(cs.err_side));
     }
-    if (want_sums) {
+    if (L.sums) {
       const double xsum = unit_fixed_sum(u);  // odd lanes: unit n / 2
       if (store && (n & 1u))
         lds_write_b64(sbase + xsb + 64u * pb + 8u * (n >> 1),
@@ -1226,48 +1180,6 @@ inline LaunchShape launch_shape(uint32_t ntiles, uint32_t tparts, uint32_t waves
   return ls;
 }
 
-// hand_off for NTOK activation vectors at once, whole tiles only: partial r
-// of the tile holds 16 rows x NTOK sums; the finishing wave stores
-// y[tok * rows + row] for every token.  In two halves for kernels that write
-// one vector's sums at a time: token_slot waits until the tile owns its ring
-// slot and returns the LDS address of this lane's row in partial pr.r (vector
-// t at + 64 t); token_slot_done counts the partial and, in the wave that
-// completes the tile, adds the partials in order and stores the rows.
-__device__ __forceinline__ uint32_t token_slot(uint32_t sbase, const Layout& L,
-                                               const FastDiv& by_slots, const Pair& pr,
-                                               uint32_t tparts, uint32_t ntok, uint32_t lane,
-                                               uint32_t& fail) {
-  const uint32_t slots = by_slots.d;
-  const uint32_t slot = pr.lt - quo(pr.lt, by_slots) * slots;
-  wait_slot(sbase + L.owner + 4u * slot, pr.lt, fail);
-  return sbase + L.part + 64u * ntok * (slot * tparts + pr.r) + 4u * (lane & 15u);
-}
-template <int NTOK>
-__device__ __forceinline__ void token_slot_done(uint32_t sbase, const Layout& L,
-                                                const FastDiv& by_slots, const Pair& pr,
-                                                uint32_t tparts, uint32_t lane, uint32_t rows,
-                                                float* __restrict__ y) {
-  const uint32_t grp = lane >> 4, n = lane & 15u;
-  const uint32_t slots = by_slots.d;
-  const uint32_t slot = pr.lt - quo(pr.lt, by_slots) * slots;
-  uint32_t old = 0u;
-  if (lane == 0u) old = lds_add_rtn(sbase + L.cnt + 4u * slot, 1u);
-  const uint32_t done = __builtin_amdgcn_readlane(old, 0);
-  if (done != tparts - 1u) return;
-  // lane group g stores tokens g, g + 4, ...
-  const uint32_t row = pr.tile * 16u + n;
-  for (uint32_t t = grp; t < (uint32_t)NTOK; t += 4u) {
-    float sum = 0.0f;
-    for (uint32_t st = 0; st < tparts; ++st)
-      sum += __uint_as_float(
-          lds_read_b32(sbase + L.part + 64u * NTOK * (slot * tparts + st) + 64u * t + 4u * n));
-    if (row < rows) y[(size_t)t * rows + row] = sum;
-  }
-  if (lane == 0u) {
-    lds_write_b32(sbase + L.cnt + 4u * slot, 0u);
-    lds_write_b32(sbase + L.owner + 4u * slot, pr.lt + slots);
-  }
-}
 // The schedule constants of a launch, or false when a multiply-high quotient
 // of the schedule could be inexact (x * d >= 2^32 for some quotient taken) or
 // the counts do not fit their fields.

@@ -1,14 +1,13 @@
 // Shared parts of the kernels that put several activation vectors in the
-// rows of the matrix-core A operand (q4k_tokens_mfma, q6k_tokens_mfma): the
-// group images of four vectors at a time, built in LDS from copies of x,
-// and the reduce kernel that adds the K slices' partial sums of a sliced
-// launch in slice order.
+// rows of the matrix-core A operand (q45_tokens_mfma, q6k_tokens_mfma): the
+// group images of four vectors at a time, built in LDS, and the reduce kernel
+// that adds the K slices' partial sums of a sliced launch in slice order.
 //
-// Group images (4 KB per block and group of four vectors): group g's block
-// b at img + 4096 (g nbl + b), unit pair p at + 1024 p, then 16 bytes per
-// A-operand lane l = 16 k + 4 t + d of v_mfma_i32_16x16x32_i8: the 8 bytes
-// of digit d of vector 4 g + t over elements 8 k .. 8 k + 7 of unit 2 p,
-// then those of unit 2 p + 1.
+// Group images: four vectors of four digits in the 16 A rows of
+// v_mfma_i32_16x16x64_i8 (lane 16 k + 4 t + d: digit d of vector t over the 16
+// elements that meet lane group k's weights).  A block is four MFMAs j, 1 KB
+// each; chunk c (elements 16 c .. 16 c + 15) is at the offset a format's map
+// gives, 1024 j + 256 k.
 #pragma once
 
 #include "mfma_common.h"
@@ -16,131 +15,6 @@
 namespace sihip {
 namespace mfma {
 namespace {
-
-// An 8-byte MFMA operand from two words.
-__device__ __forceinline__ int64_t as_i64(uint32_t lo, uint32_t hi) {
-  return (int64_t)(((uint64_t)hi << 32) | lo);
-}
-
-// The image blocks a wave owns: group-blocks q = wave, wave + WAVES, ... of
-// the ng x nbl of a launch (group q / nbl, local block q % nbl), walked
-// without a division.
-template <int WAVES, typename F>
-__device__ __forceinline__ void for_group_blocks(uint32_t ng, uint32_t nbl, uint32_t wave, F f) {
-  uint32_t g = 0u, i = wave;
-  while (i >= nbl && g < ng) {
-    i -= nbl;
-    ++g;
-  }
-  for (; g < ng;) {
-    f(g, i);
-    i += WAVES;
-    while (i >= nbl && g < ng) {
-      i -= nbl;
-      ++g;
-    }
-  }
-}
-
-// Copies of the vectors' blocks blk0 .. blk0 + nbl - 1: vector 4 g + t's
-// block blk0 + i at img + 4096 (g nbl + i) + 1024 t; the slots of vectors past
-// ntok are cleared.
-template <int WAVES>
-__device__ __forceinline__ void copy_x_group(uint8_t* smem, uint32_t img, const float* x,
-                                             uint32_t nb, uint32_t blk0, uint32_t nbl,
-                                             uint32_t ng, uint32_t ntok, uint32_t wave,
-                                             uint32_t lane) {
-  const __amdgpu_buffer_rsrc_t xr = __builtin_amdgcn_make_buffer_rsrc(
-      const_cast<float*>(x), 0, (int)(ntok * nb * 1024u), kBufferWord3);
-  for_group_blocks<WAVES>(ng, nbl, wave, [&](uint32_t g, uint32_t i) {
-    const uint32_t dst = img + 4096u * (g * nbl + i);
-#pragma unroll
-    for (uint32_t t = 0; t < 4u; ++t) {
-      const uint32_t v = 4u * g + t;
-      if (v < ntok)
-        __builtin_amdgcn_raw_ptr_buffer_load_lds(xr, (lds_void*)(smem + dst + 1024u * t), 16,
-                                                  (v * nb + blk0 + i) * 1024u + 16u * lane, 0, 0,
-                                                  0);
-      else
-        lds_write_b128((uint32_t)(uintptr_t)smem + dst + 1024u * t + 16u * lane,
-                       u32x4{0u, 0u, 0u, 0u});
-    }
-  });
-}
-
-// Group images, exponents, side lists and unit sums of the copied blocks, in
-// place: a wave converts exactly the group-blocks it copied; lane (t, c)
-// takes elements 16 c .. 16 c + 15 of vector 4 g + t.  Blocks follow
-// build_images' rules (side elements, exponent kBadBlock for blocks that
-// must take the exact path).  LIST: up to kSideMax side elements of a block
-// are listed (and zero in the image) for the kernel to add exactly; without
-// it every block with side elements is a rounded block, which the kernel
-// checks with the block's error sums instead (the two- and four-group Q4_K
-// and Q5_K kernels: the listed elements' exact decode took registers enough
-// to spill their main loops).
-template <int WAVES, bool LIST = true>
-__device__ __forceinline__ void build_group_images(uint32_t sbase, const Layout& L, uint32_t nbl,
-                                                   uint32_t ng, uint32_t wave, uint32_t lane) {
-  const uint32_t t = lane >> 4, c = lane & 15u;
-  const uint32_t u = c >> 1;                                  // unit of the lane's chunk
-  const uint32_t g0 = 2u * (c & 1u);                          // K slice of its first 8
-  const uint32_t woff = 1024u * (u >> 1) + 16u * (16u * g0 + 4u * t) + 8u * (u & 1u);
-  for_group_blocks<WAVES>(ng, nbl, wave, [&](uint32_t g, uint32_t b) {
-    const uint32_t blk = sbase + L.img + 4096u * (g * nbl + b);
-    const uint32_t v = 4u * g + t;  // the lane's vector
-    u32x4 xq[4];
-    lds_read4<16>(blk + 1024u * t + 64u * c, xq);
-    float xv[16];
-#pragma unroll
-    for (int k = 0; k < 4; ++k)
-#pragma unroll
-      for (int i = 0; i < 4; ++i) xv[4 * k + i] = __uint_as_float(xq[k][i]);
-    const ChunkSplit cs = split_chunk(xv);
-    const bool bad_blk = (__builtin_amdgcn_ballot_w64(cs.bad) >> (16u * t)) & 0xffffull;
-    const uint32_t meta = sbase + L.expo + v * L.expo_stride;
-    const uint32_t list = meta + L.side_off + kSideBytes * b;
-    uint32_t nside = 0u;
-    bool rounded;
-    if constexpr (LIST) {
-      nside = __builtin_amdgcn_ballot_w64(cs.smask != 0u)
-                  ? side_list(xv, cs.smask, c, list, !bad_blk)
-                  : 0u;
-      rounded = !bad_blk && nside > kSideMax;
-    } else {
-      rounded = !bad_blk &&
-                ((__builtin_amdgcn_ballot_w64(cs.smask != 0u) >> (16u * t)) & 0xffffull) != 0u;
-    }
-    uint32_t uq[16];
-    biased_values(cs, !rounded, uq);
-    uint32_t dg[4][4];
-#pragma unroll
-    for (int k = 0; k < 4; ++k)
-      transpose_digits(uq[4 * k], uq[4 * k + 1], uq[4 * k + 2], uq[4 * k + 3], dg[k]);
-    // the wave has read the whole block (lds_read4 waits) before any write
-#pragma unroll
-    for (int d = 0; d < 4; ++d) {
-      lds_write_b64(blk + woff + 16u * d, u32x2{dg[0][d], dg[1][d]});
-      lds_write_b64(blk + woff + 16u * d + 256u, u32x2{dg[2][d], dg[3][d]});
-    }
-    if (rounded)  // chunk c's error sum at position c (read whole by tok_side)
-      lds_write_b32(list + 4u * c, __float_as_uint(cs.err_side));
-    const float xsum = unit_fixed_sum(uq);  // odd lanes: unit c / 2 (listed elements as 0)
-    if (c & 1u)
-      lds_write_b32(sbase + L.xsum + v * L.xsum_stride + 32u * b + 4u * u, __float_as_uint(xsum));
-    if (c == 0u) {
-      lds_write_b32(meta + 4u * b, (uint32_t)(bad_blk ? kBadBlock : cs.e - kFixBits));
-      lds_write_b8(meta + count_pos(L, b), bad_blk ? 0u : rounded ? kSideRounded : nside);
-    }
-  });
-}
-
-
-// ---- Group images for v_mfma_i32_16x16x64_i8 -------------------------------
-//
-// The same four vectors of four digits per group in the 16 A rows, K = 64 (lane
-// 16 k + 4 t + d: digit d of vector t over the 16 elements that meet lane
-// group k's weights): a block is four MFMAs j, 1 KB each, chunk c (elements
-// 16 c .. 16 c + 15) at the offset a format's map gives, 1024 j + 256 k.
 
 // Plain LDS reads: the compiler places their waits, so that a block's reads
 // overlap.  (For kernels without buffer->LDS copies, which the compiler would
@@ -330,12 +204,6 @@ __device__ __forceinline__ float slice_err(const uint8_t* rerr, uint32_t nbl) {
   for (uint32_t b = 1; b < 4u; ++b)
     if (b < nbl) e += __uint_as_float(v[b]);
   return e;
-}
-
-// Sum of all 16 chunk error sums of a rounded block's side area.
-__device__ __forceinline__ float rounded_err_all(uint32_t list) {
-  return (rounded_err(list, 0u) + rounded_err(list, 1u)) +
-         (rounded_err(list, 2u) + rounded_err(list, 3u));
 }
 
 // y[t * yrows + row] = sum over the stages s of part[(s * nv + t) * rows + row],
