@@ -39,23 +39,21 @@
 //
 // Work split.  A launch cuts K into slices of four blocks: workgroup g works
 // on slice g / GS for tiles g % GS, g % GS + GS, ..., keeping that slice's
-// images in LDS; each wave takes (tile, slice) pairs and stores the vectors'
-// sums in the scratch; tok_reduce adds the slices in order.  A launch whose
-// sums exceed the scratch runs as several over row ranges.
-//
-// Weights go straight to registers: a block's pieces are loaded for the
-// wave's next tile as soon as the block is decoded, so a tile's worth of loads
-// is in flight through the arithmetic, and the LDS holds images only.  (Staged
-// in LDS by buffer->LDS copies that went out after a stage's arithmetic:
-// 17408 x 5120 M = 4 / 16 19.2 / 33.4 us against 17.8 / 28.2, part of it the
-// shorter image build.  Reading each group's images one group ahead changed
-// nothing: 18.1 / 29.2.)
+// images in LDS; each wave takes (tile, slice) pairs, their two-block stages
+// one after another through one stage buffer (buffer->LDS copies, row by row;
+// the next stage's go out once the stage is in registers), and stores the
+// vectors' sums in the scratch; tok_reduce adds the slices in order.  A launch
+// whose sums exceed the scratch runs as several over row ranges.
 //
 // Measured, 17408 x 5120 Q4_K M = 4 / 8 / 16 with the reduce (4.1-4.7 us of
-// it): 27.9 / 44.4 / 72.9 -> 17.8 / 21.2 / 28.2 us.  At M = 4 the launch is
-// bound by the weight stream behind its start (5 us until the first tile is in
-// and the images are built); at M = 16 VALU (about 180 instructions a tile and
-// block) and MFMA (36 of 16 cycles) add up to 13 of the kernel's 24 us.
+// it): 27.9 / 44.4 / 72.9 us with the scales applied to the MFMA results and
+// f32 terms; 16.3 / 20.3 / 26.9 here.  On the way: four-block stages whose copy
+// went out after the arithmetic 19.2 / 23.3 / 33.4; weights loaded straight to
+// registers, a tile ahead, 17.8 / 21.2 / 28.2 (each lane's 16 bytes a cache
+// access of its own).  At M = 4 the launch is bound by the weight stream behind
+// its start (5 us until the first stage is in and the images are built); at
+// M = 16 VALU (about 180 instructions a tile and block) and MFMA (36 of 16
+// cycles) add up to 13 of the kernel's 22 us.
 #include "mfma_common.h"
 #include "si_hip_tuned.h"
 #include "tokens_common.h"
@@ -71,6 +69,13 @@ template <int QB>
 struct Format {
   static constexpr uint32_t kBytes = QB == 5 ? kQ5Bytes : kQ4Bytes;
   static constexpr uint32_t kType = QB == 5 ? kTypeQ5K : kTypeQ4K;
+  // A stage is two blocks of 16 rows.  In LDS a row keeps its 16-byte pieces in
+  // order, an odd number of slots (kPitch) from the next row, so that 16 lanes
+  // reading one piece of the 16 rows meet all bank groups alike.
+  static constexpr uint32_t kPieces = 2u * kBytes / 16u;
+  static constexpr uint32_t kPitch = kPieces | 1u;
+  static constexpr int kCopies = (int)((16u * kPitch + 63u) / 64u);
+  static constexpr uint32_t kStage = 1024u * kCopies;
 };
 
 // Launch constants: GS workgroups per slice and its division constant.
@@ -78,26 +83,83 @@ struct Tok45Args {
   uint32_t groups_per_slice, m_gps;
 };
 
-// The lane's pieces of one block: the header, its two qs pieces and (Q5_K) the
-// two qh pieces.
+// The lane's pieces of a stage's two blocks: the header, its two qs pieces and
+// (Q5_K) the two qh pieces.
 template <int QB>
 struct Raw45 {
   u32x4 h, q[2], qh[QB == 5 ? 2 : 1];
 };
 template <int QB>
-__device__ __forceinline__ void load_block(Raw45<QB>& r, __amdgpu_buffer_rsrc_t rsrc,
-                                           uint32_t row_off, uint32_t qs_off, int b) {
-  auto ld = [&](uint32_t off) {
-    return __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(rsrc, off, 0, 0));
-  };
-  const uint32_t at = Format<QB>::kBytes * (uint32_t)b;
-  r.h = ld(row_off + at);
-  r.q[0] = ld(qs_off + at);
-  r.q[1] = ld(qs_off + at + 16u);
-  if constexpr (QB == 5) {
-    r.qh[0] = ld(row_off + at + 16u);
-    r.qh[1] = ld(row_off + at + 32u);
-  }
+__device__ __forceinline__ void read_stage(Raw45<QB> (&r)[2], uint32_t hb, uint32_t qb) {
+  if constexpr (QB == 4)
+    asm volatile(
+        "ds_read_b128 %0, %6\n"
+        "ds_read_b128 %1, %7\n"
+        "ds_read_b128 %2, %7 offset:16\n"
+        "ds_read_b128 %3, %6 offset:144\n"
+        "ds_read_b128 %4, %7 offset:144\n"
+        "ds_read_b128 %5, %7 offset:160\n"
+        "s_waitcnt lgkmcnt(0)"
+        : "=&v"(r[0].h), "=&v"(r[0].q[0]), "=&v"(r[0].q[1]), "=&v"(r[1].h), "=&v"(r[1].q[0]),
+          "=&v"(r[1].q[1])
+        : "v"(hb), "v"(qb)
+        : "memory");
+  else
+    asm volatile(
+        "ds_read_b128 %0, %10\n"
+        "ds_read_b128 %1, %10 offset:16\n"
+        "ds_read_b128 %2, %10 offset:32\n"
+        "ds_read_b128 %3, %11\n"
+        "ds_read_b128 %4, %11 offset:16\n"
+        "ds_read_b128 %5, %10 offset:176\n"
+        "ds_read_b128 %6, %10 offset:192\n"
+        "ds_read_b128 %7, %10 offset:208\n"
+        "ds_read_b128 %8, %11 offset:176\n"
+        "ds_read_b128 %9, %11 offset:192\n"
+        "s_waitcnt lgkmcnt(0)"
+        : "=&v"(r[0].h), "=&v"(r[0].qh[0]), "=&v"(r[0].qh[QB - 4]), "=&v"(r[0].q[0]),
+          "=&v"(r[0].q[1]), "=&v"(r[1].h), "=&v"(r[1].qh[0]), "=&v"(r[1].qh[QB - 4]),
+          "=&v"(r[1].q[0]), "=&v"(r[1].q[1])
+        : "v"(hb), "v"(qb)
+        : "memory");
+}
+
+// Group G's operands for block B of a stage (from the stage's first block): its
+// images (ia), unit sums (ua), the exponent of the lane's vector (ea) and
+// (Q5_K) 128 times that vector's digit sums (da).
+template <int QB, int G, int B>
+__device__ __forceinline__ void read_group(uint32_t ia, uint32_t ua, uint32_t ea, uint32_t da,
+                                           i32x4 (&a)[4], uint32_t& xs, int& e, i32x4& ds) {
+  constexpr int kGb = (int)kSliceBlocks * G + B;
+  if constexpr (QB == 5)
+    asm volatile(
+        "ds_read_b128 %0, %7 offset:%11\n"
+        "ds_read_b128 %1, %7 offset:%12\n"
+        "ds_read_b128 %2, %7 offset:%13\n"
+        "ds_read_b128 %3, %7 offset:%14\n"
+        "ds_read_b32 %4, %8 offset:%15\n"
+        "ds_read_b32 %5, %9 offset:%16\n"
+        "ds_read_b128 %6, %10 offset:%17\n"
+        "s_waitcnt lgkmcnt(0)"
+        : "=&v"(a[0]), "=&v"(a[1]), "=&v"(a[2]), "=&v"(a[3]), "=&v"(xs), "=&v"(e), "=&v"(ds)
+        : "v"(ia), "v"(ua), "v"(ea), "v"(da), "i"(4096 * kGb), "i"(4096 * kGb + 1024),
+          "i"(4096 * kGb + 2048), "i"(4096 * kGb + 3072), "i"(256 * kGb),
+          "i"(16 * (int)kSliceBlocks * G + 4 * B), "i"(64 * kGb)
+        : "memory");
+  else
+    asm volatile(
+        "ds_read_b128 %0, %6 offset:%9\n"
+        "ds_read_b128 %1, %6 offset:%10\n"
+        "ds_read_b128 %2, %6 offset:%11\n"
+        "ds_read_b128 %3, %6 offset:%12\n"
+        "ds_read_b32 %4, %7 offset:%13\n"
+        "ds_read_b32 %5, %8 offset:%14\n"
+        "s_waitcnt lgkmcnt(0)"
+        : "=&v"(a[0]), "=&v"(a[1]), "=&v"(a[2]), "=&v"(a[3]), "=&v"(xs), "=&v"(e)
+        : "v"(ia), "v"(ua), "v"(ea), "i"(4096 * kGb), "i"(4096 * kGb + 1024),
+          "i"(4096 * kGb + 2048), "i"(4096 * kGb + 3072), "i"(256 * kGb),
+          "i"(16 * (int)kSliceBlocks * G + 4 * B)
+        : "memory");
 }
 
 // One block of the lane's row, decoded: the scaled weights' two digits for
@@ -167,6 +229,7 @@ __global__ __launch_bounds__(WAVES * 64) void q45_tokens_mfma(const uint8_t* __r
                                                               Tok45Args ta) {
   using F = Format<QB>;
   extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
+  constexpr uint32_t kImages = (uint32_t)WAVES * F::kStage;  // after the stage buffers
   constexpr TokLayout L = tok64_layout(kSliceBlocks, NG, true, QB == 5);
   const uint32_t wave = uniform(threadIdx.x >> 6);
   const uint32_t lane = threadIdx.x & 63u;
@@ -174,115 +237,135 @@ __global__ __launch_bounds__(WAVES * 64) void q45_tokens_mfma(const uint8_t* __r
   const uint32_t row_bytes = nb * F::kBytes;
   const uint32_t ntiles = (rows + 15u) / 16u;
   const uint32_t sbase = (uint32_t)(uintptr_t)smem;
+  uint8_t* const wstage = smem + wave * F::kStage;
 
-  // this workgroup's slice k (blocks blk0 .. blk0 + nbl - 1) and its tiles
-  // tg, tg + GS, ...; the wave's are tiles wave, wave + WAVES, ... of those
+  // this workgroup's slice k (blocks blk0 .. blk0 + nbl - 1, nst stages) and
+  // its tiles tg, tg + GS, ...; the wave's are tiles wave, wave + WAVES, ...
   const FastDiv by_gps{ta.groups_per_slice, ta.m_gps};
   const uint32_t k = quo(blockIdx.x, by_gps);
   const uint32_t tg = blockIdx.x - k * ta.groups_per_slice;
   const uint32_t blk0 = kSliceBlocks * k, nbl = min(kSliceBlocks, nb - blk0);
+  const uint32_t nst = (nbl + 1u) / 2u;
   const uint32_t ntw = tg < ntiles ? quo(ntiles - 1u - tg, by_gps) + 1u : 0u;
 
-  // 1. the activations of the wave's image blocks, then the blocks of its
-  //    first tile, into registers
+  // 1. the activations of the wave's image blocks into registers, then the
+  //    copy of its first stage: copy i's slot c = 64 i + lane is piece
+  //    c % kPitch of row c / kPitch, so consecutive lanes read consecutive
+  //    pieces of a row (a row's spare slot re-reads its last piece; rows past
+  //    the matrix read zero)
   constexpr int kShare = (NG * (int)kSliceBlocks + WAVES - 1) / WAVES;
   u32x4 xq[kShare][4];
   load_group_x<WAVES, kShare>(xq, x, nb, blk0, nbl, NG, ntok, wave, lane);
-  const uint32_t row_off = n * row_bytes;
-  const uint32_t qs_off = row_off + F::kBytes - 128u + 32u * grp;
-  auto tile_rsrc = [&](uint32_t lt) {
-    // rows past the matrix read zero
+  uint32_t vo[F::kCopies];
+  copy_offsets<F::kCopies, F::kPitch, F::kPieces>(row_bytes, lane, vo);
+  auto issue = [&](uint32_t lt, uint32_t sl) {
     const uint32_t row0 = (tg + lt * ta.groups_per_slice) * 16u;
     const uint32_t nrows = min(16u, rows - row0);
-    return __builtin_amdgcn_make_buffer_rsrc(
-        const_cast<uint8_t*>(w + (size_t)row0 * row_bytes + F::kBytes * blk0), 0,
-        (int)(nrows * row_bytes - F::kBytes * blk0), kBufferWord3);
-  };
-  Raw45<QB> raw[kSliceBlocks];
-  if (wave < ntw) {
-    const __amdgpu_buffer_rsrc_t rsrc = tile_rsrc(wave);
+    const uint32_t at = F::kBytes * (blk0 + 2u * sl);
+    const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<uint8_t*>(w + (size_t)row0 * row_bytes + at), 0, (int)(nrows * row_bytes - at),
+        kBufferWord3);
 #pragma unroll
-    for (int b = 0; b < (int)kSliceBlocks; ++b)
-      if ((uint32_t)b < nbl) load_block<QB>(raw[b], rsrc, row_off, qs_off, b);
-  }
+    for (int i = 0; i < F::kCopies; ++i) {
+      const uint32_t off = vo[i];
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, (lds_void*)(wstage + 1024 * i), 16, off, 0, 0,
+                                                0);
+    }
+  };
+  if (wave < ntw) issue(wave, 0u);
 
   // 2. the group images (chunk 4 p + j: MFMA j, lane group p)
   build_group_images64<WAVES, kShare, true, QB == 5>(
-      sbase, L, xq, nbl, NG, wave, lane,
+      sbase + kImages, L, xq, nbl, NG, wave, lane,
       [](uint32_t c) { return 1024u * (c & 3u) + 256u * (c >> 2); });
   lds_wait();
   __builtin_amdgcn_s_barrier();
   asm volatile("" ::: "memory");
-
-  // 3. the wave's tiles: lane (grp, n) accumulates, for each group G, vector
-  //    4 G + grp, row n
-  const uint8_t* const img = smem + L.img + 16u * lane;
-  const uint8_t* const usum = smem + L.usum + 4u * lane;
-  const uint8_t* const dsum = smem + L.dsum + 16u * grp;
-  const uint8_t* const expo = smem + L.expo + 16u * grp;
   float side[NG];
 #pragma unroll
-  for (int G = 0; G < NG; ++G) side[G] = slice_err(smem + L.rerr + 64 * G + 16u * grp, nbl);
-  for (uint32_t lt = wave; lt < ntw; lt += WAVES) {
-    const bool more = lt + WAVES < ntw;
-    const __amdgpu_buffer_rsrc_t next = tile_rsrc(more ? lt + WAVES : lt);
-    double acc[NG], sum_abs[NG];
-    bool redo[NG];  // the lane leaves group G's stage to tok_reduce
-    float most = 0.0f;  // bound on the row's |w| over the slice
+  for (int G = 0; G < NG; ++G)
+    side[G] = slice_err(smem + kImages + L.rerr + 64 * G + 16u * grp, nbl);
+
+  // 3. the wave's tiles, stage by stage: lane (grp, n) accumulates, for each
+  //    group G, vector 4 G + grp, row n
+  const uint32_t hb = sbase + wave * F::kStage + 16u * F::kPitch * n;
+  const uint32_t qb = hb + F::kBytes - 128u + 32u * grp;
+  const uint32_t ia0 = sbase + kImages + L.img + 16u * lane;
+  const uint32_t ua0 = sbase + kImages + L.usum + 4u * lane;
+  const uint32_t ea0 = sbase + kImages + L.expo + 16u * grp;
+  const uint32_t da0 = sbase + kImages + L.dsum + 16u * grp;
+  double acc[NG], sum_abs[NG];
+  bool redo[NG];  // the lane leaves group G's slice to tok_reduce
+  float most = 0.0f;  // bound on the row's |w| over the slice
 #pragma unroll
-    for (int G = 0; G < NG; ++G) {
-      acc[G] = sum_abs[G] = 0.0;
-      redo[G] = false;
-    }
-#pragma unroll
-    for (int b = 0; b < (int)kSliceBlocks; ++b) {
-      if ((uint32_t)b >= nbl) continue;
+  for (int G = 0; G < NG; ++G) {
+    acc[G] = sum_abs[G] = 0.0;
+    redo[G] = false;
+  }
+  uint32_t sl = 0u;
+  for (uint32_t lt = wave; lt < ntw;) {
+    __builtin_amdgcn_s_waitcnt(waitcnt_vm(0));
+    Raw45<QB> raw[2];
+    read_stage<QB>(raw, hb, qb);
+    // the stage is in registers: the buffer takes the next one
+    const bool last = sl + 1u == nst;
+    const uint32_t lt_next = last ? lt + WAVES : lt, sl_next = last ? 0u : sl + 1u;
+    if (lt_next < ntw) issue(lt_next, sl_next);
+    const uint32_t ia = ia0 + 8192u * sl, ua = ua0 + 512u * sl, ea = ea0 + 8u * sl,
+                   da = da0 + 128u * sl;
+    static_for<2>([&](auto bc) {
+      constexpr int b = decltype(bc)::value;
+      if (2u * sl + b >= nbl) return;  // (an odd block count's last stage)
       const Block45 bw = decode_block<QB>(raw[b], grp);
       most = fmaxf(most, fmaf(fabsf(bw.df), QB == 5 ? 31.0f * 63.0f : 15.0f * 63.0f,
                               63.0f * fabsf(bw.dminf)));
       const double bd = (double)bw.df, bdmin = (double)bw.dminf;
-      if (more) load_block<QB>(raw[b], next, row_off, qs_off, b);
-#pragma unroll
-      for (int G = 0; G < NG; ++G) {
-        const int gb = G * (int)kSliceBlocks + b;
-        i32x4 c0 = {0, 0, 0, 0};
-        if constexpr (QB == 5) c0 = __builtin_bit_cast(i32x4, lds_u32x4(dsum + 64 * gb));
+      static_for<NG>([&](auto gc) {
+        constexpr int G = decltype(gc)::value;
+        i32x4 a[4], c0 = {0, 0, 0, 0};
+        uint32_t xw;
+        int e;
+        read_group<QB, G, b>(ia, ua, ea, da, a, xw, e, c0);
         i32x4 ch = c0, cl = c0;
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          const i32x4 a = __builtin_bit_cast(i32x4, lds_u32x4(img + 4096 * gb + 1024 * j));
-          ch = __builtin_amdgcn_mfma_i32_16x16x64_i8(a, bw.hi[j], ch, 0, 0, 0);
-          cl = __builtin_amdgcn_mfma_i32_16x16x64_i8(a, bw.lo[j], cl, 0, 0, 0);
-        }
-        const f16x2 xs = __builtin_bit_cast(f16x2, lds_u32(usum + 256 * gb));
+        const f16x2 xs = __builtin_bit_cast(f16x2, xw);
         const f32x4 cm = __builtin_amdgcn_mfma_f32_16x16x16f16(
             f16x4{xs[0], xs[1], (_Float16)0.0f, (_Float16)0.0f}, bw.mins,
             f32x4{0.0f, 0.0f, 0.0f, 0.0f}, 0, 0, 0);
-        const int e = (int)lds_u32(expo + 64 * G + 4 * b);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          ch = __builtin_amdgcn_mfma_i32_16x16x64_i8(a[j], bw.hi[j], ch, 0, 0, 0);
+          cl = __builtin_amdgcn_mfma_i32_16x16x64_i8(a[j], bw.lo[j], cl, 0, 0, 0);
+        }
+        const double m = fma(fma((double)cm[2], 4096.0, (double)cm[1]), 4096.0, (double)cm[0]);
         double t = (double)(8 * ch[3] + cl[3]);
 #pragma unroll
         for (int d = 2; d >= 0; --d) t = fma(t, 256.0, (double)(8 * ch[d] + cl[d]));
-        const double m = fma(fma((double)cm[2], 4096.0, (double)cm[1]), 4096.0, (double)cm[0]);
         t *= bd;
         const double p = fma(-bdmin, m, t);
         redo[G] |= cancels(p, t);
         const double v = __builtin_amdgcn_ldexp(p, e);  // 0 for kBadTok
         acc[G] += v;
         sum_abs[G] += fabs(v);
-      }
-    }
-    const uint32_t row = (tg + lt * ta.groups_per_slice) * 16u + n;
+      });
+    });
+    if (last) {
+      const uint32_t row = (tg + lt * ta.groups_per_slice) * 16u + n;
 #pragma unroll
-    for (int G = 0; G < NG; ++G) {
-      const float part = (float)acc[G];
-      redo[G] |= !(fabsf(part) < __builtin_huge_valf());
-      const float err = most * side[G];
-      redo[G] |= !(err * 1.01f <= kStageTol * ((float)sum_abs[G] - err));
-      const uint32_t v = 4u * G + grp;
-      if (row < rows && v < ntok)
-        part_out[((size_t)k * 4u * NG + v) * rows + row] =
-            redo[G] ? __uint_as_float(kPartRedo) : part;
+      for (int G = 0; G < NG; ++G) {
+        const float part = (float)acc[G], err = most * side[G];
+        const bool bad = redo[G] || !(fabsf(part) < __builtin_huge_valf()) ||
+                         !(err * 1.01f <= kStageTol * ((float)sum_abs[G] - err));
+        const uint32_t v = 4u * G + grp;
+        if (row < rows && v < ntok)
+          part_out[((size_t)k * 4u * NG + v) * rows + row] =
+              bad ? __uint_as_float(kPartRedo) : part;
+        acc[G] = sum_abs[G] = 0.0;
+        redo[G] = false;
+      }
+      most = 0.0f;
     }
+    lt = lt_next;
+    sl = sl_next;
   }
 }
 
@@ -293,8 +376,9 @@ bool launch_tok45(const uint8_t* w, const float* x, float* y, uint32_t rows, uin
   using F = Format<QB>;
   const uint32_t cus = (uint32_t)cu_count();
   const uint32_t slices = (nb + kSliceBlocks - 1u) / kSliceBlocks;
-  constexpr TokLayout L = tok64_layout(kSliceBlocks, NG, true, QB == 5);
-  static_assert(L.total <= kLdsBytes, "the images fit the LDS");
+  constexpr uint32_t kLds =
+      (uint32_t)W * F::kStage + tok64_layout(kSliceBlocks, NG, true, QB == 5).total;
+  static_assert(kLds <= kLdsBytes, "the stage buffers and the images fit the LDS");
   if (slices > cus) return false;
   // the rows of one launch: all, or as many whole tiles as the scratch holds
   const size_t row_part = (size_t)slices * 4u * NG * sizeof(float);
@@ -314,7 +398,7 @@ bool launch_tok45(const uint8_t* w, const float* x, float* y, uint32_t rows, uin
     ta.groups_per_slice = min(cus / slices, (nr + 15u) / 16u);
     ta.m_gps = div_magic(ta.groups_per_slice);
     hipLaunchKernelGGL((q45_tokens_mfma<W, NG, QB>), dim3(ta.groups_per_slice * slices),
-                       dim3(W * 64), L.total, s, wr, x, nr, nb, ntok, ws.scratch, ta);
+                       dim3(W * 64), kLds, s, wr, x, nr, nb, ntok, ws.scratch, ta);
     *err = hipGetLastError();
     if (*err != hipSuccess) break;
     launch_tok_reduce<F::kType>(ws.scratch, y + r0, nr, rows, slices, 4u * NG, ntok, wr, x, nb,
@@ -330,12 +414,11 @@ bool launch_tok45_any(const uint8_t* w, const float* x, float* y, uint32_t rows,
   // Waves, measured (17408 x 5120, us, 12 / 8 waves): Q4_K M = 4 17.8 / 18.5,
   // M = 8 21.2 / 21.3, M = 16 29.6 (spills) / 28.2; Q5_K, whose blocks take
   // more registers, M = 4 21.7 / 21.0, M = 8 26.9 / 25.1.
-  constexpr int kWaves = QB == 5 ? 8 : 12;
-  if (ntok <= 4u) return launch_tok45<kWaves, 1, QB>(w, x, y, rows, nb, ntok, ws, s, err);
-  if (ntok <= 8u) return launch_tok45<kWaves, 2, QB>(w, x, y, rows, nb, ntok, ws, s, err);
-  if (ntok <= 12u)
-    return launch_tok45<QB == 5 ? 8 : 10, 3, QB>(w, x, y, rows, nb, ntok, ws, s, err);
-  return launch_tok45<8, 4, QB>(w, x, y, rows, nb, ntok, ws, s, err);
+  // (8 waves: M = 4 / 16 17.2 / 28.7 us against 16.3 / 26.9; 16 the same)
+  if (ntok <= 4u) return launch_tok45<12, 1, QB>(w, x, y, rows, nb, ntok, ws, s, err);
+  if (ntok <= 8u) return launch_tok45<12, 2, QB>(w, x, y, rows, nb, ntok, ws, s, err);
+  if (ntok <= 12u) return launch_tok45<12, 3, QB>(w, x, y, rows, nb, ntok, ws, s, err);
+  return launch_tok45<12, 4, QB>(w, x, y, rows, nb, ntok, ws, s, err);
 }
 
 }  // namespace

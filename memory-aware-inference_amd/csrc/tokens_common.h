@@ -85,6 +85,18 @@ __device__ __forceinline__ void load_group_x(u32x4 (&xq)[SHARE][4], const float*
   }
 }
 
+// The lane's offsets, from a stage's first row, of the copies that fill PITCH
+// 16-byte slots a row in order (PIECES of them distinct).
+template <int COPIES, uint32_t PITCH, uint32_t PIECES>
+__device__ __forceinline__ void copy_offsets(uint32_t row_bytes, uint32_t lane,
+                                             uint32_t (&vo)[COPIES]) {
+#pragma unroll
+  for (int i = 0; i < COPIES; ++i) {
+    const uint32_t c = min(64u * (uint32_t)i + lane, 16u * PITCH - 1u), row = c / PITCH;
+    vo[i] = row * row_bytes + 16u * min(c - PITCH * row, PIECES - 1u);
+  }
+}
+
 // Sum over a DPP row's 16 lanes (valid in lane 15).
 __device__ __forceinline__ uint32_t row_sum_u(uint32_t v) {
   v += dpp_u<kRowShr1>(v);
