@@ -9,10 +9,10 @@
 // A block with smaller non-zero elements ("side" elements) is a "rounded"
 // block (side count kSideRounded), so that the dot stays within its bar of
 // 2e-5 * sum|w x| for any weights: the side elements stay in the fixed point,
-// rounded like the rest, and the block keeps, per 16-element chunk, the sum
-// of their rounding errors |x_i - X_i 2^(e_b - 30)|.  The kernel bounds a
-// row's error from those blocks by (largest |w| the block header allows) x
-// (that sum), and compares it with the sum of |partial dot| over the row's
+// rounded like the rest, and the block keeps, per 16-element chunk, a bound on
+// the sum of their rounding errors (half a unit 2^(e_b - 30) each).  The kernel
+// bounds a row's error from those blocks by (largest |w| the block header
+// allows) x (that bound), and compares it with the sum of |partial dot| over the row's
 // stage, which is at most sum|w x| over the stage.  A row whose bound exceeds
 // kRoundedTol of it recomputes its rounded blocks exactly.  (The kernels of
 // several vectors build their own images, tokens_common.h.)
@@ -56,7 +56,7 @@ constexpr int kFixBits = 30;
 constexpr uint32_t kLdsBytes = 163840u;
 constexpr int kBadBlock = 0x40000000;  // exponent slot of a block taking the exact path
 // Side elements: non-zero |x| below 2^(e_b - kSideShift).  Each block has
-// kSideBytes of LDS: for a rounded block, 16 f32 error sums, the one of chunk c
+// kSideBytes of LDS: for a rounded block, 16 f32 error bounds, that of chunk c
 // at position 4 p + t for the chunk in MFMA t of lane group p (the four of a
 // lane group side by side).
 constexpr int kSideShift = 14;
@@ -285,99 +285,69 @@ __device__ __forceinline__ void copy_x(uint8_t* smem, uint32_t img, const float*
   }
 }
 
-// The fixed-point split of one lane's 16 activations (a 16-element chunk of a
-// block whose 16 lanes form one DPP row): the row's exponent e (largest |x|
-// below 2^e), the fixed-point values X (two's complement), the mask of side
-// elements, the f32 sum of all 16, the sum of the side elements' rounding
-// errors, and whether the chunk alone forces the exact path.
-struct ChunkSplit {
+// Largest of a DPP row's 16 values, in every lane.
+__device__ __forceinline__ uint32_t row_max_u(uint32_t v) {
+  v = max(v, dpp_u<kRowShr1>(v));
+  v = max(v, dpp_u<kRowShr2>(v));
+  v = max(v, dpp_u<kRowShr4>(v));
+  v = max(v, dpp_u<kRowShr8>(v));
+  return dpp_u<kRowBcast15>(v);
+}
+
+// The fixed point of one lane's 16 activations (f32 bits; a 16-element chunk
+// of a block whose 16 lanes form one DPP row): the block's exponent e (largest
+// |x| below 2^e), whether it must take the exact path (an activation that is
+// not finite or reaches 2^100), the number of the chunk's side elements (each
+// rounded by at most half a unit 2^(e - 30)), the digit bytes dg[quad][digit]
+// and the chunk's digit sums (|.| <= 2^11).  Every workgroup does this for all
+// of x before its first arithmetic, so it is written for few instructions:
+// one pass over the shifted bits finds the maximum and the non-finite values,
+// side elements are only counted, and the sums come from the bytes (v_dot4).
+struct ChunkDigits {
   int e;
-  uint32_t fx[16];
-  uint32_t smask;
-  float xsum, err_side;
   bool bad;
+  uint32_t nside;
+  uint32_t dg[4][4];
+  int sum[4];
 };
-__device__ __forceinline__ ChunkSplit split_chunk(const float (&xv)[16]) {
-  ChunkSplit r;
-  float amax = 0.0f, amin = __builtin_huge_valf();
-  r.xsum = 0.0f;
+template <typename Bits>
+__device__ __forceinline__ ChunkDigits chunk_digits(Bits bits) {
+  ChunkDigits r;
+  uint32_t top = 0u;  // 2 |bits| of the largest |x|
 #pragma unroll
-  for (int k = 0; k < 16; ++k) {
-    amax = fmaxf(amax, fabsf(xv[k]));
-    amin = fminf(amin, fabsf(xv[k]));
-    r.xsum += xv[k];
+  for (int k = 0; k < 16; ++k) top = max(top, bits(k) << 1);
+  top = row_max_u(top);
+  r.bad = top >= 2u * 0x71800000u;  // 2^100 and above, infinities, NaN
+  r.e = __builtin_amdgcn_frexp_expf(__uint_as_float(top >> 1));  // 0 for a block of zeros
+  const uint32_t side = 2u * __float_as_uint(__builtin_amdgcn_ldexpf(1.0f, r.e - kSideShift)) - 2u;
+  r.nside = 0u;
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    uint32_t u[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const uint32_t v = bits(4 * k + j);
+      r.nside += (uint32_t)((v << 1) - 2u < side);  // 0 < |x| < 2^(e - kSideShift)
+      u[j] = (uint32_t)__float2int_rn(
+                 __builtin_amdgcn_ldexpf(__uint_as_float(v), kFixBits - r.e)) +
+             0x80808080u;
+    }
+    transpose_digits(u[0], u[1], u[2], u[3], r.dg[k]);
   }
-  // not finite or huge: a NaN shows in the sum (which cannot overflow below
-  // 2^100), an infinity in the maximum
-  r.bad = !(amax < 0x1p100f) || r.xsum != r.xsum;
-  amax = fmaxf(amax, dpp<kRowShr1>(amax));
-  amax = fmaxf(amax, dpp<kRowShr2>(amax));
-  amax = fmaxf(amax, dpp<kRowShr4>(amax));
-  amax = fmaxf(amax, dpp<kRowShr8>(amax));
-  amax = dpp<kRowBcast15>(amax);
-  r.e = __builtin_amdgcn_frexp_expf(amax);  // amax < 2^e; 0 for amax == 0
-  const float thr = __builtin_amdgcn_ldexpf(1.0f, r.e - kSideShift);
 #pragma unroll
-  for (int k = 0; k < 16; ++k)
-    r.fx[k] = (uint32_t)__float2int_rn(__builtin_amdgcn_ldexpf(xv[k], kFixBits - r.e));
-  r.smask = 0u;
-  r.err_side = 0.0f;
-  // (rare for dense activations: some |x| below the threshold, or a zero).
-  // The empty asm keeps the compiler from hoisting this work above the
-  // branch, into every block's build.
-  if (__builtin_amdgcn_ballot_w64(amin < thr) != 0u) {
-    float xs[16];
-    uint32_t fs[16];
+  for (int d = 0; d < 4; ++d) {
+    r.sum[d] = 0;
 #pragma unroll
-    for (int k = 0; k < 16; ++k) {
-      xs[k] = xv[k];
-      fs[k] = r.fx[k];
-      asm volatile("" : "+v"(xs[k]), "+v"(fs[k]));
-    }
-    // side: 0 < |x| < thr, as integers: bits(|x|) - 1 below bits(thr) - 1
-    const uint32_t tb = __float_as_uint(thr) - 1u;
-#pragma unroll
-    for (int k = 0; k < 16; ++k) {
-      const bool side = ((__float_as_uint(xs[k]) & 0x7fffffffu) - 1u) < tb;
-      r.smask |= (uint32_t)side << k;
-      // |X| < 2^16 for a side element, so (float)X and the difference are exact
-      const float err =
-          fabsf(xs[k] - __builtin_amdgcn_ldexpf((float)(int)fs[k], r.e - kFixBits));
-      r.err_side += side ? err : 0.0f;
-    }
+    for (int k = 0; k < 4; ++k)
+      r.sum[d] = __builtin_amdgcn_sdot4((int)r.dg[k][d], 0x01010101, r.sum[d], false);
   }
   return r;
 }
 
-// The biased digit words of a chunk: X + 0x80808080.
-__device__ __forceinline__ void biased_values(const ChunkSplit& cs, uint32_t (&u)[16]) {
-#pragma unroll
-  for (int k = 0; k < 16; ++k) u[k] = cs.fx[k] + 0x80808080u;
-}
-
-// Sum of the fixed-point values X of a 32-element unit whose two 16-element
-// halves are held by this lane (biased digit words u = X + 0x80808080) and the
-// lane before it in its DPP row; the result is valid in the odd lanes.  The
-// sum is exact (X = hi 2^15 + lo with both parts summed as integers below
-// 2^20, |sum| <= 2^35), so the min term d_min * m * sum X of a unit sees the
-// activations rounded exactly as the MFMA digit sums do.
-__device__ __forceinline__ double unit_fixed_sum(const uint32_t (&u)[16]) {
-  uint32_t hi = 0u, lo = 0u;
-#pragma unroll
-  for (int k = 0; k < 16; ++k) {
-    const int32_t X = (int32_t)(u[k] - 0x80808080u);
-    hi += (uint32_t)(X >> 15);
-    lo += (uint32_t)X & 0x7fffu;
-  }
-  hi += dpp_u<kRowShr1>(hi);
-  lo += dpp_u<kRowShr1>(lo);
-  return fma((double)(int32_t)hi, 32768.0, (double)lo);
-}
-
-// Turns the copied blocks of x into digit images in place, plus exponents, the error sums of rounded blocks, side counts
-// (kSideRounded or 0) and, when the layout keeps them, the sums of each
-// 32-element unit's fixed-point values (unit_fixed_sum, in units of
-// 2^(e_b - 30)).  The caller has waited for the copies.  CHUNK_SLOT(c)
+// Turns the copied blocks of x into digit images in place, plus exponents, the
+// rounded blocks' error bounds, side counts (kSideRounded or 0) and, when the
+// layout keeps them, the exact sums of each 32-element unit's fixed-point
+// values (f64, in units of 2^(e_b - 30)).  The caller has waited for the copies.  CHUNK_SLOT(c)
 // gives the byte offset, inside the block's 1 KB, of the A row 4 p (digit 0)
 // of MFMA t that holds chunk c (elements 16 c .. 16 c + 15): 256 t + 64 p.  A
 // block with an activation that is not finite or reaches 2^100 gets exponent
@@ -396,22 +366,12 @@ __device__ __forceinline__ void build_images(uint32_t sbase, const Layout& L, ui
     const uint32_t pbc = pb < nb ? pb : nb - 1u;  // lanes past K redo the last block, unstored
     u32x4 xq[4];
     lds_read4<16>(sbase + img + 1024u * pbc + 64u * n, xq);
-    float xv[16];
-#pragma unroll
-    for (int k = 0; k < 4; ++k)
-#pragma unroll
-      for (int c = 0; c < 4; ++c) xv[4 * k + c] = __uint_as_float(xq[k][c]);
-    const ChunkSplit cs = split_chunk(xv);
+    const ChunkDigits cd = chunk_digits([&](int k) { return xq[k >> 2][k & 3]; });
     const bool store = pb < nb;
-    const bool bad_blk = (__builtin_amdgcn_ballot_w64(cs.bad) >> (16u * grp)) & 0xffffull;
     const uint32_t list = sbase + sdb + kSideBytes * pb;
     const bool rounded =
-        !bad_blk && ((__builtin_amdgcn_ballot_w64(cs.smask != 0u) >> (16u * grp)) & 0xffffull);
-    uint32_t u[16];
-    biased_values(cs, u);
-    uint32_t dg[4][4];  // [element quad][digit]
-#pragma unroll
-    for (int k = 0; k < 4; ++k) transpose_digits(u[4 * k], u[4 * k + 1], u[4 * k + 2], u[4 * k + 3], dg[k]);
+        !cd.bad && ((__builtin_amdgcn_ballot_w64(cd.nside != 0u) >> (16u * grp)) & 0xffffull);
+    const auto& dg = cd.dg;
     // all lanes of the group have read the block before any lane writes it
     const uint32_t slot = chunk_slot(n);
     const uint32_t ib = sbase + img + 1024u * pbc + slot;
@@ -421,16 +381,20 @@ __device__ __forceinline__ void build_images(uint32_t sbase, const Layout& L, ui
         lds_write_b128(ib + 16u * d, u32x4{dg[0][d], dg[1][d], dg[2][d], dg[3][d]});
       if (rounded)  // position 4 p + t
         lds_write_b32(list + 4u * (4u * ((slot >> 6) & 3u) + (slot >> 8)),
-                      __float_as_uint(cs.err_side));
+                      __float_as_uint(__builtin_amdgcn_ldexpf((float)cd.nside, cd.e - kFixBits - 1)));
     }
     if (L.sums) {
-      const double xsum = unit_fixed_sum(u);  // odd lanes: unit n / 2
+      // unit n / 2, whose two chunks meet in the odd lane: exact
+      int lo = cd.sum[0] + 256 * cd.sum[1], hi = cd.sum[2] + 256 * cd.sum[3];
+      lo += (int)dpp_u<kRowShr1>((uint32_t)lo);
+      hi += (int)dpp_u<kRowShr1>((uint32_t)hi);
+      const double xsum = fma((double)hi, 65536.0, (double)lo);
       if (store && (n & 1u))
         lds_write_b64(sbase + xsb + 64u * pb + 8u * (n >> 1),
                       __builtin_bit_cast(u32x2, xsum));
     }
     if (store && n == 0u) {
-      lds_write_b32(sbase + exb + 4u * pb, (uint32_t)(bad_blk ? kBadBlock : cs.e - kFixBits));
+      lds_write_b32(sbase + exb + 4u * pb, (uint32_t)(cd.bad ? kBadBlock : cd.e - kFixBits));
       lds_write_b8(sbase + exb + count_pos(L, pb), rounded ? kSideRounded : 0u);
     }
   }

@@ -106,14 +106,9 @@ __device__ __forceinline__ uint32_t row_sum_u(uint32_t v) {
 }
 
 // Turns the wave's share of activations (load_group_x) into images, with what
-// else the layout keeps of them: the fixed point of mfma_common.h.  Every
-// workgroup of a slice does this for itself, so it is written for few
-// instructions (about 270 a group-block; with the error sums and unit sums of
-// the one-vector kernels' build 540, a quarter of a sixteen-vector launch):
-// one pass over the shifted bits finds the block's largest |x| and whether
-// an element is not finite, the sums come from the digit bytes (v_dot4), and
-// a side element (0 < |x| < 2^(e - kSideShift)) is only counted, for the bound
-// of half a unit 2^(e - 30) each on its rounding.
+// else the layout keeps of them (chunk_digits: about 270 instructions a
+// group-block; a build that summed the side elements' rounding errors and the
+// units apart took 540, a quarter of a sixteen-vector launch).
 template <int WAVES, int SHARE, bool MINS, bool DSUM, typename ChunkSlot>
 __device__ __forceinline__ void build_group_images64(uint32_t sbase, const TokLayout& L,
                                                      const u32x4 (&xr)[SHARE][4], uint32_t nbl,
@@ -128,46 +123,12 @@ __device__ __forceinline__ void build_group_images64(uint32_t sbase, const TokLa
     const uint32_t gb = L.stride * g + b;
     const uint32_t blk = sbase + L.img + 4096u * gb;
     const uint32_t vec = 4u * L.stride * (4u * g + t) + 4u * b;
-    auto bits = [&](int k) { return xr[i][k >> 2][k & 3]; };
-    uint32_t top = 0u;  // 2 |bits| of the largest |x|, of the chunk, then of the block
-#pragma unroll
-    for (int k = 0; k < 16; ++k) top = max(top, bits(k) << 1);
-    top = max(top, dpp_u<kRowShr1>(top));
-    top = max(top, dpp_u<kRowShr2>(top));
-    top = max(top, dpp_u<kRowShr4>(top));
-    top = max(top, dpp_u<kRowShr8>(top));
-    top = dpp_u<kRowBcast15>(top);
-    const bool bad = top >= 2u * 0x71800000u;  // 2^100 and above, infinities, NaN
-    const int e = __builtin_amdgcn_frexp_expf(__uint_as_float(top >> 1));
-    const uint32_t side = 2u * __float_as_uint(__builtin_amdgcn_ldexpf(1.0f, e - kSideShift)) - 2u;
-    uint32_t nside = 0u;
-    uint32_t dg[4][4];
-#pragma unroll
-    for (int k = 0; k < 4; ++k) {
-      uint32_t u[4];
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const uint32_t v = bits(4 * k + j);
-        nside += (uint32_t)((v << 1) - 2u < side);
-        u[j] = (uint32_t)__float2int_rn(
-                   __builtin_amdgcn_ldexpf(__uint_as_float(v), kFixBits - e)) +
-               0x80808080u;
-      }
-      transpose_digits(u[0], u[1], u[2], u[3], dg[k]);
-    }
+    const ChunkDigits cd = chunk_digits([&](int k) { return xr[i][k >> 2][k & 3]; });
+    const auto& dg = cd.dg;
+    const auto& sum = cd.sum;
 #pragma unroll
     for (int d = 0; d < 4; ++d)
       lds_write_b128(blk + woff + 16u * d, u32x4{dg[0][d], dg[1][d], dg[2][d], dg[3][d]});
-    int sum[4];  // the chunk's digit sums, |.| <= 2^11
-#pragma unroll
-    for (int d = 0; d < 4; ++d) {
-      sum[d] = 0;
-      if constexpr (MINS || DSUM) {
-#pragma unroll
-        for (int k = 0; k < 4; ++k)
-          sum[d] = __builtin_amdgcn_sdot4((int)dg[k][d], 0x01010101, sum[d], false);
-      }
-    }
     if constexpr (MINS) {
       // unit c / 2 (its two chunks meet in the odd lane): X_u = hi 2^16 + lo
       // in 12-bit signed pieces, the last what is left (|X_u| <= 2^35, so at
@@ -197,12 +158,12 @@ __device__ __forceinline__ void build_group_images64(uint32_t sbase, const TokLa
       if (c == 15u)
         lds_write_b128(sbase + L.dsum + 64u * gb + 16u * t, u32x4{s[0], s[1], s[2], s[3]});
     }
-    nside = row_sum_u(nside);
+    const uint32_t nside = row_sum_u(cd.nside);
     if (c == 15u) {
-      lds_write_b32(sbase + L.expo + vec, (uint32_t)(bad ? kBadTok : e - kFixBits));
+      lds_write_b32(sbase + L.expo + vec, (uint32_t)(cd.bad ? kBadTok : cd.e - kFixBits));
       lds_write_b32(sbase + L.rerr + vec,
-                    bad ? 0x7f800000u
-                        : __float_as_uint(__builtin_amdgcn_ldexpf((float)nside, e - kFixBits - 1)));
+                    cd.bad ? 0x7f800000u
+                        : __float_as_uint(__builtin_amdgcn_ldexpf((float)nside, cd.e - kFixBits - 1)));
     }
   }
 }
