@@ -140,7 +140,53 @@ __global__ __launch_bounds__(256) void fused_gate_up_generic_kernel(
   if (lane == 0) h[row] = silu_times(g, u);
 }
 
-// Exact dequantisation of whole blocks: one thread per 32-weight unit.
+// A little-endian word at any alignment.
+__device__ __forceinline__ uint32_t load_word(const uint8_t* p) {
+  uint32_t v;
+  __builtin_memcpy(&v, p, 4);
+  return v;
+}
+
+// The exact values of elements i .. i + 3 (i a multiple of 4) of a block, as
+// decode_unit_exact gives them (quant.rs order).
+template <uint32_t T>
+__device__ __forceinline__ float4 decode_four_exact(const uint8_t* __restrict__ blk, uint32_t i) {
+  float v[4];
+  const uint32_t l = i & 31u;
+  if constexpr (T == kTypeQ4K || T == kTypeQ5K) {
+    const uint32_t unit = i >> 5, s = unit & 3u, dd = load_word(blk);
+    const uint32_t w0 = load_word(blk + 4) >> (8u * s), w1 = load_word(blk + 8) >> (8u * s);
+    const uint32_t w2 = load_word(blk + 12) >> (8u * s);
+    // scale_min_k4 on byte s of the three words
+    const uint32_t sc = unit < 4u ? w0 & 63u : (w2 & 0x0fu) | ((w0 >> 2) & 0x30u);
+    const uint32_t mn = unit < 4u ? w1 & 63u : ((w2 >> 4) & 0x0fu) | ((w1 >> 2) & 0x30u);
+    const float d1 = __fmul_rn(half_bits_to_float_exact(dd & 0xffffu), (float)sc);
+    const float m1 = __fmul_rn(half_bits_to_float_exact(dd >> 16), (float)mn);
+    uint32_t q = (load_word(blk + (T == kTypeQ4K ? 16 : 48) + 32u * (unit >> 1) + l) >>
+                  (4u * (unit & 1u))) & 0x0f0f0f0fu;
+    if constexpr (T == kTypeQ5K) q |= ((load_word(blk + 16 + l) >> unit) & 0x01010101u) << 4;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) v[k] = k4_value_exact(d1, m1, (q >> (8 * k)) & 0xffu);
+  } else {
+    const uint32_t half = i >> 7, quartet = (i >> 5) & 3u;
+    const float d = half_bits_to_float_exact(blk[208] | (blk[209] << 8));
+    const int sc = (int8_t)blk[192 + (i >> 4)];
+    const uint32_t q =
+        ((load_word(blk + 64u * half + 32u * (quartet & 1u) + l) >> (4u * (quartet >> 1))) &
+         0x0f0f0f0fu) |
+        (((load_word(blk + 128u + 32u * half + l) >> (2u * quartet)) & 0x03030303u) << 4);
+#pragma unroll
+    for (int k = 0; k < 4; ++k) v[k] = k6_value_exact(d, sc, (int)((q >> (8 * k)) & 0xffu) - 32);
+  }
+  return make_float4(v[0], v[1], v[2], v[3]);
+}
+
+// Exact dequantisation of whole blocks, four elements a thread, so that a
+// wave's loads are a block's consecutive words and its stores whole lines; a
+// workgroup takes 1024 consecutive elements (chunk blockIdx.x % chunks) of
+// one output row, so the row's index and the division are uniform.  (One
+// 32-weight unit a thread, its bytes loaded one by one and 64-bit divisions
+// per thread: 64 rows of 5120 4.2 us in a graph, near all of it the launch; so 3.9.)
 // `row_index` (optional) maps output row r to source row row_index[r]
 // (the embedding gather); otherwise output row r is source row r.  An index
 // of table_rows or more reads nothing: its output row is NaN and the kernel
@@ -148,36 +194,24 @@ __global__ __launch_bounds__(256) void fused_gate_up_generic_kernel(
 template <uint32_t T>
 __global__ __launch_bounds__(256) void dequant_kernel(const uint8_t* __restrict__ w,
                                                       const uint32_t* __restrict__ row_index,
-                                                      float* __restrict__ out, uint32_t out_rows,
-                                                      uint32_t cols, uint32_t table_rows,
+                                                      float* __restrict__ out, uint32_t nb,
+                                                      uint32_t chunks, uint32_t table_rows,
                                                       void* ws) {
   constexpr uint32_t BB = BlockBytes<T>::value;
-  const uint32_t nb = cols / kBlockElems;
-  const uint64_t units_total = (uint64_t)out_rows * nb * 8u;
-  const uint64_t id = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (id >= units_total) return;
-  const uint32_t r = (uint32_t)(id / ((uint64_t)nb * 8u));
-  const uint32_t rem = (uint32_t)(id % ((uint64_t)nb * 8u));
-  const uint32_t blk = rem >> 3;
-  const uint32_t unit = rem & 7u;
+  const uint32_t r = blockIdx.x / chunks, chunk = blockIdx.x - r * chunks;
+  const uint32_t blk = 4u * chunk + (threadIdx.x >> 6);
+  if (blk >= nb) return;
   const uint64_t src_row = row_index ? row_index[r] : r;
-  float v[32];
+  const uint32_t i = 4u * (threadIdx.x & 63u);
+  float4 v;
   if (src_row < table_rows) {
-    decode_unit_exact<T>(w + (src_row * nb + blk) * BB, unit, v);
+    v = decode_four_exact<T>(w + (src_row * nb + blk) * BB, i);
   } else {
-#pragma unroll
-    for (int i = 0; i < 32; ++i) v[i] = __builtin_nanf("");
-    if (ws && blk == 0u && unit == 0u) report_device_error(ws, kDevErrTokenId);
+    const float nan = __builtin_nanf("");
+    v = make_float4(nan, nan, nan, nan);
+    if (ws && blk == 0u && i == 0u) report_device_error(ws, kDevErrTokenId);
   }
-  uint32_t col0;
-  if constexpr (T == kTypeQ6K) {
-    col0 = blk * 256u + (unit >> 2) * 128u + (unit & 3u) * 32u;
-  } else {
-    col0 = blk * 256u + unit * 32u;
-  }
-  float4* o = reinterpret_cast<float4*>(out + (uint64_t)r * cols + col0);
-#pragma unroll
-  for (int i = 0; i < 8; ++i) o[i] = make_float4(v[4 * i], v[4 * i + 1], v[4 * i + 2], v[4 * i + 3]);
+  *reinterpret_cast<float4*>(out + ((uint64_t)r * nb + blk) * kBlockElems + i) = v;
 }
 
 }  // namespace
@@ -238,20 +272,30 @@ hipError_t launch_fused_gate_up_generic(const uint8_t* gate, const uint8_t* up, 
 hipError_t launch_dequant(uint32_t type, const uint8_t* w, const uint32_t* row_index, float* out,
                           uint32_t out_rows, uint32_t cols, hipStream_t s, uint32_t table_rows,
                           void* ws) {
-  const uint64_t units = (uint64_t)out_rows * (cols / kBlockElems) * 8u;
-  const dim3 grid((uint32_t)((units + 255) / 256));
+  // without an index the rows follow each other: one row of all their blocks
+  uint64_t nb = cols / kBlockElems, nrows = out_rows;
+  if (row_index == nullptr) {
+    nb *= nrows;
+    nrows = 1u;
+    table_rows = 1u;
+  }
+  const uint64_t groups = nrows * ((nb + 3u) / 4u);
+  if (nb == 0u || nb > 0xfffffffcu || groups == 0u || groups > 0x7fffffffu)
+    return hipErrorInvalidValue;
+  const uint32_t chunks = (uint32_t)((nb + 3u) / 4u);
+  const dim3 grid((uint32_t)groups);
   switch (type) {
     case kTypeQ4K:
       hipLaunchKernelGGL(dequant_kernel<kTypeQ4K>, grid, dim3(256), 0, s, w, row_index, out,
-                         out_rows, cols, table_rows, ws);
+                         (uint32_t)nb, chunks, table_rows, ws);
       break;
     case kTypeQ5K:
       hipLaunchKernelGGL(dequant_kernel<kTypeQ5K>, grid, dim3(256), 0, s, w, row_index, out,
-                         out_rows, cols, table_rows, ws);
+                         (uint32_t)nb, chunks, table_rows, ws);
       break;
     case kTypeQ6K:
       hipLaunchKernelGGL(dequant_kernel<kTypeQ6K>, grid, dim3(256), 0, s, w, row_index, out,
-                         out_rows, cols, table_rows, ws);
+                         (uint32_t)nb, chunks, table_rows, ws);
       break;
     default:
       return hipErrorInvalidValue;

@@ -90,6 +90,26 @@ SHAPES = [(1, 256), (7, 512), (64, 1024), (40, 2304), (300, 5120), (48, 5376), (
 
 
 @pytest.mark.parametrize("t", [12, 13, 14])
+@pytest.mark.parametrize("nb", [1, 2, 3, 4, 5, 7])
+def test_dequantize_partial_workgroups(hip_ctx, t, nb):
+    """Block counts around a workgroup's four, and embedding rows of as many
+    blocks gathered out of order with repeats (Q4_K)."""
+    row = nb * si_hip.BLOCK_BYTES[t]
+    raw = np.random.default_rng(60 * t + nb).integers(0, 256, 9 * row, dtype=np.uint8).tobytes()
+    assert same_bits(hip_ctx.dequantize(t, raw[:row], nb * 256),
+                     O.dequantize(t, raw[:row], nb * 256))
+    if t == 12:
+        ids = np.array([8, 0, 3, 3, 7, 8, 1], dtype=np.uint32)
+        T = hip_ctx.upload_quant_weight_private(raw, 12)
+        try:
+            got = hip_ctx.q4_k_embedding_tokens(T, (nb * 256, 9), ids)
+            for g, i in zip(np.asarray(got).reshape(len(ids), -1), ids):
+                assert same_bits(g, O.dequantize(12, raw[i * row:(i + 1) * row], nb * 256))
+        finally:
+            T.free()
+
+
+@pytest.mark.parametrize("t", [12, 13, 14])
 @pytest.mark.parametrize("rows,cols", SHAPES)
 def test_matvec_within_tolerance(ctx, t, rows, cols):
     log(f"matvec t={t} {rows}x{cols}")
