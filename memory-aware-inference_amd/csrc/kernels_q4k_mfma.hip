@@ -870,7 +870,7 @@ __global__ __launch_bounds__(WAVES * 64) void q4k_matvec_mfma(const uint8_t* __r
     if constexpr (SLICED)
       hand_off_slice(sbase, L, ss, pr, rowsum, lane, rows, y, ws, fail);
     else
-      hand_off<MATS>(sbase, L, slots, sc, sa, pr, nstages, rowsum, lane, rows, y, ws, fail);
+      hand_off<MATS>(sbase, L, slots, sc, pr, nstages, rowsum, lane, rows, y, ws, fail);
   }
   if (fail != 0u) report_device_error(wsp, fail);
 }
@@ -971,7 +971,7 @@ bool launch_sliced(const uint8_t* w, const float* x, float* y, uint32_t rows, ui
 uint64_t busiest_pairs(uint32_t ntiles, uint32_t tparts, uint32_t waves, size_t ws_bytes) {
   const LaunchShape ls = launch_shape(ntiles, tparts, waves, ws_bytes, 1u);
   const uint64_t g = ls.groups, q = ntiles / g, lp = (ntiles - q * g) * (uint64_t)tparts;
-  return ls.split ? q * tparts + (lp + g - 1u) / g : (ntiles + g - 1u) / g * tparts;
+  return ls.width != 0u ? q * tparts + (lp + g - 1u) / g : (ntiles + g - 1u) / g * tparts;
 }
 
 // Whether an unsliced one-vector launch of W waves and SB-block stages fits

@@ -484,7 +484,7 @@ __global__ __launch_bounds__(WAVES * 64) void q6k_matvec_mfma(const uint8_t* __r
       if constexpr (SLICED)
         hand_off_slice<true>(sbase, L, ss, pr, ra, lane, rows, y, ws, fail, rb);
       else
-        hand_off<1, ARGMAX, true>(sbase, L, slots, sc, sa, pr, nstages, ra, lane, rows, y, ws,
+        hand_off<1, ARGMAX, true>(sbase, L, slots, sc, pr, nstages, ra, lane, rows, y, ws,
                                   fail, &best, aa.rule, rb);
       continue;
     }
@@ -496,7 +496,7 @@ __global__ __launch_bounds__(WAVES * 64) void q6k_matvec_mfma(const uint8_t* __r
     if constexpr (SLICED)
       hand_off_slice(sbase, L, ss, pr, rowsum, lane, rows, y, ws, fail);
     else
-      hand_off<1, ARGMAX>(sbase, L, slots, sc, sa, pr, nstages, rowsum, lane, rows, y, ws, fail,
+      hand_off<1, ARGMAX>(sbase, L, slots, sc, pr, nstages, rowsum, lane, rows, y, ws, fail,
                           &best, aa.rule);
   }
   if (fail != 0u) report_device_error(wsp, fail);
@@ -852,7 +852,7 @@ uint32_t q6_slices(uint32_t ntiles, uint32_t nb, size_t ws_bytes) {
   const LaunchShape ls = launch_shape(ntiles, nst, 12u, ws_bytes, 1u);
   const uint64_t g1 = ls.groups;
   const uint64_t q = ntiles / g1, lp = (ntiles - q * g1) * nst;
-  const uint64_t most0 = ls.split ? q * nst + (lp + g1 - 1u) / g1 : (ntiles + g1 - 1u) / g1 * nst;
+  const uint64_t most0 = ls.width != 0u ? q * nst + (lp + g1 - 1u) / g1 : (ntiles + g1 - 1u) / g1 * nst;
   auto most = [&](uint32_t S) {  // the busiest sliced workgroup's pairs
     const uint64_t gs = std::min<uint64_t>(ntiles, cus / S);
     return (ntiles + gs - 1u) / gs * ((nst + S - 1u) / S);

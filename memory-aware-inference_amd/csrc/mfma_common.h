@@ -528,10 +528,11 @@ __device__ __forceinline__ uint32_t quo(uint32_t x, const FastDiv& f) {
 }
 
 // The launch constants of the work split below, one kernel argument: the ring
-// slot count (bits 0-7), the split flag (bit 8) and the workgroup count G
-// (bits 16-31), then the division constants of G, the partials per tile and
-// the slot count.  Kept to 16 bytes so a kernel's arguments stay within the
-// first 64-byte line of its argument block (one memory round trip).
+// slot count (bits 0-7), the split width (bits 8-15; 0: no tile is split) and
+// the workgroup count G (bits 16-31), then the division constants of G, the
+// partials per tile and the slot count.  Kept to 16 bytes so a kernel's
+// arguments stay within the first 64-byte line of its argument block (one
+// memory round trip).
 struct SchedArgs {
   uint32_t packed;
   uint32_t m_groups, m_parts, m_slots;
@@ -566,19 +567,21 @@ __device__ __forceinline__ void load_group_args_early(const GroupArgs& ga) {
 // round of pairs more than others (rounds = pairs / waves, rounded up), the
 // launch "splits": workgroup g keeps q = T / G whole tiles g, g + G, ...,
 // g + (q - 1) G, and the L = (T - q G) S pairs of the leftover tiles are cut
-// into G contiguous ranges, so every workgroup gets the same number of pairs
-// to within one.  A leftover tile whose pairs fall into two or more ranges is
-// "split": each of its workgroups sums its own partials, publishes them in a
-// small global workspace and counts them on the tile's global counter; the
-// workgroup that completes the count adds the published sums in workgroup
-// order and stores the rows (deterministic for a given grid).  That exchange
-// costs a wave a few microseconds of waiting, so the leftover pairs go to the
-// last waves of the first round -- waves with a pair less than the others --
-// when the ring has a slot for every tile of the workgroup (tiles are then
-// not taken in slot order), and first otherwise.
+// into contiguous ranges of X pairs, one for each of the first ceil(L / X)
+// workgroups (launch_shape picks X).  (Ranges of X and X - 1 pairs over all G
+// workgroups cost more to work out than the evener shares give: 4096 x 5120
+// Q4_K 6.15 us, so 6.35; 17408 x 5120 12.5 both.)  A leftover tile whose pairs fall into
+// two or more ranges is "split": each of its workgroups sums its own partials,
+// publishes them in a small global workspace and counts them on the tile's
+// global counter; the workgroup that completes the count adds the published
+// sums in workgroup order and stores the rows (deterministic for a given
+// grid).  That exchange costs a wave a few microseconds of waiting, so the
+// leftover pairs go to the last waves of the first round -- waves with a pair
+// less than the others -- when the ring has a slot for every tile of the
+// workgroup (tiles are then not taken in slot order), and first otherwise.
 struct Sched {
   uint32_t a, b;        // [a, b): this workgroup's leftover pairs
-  uint32_t lpairs;      // L
+  uint32_t width;       // X
   uint32_t split_base;  // first leftover tile, q G
   uint32_t nsplit;      // leftover tiles this workgroup touches
   uint32_t nwhole;      // whole tiles g + G t, t < nwhole (g = blockIdx.x)
@@ -588,41 +591,33 @@ struct Sched {
   FastDiv by_parts, by_slots;
   uint32_t t_a;         // first leftover tile index (a / parts)
 };
-// First leftover pair of workgroup g: floor(g L / G).
-__device__ __forceinline__ uint32_t range_start(uint32_t g, uint32_t lpairs,
-                                                const FastDiv& by_groups) {
-  return quo(g * lpairs, by_groups);
+// First leftover pair of workgroup g.
+__device__ __forceinline__ uint32_t range_start(uint32_t g, uint32_t lpairs, uint32_t width) {
+  return min(g * width, lpairs);
 }
-// (the division constant of G is taken from the kernel argument where it is
-// needed rather than kept in the schedule, which would hold a scalar register
-// through the whole kernel)
-__device__ __forceinline__ uint32_t range_start(const Sched& s, const SchedArgs& sa, uint32_t g) {
-  return range_start(g, s.lpairs, FastDiv{s.groups, sa.m_groups});
-}
-// The workgroup whose range holds leftover pair p (p < L), i.e. the g with
-// range_start(g) <= p < range_start(g + 1): p G / L in floating point (with
-// the approximate reciprocal) is within one or two of it, and the loops
+// The workgroup whose range holds leftover pair p (p < L), p / X: in floating
+// point (with the approximate reciprocal) it is within one, and the loops
 // settle the rest.
-__device__ __forceinline__ uint32_t range_of(const Sched& s, const SchedArgs& sa, uint32_t p) {
-  const uint32_t G = s.groups;
-  uint32_t g = min((uint32_t)((float)p * (float)G * __builtin_amdgcn_rcpf((float)s.lpairs)), G - 1u);
-  while (g > 0u && range_start(s, sa, g) > p) --g;
-  while (g + 1u < G && range_start(s, sa, g + 1u) <= p) ++g;
+__device__ __forceinline__ uint32_t range_of(const Sched& s, uint32_t p) {
+  uint32_t g = (uint32_t)((float)p * __builtin_amdgcn_rcpf((float)s.width));
+  while (g * s.width > p) --g;
+  while ((g + 1u) * s.width <= p) ++g;
   return g;
 }
 __device__ __forceinline__ Sched make_sched(uint32_t ntiles, uint32_t tparts, uint32_t waves,
                                             const SchedArgs& sa) {
   Sched s;
   const uint32_t G = sa.packed >> 16, g = blockIdx.x, slots = sa.packed & 0xffu;
-  const bool split = (sa.packed & 0x100u) != 0u;
+  const uint32_t width = (sa.packed >> 8) & 0xffu;
+  const bool split = width != 0u;
   const FastDiv by_parts{tparts, sa.m_parts}, by_groups{G, sa.m_groups};
   // (plain locals first: the struct is filled in once at the end)
   const uint32_t nwhole = split ? quo(ntiles, by_groups)
                                 : (g < ntiles ? quo(ntiles - 1u - g, by_groups) + 1u : 0u);
   const uint32_t split_base = split ? nwhole * G : ntiles;
   const uint32_t lpairs = split ? (ntiles - split_base) * tparts : 0u;
-  const uint32_t a = split ? range_start(g, lpairs, by_groups) : 0u;
-  const uint32_t b = split ? range_start(g + 1u, lpairs, by_groups) : 0u;
+  const uint32_t a = range_start(g, lpairs, width);
+  const uint32_t b = range_start(g + 1u, lpairs, width);
   const uint32_t t_a = quo(a, by_parts);
   s.by_parts = by_parts;
   s.by_slots = FastDiv{slots, sa.m_slots};
@@ -630,7 +625,7 @@ __device__ __forceinline__ Sched make_sched(uint32_t ntiles, uint32_t tparts, ui
   s.slack0 = 0u;
   s.nwhole = nwhole;
   s.split_base = split_base;
-  s.lpairs = lpairs;
+  s.width = width;
   s.a = a;
   s.b = b;
   s.t_a = t_a;
@@ -733,8 +728,7 @@ __device__ __forceinline__ void wait_slot(uint32_t owner_at, uint32_t lt, uint32
 // 2 r + 1 at partial nparts + pr.r; the two sums are added and stored apart.
 template <int MATS, bool ARGMAX = false, bool PAIRED = false>
 __device__ __forceinline__ void hand_off(uint32_t sbase, const Layout& L, uint32_t slots,
-                                         const Sched& sc, const SchedArgs& sa, const Pair& pr,
-                                         uint32_t nparts,
+                                         const Sched& sc, const Pair& pr, uint32_t nparts,
                                          float rowsum, uint32_t lane, uint32_t rows,
                                          float* __restrict__ y, SplitWs ws, uint32_t& fail,
                                          uint64_t* best = nullptr, uint32_t rule = 0u,
@@ -813,16 +807,14 @@ __device__ __forceinline__ void hand_off(uint32_t sbase, const Layout& L, uint32
       store_coherent(ws.part + (e * kSums) * 16u + n, sum);
       if (kTwo) store_coherent(ws.part + (e * kSums + 1u) * 16u + n, sum2);
     }
-    const uint32_t g0 = range_of(sc, sa, t * tparts);
-    const uint32_t g1 = range_of(sc, sa, t * tparts + tparts - 1u);
+    const uint32_t g0 = range_of(sc, t * tparts);
+    const uint32_t g1 = range_of(sc, t * tparts + tparts - 1u);
     // float offset of share wg's entry for this tile in ws.part, or kNoEntry
     // when wg holds none of its pairs
     constexpr uint32_t kNoEntry = 0xffffffffu;
     auto entry = [&](uint32_t wg) -> uint32_t {
       if (wg > g1) return kNoEntry;
-      const uint32_t wa = range_start(sc, sa, wg);
-      if (wa == range_start(sc, sa, wg + 1u)) return kNoEntry;  // no leftover pairs
-      const uint32_t t0 = quo(wa, sc.by_parts);
+      const uint32_t t0 = quo(wg * sc.width, sc.by_parts);
       return (2u * wg + (t == t0 ? 0u : 1u)) * kSums * 16u + n;
     };
     // this workgroup's own share is taken from registers, not read back
@@ -1112,7 +1104,7 @@ inline int cu_count() {
 // least three rounds), and the most tiles one workgroup touches.
 struct LaunchShape {
   uint32_t groups;
-  bool split;
+  uint32_t width;  // pairs in a leftover range, 0: no tile is split
   uint32_t tiles_per_group;
 };
 // Pair and tile indices divided with FastDiv stay below ntiles * tparts and
@@ -1135,12 +1127,27 @@ inline LaunchShape launch_shape(uint32_t ntiles, uint32_t tparts, uint32_t waves
   const uint64_t lpairs = (uint64_t)(ntiles - q * g1) * tparts;
   const uint64_t most = (uint64_t)q * tparts + (lpairs + g1 - 1u) / g1;
   const uint64_t rounds1 = (most + waves - 1u) / waves;
+  // The width of the leftover ranges: an eighth of a tile, within the rounds
+  // that the narrowest ranges (every workgroup's share equal) take.  The
+  // workgroup that completes a tile reads its shares four at a time, about a
+  // microsecond a batch: with one leftover tile over all workgroups Q6_K
+  // 8210 x 11008 took 63.1 us (so 36.9), 4112 x 14336 43.1 (16.7), Q4_K
+  // 8208 x 16384 46.5 (23.8), 4112 x 5120 7.3 (7.0).
+  const uint64_t narrow = (lpairs + g1 - 1u) / g1;
+  const uint64_t width =
+      q == 0u ? narrow
+              : max(narrow, min(((uint64_t)tparts + 7u) / 8u, rounds1 * waves - (uint64_t)q * tparts));
   // the cross-workgroup exchange costs about a round in a short launch, so
   // split only launches of three or more rounds
-  ls.split = rounds1 < rounds0 && rounds0 >= 3u && split_ws_fits(ws_bytes, g1, ntiles, mats);
-  ls.groups = ls.split ? g1 : g0;
-  ls.tiles_per_group = ls.split ? q + (uint32_t)(((lpairs + g1 - 1u) / g1 + tparts - 1u) / tparts) + 1u
-                                : (ntiles + g0 - 1u) / g0;
+  const bool split = rounds1 < rounds0 && rounds0 >= 3u && width <= 0xffu &&
+                     split_ws_fits(ws_bytes, g1, ntiles, mats);
+  // (without a whole tile each, only the workgroups with a range)
+  ls.groups = !split ? g0 : (q == 0u ? (uint32_t)((lpairs + width - 1u) / width) : g1);
+  ls.width = split ? (uint32_t)width : 0u;
+  // (a range of X > 1 pairs touches a tile more than its whole ones hold)
+  ls.tiles_per_group =
+      split ? q + min(ntiles - q * g1, (uint32_t)((width + tparts - 2u) / tparts) + 1u)
+            : (ntiles + g0 - 1u) / g0;
   return ls;
 }
 
@@ -1152,11 +1159,7 @@ inline bool make_sched_args(uint32_t ntiles, uint32_t tparts, uint32_t slots,
   const uint64_t G = ls.groups;
   if (G == 0u || G > 0xffffu || slots == 0u || slots > 0xffu) return false;
   if ((uint64_t)ntiles * G >= (1ull << 32)) return false;  // tile / G quotients
-  if (ls.split) {
-    const uint64_t lpairs = (uint64_t)(ntiles - ntiles / ls.groups * ls.groups) * tparts;
-    if (lpairs * G * G >= (1ull << 32)) return false;  // range starts: (g + 1) L / G
-  }
-  out->packed = (uint32_t)(G << 16) | (ls.split ? 0x100u : 0u) | slots;
+  out->packed = (uint32_t)(G << 16) | (ls.width << 8) | slots;
   out->m_groups = div_magic((uint32_t)G);
   out->m_parts = div_magic(tparts);
   out->m_slots = div_magic(slots);
