@@ -235,7 +235,36 @@ __device__ __forceinline__ float q6_bound(const int (&sc)[4], float d) {
 // stages and their copies are the even case's.  Block b of a launch row
 // meets x block b mod nr (x sits twice in the image area); the sums of its
 // blocks b < nr go to y[2 r] and the rest to y[2 r + 1], the stage that
-// holds blocks nr - 1 and nr handing one sum to each.
+// holds blocks nr - 1 and nr handing one sum to each.  A workgroup past those
+// of the schedule takes the last row of an odd row count, alone, on the exact
+// per-weight path (the launch then leaves it a CU): as a launch of its own that
+// row took 4097 x 11008 to 20.5 us, here it takes 16.0.
+
+// y[0] = the dot of one row (w: its nr blocks) with x, by a whole workgroup:
+// thread t decodes units t, t + 64 WAVES, ... as quant.rs does.
+template <int WAVES>
+__device__ __forceinline__ void last_row_dot(const uint8_t* __restrict__ w,
+                                             const float* __restrict__ x, float* __restrict__ y,
+                                             uint32_t nr, uint8_t* smem) {
+  float acc = 0.0f;
+  for (uint32_t u = threadIdx.x; u < 8u * nr; u += 64u * WAVES) {
+    float v[32];
+    decode_unit_exact<kTypeQ6K>(w + (size_t)(u >> 3) * kQ6Bytes, u & 7u, v);
+    const float* const xu = x + 32u * (size_t)u;
+#pragma unroll
+    for (int i = 0; i < 32; ++i) acc = fmaf(v[i], xu[i], acc);
+  }
+#pragma unroll
+  for (int h = 32; h > 0; h >>= 1) acc += __shfl_xor(acc, h, 64);
+  float* const part = reinterpret_cast<float*>(smem);
+  if ((threadIdx.x & 63u) == 0u) part[threadIdx.x >> 6] = acc;
+  __syncthreads();
+  if (threadIdx.x == 0u) {
+    for (int k = 1; k < WAVES; ++k) acc += part[k];
+    y[0] = acc;
+  }
+}
+
 struct ArgmaxArgs {
   uint64_t* result;
   uint32_t rule;
@@ -255,6 +284,13 @@ __global__ __launch_bounds__(WAVES * 64) void q6k_matvec_mfma(const uint8_t* __r
   static_assert(!(PAIRED && SLICED && ARGMAX), "sliced row pairs: no argmax");
   extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
   if constexpr (GROUPED) load_group_args_early(ga);
+  if constexpr (PAIRED && !ARGMAX) {
+    if (blockIdx.x >= (SLICED ? sla.slices * sla.tgroups : sa.packed >> 16)) {
+      last_row_dot<WAVES>(w + (size_t)rows * nb * kQ6Bytes, x, y + 2u * (size_t)rows, nb / 2u,
+                          smem);
+      return;
+    }
+  }
   const uint32_t slots = sa.packed & 0xffu;
   const uint32_t ntiles = (rows + 15u) / 16u;
   const uint32_t nstages = (nb + 1u) / 2u;
@@ -744,10 +780,12 @@ __global__ __launch_bounds__(WAVES * 64) void q6k_tokens_mfma(const uint8_t* __r
 template <int W, int D, bool G = false, bool AM = false, bool P = false>
 bool launch_wd(const uint8_t* w, const float* x, float* y, uint32_t rows, uint32_t nb,
                const Workspace& ws, hipStream_t s, hipError_t* err,
-               const GroupArgs& ga = GroupArgs{}, const ArgmaxArgs& aa = ArgmaxArgs{}) {
+               const GroupArgs& ga = GroupArgs{}, const ArgmaxArgs& aa = ArgmaxArgs{},
+               bool last_row = false) {
   const uint32_t ntiles = (rows + 15u) / 16u;
   const uint32_t nstages = (nb + 1u) / 2u;
-  const LaunchShape ls = launch_shape(ntiles, nstages, W, ws.bytes, P ? 2u : 1u);
+  const LaunchShape ls = launch_shape(ntiles, nstages, W, ws.bytes, P ? 2u : 1u,
+                                      (uint32_t)cu_count() - (last_row ? 1u : 0u));
   const uint32_t grid = ls.groups;
   const uint32_t slots = ring_slots(W, D, ls.tiles_per_group, P ? 2u * nstages : nstages);
   // One pair touched ahead pays where the image build is long (the 68-block
@@ -769,9 +807,9 @@ bool launch_wd(const uint8_t* w, const float* x, float* y, uint32_t rows, uint32
     *err = attr;
     return true;
   }
-  hipLaunchKernelGGL((q6k_matvec_mfma<W, D, G, AM, false, P>), dim3(grid), dim3(W * 64), lds,
-                     s, w, x, y, rows, nb, ws.ptr, sa, D == 1 ? prefetch : 0u, ga, aa,
-                     SliceArgs{});
+  hipLaunchKernelGGL((q6k_matvec_mfma<W, D, G, AM, false, P>),
+                     dim3(grid + (last_row ? 1u : 0u)), dim3(W * 64), lds, s, w, x, y, rows, nb,
+                     ws.ptr, sa, D == 1 ? prefetch : 0u, ga, aa, SliceArgs{});
   *err = hipGetLastError();
   return true;
 }
@@ -780,7 +818,8 @@ bool launch_wd(const uint8_t* w, const float* x, float* y, uint32_t rows, uint32
 // P: row pairs, rows and nb being the pairs' (rows / 2 rows of 2 nr blocks).
 template <int W, int D, bool P = false>
 bool launch_sliced(const uint8_t* w, const float* x, float* y, uint32_t rows, uint32_t nb,
-                   uint32_t S, const Workspace& ws, hipStream_t s, hipError_t* err) {
+                   uint32_t S, const Workspace& ws, hipStream_t s, hipError_t* err,
+                   bool last_row = false) {
   const uint32_t ntiles = (rows + 15u) / 16u;
   const uint32_t nstages = nb / 2u;
   // even nb (4-byte aligned rows and stages); in-tile offsets (16 rows) and
@@ -788,7 +827,8 @@ bool launch_sliced(const uint8_t* w, const float* x, float* y, uint32_t rows, ui
   if (rows == 0u || nb == 0u || (nb & 1u) != 0u || (uint64_t)nb * kQ6Bytes * 16u > 0x7fffffffu)
     return false;
   SliceShape sh;
-  if (!slice_shape(ntiles, nstages, S, (uint32_t)cu_count(), ws.bytes, &sh, P ? 128u : 64u))
+  if (!slice_shape(ntiles, nstages, S, (uint32_t)cu_count() - (last_row ? 1u : 0u), ws.bytes, &sh,
+                   P ? 128u : 64u))
     return false;
   if (2u * sh.ns_max > kMaxMetaBlocks) return false;
   const uint32_t slots = ring_slots(W, D, sh.tiles_per_group, sh.ns_max);
@@ -807,8 +847,8 @@ bool launch_sliced(const uint8_t* w, const float* x, float* y, uint32_t rows, ui
     *err = attr;
     return true;
   }
-  hipLaunchKernelGGL((q6k_matvec_mfma<W, D, false, false, true, P>), dim3(sh.groups), dim3(W * 64),
-                     lds, s, w, x, y, rows, nb, ws.ptr, sa, prefetch, GroupArgs{}, ArgmaxArgs{},
+  hipLaunchKernelGGL((q6k_matvec_mfma<W, D, false, false, true, P>),
+                     dim3(sh.groups + (last_row ? 1u : 0u)), dim3(W * 64), lds, s, w, x, y, rows, nb, ws.ptr, sa, prefetch, GroupArgs{}, ArgmaxArgs{},
                      sh.args);
   *err = hipGetLastError();
   return true;
@@ -829,39 +869,52 @@ bool launch_sliced(const uint8_t* w, const float* x, float* y, uint32_t rows, ui
 //   8192 x 28672       57.0     52.4    56.0
 //   2048 x 32768       50.4     20.2
 //   2560 x 9728         9.5              9.7
-// So: four slices when the unsliced launch's busiest workgroup has at most
-// two rounds of pairs (24; its build is then exposed) and slicing adds it
-// none or the rows are long (48 blocks or more); with more pairs, only when
-// the unsliced images leave room for fewer than eight waves (very long
-// rows), in the fewest slices that add no pairs to the busiest workgroup.
-uint32_t q6_slices(uint32_t ntiles, uint32_t nb, size_t ws_bytes) {
+// and, rows of odd block counts taken as pairs (S = 2 / 3 / 4, four waves
+// unsliced): 4096 x 11008 13.8 / 16.0 / 14.6, 2047 x 11008 12.1 / 9.9 / 12.6,
+// 8192 x 11008 22.4 / 26.0 / 22.1 (unsliced 64), 4097 x 17152 - / 21.9 / 23.6;
+// 2560 x 17408 S = 3 / 4 14.4 / 14.9, 1360 x 17408 9.4 / 10.1.
+// So: four slices, or three where that leaves the busiest workgroup fewer
+// pairs, when the unsliced launch's busiest workgroup has at most two rounds
+// of pairs (24; its build is then exposed) and slicing adds it none or the
+// rows are long (48 blocks or more); with more pairs, only when the unsliced
+// images leave room for fewer than eight waves (very long rows), in the
+// number of two to four that gives the busiest workgroup the fewest.
+uint32_t q6_slices(uint32_t ntiles, uint32_t nb, size_t ws_bytes, bool pairs = false,
+                   uint64_t cus = (uint64_t)cu_count()) {
   static const int env = env_int("SI_HIP_Q6K_SLICES", -1);
   if (env >= 0) return (uint32_t)env;
   const uint32_t nst = nb / 2u;
   if (nst < 16u) return 0u;
-  const uint64_t cus = (uint64_t)cu_count();
+  auto most = [&](uint32_t S) {  // the busiest sliced workgroup's pairs
+    const uint64_t gs = std::min<uint64_t>(ntiles, cus / S);
+    return (ntiles + gs - 1u) / gs * ((nst + S - 1u) / S);
+  };
   if (nb > kMaxMetaBlocks) {
     // rows longer than the unsliced kernel takes must slice: the fewest
     // slices (from four) whose images (64 blocks at most) leave the stage
     // buffers of 12 waves room in the LDS
     uint32_t S = 4u;
     while (S < 64u && S < cus && (nst + S - 1u) / S > 32u) S *= 2u;
-    return S;
+    return S == 4u && cus >= 4u && (nst + 2u) / 3u <= 32u && most(3u) < most(4u) ? 3u : S;
   }
   // the unsliced launch's busiest workgroup (launch_shape's choice at 12 waves)
-  const LaunchShape ls = launch_shape(ntiles, nst, 12u, ws_bytes, 1u);
+  const LaunchShape ls = launch_shape(ntiles, nst, 12u, ws_bytes, 1u, (uint32_t)cus);
   const uint64_t g1 = ls.groups;
   const uint64_t q = ntiles / g1, lp = (ntiles - q * g1) * nst;
   const uint64_t most0 = ls.width != 0u ? q * nst + (lp + g1 - 1u) / g1 : (ntiles + g1 - 1u) / g1 * nst;
-  auto most = [&](uint32_t S) {  // the busiest sliced workgroup's pairs
-    const uint64_t gs = std::min<uint64_t>(ntiles, cus / S);
-    return (ntiles + gs - 1u) / gs * ((nst + S - 1u) / S);
-  };
-  if (most0 <= 24u) return most(4u) <= most0 || nb >= 48u ? 4u : 0u;
-  if (layout(8u, 1u, nb, 2u).total <= kLdsBytes) return 0u;
-  for (uint32_t S : {2u, 4u})
-    if (most(S) <= most0) return S;
-  return 0u;
+  if (cus < 4u) return 0u;
+  if (most0 <= 24u) {
+    const uint32_t S = most(3u) < most(4u) ? 3u : 4u;
+    return most(S) <= most0 || nb >= 48u ? S : 0u;
+  }
+  const uint32_t slots =
+      ring_slots(8u, 1u, launch_shape(ntiles, nst, 8u, ws_bytes, 1u, (uint32_t)cus).tiles_per_group,
+                 pairs ? 2u * nst : nst);
+  if (layout(8u, 1u, nb, slots, pairs ? 2u : 1u).total <= kLdsBytes) return 0u;
+  uint32_t best = 2u;
+  for (uint32_t S : {3u, 4u})
+    if (most(S) < most(best)) best = S;
+  return best;
 }
 
 // An odd block count over an even row count runs as row pairs (PAIRED) of
@@ -884,24 +937,28 @@ bool q6_shape_ok(uint32_t rows, uint32_t nb) {
 }  // namespace
 
 namespace {
-// An odd block count nb over an even row count: row pairs, K-sliced by the
-// rule of the even case (and always past 64 blocks, where the pairs' rows
-// exceed what the unsliced kernel takes), else unsliced.
+// An odd block count nb: row pairs, K-sliced by the rule of the even case (and
+// always past 64 blocks, where the pairs' rows exceed what the unsliced
+// kernel takes), else unsliced; the last row of an odd row count beside them.
 bool launch_pairs(const uint8_t* w, const float* x, float* y, uint32_t rows, uint32_t nb,
                   bool may_slice, const Workspace& ws, hipStream_t s, hipError_t* err) {
-  if ((nb & 1u) == 0u || rows < 2u || (rows & 1u) == 1u) return false;
+  if ((nb & 1u) == 0u || rows < 2u) return false;
   const uint32_t prows = rows / 2u, pnb = 2u * nb;
+  const bool last = (rows & 1u) != 0u;
   if (may_slice) {
-    const uint32_t S = q6_slices((prows + 15u) / 16u, pnb, ws.bytes);
-    if (S >= 2u && (launch_sliced<12, 1, true>(w, x, y, prows, pnb, S, ws, s, err) ||
-                    launch_sliced<8, 1, true>(w, x, y, prows, pnb, S, ws, s, err)))
+    const uint32_t S = q6_slices((prows + 15u) / 16u, pnb, ws.bytes, true,
+                                 (uint64_t)cu_count() - (last ? 1u : 0u));
+    if (S >= 2u && (launch_sliced<12, 1, true>(w, x, y, prows, pnb, S, ws, s, err, last) ||
+                    launch_sliced<8, 1, true>(w, x, y, prows, pnb, S, ws, s, err, last)))
       return true;
   }
-  return paired_ok(rows, nb) &&
-         (launch_wd<12, 1, false, false, true>(w, x, y, prows, pnb, ws, s, err) ||
-          launch_wd<10, 1, false, false, true>(w, x, y, prows, pnb, ws, s, err) ||
-          launch_wd<8, 1, false, false, true>(w, x, y, prows, pnb, ws, s, err) ||
-          launch_wd<4, 1, false, false, true>(w, x, y, prows, pnb, ws, s, err));
+  const GroupArgs ga{};
+  const ArgmaxArgs aa{};
+  return q6_shape_ok(prows, pnb) &&
+         (launch_wd<12, 1, false, false, true>(w, x, y, prows, pnb, ws, s, err, ga, aa, last) ||
+          launch_wd<10, 1, false, false, true>(w, x, y, prows, pnb, ws, s, err, ga, aa, last) ||
+          launch_wd<8, 1, false, false, true>(w, x, y, prows, pnb, ws, s, err, ga, aa, last) ||
+          launch_wd<4, 1, false, false, true>(w, x, y, prows, pnb, ws, s, err, ga, aa, last));
 }
 
 // ntok <= 4 NG vectors in one pass; false when the shape does not fit.
@@ -957,18 +1014,16 @@ bool launch_q6k_matvec_mfma(const uint8_t* w, const float* x, float* y, uint32_t
                             uint32_t cols, const Workspace& ws, hipStream_t s, hipError_t* err) {
   const uint32_t nb = cols / kBlockElems;
   static const int cfg = env_int("SI_HIP_Q6K_MFMA_CFG", 0);
-  if ((nb & 1u) == 1u && (rows & 1u) == 0u)
+  // An odd row count as well: pairs where the generic kernel (one wave per
+  // row) is slower.  Its time grows with the row, 257 x 5376 6.9 us to 6.5 of
+  // the pairs, 65 x 6912 6.9 / 6.7, 65 x 8448 9.2 / 7.5, 17 x 65280 59 / 15.6,
+  // and with the rows from about four a SIMD, 4097 x 256 4.7 / 4.8,
+  // 8193 x 1280 10.0 / 6.3, 3073 x 2816 8.7 / 7.6; below, 2049 x 2816 7.1 / 7.4,
+  // 2049 x 1280 4.4 / 5.7, 129 x 2816 4.4 / 6.8.
+  const bool pairs = (rows & 1u) == 0u ||
+                     (rows >= 3u && (rows >= 4096u || nb >= 27u || (uint64_t)rows * nb >= 32768u));
+  if ((nb & 1u) == 1u && pairs)
     return launch_pairs(w, x, y, rows, nb, cfg == 0, ws, s, err);
-  if ((nb & 1u) == 1u && rows >= 3u && (uint64_t)rows * nb >= 65536u) {
-    // an odd row count as well: the pairs of all rows but the last, then the
-    // last row alone (one workgroup).  The second launch costs 3-5 us, so
-    // below 64K blocks the generic kernel (one wave per row) is faster.
-    if (!launch_pairs(w, x, y, rows - 1u, nb, cfg == 0, ws, s, err)) return false;
-    if (*err == hipSuccess)
-      *err = launch_row_dot(kTypeQ6K, w + (size_t)(rows - 1u) * nb * kQ6Bytes, x, y + (rows - 1u),
-                            cols, s);
-    return true;
-  }
   if (cfg == 0 && nb > kMaxMetaBlocks) {  // (q6_shape_ok takes none of these)
     const uint32_t S = q6_slices((rows + 15u) / 16u, nb, ws.bytes);
     return S >= 2u && (launch_sliced<12, 1>(w, x, y, rows, nb, S, ws, s, err) ||

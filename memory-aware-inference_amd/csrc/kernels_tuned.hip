@@ -32,6 +32,12 @@ bool launch_matvec_tuned(uint32_t type, const uint8_t* w, const float* x, float*
   if (type == kTypeQ6K && batch > 1 &&
       launch_q6k_matmul_mfma(w, x, y, rows, cols, batch, ws, s, err))
     return true;
+  // Odd row and block counts, a few vectors: the generic kernel reads the
+  // weights once for all of them (1025 x 6912, 4 vectors: 21 us to 28 one by
+  // one), up to the size where its time per vector is the longer.
+  if (type == kTypeQ6K && batch > 1 && (rows & 1u) != 0u && ((cols / kBlockElems) & 1u) != 0u &&
+      (uint64_t)rows * (cols / kBlockElems) < 65536u)
+    return false;
   if (type == kTypeQ6K || (q4_mfma && batch > 1)) {
     // several candidates (batch-major x and y, metal.rs:1104-1126): one
     // matrix-core matvec per candidate, each bit-identical to its M = 1 call

@@ -1117,9 +1117,9 @@ inline bool quotients_fit(uint32_t ntiles, uint32_t tparts) {
 }
 
 inline LaunchShape launch_shape(uint32_t ntiles, uint32_t tparts, uint32_t waves,
-                                size_t ws_bytes, uint32_t mats) {
+                                size_t ws_bytes, uint32_t mats,
+                                uint32_t cus = (uint32_t)cu_count()) {
   LaunchShape ls;
-  const uint32_t cus = (uint32_t)cu_count();
   const uint32_t g0 = min(ntiles, cus);
   const uint64_t rounds0 = ((uint64_t)(ntiles + g0 - 1u) / g0 * tparts + waves - 1u) / waves;
   const uint32_t g1 = (uint32_t)min((uint64_t)cus, (uint64_t)ntiles * tparts);

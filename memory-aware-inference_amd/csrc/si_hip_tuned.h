@@ -37,9 +37,7 @@ constexpr size_t kMaxGroupWeights = 8;  // = kMaxGroup of the kernels
 bool launch_matvec_group(uint32_t type, const uint8_t* const* w, const uint32_t* rows,
                          uint32_t count, uint32_t cols, const float* x, float* y,
                          const Workspace& ws, hipStream_t s, hipError_t* err);
-// Q6_K, one vector / batch >= 2 vectors (two in one pass of the per-vector
-// loop, three to sixteen in one pass of the vectors-in-rows kernel), on the
-// matrix cores.
+// Q6_K, one vector / batch = 2..16 vectors in one pass, on the matrix cores.
 bool launch_q6k_matvec_mfma(const uint8_t* w, const float* x, float* y, uint32_t rows,
                             uint32_t cols, const Workspace& ws, hipStream_t s, hipError_t* err);
 // The Q6_K matvec with the greedy argmax of its output fused (rule: an

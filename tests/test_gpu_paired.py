@@ -9,9 +9,9 @@ to its own row of the pair -- the stage holding blocks nb - 1 and nb hands
 one sum to each.  Long pair rows over few tiles, and every pair row past 128
 blocks (nb > 64), run K-sliced: a workgroup holds the images of its slice's
 stretch of the doubled x, and the slice hand-off carries both sums of each
-row.  An odd row count over 64K blocks or more runs its first rows - 1 rows
-as pairs and the last row alone (one workgroup); smaller odd row counts run
-the generic kernel.
+row.  An odd row count runs its first rows - 1 rows as pairs and the last row
+in a workgroup of its own beside them, from 4096 rows, 27 blocks a row or 32K
+blocks; smaller odd row counts run the generic kernel.
 
 Bar: rows within 2e-5 * sum|w*x| of the f64 dot, +-inf / NaN rows where
 per-weight f32 products give them, the same bits on every call, and the
@@ -40,7 +40,7 @@ def log(msg):
 # 9 blocks over a partial tile of pairs (17 pairs); the Gemma-class head
 # width 5376 (21 blocks); the Llama-2-7B down projection (43 blocks, K-sliced
 # pairs); a head of 32000 rows (a split launch of 1000 pair tiles); odd row
-# counts (generic below 64K blocks: 41 rows, three rows of one block, one row;
+# counts (generic: 41 rows, three rows of one block, one row;
 # pairs, then the last row alone: 4097 rows of sliced pairs, a 32001-row
 # head); pair rows past 128 blocks, which must slice (67, 65 and 129 blocks;
 # 135 blocks: eight slices), and the same with an odd row count
@@ -124,7 +124,7 @@ def test_sliced_pairs_special_activations(hip_ctx):
 def test_odd_rows_split_special_activations(hip_ctx):
     """An odd row count split into sliced pairs and the last row alone: huge,
     side and zero blocks within the bound, then one infinite or NaN
-    activation at a time, every row (the last one's own launch included) in
+    activation at a time, every row (the last one's own workgroup included) in
     the category that per-weight f32 products give."""
     rows, cols = 1001, 17152
     w = si_hip.synth_matrix(Q6, seed=4650, rows=rows, cols=cols, threads=8)
@@ -295,4 +295,33 @@ def test_random_odd_block_counts(hip_ctx, seed):
         assert_dot_close(y, y64, ab, what=f"{rows}x{cols}")
         assert same_bits(hip_ctx.gguf_quant_matvec_weight(W, rows, cols, x), y)
     finally:
+        W.free()
+
+
+@pytest.mark.parametrize("rows,cols", [
+    (3, 6912), (3, 17152), (5, 8448), (4095, 2304), (4097, 256), (4097, 1280), (1187, 7424),
+    (255, 33024), (2047, 11008), (8191, 8448), (8225, 5376)])
+def test_odd_rows_beside_pairs(hip_ctx, rows, cols):
+    """The last row's workgroup beside unsliced, split and sliced pairs (three
+    slices: 2047 rows), at the edges of the rule, against the oracle and the
+    generic kernel; the last row also with an infinite activation."""
+    log(f"odd rows {rows}x{cols}")
+    w = si_hip.synth_matrix(Q6, seed=rows * 7 + cols, rows=rows, cols=cols, threads=8)
+    x = si_hip.synth_normal(rows + 5 * cols, cols)
+    _, y64, ab = O.matvec(Q6, w, rows, cols, x, threads=8)
+    W = hip_ctx.upload_quant_weight_private(w, Q6)
+    try:
+        y = hip_ctx.gguf_quant_matvec_weight(W, rows, cols, x)
+        assert_dot_close(y, y64, ab, what=f"{rows}x{cols}")
+        assert same_bits(hip_ctx.gguf_quant_matvec_weight(W, rows, cols, x), y)
+        hip_ctx.set_kernel_policy(si_hip.KERNEL_GENERIC)
+        g = hip_ctx.gguf_quant_matvec_weight(W, rows, cols, x)
+        assert np.all(np.abs(g.astype(np.float64) - y) <= 4e-5 * ab + 1e-30)
+        x[cols - 1] = np.inf
+        g = hip_ctx.gguf_quant_matvec_weight(W, rows, cols, x)
+        hip_ctx.set_kernel_policy(si_hip.KERNEL_AUTO)
+        y = hip_ctx.gguf_quant_matvec_weight(W, rows, cols, x)
+        assert np.array_equal(_category(y), _category(g))
+    finally:
+        hip_ctx.set_kernel_policy(si_hip.KERNEL_AUTO)
         W.free()
