@@ -411,10 +411,8 @@ bool launch_tok45(const uint8_t* w, const float* x, float* y, uint32_t rows, uin
 template <int QB>
 bool launch_tok45_any(const uint8_t* w, const float* x, float* y, uint32_t rows, uint32_t nb,
                       uint32_t ntok, const Workspace& ws, hipStream_t s, hipError_t* err) {
-  // Waves, measured (17408 x 5120, us, 12 / 8 waves): Q4_K M = 4 17.8 / 18.5,
-  // M = 8 21.2 / 21.3, M = 16 29.6 (spills) / 28.2; Q5_K, whose blocks take
-  // more registers, M = 4 21.7 / 21.0, M = 8 26.9 / 25.1.
-  // (8 waves: M = 4 / 16 17.2 / 28.7 us against 16.3 / 26.9; 16 the same)
+  // Twelve waves; 8 measured 17.2 / 28.7 us at M = 4 / 16 against 16.3 / 26.9
+  // (Q4_K 17408 x 5120), 16 the same.
   if (ntok <= 4u) return launch_tok45<12, 1, QB>(w, x, y, rows, nb, ntok, ws, s, err);
   if (ntok <= 8u) return launch_tok45<12, 2, QB>(w, x, y, rows, nb, ntok, ws, s, err);
   if (ntok <= 12u) return launch_tok45<12, 3, QB>(w, x, y, rows, nb, ntok, ws, s, err);

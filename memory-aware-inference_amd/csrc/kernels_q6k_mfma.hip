@@ -579,10 +579,20 @@ __global__ __launch_bounds__(WAVES * 64) void q6k_matvec_mfma(const uint8_t* __r
 // whose side elements (half a unit each times 4096 |d|, the largest |w| a
 // block can hold) could be off by more than kRoundedTol of its sum |block
 // term| stores kPartRedo for the slice, and tok_reduce recomputes it exactly.
+//
+// PAIRED (odd block counts, where a row starts 2 bytes off 4 every second
+// time): the even rows and the odd rows as two matrices of row stride 2 nb
+// blocks, nb + 1 blocks wide so that both start aligned and the stages are
+// whole: an even row with the block after it, an odd row with the block before
+// it, whose activations read as zero.  Slices 0 .. `slices` - 1 are the even
+// rows', the next `slices` the odd rows', and a "row" here is a pair.
+// 4096 x 11008, M = 2 / 4 / 8 / 16: 28.3 / 55.3 / 108.5 / 215.6 us one vector
+// at a time, 15.3 / 15.5 / 17.4 / 20.5 so.
 constexpr uint32_t kTokBlocks = 4u;
 
 struct Q6TokArgs {
   uint32_t groups_per_slice, m_gps;
+  uint32_t slices;  // PAIRED
 };
 
 // The two digits of the lane's 64 scaled weights of a block: set t's four
@@ -624,7 +634,7 @@ __device__ __forceinline__ void lds_read_group(uint32_t ia, uint32_t ea, i32x4 (
       : "memory");
 }
 
-template <int WAVES, int NG>
+template <int WAVES, int NG, bool PAIRED>
 __global__ __launch_bounds__(WAVES * 64) void q6k_tokens_mfma(const uint8_t* __restrict__ w,
                                                               const float* __restrict__ x,
                                                               uint32_t rows, uint32_t nb,
@@ -638,8 +648,7 @@ __global__ __launch_bounds__(WAVES * 64) void q6k_tokens_mfma(const uint8_t* __r
   const uint32_t lane = threadIdx.x & 63u;
   const uint32_t grp = lane >> 4, n = lane & 15u;
   const uint32_t half = grp >> 1, sub = grp & 1u;
-  const uint32_t row_bytes = nb * kQ6Bytes;
-  const uint32_t ntiles = (rows + 15u) / 16u;
+  const uint32_t row_bytes = (PAIRED ? 2u : 1u) * nb * kQ6Bytes;
   const uint32_t sbase = (uint32_t)(uintptr_t)smem;
   uint8_t* const wstage = smem + wave * kStageBytes;
 
@@ -648,22 +657,34 @@ __global__ __launch_bounds__(WAVES * 64) void q6k_tokens_mfma(const uint8_t* __r
   const FastDiv by_gps{ta.groups_per_slice, ta.m_gps};
   const uint32_t k = quo(blockIdx.x, by_gps);
   const uint32_t tg = blockIdx.x - k * ta.groups_per_slice;
-  const uint32_t blk0 = kTokBlocks * k, nbl = min(kTokBlocks, nb - blk0), nst = nbl / 2u;
+  const uint32_t odd = PAIRED && k >= ta.slices ? 1u : 0u;
+  const uint32_t blk0 = kTokBlocks * (PAIRED ? k - odd * ta.slices : k);
+  const uint32_t nbl = min(kTokBlocks, nb + (PAIRED ? 1u : 0u) - blk0), nst = nbl / 2u;
+  const uint32_t places = PAIRED ? (rows + 1u) / 2u : rows;  // of the partials
+  const uint32_t trows = odd ? rows / 2u : places;           // the slice's rows
+  const uint32_t ntiles = (trows + 15u) / 16u;
   const uint32_t ntw = tg < ntiles ? quo(ntiles - 1u - tg, by_gps) + 1u : 0u;
 
   // 1. the activations of the wave's image blocks into registers, then the
   //    copy of its first stage (copy_offsets; rows past the matrix read zero)
   constexpr int kShare = (NG * (int)kTokBlocks + WAVES - 1) / WAVES;
   u32x4 xq[kShare][4];
-  load_group_x<WAVES, kShare>(xq, x, nb, blk0, nbl, NG, ntok, wave, lane);
+  load_group_x<WAVES, kShare>(xq, x, nb, blk0 - odd, nbl, NG, ntok, wave, lane);
   uint32_t vo[kCopies];
   copy_offsets(row_bytes, lane, vo);
   auto issue = [&](uint32_t lt, uint32_t sl) {
     const uint32_t row0 = (tg + lt * ta.groups_per_slice) * 16u;
-    const uint32_t nrows = min(16u, rows - row0);
-    const uint32_t at = kQ6Bytes * blk0 + kStageRowBytes * sl;
+    const uint32_t nrows = min(16u, trows - row0);
+    uint32_t at = kQ6Bytes * blk0 + kStageRowBytes * sl;
+    if constexpr (PAIRED) at += odd * (nb - 1u) * kQ6Bytes;
+    uint32_t size = nrows * row_bytes;
+    if constexpr (PAIRED) {
+      // the last pair of an odd row count is one row, its last 2 bytes the
+      // lower half of a word
+      if (2u * (row0 + nrows) > rows) size = (size - nb * kQ6Bytes + 3u) & ~3u;
+    }
     const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc(
-        const_cast<uint8_t*>(w + (size_t)row0 * row_bytes + at), 0, (int)(nrows * row_bytes - at),
+        const_cast<uint8_t*>(w + (size_t)row0 * row_bytes + at), 0, (int)(size - at),
         kBufferWord3);
 #pragma unroll
     for (int i = 0; i < (int)kCopies; ++i)
@@ -765,8 +786,8 @@ __global__ __launch_bounds__(WAVES * 64) void q6k_tokens_mfma(const uint8_t* __r
         const bool redo = !(fabsf(part) < __builtin_huge_valf()) ||
                           !(err * 1.01f <= kRoundedTol * ((float)sum_abs[G] - err));
         const uint32_t vec = 4u * G + grp;
-        if (row < rows && vec < ntok)
-          part_out[((size_t)k * 4u * NG + vec) * rows + row] =
+        if (row < trows && vec < ntok)
+          part_out[((size_t)k * 4u * NG + vec) * places + row] =
               redo ? __uint_as_float(kPartRedo) : part;
         acc[G] = sum_abs[G] = 0.0;
       }
@@ -962,38 +983,44 @@ bool launch_pairs(const uint8_t* w, const float* x, float* y, uint32_t rows, uin
 }
 
 // ntok <= 4 NG vectors in one pass; false when the shape does not fit.
-template <int W, int NG>
+template <int W, int NG, bool P>
 bool launch_tok6(const uint8_t* w, const float* x, float* y, uint32_t rows, uint32_t nb,
                  uint32_t ntok, const Workspace& ws, hipStream_t s, hipError_t* err) {
   constexpr uint32_t kLds =
       (uint32_t)W * kStageBytes + tok64_layout(kTokBlocks, NG, false, false).total;
   static_assert(kLds <= kLdsBytes, "the stage buffers and the images fit the LDS");
+  constexpr uint32_t kPer = P ? 2u : 1u;  // rows a place of the partials
   const uint32_t cus = (uint32_t)cu_count();
-  const uint32_t slices = (nb + kTokBlocks - 1u) / kTokBlocks;
-  if (slices > cus || !q6_shape_ok(rows, nb)) return false;
+  const uint32_t slices = (nb + (P ? 1u : 0u) + kTokBlocks - 1u) / kTokBlocks;
+  // 32-bit offsets of the weights in a tile and of the activations
+  if (kPer * slices > cus || (uint64_t)nb * kPer * kQ6Bytes * 16u > 0x7fffffffu ||
+      (uint64_t)ntok * nb * 1024u > 0x7fffffffu)
+    return false;
+  if (!P && !q6_shape_ok(rows, nb)) return false;
   // the rows of one launch: all, or as many whole tiles as the scratch holds
-  const size_t row_part = (size_t)slices * 4u * NG * sizeof(float);
-  const uint32_t chunk =
-      (uint32_t)min((uint64_t)rows, (uint64_t)(ws.scratch_bytes / row_part / 16u * 16u));
+  const size_t place_part = (size_t)kPer * slices * 4u * NG * sizeof(float);
+  const uint64_t fit = ws.scratch_bytes / place_part / 16u * 16u * kPer;
+  const uint32_t chunk = (uint32_t)min((uint64_t)rows, fit);
   if (chunk == 0u) return false;
   // block and tile indices divided by GS <= cus
   if ((uint64_t)(cus + (chunk + 15u) / 16u) * cus >= (1ull << 32)) return false;
   static const hipError_t attr =
-      hipFuncSetAttribute(reinterpret_cast<const void*>(&q6k_tokens_mfma<W, NG>),
+      hipFuncSetAttribute(reinterpret_cast<const void*>(&q6k_tokens_mfma<W, NG, P>),
                           hipFuncAttributeMaxDynamicSharedMemorySize, (int)kLdsBytes);
   *err = attr;
   for (uint32_t r0 = 0; r0 < rows && *err == hipSuccess; r0 += chunk) {
     const uint32_t nr = min(chunk, rows - r0);
     const uint8_t* const wr = w + (size_t)r0 * nb * kQ6Bytes;
     Q6TokArgs ta{};
-    ta.groups_per_slice = min(cus / slices, (nr + 15u) / 16u);
+    ta.slices = slices;
+    ta.groups_per_slice = min(cus / (kPer * slices), ((nr + kPer - 1u) / kPer + 15u) / 16u);
     ta.m_gps = div_magic(ta.groups_per_slice);
-    hipLaunchKernelGGL((q6k_tokens_mfma<W, NG>), dim3(ta.groups_per_slice * slices), dim3(W * 64),
-                       kLds, s, wr, x, nr, nb, ntok, ws.scratch, ta);
+    hipLaunchKernelGGL((q6k_tokens_mfma<W, NG, P>), dim3(ta.groups_per_slice * kPer * slices),
+                       dim3(W * 64), kLds, s, wr, x, nr, nb, ntok, ws.scratch, ta);
     *err = hipGetLastError();
     if (*err != hipSuccess) break;
-    launch_tok_reduce<kTypeQ6K>(ws.scratch, y + r0, nr, rows, slices, 4u * NG, ntok, wr, x, nb,
-                                kTokBlocks, s);
+    launch_tok_reduce<kTypeQ6K, P>(ws.scratch, y + r0, nr, rows, slices, 4u * NG, ntok, wr, x, nb,
+                                   kTokBlocks, s);
     *err = hipGetLastError();
   }
   return true;
@@ -1001,12 +1028,13 @@ bool launch_tok6(const uint8_t* w, const float* x, float* y, uint32_t rows, uint
 
 // Twelve waves; 8 and 16 measured the same within 1 % up to eight vectors, 8
 // took 198 against 193 us at sixteen (151936 x 5120).
+template <bool P>
 bool launch_tok6_any(const uint8_t* w, const float* x, float* y, uint32_t rows, uint32_t nb,
                      uint32_t ntok, const Workspace& ws, hipStream_t s, hipError_t* err) {
-  if (ntok <= 4u) return launch_tok6<12, 1>(w, x, y, rows, nb, ntok, ws, s, err);
-  if (ntok <= 8u) return launch_tok6<12, 2>(w, x, y, rows, nb, ntok, ws, s, err);
-  if (ntok <= 12u) return launch_tok6<12, 3>(w, x, y, rows, nb, ntok, ws, s, err);
-  return launch_tok6<12, 4>(w, x, y, rows, nb, ntok, ws, s, err);
+  if (ntok <= 4u) return launch_tok6<12, 1, P>(w, x, y, rows, nb, ntok, ws, s, err);
+  if (ntok <= 8u) return launch_tok6<12, 2, P>(w, x, y, rows, nb, ntok, ws, s, err);
+  if (ntok <= 12u) return launch_tok6<12, 3, P>(w, x, y, rows, nb, ntok, ws, s, err);
+  return launch_tok6<12, 4, P>(w, x, y, rows, nb, ntok, ws, s, err);
 }
 }  // namespace
 
@@ -1060,12 +1088,23 @@ bool launch_q6k_matvec_argmax_mfma(const uint8_t* w, const float* x, float* y, u
          launch_wd<8, 1, false, true>(w, x, y, rows, nb, ws, s, err, GroupArgs{}, aa);
 }
 
-// (odd block counts and rows past kMaxMetaBlocks run one vector at a time)
+// (even block counts past kMaxMetaBlocks run one vector at a time)
 bool launch_q6k_matmul_mfma(const uint8_t* w, const float* x, float* y, uint32_t rows,
                             uint32_t cols, uint32_t batch, const Workspace& ws, hipStream_t s,
                             hipError_t* err) {
   if (batch < 2u || batch > 16u) return false;
-  return launch_tok6_any(w, x, y, rows, cols / kBlockElems, batch, ws, s, err);
+  const uint32_t nb = cols / kBlockElems;
+  // Odd row and block counts: the generic kernel, which takes any, where it is
+  // faster, short rows and few vectors (us, generic / here: 129 x 2816 M = 2 / 3
+  // 6.5 / 7.2, 8.0 / 7.2; 1025 x 1280 M = 5 / 8 7.8 / 9.0, 10.9 / 9.0; 4097 x 256
+  // M = 2 / 4 6.0 / 6.8, 8.8 / 7.0; 33 x 5376 M = 2 9.0 / 7.2; 2049 x 2816 M = 2
+  // 10.2 / 8.6; a single row of 2816 M = 5 / 8 7.7 / 8.0, 10.6 / 8.2).
+  if ((nb & 1u) != 0u && (rows & 1u) != 0u && nb < 16u && (uint64_t)rows * nb < 16384u &&
+      rows * batch < 12288u &&
+      (rows < 16u ? batch * nb < 64u : batch < 8u && batch * nb < 33u))
+    return false;
+  return (nb & 1u) != 0u ? launch_tok6_any<true>(w, x, y, rows, nb, batch, ws, s, err)
+                         : launch_tok6_any<false>(w, x, y, rows, nb, batch, ws, s, err);
 }
 
 bool mfma::launch_q6k_matvec_group(const GroupArgs& ga, uint32_t total_rows, uint32_t cols,

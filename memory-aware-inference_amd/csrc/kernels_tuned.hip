@@ -32,9 +32,9 @@ bool launch_matvec_tuned(uint32_t type, const uint8_t* w, const float* x, float*
   if (type == kTypeQ6K && batch > 1 &&
       launch_q6k_matmul_mfma(w, x, y, rows, cols, batch, ws, s, err))
     return true;
-  // Odd row and block counts, a few vectors: the generic kernel reads the
-  // weights once for all of them (1025 x 6912, 4 vectors: 21 us to 28 one by
-  // one), up to the size where its time per vector is the longer.
+  // Odd row and block counts that launch left: the generic kernel reads the
+  // weights once for all the vectors, up to the size where one vector at a time
+  // is faster.
   if (type == kTypeQ6K && batch > 1 && (rows & 1u) != 0u && ((cols / kBlockElems) & 1u) != 0u &&
       (uint64_t)rows * (cols / kBlockElems) < 65536u)
     return false;

@@ -65,7 +65,8 @@ __host__ __device__ constexpr TokLayout tok64_layout(uint32_t stride, uint32_t n
 // The wave's share of the image blocks: group-blocks q = wave + i WAVES, i <
 // SHARE, of the ng groups in order of group and of the blocks 0 .. stride - 1
 // (those past nbl hold nothing); lane (t, c) takes elements 16 c .. 16 c + 15 of
-// vector 4 g + t.  Vectors past ntok read as zero.
+// vector 4 g + t.  Vectors past ntok and blocks outside the row's nb read as
+// zero.
 template <int WAVES, int SHARE>
 __device__ __forceinline__ void load_group_x(u32x4 (&xq)[SHARE][4], const float* x, uint32_t nb,
                                              uint32_t blk0, uint32_t nbl, uint32_t ng,
@@ -76,7 +77,8 @@ __device__ __forceinline__ void load_group_x(u32x4 (&xq)[SHARE][4], const float*
   for (int i = 0; i < SHARE; ++i) {
     const uint32_t q = wave + (uint32_t)i * WAVES, g = q >> 2, b = q & 3u;
     if (g < ng && b < nbl) {
-      const uint32_t off = ((4u * g + (lane >> 4)) * nb + blk0 + b) * 1024u + 64u * (lane & 15u);
+      const uint32_t at = ((4u * g + (lane >> 4)) * nb + blk0 + b) * 1024u + 64u * (lane & 15u);
+      const uint32_t off = blk0 + b < nb ? at : 0x80000000u;
 #pragma unroll
       for (int j = 0; j < 4; ++j)
         xq[i][j] = __builtin_bit_cast(
@@ -193,6 +195,10 @@ __device__ __forceinline__ float slice_err(const uint8_t* rerr, uint32_t nbl) {
 // partials again in stage order, the first eight stages kept in registers.
 // R rows per thread: 1, or 4 with 16-byte loads and stores (launch_tok_reduce
 // takes 4 when the rows, y and the grid allow it); each row's sum is the same.
+// PAIRED: rows 2 r and 2 r + 1 share place r of the partials, of ceil(rows / 2);
+// the first nstages stages are the even rows' and the next nstages the odd
+// rows', whose stage s starts a block earlier (the block before the row is no
+// part of it).
 constexpr uint32_t kRedoQueue = 64;
 template <uint32_t T>
 __device__ __noinline__ float stage_exact(const uint8_t* __restrict__ w, uint32_t row,
@@ -213,14 +219,14 @@ __device__ __noinline__ float stage_exact(const uint8_t* __restrict__ w, uint32_
   return (float)acc;
 }
 
-template <uint32_t T, int R>
+template <uint32_t T, int R, bool PAIRED>
 __global__ __launch_bounds__(256) void tok_reduce(const float* __restrict__ part,
                                                   float* __restrict__ y, uint32_t rows,
                                                   uint32_t yrows, uint32_t nstages, uint32_t nv,
                                                   const uint8_t* __restrict__ w,
                                                   const float* __restrict__ x, uint32_t nb,
                                                   uint32_t bps) {
-  static_assert(R == 1 || R == 4, "one or four rows per thread");
+  static_assert(R == 1 || (R == 4 && !PAIRED), "one or four rows per thread");
   constexpr uint32_t kBytes = BlockBytes<T>::value;
   __shared__ uint32_t queue[kRedoQueue];  // (row in the workgroup) << 16 | stage
   __shared__ float value[kRedoQueue];
@@ -228,9 +234,11 @@ __global__ __launch_bounds__(256) void tok_reduce(const float* __restrict__ part
   const uint32_t tid = threadIdx.x, t = blockIdx.y;
   const uint32_t rw = (uint32_t)R * tid;                    // the thread's first row in the workgroup
   const uint32_t row = blockIdx.x * (256u * R) + rw;        // its rows row .. row + R - 1
-  const float* const p = part + (size_t)t * rows + row;
+  const uint32_t places = PAIRED ? (rows + 1u) / 2u : rows;
+  const size_t step = (size_t)nv * places;
+  const float* const p = part + (size_t)t * places +
+                         (PAIRED ? (row >> 1) + (row & 1u) * nstages * step : (size_t)row);
   const float* const xt = x + (size_t)t * nb * kBlockElems;
-  const size_t step = (size_t)nv * rows;
   if (tid == 0u) queued = 0u;
   __syncthreads();
   // stages base .. base + 7 of the thread's rows, eight loads in flight
@@ -291,8 +299,9 @@ __global__ __launch_bounds__(256) void tok_reduce(const float* __restrict__ part
       double acc = 0.0;
       if (k < nq) {
         const uint32_t r = blockIdx.x * (256u * R) + (queue[k] >> 16), st = queue[k] & 0xffffu;
+        const uint32_t early = PAIRED ? r & 1u : 0u;
         for (uint32_t uu = l; uu < 8u * bps; uu += 32u) {
-          const uint32_t b = bps * st + (uu >> 3), u = uu & 7u;  // unit u of block b
+          const uint32_t b = bps * st + (uu >> 3) - early, u = uu & 7u;  // unit u of block b
           if (b < nb) {
             float wv[32];
             decode_unit_exact<T>(w + ((size_t)r * nb + b) * kBytes, u, wv);
@@ -310,6 +319,7 @@ __global__ __launch_bounds__(256) void tok_reduce(const float* __restrict__ part
   }
   if (row >= rows) return;
   if (mine) {  // the sums again, with the recomputed stages (unchanged for rows without one)
+    const uint32_t early = PAIRED ? row & 1u : 0u;
     const uint32_t nq = min(queued, kRedoQueue);
 #pragma unroll
     for (int c = 0; c < R; ++c) sum[c] = 0.0f;
@@ -335,8 +345,9 @@ __global__ __launch_bounds__(256) void tok_reduce(const float* __restrict__ part
             uint32_t k = 0;
             while (k < nq && queue[k] != key) ++k;
             vc = k < nq ? value[k]
-                        : stage_exact<T>(w, row + (uint32_t)c, nb, bps * st,
-                                         min(bps * st + bps, nb), xt);
+                        : stage_exact<T>(w, row + (uint32_t)c, nb,
+                                         bps * st - (early != 0u && st != 0u ? 1u : 0u),
+                                         min(bps * st + bps - early, nb), xt);
           }
           sum[c] += vc;
         }
@@ -352,22 +363,22 @@ __global__ __launch_bounds__(256) void tok_reduce(const float* __restrict__ part
 }
 
 // The reduce of a sliced launch of ntok vectors: four rows a thread when the
-// row counts (of the launch, and yrows of a vector's outputs) are multiples
-// of 4, y is 16-byte aligned (the scratch always is) and the grid still gives every CU two workgroups, else one.  The Q6_K head
-// (151,936 rows) at M = 4 / 8 / 16: 144.6 / 180.1 / 321.5 -> 143.6 / 176.8 /
-// 317.4 us a call; Q4_K 17408 rows at M = 16 (one workgroup a CU) lost
-// 0.4 us, so it keeps one row a thread.
-template <uint32_t T>
+// row counts (of the launch, and yrows of a vector's outputs) are multiples of
+// 4, y is 16-byte aligned (the scratch always is) and the grid still gives
+// every CU two workgroups, else one.  (With one row a thread the Q6_K head,
+// 151,936 rows, takes 1 us more at M = 4 and 4 us at M = 16; Q4_K 17408 rows
+// at M = 16, one workgroup a CU, loses 0.4 us with four.)
+template <uint32_t T, bool PAIRED = false>
 void launch_tok_reduce(const float* part, float* y, uint32_t rows, uint32_t yrows,
                        uint32_t nstages, uint32_t nv, uint32_t ntok, const uint8_t* w,
                        const float* x, uint32_t nb, uint32_t bps, hipStream_t s) {
   const uint32_t g4 = (rows + 1023u) / 1024u;
-  if (rows % 4u == 0u && yrows % 4u == 0u && ((uintptr_t)y & 15u) == 0u &&
+  if (!PAIRED && rows % 4u == 0u && yrows % 4u == 0u && ((uintptr_t)y & 15u) == 0u &&
       (uint64_t)g4 * ntok >= 2u * (uint64_t)cu_count())
-    hipLaunchKernelGGL((tok_reduce<T, 4>), dim3(g4, ntok), dim3(256), 0, s, part, y, rows, yrows,
+    hipLaunchKernelGGL((tok_reduce<T, 4, false>), dim3(g4, ntok), dim3(256), 0, s, part, y, rows, yrows,
                        nstages, nv, w, x, nb, bps);
   else
-    hipLaunchKernelGGL((tok_reduce<T, 1>), dim3((rows + 255u) / 256u, ntok), dim3(256), 0, s, part,
+    hipLaunchKernelGGL((tok_reduce<T, 1, PAIRED>), dim3((rows + 255u) / 256u, ntok), dim3(256), 0, s, part,
                        y, rows, yrows, nstages, nv, w, x, nb, bps);
 }
 

@@ -259,8 +259,7 @@ def test_odd_block_count_head_argmax(hip_ctx, rows, cols):
 
 
 def test_odd_block_count_matmul_many(hip_ctx):
-    """Several vectors over an odd-block matrix: one paired launch per
-    vector, each within its bound."""
+    """Several vectors over an odd-block matrix, each within its bound."""
     rows, cols, batch = 1000, 5376, 3
     w = si_hip.synth_matrix(Q6, seed=4500, rows=rows, cols=cols, threads=8)
     X = si_hip.synth_normal(4501, batch * cols).reshape(batch, cols)
@@ -278,8 +277,8 @@ def test_odd_block_count_matmul_many(hip_ctx):
 def test_random_odd_block_counts(hip_ctx, seed):
     """Seeded random Q6_K shapes with odd block counts and row counts of either
     parity up to 300K blocks: unsliced and sliced row pairs, the odd row
-    count's pairs plus one-workgroup last row, and the generic kernel below
-    64K blocks; every row within the oracle's bound and repeating its bits."""
+    count's pairs plus one-workgroup last row, and the generic kernel for the
+    smallest; every row within the oracle's bound and repeating its bits."""
     rng = np.random.default_rng(9800 + seed)
     nb = int(rng.choice([1, 9, 21, 43, 67, 135]))
     rows = int(rng.integers(1, min(8000, 300000 // nb) + 1))

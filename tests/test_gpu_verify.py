@@ -1,0 +1,88 @@
+"""GPU: several activation vectors over one weight matrix (verify), M = 2..16.
+
+The vectors sit in the rows of the matrix-core operand, four to a group, and a
+launch is cut into K slices of four blocks: sizes here are the edges of the
+groups (M = 2, 4, 5, 8, 9, 12, 13, 16), of the 16-row tiles, and of the slices
+and their two-block stages (1 to 9 blocks, whole and short last slices).  Odd
+Q6_K block counts run their even and odd rows as two matrices of twice the row
+stride, either row count parity.
+
+Bar: every row within 2e-5 * sum|w*x| of the f64 dot; non-finite rows in the
+category that per-weight f32 products give.
+"""
+import numpy as np
+import pytest
+
+import oracle_lib as O
+import si_hip
+from test_gpu_parity import _category, assert_dot_close, log, same_bits
+
+pytestmark = pytest.mark.gpu
+
+SIZES = [(1, 256, 2), (15, 512, 3), (17, 768, 4), (33, 1024, 5), (16, 1280, 8), (47, 1536, 9),
+         (3, 1792, 12), (130, 2048, 13), (256, 2304, 16), (1001, 5376, 6), (4100, 2560, 16),
+         (2, 11008, 16), (999, 17152, 7)]
+
+
+@pytest.mark.parametrize("t", [12, 13, 14])
+@pytest.mark.parametrize("rows,cols,batch", SIZES)
+def test_verify_edges(hip_ctx, t, rows, cols, batch):
+    log(f"verify t={t} {rows}x{cols} M={batch}")
+    w = si_hip.synth_matrix(t, seed=rows + cols + t, rows=rows, cols=cols, threads=8)
+    X = si_hip.synth_normal(rows * 3 + cols + batch, batch * cols).reshape(batch, cols).copy()
+    X[:, ::97] *= np.float32(300.0)  # a few large channels
+    X[batch - 1, :256] = 0.0
+    W = hip_ctx.upload_quant_weight_private(w, t)
+    try:
+        outs = [o.copy() for o in hip_ctx.gguf_quant_matmul_many_weight(W, rows, cols, batch, X)]
+        for b in range(batch):
+            _, y64, ab = O.matvec(t, w, rows, cols, X[b], threads=8)
+            assert_dot_close(outs[b], y64, ab, what=f"vector {b}")
+        again = hip_ctx.gguf_quant_matmul_many_weight(W, rows, cols, batch, X)
+        assert all(same_bits(a, o) for a, o in zip(again, outs))
+    finally:
+        W.free()
+
+
+@pytest.mark.parametrize("t,rows,cols", [(12, 37, 1792), (13, 37, 1792), (14, 37, 1792),
+                                         (14, 38, 2304), (14, 38, 2560)])
+def test_verify_special_blocks(hip_ctx, t, rows, cols):
+    """Huge, subnormal and side blocks within the bound, and one infinite or NaN
+    activation in the first and the last block of a vector (its neighbours'
+    rows stay finite)."""
+    batch = 6
+    w = si_hip.synth_matrix(t, seed=77 * t + cols, rows=rows, cols=cols, threads=8)
+    X = si_hip.synth_normal(78 * t + rows, batch * cols).reshape(batch, cols).copy()
+    X[1, 100:140] = np.float32(3e30)
+    X[2, 300] = np.float32(1e-9)
+    X[2, 512:768] = np.float32(1e-41)
+    X[3, cols - 1] = np.inf
+    X[4, 0] = np.nan
+    X[5, 3] = -np.inf
+    W = hip_ctx.upload_quant_weight_private(w, t)
+    try:
+        outs = hip_ctx.gguf_quant_matmul_many_weight(W, rows, cols, batch, X)
+        for b in range(batch):
+            y32, y64, ab = O.matvec(t, w, rows, cols, X[b], threads=8)
+            assert np.array_equal(_category(outs[b]), _category(y32)), f"vector {b}"
+            if b < 3:
+                assert_dot_close(outs[b], y64, ab, what=f"vector {b}")
+    finally:
+        W.free()
+
+
+@pytest.mark.parametrize("t", [12, 13])
+@pytest.mark.parametrize("rows,cols", [(48, 512), (80, 5120), (33, 2816)])
+def test_matvec_cancelling_terms(hip_ctx, t, rows, cols):
+    """One vector: a constant vector against weights of nearly zero mean in
+    every block, so that the scale and the minimum terms cancel: the row's
+    error stays far under its terms' size."""
+    w = si_hip.synth_matrix(t, seed=rows + 9 * cols + t, rows=rows, cols=cols, threads=8)
+    dq = O.dequantize(t, w, rows * cols).reshape(rows, cols).astype(np.float64)
+    x = (np.ones(cols) + 1e-3 * si_hip.synth_normal(cols, cols)).astype(np.float32)
+    W = hip_ctx.upload_quant_weight_private(w, t)
+    try:
+        y = hip_ctx.gguf_quant_matvec_weight(W, rows, cols, x)
+        assert_dot_close(y, dq @ x.astype(np.float64), np.abs(dq) @ np.abs(x.astype(np.float64)))
+    finally:
+        W.free()
