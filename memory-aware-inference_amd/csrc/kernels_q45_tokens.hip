@@ -1,4 +1,4 @@
-// Multi-token verify of Q4_K and Q5_K on the gfx950 int8 matrix cores: three
+// Multi-token verify of Q4_K and Q5_K on the gfx950 int8 matrix cores: two
 // to sixteen activation vectors in one pass over the weights (matmul-many,
 // replacing si_q4_k_matmul_many, metal.rs:1052-1262).
 //
