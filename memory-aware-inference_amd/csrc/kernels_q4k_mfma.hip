@@ -1196,7 +1196,8 @@ bool launch_matvec_group(uint32_t type, const uint8_t* const* w, const uint32_t*
   for (uint32_t k = 0; k < kMaxGroup; ++k) ga.tile_end[k] = 0xffffffffu;
   uint64_t tiles = 0, total = 0;
   for (uint32_t k = 0; k < count; ++k) {
-    if (rows[k] == 0u || (k + 1u < count && rows[k] % 16u != 0u)) return false;
+    if (rows[k] == 0u || (k + 1u < count && rows[k] % 16u != 0u) || !word_aligned(w[k]))
+      return false;
     ga.w[k] = w[k];
     ga.rows[k] = rows[k];
     total += rows[k];

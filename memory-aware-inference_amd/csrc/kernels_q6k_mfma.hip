@@ -1076,6 +1076,7 @@ bool launch_q6k_matvec_mfma(const uint8_t* w, const float* x, float* y, uint32_t
 bool launch_q6k_matvec_argmax_mfma(const uint8_t* w, const float* x, float* y, uint32_t rows,
                                    uint32_t cols, uint32_t rule, uint64_t* result,
                                    const Workspace& ws, hipStream_t s, hipError_t* err) {
+  if (!word_aligned(w)) return false;
   const uint32_t nb = cols / kBlockElems;
   const ArgmaxArgs aa{result, rule};
   if (paired_ok(rows, nb))

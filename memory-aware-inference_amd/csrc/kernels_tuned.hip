@@ -20,7 +20,7 @@ int env_flag(const char* name, int fallback) {
 bool launch_matvec_tuned(uint32_t type, const uint8_t* w, const float* x, float* y, uint32_t rows,
                          uint32_t cols, uint32_t batch, const Workspace& ws, hipStream_t s,
                          hipError_t* err) {
-  if (batch == 0) return false;
+  if (batch == 0 || !word_aligned(w)) return false;
   const bool q4_mfma = type == kTypeQ4K;
   static const int tokens_per_pass = env_flag("SI_HIP_Q4K_BATCH_PASS", 1);
   if (q4_mfma && batch > 1 && tokens_per_pass &&
@@ -58,7 +58,8 @@ bool launch_matvec_tuned(uint32_t type, const uint8_t* w, const float* x, float*
 bool launch_fused_gate_up_tuned(const uint8_t* gate, const uint8_t* up, const float* x, float* h,
                                 uint32_t rows, uint32_t cols, const Workspace& ws, hipStream_t s,
                                 hipError_t* err) {
-  return launch_q4k_gate_up_mfma(gate, up, x, h, rows, cols, ws, s, err);
+  return word_aligned(gate) && word_aligned(up) &&
+         launch_q4k_gate_up_mfma(gate, up, x, h, rows, cols, ws, s, err);
 }
 
 }  // namespace sihip

@@ -10,6 +10,12 @@
 
 namespace sihip {
 
+// Whether the matrix-core kernels can read a matrix that starts at w: their
+// 16-byte copies into LDS need word-aligned addresses.  (A row range or a view
+// of a Q6_K matrix with an odd block count may start 2 bytes off a word; the
+// generic kernels take any address.)
+inline bool word_aligned(const uint8_t* w) { return ((uintptr_t)w & 3u) == 0u; }
+
 bool launch_matvec_tuned(uint32_t type, const uint8_t* w, const float* x, float* y, uint32_t rows,
                          uint32_t cols, uint32_t batch, const Workspace& ws, hipStream_t s,
                          hipError_t* err);

@@ -86,3 +86,33 @@ def test_matvec_cancelling_terms(hip_ctx, t, rows, cols):
         assert_dot_close(y, dq @ x.astype(np.float64), np.abs(dq) @ np.abs(x.astype(np.float64)))
     finally:
         W.free()
+
+
+@pytest.mark.parametrize("rows,cols,start", [(3, 256, 1), (64, 1280, 3), (129, 6912, 5),
+                                             (4097, 1280, 1), (40, 1280, 2)])
+def test_q6k_rows_off_a_word(hip_ctx, rows, cols, start):
+    """Q6_K matrices that start inside another one: with an odd block count an odd
+    row starts 2 bytes off a word, where the copies into LDS cannot."""
+    log(f"q6k rows {start}..{start + rows} of {cols}")
+    total, rb = rows + start + 1, cols // 256 * 210
+    w = si_hip.synth_matrix(14, seed=rows + cols, rows=total, cols=cols, threads=8)
+    part = w[start * rb:(start + rows) * rb]
+    X = si_hip.synth_normal(rows + 7 * cols, 5 * cols).reshape(5, cols).copy()
+    ref = [O.matvec(14, part, rows, cols, X[b], threads=8)[1:] for b in range(5)]
+    W = hip_ctx.upload_quant_weight_private(w, 14)
+    V = W.view(start * rb, rows * rb, 14)
+    try:
+        y = hip_ctx.gguf_quant_matvec_tensor_rows(W, (cols, total), start, rows, X[0])
+        assert_dot_close(y, *ref[0], what="row range")
+        _, logits = hip_ctx.gguf_quant_matvec_argmax_weight(V, rows, cols, X[0])
+        assert_dot_close(logits, *ref[0], what="head")
+        for batch in (2, 5):
+            outs = hip_ctx.gguf_quant_matmul_many_weight(V, rows, cols, batch, X[:batch])
+            for b in range(batch):
+                assert_dot_close(outs[b], *ref[b], what=f"vector {b} of {batch}")
+        both = hip_ctx.gguf_quant_matvec_many_weights([V, V], [rows, rows], cols, X[0])
+        for y in both:
+            assert_dot_close(y, *ref[0], what="group")
+    finally:
+        V.free()
+        W.free()
