@@ -33,9 +33,9 @@
 // with a block whose activations are not finite or reach 2^100; one whose
 // sum is not finite; one with a block whose two terms cancel to below 2^-30
 // of the first, so that f64 rounding could show (weights that all decode to
-// zero); and one whose side elements (mfma_common.h; bounded by half a unit
-// each times the largest weight that d and dmin allow) could be off by more
-// than kStageTol of its sum |block term|.
+// zero); and one whose side elements (bounded by half a unit each times the
+// largest weight that d and dmin allow) could be off by more than they may be
+// (kFewTol, tokens_common.h).
 //
 // Work split.  A launch cuts K into slices of four blocks: workgroup g works
 // on slice g / GS for tiles g % GS, g % GS + GS, ..., keeping that slice's
@@ -352,9 +352,9 @@ __global__ __launch_bounds__(WAVES * 64) void q45_tokens_mfma(const uint8_t* __r
       const uint32_t row = (tg + lt * ta.groups_per_slice) * 16u + n;
 #pragma unroll
       for (int G = 0; G < NG; ++G) {
-        const float part = (float)acc[G], err = most * side[G];
+        const float part = (float)acc[G];
         const bool bad = redo[G] || !(fabsf(part) < __builtin_huge_valf()) ||
-                         !(err * 1.01f <= kStageTol * ((float)sum_abs[G] - err));
+                         !side_ok(most, side[G], (float)sum_abs[G]);
         const uint32_t v = 4u * G + grp;
         if (row < rows && v < ntok)
           part_out[((size_t)k * 4u * NG + v) * rows + row] =

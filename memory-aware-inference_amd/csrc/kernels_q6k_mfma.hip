@@ -577,8 +577,9 @@ __global__ __launch_bounds__(WAVES * 64) void q6k_matvec_mfma(const uint8_t* __r
 // whose sums exceed the scratch runs as several over row ranges.  A (vector,
 // row) that meets a block on the exact path, whose sum is not finite, or
 // whose side elements (half a unit each times 4096 |d|, the largest |w| a
-// block can hold) could be off by more than kRoundedTol of its sum |block
-// term| stores kPartRedo for the slice, and tok_reduce recomputes it exactly.
+// block can hold) could be off by more than they may be (kFewTol,
+// tokens_common.h) stores kPartRedo for the slice, and tok_reduce recomputes it
+// exactly.
 //
 // PAIRED (odd block counts, where a row starts 2 bytes off 4 every second
 // time): the even rows and the odd rows as two matrices of row stride 2 nb
@@ -782,9 +783,9 @@ __global__ __launch_bounds__(WAVES * 64) void q6k_tokens_mfma(const uint8_t* __r
       const uint32_t row = (tg + lt * ta.groups_per_slice) * 16u + n;
 #pragma unroll
       for (int G = 0; G < NG; ++G) {
-        const float part = (float)acc[G], err = most * side[G];
+        const float part = (float)acc[G];
         const bool redo = !(fabsf(part) < __builtin_huge_valf()) ||
-                          !(err * 1.01f <= kRoundedTol * ((float)sum_abs[G] - err));
+                          !side_ok(most, side[G], (float)sum_abs[G]);
         const uint32_t vec = 4u * G + grp;
         if (row < trows && vec < ntok)
           part_out[((size_t)k * 4u * NG + vec) * places + row] =

@@ -37,6 +37,17 @@ __device__ __forceinline__ void lds_write_b16(uint32_t addr, uint32_t v) {
 // zero.
 constexpr int kBadTok = -(1 << 20);
 
+// What a vector's side elements (mfma_common.h) may cost its dot with a row
+// over a slice: 2^-22 of the row's sum |block term| where no block has more
+// than eight of them, which is what the f32 rounding of such sums would be
+// (the terms here are f64), and kRoundedTol of it for the blocks that have
+// more.  A (vector, row) past that takes the slice's exact dot.  (Up to eight
+// per block used to be listed and added from the exact weights; held to
+// kRoundedTol like the rest, a dot that rides on them was up to 7.6e-6 off.)
+// Slices of ordinary activations reach 1e-8 of the sum.
+constexpr uint32_t kFewSide = 8;
+constexpr float kFewTol = 0x1p-22f;
+
 // LDS map of a launch whose workgroups keep up to stride = 4 blocks of ng
 // groups (group g's block b is group-block gb = stride g + b): the
 // group images (4 KB per group-block); with `mins`, the unit sums (256 bytes
@@ -44,7 +55,8 @@ constexpr int kBadTok = -(1 << 20);
 // 64 k + 4 (4 t + p), piece p of vector t); with `dsum`, 128 times each
 // vector's digit sums (64 bytes per group-block, vector t's four at 16 t); per
 // vector v, 4 stride bytes each, the exponents and the bounds on the side
-// elements' rounding (infinite for a block on the exact path).
+// elements' rounding over the tolerance they are held to (kFewTol or
+// kRoundedTol; infinite for a block on the exact path).
 struct TokLayout {
   uint32_t img, usum, dsum, expo, rerr, total;
   uint32_t stride;
@@ -107,6 +119,14 @@ __device__ __forceinline__ uint32_t row_sum_u(uint32_t v) {
   return v + dpp_u<kRowShr8>(v);
 }
 
+// Whether a (vector, row) keeps its sum over the slice: `most` the largest |w|
+// the row's blocks can hold, `side` the vector's slice_err, `sum_abs` the sum of
+// |block term|, which is at most sum|w x| plus the bound itself (under 1 % of
+// it); the factor also covers the f32 rounding here.
+__device__ __forceinline__ bool side_ok(float most, float side, float sum_abs) {
+  return most * side * 1.02f <= sum_abs;
+}
+
 // Turns the wave's share of activations (load_group_x) into images, with what
 // else the layout keeps of them (chunk_digits: about 270 instructions a
 // group-block; a build that summed the side elements' rounding errors and the
@@ -162,16 +182,18 @@ __device__ __forceinline__ void build_group_images64(uint32_t sbase, const TokLa
     }
     const uint32_t nside = row_sum_u(cd.nside);
     if (c == 15u) {
+      const float n = (float)nside * (nside <= kFewSide ? 1.0f / kFewTol : 1.0f / kRoundedTol);
       lds_write_b32(sbase + L.expo + vec, (uint32_t)(cd.bad ? kBadTok : cd.e - kFixBits));
       lds_write_b32(sbase + L.rerr + vec,
                     cd.bad ? 0x7f800000u
-                        : __float_as_uint(__builtin_amdgcn_ldexpf((float)nside, cd.e - kFixBits - 1)));
+                        : __float_as_uint(__builtin_amdgcn_ldexpf(n, cd.e - kFixBits - 1)));
     }
   }
 }
 
-// A vector's bound on the rounding of its side elements over the nbl blocks
-// of the slice (infinite when a block takes the exact path).
+// A vector's bound on the rounding of its side elements, over its tolerance,
+// summed over the nbl blocks of the slice (infinite when a block takes the
+// exact path).
 __device__ __forceinline__ float slice_err(const uint8_t* rerr, uint32_t nbl) {
   const u32x4 v = lds_u32x4(rerr);
   float e = __uint_as_float(v[0]);

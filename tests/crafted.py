@@ -89,3 +89,38 @@ def crafted_x(cols: int, case: str, seed: int) -> np.ndarray:
     else:
         raise ValueError(case)
     return x.reshape(-1).astype(np.float32)
+
+
+def small_dot(t: int, rows: int, cols: int, nside: int = 8):
+    """A matrix of equal blocks and a vector whose dot rides on small
+    activations: per block an activation of 1 on a zero weight, `nside`
+    elements half a fixed-point unit below the side threshold on the largest
+    weight the block's header allows (each rounds up by that half unit, 2^-17
+    of itself), and for Q6_K nine more exactly on the threshold."""
+    blk = np.zeros((1, BLOCK[t]), np.uint8)
+    half = np.array([0.01], np.float16).view(np.uint8)
+    pos = 3 + 11 * np.arange(nside)
+    kept = 2 + 11 * np.arange(9 if t == 14 else 0)
+    if t == 14:
+        blk[:, 128:192] = 0xAA        # q = 32 everywhere
+        blk[:, 192:208] = 127
+        blk[:, 208:210] = half
+    else:
+        blk[:, 0:2] = half
+        blk[:, 4:8] = 0xFF            # every scale 63, every min 0
+        blk[:, 12:16] = 0x0F
+    for i in np.concatenate([pos, kept]).astype(int):
+        if t == 14:
+            h, t4, l = i // 128, (i % 128) // 32, i % 32
+            _set_nibble(blk, 64 * h + l + 32 * (t4 & 1), t4 >> 1, 15)
+            blk[:, 128 + 32 * h + l] |= np.uint8(3 << (2 * t4))
+        else:
+            u, l = i // 32, i % 32
+            _set_nibble(blk, (16 if t == 12 else 48) + 32 * (u // 2) + l, u & 1, 15)
+            if t == 13:
+                blk[:, 16 + l] |= np.uint8(1 << u)
+    x = np.zeros((cols // 256, 256), np.float32)
+    x[:, 0] = 1.0
+    x[:, pos] = 65535.5 * 2.0 ** -29
+    x[:, kept] = 2.0 ** -13
+    return np.tile(blk, (rows * (cols // 256), 1)).reshape(-1), x.reshape(-1)

@@ -13,6 +13,7 @@ category that per-weight f32 products give.
 import numpy as np
 import pytest
 
+import crafted
 import oracle_lib as O
 import si_hip
 from test_gpu_parity import _category, assert_dot_close, log, same_bits
@@ -115,4 +116,24 @@ def test_q6k_rows_off_a_word(hip_ctx, rows, cols, start):
             assert_dot_close(y, *ref[0], what="group")
     finally:
         V.free()
+        W.free()
+
+
+@pytest.mark.parametrize("t,cols", [(12, 2048), (13, 2304), (14, 2048), (14, 2304)])
+@pytest.mark.parametrize("batch", [2, 4, 5, 16])
+def test_verify_dot_on_small_activations(hip_ctx, t, cols, batch):
+    """A dot that eight side elements a block carry keeps f32 precision: they may
+    cost 2^-22 of sum|w*x|, and each slice of four blocks and the sum over the
+    slices round once to f32 (2^-24)."""
+    rows = 20
+    w, x = crafted.small_dot(t, rows, cols)
+    _, y64, ab = O.matvec(t, w, rows, cols, x, threads=8)
+    assert ab.min() > 0.0
+    slices = (cols // 256 + 4) // 4
+    W = hip_ctx.upload_quant_weight_private(w, t)
+    try:
+        outs = hip_ctx.gguf_quant_matmul_many_weight(W, rows, cols, batch, np.stack([x] * batch))
+        for b in range(batch):
+            assert_dot_close(outs[b], y64, ab, 2.0 ** -22 + (slices + 1) * 2.0 ** -24, f"vector {b}")
+    finally:
         W.free()
