@@ -568,7 +568,7 @@ __device__ __forceinline__ float stage_rowsum(const StageRegs<QB, SB>& v, uint32
     float apart = 0.0f;
 #pragma unroll
     for (int b = 0; b < SB; ++b) apart += fabsf(part[b]);
-    redo |= !stage_ok(err, apart);
+    redo |= !rounded_ok(err, apart);
   }
   float sum = (float)acc;
   if (bad_any || __builtin_amdgcn_ballot_w64(redo) != 0u) {

@@ -65,12 +65,6 @@ constexpr uint32_t kSideRounded = 0xffu;  // side count of a rounded block
 // A row's stage passes when (error bound) * 1.01 <= kRoundedTol *
 // (sum |partial| - error bound); 1.01 covers the f32 rounding of both sums.
 constexpr float kRoundedTol = 4e-6f;
-// The Q4_K / Q5_K kernels form a block's terms in f64 from exact integers, so
-// their rounded blocks' bound has kStageTol of the row's sum |partial| to
-// itself.  With the fixed point's 2^-17 on kept elements and the f32
-// accumulation of the partials (under 3e-6) the dot stays within
-// 2e-5 * sum|w x|.
-constexpr float kStageTol = 8e-6f;
 // A stage partial the vectors-in-rows kernel leaves for its reduce kernel to
 // recompute exactly (its lane failed the stage check): a signalling-NaN
 // pattern, which no arithmetic result has.
@@ -470,15 +464,6 @@ __device__ __forceinline__ float rounded_bound(uint32_t list, uint32_t rmask, ui
   return err;
 }
 
-// The rounded-block check of the Q4_K / Q5_K kernels: whether the row of this
-// lane passes with `err`, the lane's bound on the error of its rounded
-// blocks, and `abs_part`, its sum of |partial| (both summed over the row's
-// four lane groups here).  A row that fails recomputes the stage on the
-// exact per-weight path.
-__device__ __forceinline__ bool stage_ok(float err, float abs_part) {
-  const float e = sum_lane_groups(err), a = sum_lane_groups(abs_part);
-  return e * 1.01f <= kStageTol * (a - e);
-}
 // The f64 difference p of a block's two terms, the first of them `first`: whether
 // its rounding (2^-52 of the first term) can show, that is p below 2^-30 of
 // it -- weights that cancel inside their own decode -- or not a number.

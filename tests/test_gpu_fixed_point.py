@@ -123,3 +123,20 @@ def test_crafted_head_argmax(ctx, case):
     if top2[1] - top2[0] > 4e-5 * ab.max():
         assert token == int(np.argmax(y64))
     assert token == int(np.argmax(logits))
+
+
+@pytest.mark.parametrize("t", [12, 13])
+@pytest.mark.parametrize("rows,cols", [(20, 2048), (640, 17408), (8192, 8192), (17408, 5120)])
+def test_dot_on_small_activations(hip_ctx, t, rows, cols):
+    """A dot that eight side elements a block carry, one vector: their rounding may
+    cost 4e-6 of sum|w*x|, and at most 34 f32 partials of one sign are added up
+    (2^-24 each; a row of 68 blocks is at least four slices)."""
+    log(f"small activations t={t} {rows}x{cols}")
+    w, x = crafted.small_dot(t, rows, cols)
+    _, y64, ab = O.matvec(t, w, rows, cols, x, threads=8)
+    W = hip_ctx.upload_quant_weight_private(w, t)
+    try:
+        y = hip_ctx.gguf_quant_matvec_weight(W, rows, cols, x)
+        assert_dot_close(y, y64, ab, 4e-6 + 34 * 2.0 ** -24, f"type {t} {rows}x{cols}")
+    finally:
+        W.free()
