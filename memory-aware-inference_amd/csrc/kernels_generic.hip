@@ -147,10 +147,9 @@ __device__ __forceinline__ float4 decode_four_exact(const uint8_t* __restrict__ 
 }
 
 // Exact dequantisation of whole blocks, four elements a thread, so that a
-// wave's loads are a block's consecutive words and its stores whole lines; a
-// workgroup takes 1024 consecutive elements (chunk blockIdx.x % chunks) of
-// one output row, so the row's index and the division are uniform.  (One
-// 32-weight unit a thread, its bytes loaded one by one and 64-bit divisions
+// wave's loads are a block's consecutive words and its stores whole lines;
+// workgroup (c, r) takes 1024 consecutive elements (chunk c) of output row r.
+// (One 32-weight unit a thread, its bytes loaded one by one and 64-bit divisions
 // per thread: 64 rows of 5120 4.1 us by kernel trace, of which an empty launch
 // is 1.7; so 2.7.)
 // `row_index` (optional) maps output row r to source row row_index[r]
@@ -161,11 +160,9 @@ template <uint32_t T>
 __global__ __launch_bounds__(256) void dequant_kernel(const uint8_t* __restrict__ w,
                                                       const uint32_t* __restrict__ row_index,
                                                       float* __restrict__ out, uint32_t nb,
-                                                      uint32_t chunks, uint32_t table_rows,
-                                                      void* ws) {
+                                                      uint32_t table_rows, void* ws) {
   constexpr uint32_t BB = BlockBytes<T>::value;
-  const uint32_t r = blockIdx.x / chunks, chunk = blockIdx.x - r * chunks;
-  const uint32_t blk = 4u * chunk + (threadIdx.x >> 6);
+  const uint32_t r = blockIdx.y, blk = 4u * blockIdx.x + (threadIdx.x >> 6);
   if (blk >= nb) return;
   const uint64_t src_row = row_index ? row_index[r] : r;
   const uint32_t i = 4u * (threadIdx.x & 63u);
@@ -220,35 +217,43 @@ hipError_t launch_fused_gate_up_generic(const uint8_t* gate, const uint8_t* up, 
 hipError_t launch_dequant(uint32_t type, const uint8_t* w, const uint32_t* row_index, float* out,
                           uint32_t out_rows, uint32_t cols, hipStream_t s, uint32_t table_rows,
                           void* ws) {
+  const uint64_t row_blocks = cols / kBlockElems;
+  if (row_blocks == 0u || out_rows == 0u) return hipErrorInvalidValue;
   // without an index the rows follow each other: one row of all their blocks
-  uint64_t nb = cols / kBlockElems, nrows = out_rows;
-  if (row_index == nullptr) {
-    nb *= nrows;
-    nrows = 1u;
-    table_rows = 1u;
+  const uint64_t nb = row_index ? row_blocks : row_blocks * out_rows;
+  const uint64_t nrows = row_index ? out_rows : 1u;
+  if (!row_index) table_rows = 1u;
+  // A launch takes less than 2^32 threads and 2^16 workgroups in y; more rows
+  // (or blocks of the one row) run as several.
+  constexpr uint64_t kRows = 32768u, kBlocks = 1u << 24;
+  for (uint64_t r0 = 0; r0 < nrows; r0 += kRows) {
+    for (uint64_t b0 = 0; b0 < nb; b0 += row_index ? nb : kBlocks) {
+      // (an indexed row's blocks, less than 2^24, are one launch's)
+      const uint32_t n = (uint32_t)(row_index ? nb : min(nb - b0, kBlocks));
+      const uint32_t* const ids = row_index ? row_index + r0 : nullptr;
+      float* const o = out + (r0 * nb + b0) * kBlockElems;
+      const dim3 grid((n + 3u) / 4u, (uint32_t)min(nrows - r0, kRows));
+      switch (type) {
+        case kTypeQ4K:
+          hipLaunchKernelGGL(dequant_kernel<kTypeQ4K>, grid, dim3(256), 0, s, w + b0 * kQ4Bytes,
+                             ids, o, n, table_rows, ws);
+          break;
+        case kTypeQ5K:
+          hipLaunchKernelGGL(dequant_kernel<kTypeQ5K>, grid, dim3(256), 0, s, w + b0 * kQ5Bytes,
+                             ids, o, n, table_rows, ws);
+          break;
+        case kTypeQ6K:
+          hipLaunchKernelGGL(dequant_kernel<kTypeQ6K>, grid, dim3(256), 0, s, w + b0 * kQ6Bytes,
+                             ids, o, n, table_rows, ws);
+          break;
+        default:
+          return hipErrorInvalidValue;
+      }
+      const hipError_t e = hipGetLastError();
+      if (e != hipSuccess) return e;
+    }
   }
-  const uint64_t groups = nrows * ((nb + 3u) / 4u);
-  if (nb == 0u || nb > 0xfffffffcu || groups == 0u || groups > 0x7fffffffu)
-    return hipErrorInvalidValue;
-  const uint32_t chunks = (uint32_t)((nb + 3u) / 4u);
-  const dim3 grid((uint32_t)groups);
-  switch (type) {
-    case kTypeQ4K:
-      hipLaunchKernelGGL(dequant_kernel<kTypeQ4K>, grid, dim3(256), 0, s, w, row_index, out,
-                         (uint32_t)nb, chunks, table_rows, ws);
-      break;
-    case kTypeQ5K:
-      hipLaunchKernelGGL(dequant_kernel<kTypeQ5K>, grid, dim3(256), 0, s, w, row_index, out,
-                         (uint32_t)nb, chunks, table_rows, ws);
-      break;
-    case kTypeQ6K:
-      hipLaunchKernelGGL(dequant_kernel<kTypeQ6K>, grid, dim3(256), 0, s, w, row_index, out,
-                         (uint32_t)nb, chunks, table_rows, ws);
-      break;
-    default:
-      return hipErrorInvalidValue;
-  }
-  return hipGetLastError();
+  return hipSuccess;
 }
 
 }  // namespace sihip

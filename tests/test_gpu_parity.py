@@ -5,6 +5,7 @@ f32 dot within 2e-5 * sum|w*x| of the f64 value of the exact products;
 greedy argmax identical.  Tests that restate the reference's own Metal tests
 (src/metal.rs:7445-7602) keep their inputs and tolerances.
 """
+import ctypes
 import gc
 import json
 import struct
@@ -1106,3 +1107,32 @@ def test_graph_capture_state_errors(hip_ctx):
         g = hip_ctx.capture_end()
     assert g.calls == 0
     g.free()
+
+
+@pytest.mark.parametrize("tokens,cols", [(32769, 512), (70001, 256), ((1 << 24) + 3, 256)])
+def test_embedding_many_tokens(hip_ctx, tokens, cols):
+    """More tokens than one launch's workgroups reach: the rows at both ends, at
+    the edges of a launch's share and at the most that 2^32 threads would cover."""
+    log(f"embedding {tokens} x {cols}")
+    vocab = 5
+    table = si_hip.synth_matrix(12, seed=tokens, rows=vocab, cols=cols)
+    exp = O.dequantize(12, table, vocab * cols).reshape(vocab, cols).view(np.uint32)
+    ids = (np.arange(tokens, dtype=np.uint32) * np.uint32(7)) % np.uint32(vocab)
+    T = hip_ctx.upload_quant_weight_private(table, 12)
+    d_ids = hip_ctx.device_alloc(4 * tokens)
+    d_out = hip_ctx.device_alloc(4 * tokens * cols)
+    try:
+        hip_ctx.to_device(d_ids, ids)
+        rc = si_hip.lib().si_hip_embedding_device(hip_ctx.handle, T.handle, cols, vocab,
+                                                  ctypes.c_void_p(d_ids), tokens,
+                                                  ctypes.c_void_p(d_out))
+        assert rc == 0, si_hip.last_error()
+        hip_ctx.synchronize()
+        for at in (0, 32766, 65534, (1 << 24) - 2, tokens - 4):
+            if at + 4 <= tokens:
+                got = hip_ctx.from_device(d_out + 4 * at * cols, 4 * cols).view(np.uint32)
+                assert np.array_equal(got.reshape(4, cols), exp[ids[at:at + 4]]), at
+    finally:
+        hip_ctx.device_free(d_ids)
+        hip_ctx.device_free(d_out)
+        T.free()
