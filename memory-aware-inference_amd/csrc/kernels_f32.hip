@@ -217,15 +217,21 @@ void launch_norm_units(const float* x, const float* gate, const float* w, float*
   auto threads = [&](uint32_t upt) {
     return (uint32_t)min((uint64_t)1024u, (((uint64_t)n + upt - 1u) / upt + 63u) / 64u * 64u);
   };
+  auto launch = [&](auto upt, auto kernel) {
+    // (a launch takes less than 2^32 threads: more heads run as several)
+    const uint32_t t = threads(upt), most = 0xffffffffu / t;
+    for (uint32_t h0 = 0; h0 < heads; h0 += min(most, heads - h0)) {
+      const size_t at = (size_t)h0 * head_dim;
+      hipLaunchKernelGGL(kernel, dim3(min(most, heads - h0)), dim3(t), 0, s, x + at,
+                         gate ? gate + at : nullptr, w, y + at, head_dim, eps);
+    }
+  };
   if (n <= 1024u)
-    hipLaunchKernelGGL((rms_norm_kernel<MODE, U, 1>), dim3(heads), dim3(threads(1u)), 0, s, x, gate,
-                       w, y, head_dim, eps);
+    launch(1u, &rms_norm_kernel<MODE, U, 1>);
   else if (n <= 2048u)
-    hipLaunchKernelGGL((rms_norm_kernel<MODE, U, 2>), dim3(heads), dim3(threads(2u)), 0, s, x, gate,
-                       w, y, head_dim, eps);
+    launch(2u, &rms_norm_kernel<MODE, U, 2>);
   else
-    hipLaunchKernelGGL((rms_norm_kernel<MODE, U, 4>), dim3(heads), dim3(threads(4u)), 0, s, x, gate,
-                       w, y, head_dim, eps);
+    launch(4u, &rms_norm_kernel<MODE, U, 4>);
 }
 
 template <int MODE>

@@ -369,3 +369,31 @@ def test_rms_norm_register_passes(hip_ctx, mode, heads, hd):
     else:
         y = hip_ctx.rms_norm_gated(x, g, w, heads, hd, 1e-6)
     assert_rms_close(y, f64_rms(mode, x, w, heads, hd, 1e-6, g), f"mode {mode}")
+
+
+@pytest.mark.gpu
+def test_rms_norm_many_heads(hip_ctx):
+    """More heads than 2^32 threads cover at 832 a head: the first, the last and
+    those at the edge of a launch's share."""
+    hd, heads = 769, 2 ** 32 // 832 + 3
+    print(f"rms_norm {heads} heads of {hd}", flush=True)
+    rng = np.random.default_rng(11)
+    x = rng.standard_normal((3, hd)).astype(np.float32)
+    w = rng.standard_normal(hd).astype(np.float32)
+    at = [0, heads - 5, heads - 1]
+    dx, dw, dy = (hip_ctx.device_alloc(4 * n) for n in (heads * hd, hd, heads * hd))
+    try:
+        hip_ctx.to_device(dw, w)
+        for h, v in zip(at, x):
+            hip_ctx.to_device(dx + 4 * h * hd, v)
+            hip_ctx.to_device(dy + 4 * h * hd, np.full(hd, np.nan, np.float32))
+        rc = si_hip.lib().si_hip_rms_norm_device(hip_ctx.handle, 1, C.c_void_p(dx), None,
+                                                 C.c_void_p(dw), heads, hd, C.c_float(1e-6),
+                                                 C.c_void_p(dy))
+        assert rc == 0, si_hip.last_error()
+        hip_ctx.synchronize()
+        y = np.concatenate([hip_ctx.from_device(dy + 4 * h * hd, hd) for h in at])
+        assert_rms_close(y, f64_rms(1, x.reshape(-1), w, 3, hd, 1e-6, None), "many heads")
+    finally:
+        for p in (dx, dw, dy):
+            hip_ctx.device_free(p)
