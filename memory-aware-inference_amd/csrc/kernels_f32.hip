@@ -40,17 +40,17 @@ __device__ __forceinline__ void clear(float4& p) { p = make_float4(0.0f, 0.0f, 0
 // y[r] = sum_c w[r * cols + c] * x[c], WPR waves per row: thread t of the
 // row's 64 WPR takes units t, t + 64 WPR, ... of the row's n (a unit is a
 // float4 where cols % 4 == 0 and w, x are 16-byte aligned, else a float),
-// eight at a time with all their loads in flight, in two accumulators; then
-// the waves' sums are added in wave order.  One wave a row and two loads in
-// flight took 48 x 5120 (the gates beside a block's norm) 5.0 us, a row's ten
-// dependent trips to memory; sixteen waves a row, two loads a thread, 2.0 us.
-template <typename U, int WPR>
+// FLIGHT (1, 2 or 8) at a time with all their loads in flight, in two
+// accumulators; then the waves' sums are added in wave order.  One wave a row and
+// two loads in flight took 48 x 5120 (the gates beside a block's norm) 5.0 us, a
+// row's ten dependent trips to memory; sixteen waves a row, two loads a thread,
+// 2.0 us.
+template <typename U, int WPR, int FLIGHT>
 __global__ __launch_bounds__(WPR > 4 ? 64 * WPR : 256) void f32_matvec_kernel(
     const float* __restrict__ w, const float* __restrict__ x, float* __restrict__ y,
     uint32_t rows, uint32_t cols) {
   constexpr uint32_t kRows = WPR > 4 ? 1u : 4u / WPR;  // rows per workgroup
   constexpr uint32_t kStep = 64u * WPR;
-  constexpr int kFlight = 8;
   __shared__ float red[WPR > 4 ? WPR : 4];
   const uint32_t wave = threadIdx.x >> 6, lane = threadIdx.x & 63u;
   const uint32_t row = blockIdx.x * kRows + wave / WPR;
@@ -60,10 +60,10 @@ __global__ __launch_bounds__(WPR > 4 ? 64 * WPR : 256) void f32_matvec_kernel(
     const U* const xr = reinterpret_cast<const U*>(x);
     const uint32_t n = cols / (uint32_t)(sizeof(U) / sizeof(float));
     float a0 = 0.0f, a1 = 0.0f;
-    for (size_t i = (wave % WPR) * 64u + lane; i < n; i += kFlight * kStep) {
-      U p[kFlight], q[kFlight];
+    for (size_t i = (wave % WPR) * 64u + lane; i < n; i += FLIGHT * kStep) {
+      U p[FLIGHT], q[FLIGHT];
 #pragma unroll
-      for (int k = 0; k < kFlight; ++k) {
+      for (int k = 0; k < FLIGHT; ++k) {
         const size_t j = i + (uint32_t)k * kStep;
         clear(p[k]);
         clear(q[k]);
@@ -73,7 +73,7 @@ __global__ __launch_bounds__(WPR > 4 ? 64 * WPR : 256) void f32_matvec_kernel(
         }
       }
 #pragma unroll
-      for (int k = 0; k < kFlight; ++k) fma_unit(p[k], q[k], (k & 1) ? a1 : a0);
+      for (int k = 0; k < FLIGHT; ++k) fma_unit(p[k], q[k], (k & 1) ? a1 : a0);
     }
     total = wave_sum(a0 + a1);
   }
@@ -89,14 +89,24 @@ __global__ __launch_bounds__(WPR > 4 ? 64 * WPR : 256) void f32_matvec_kernel(
   }
 }
 
-// The workgroup's sum of per-wave partials, in wave order, in every thread.
-__device__ __forceinline__ float group_sum(float v, float* red) {
-  const uint32_t wave = threadIdx.x >> 6, lane = threadIdx.x & 63u;
+// The workgroup's sum of per-wave partials, in wave order, in every thread (at
+// most 16 waves; the slots of waves it does not have hold zero, so that all the
+// reads go out at once).
+__device__ __forceinline__ float group_sum(float v, float4 (&red)[4]) {
+  const uint32_t wave = threadIdx.x >> 6, lane = threadIdx.x & 63u, waves = blockDim.x >> 6;
   v = wave_sum(v);
-  if (lane == 0u) red[wave] = v;
+  float* const slot = reinterpret_cast<float*>(red);
+  if (lane == 0u) slot[wave] = v;
+  if (wave == 0u && lane >= waves && lane < 16u) slot[lane] = 0.0f;
   __syncthreads();
-  float t = red[0];
-  for (uint32_t k = 1; k < blockDim.x / 64u; ++k) t += red[k];
+  const float4 a = red[0];
+  float t = ((a.x + a.y) + a.z) + a.w;
+  if (waves > 4u) {
+    const float4 b = red[1], c = red[2], d = red[3];
+    t = (((t + b.x) + b.y) + b.z) + b.w;
+    t = (((t + c.x) + c.y) + c.z) + c.w;
+    t = (((t + d.x) + d.y) + d.z) + d.w;
+  }
   return t;
 }
 
@@ -138,7 +148,7 @@ __global__ __launch_bounds__(1024) void rms_norm_kernel(const float* __restrict_
                                                         const float* __restrict__ w,
                                                         float* __restrict__ y, uint32_t head_dim,
                                                         float eps) {
-  __shared__ float red[16];
+  __shared__ float4 red[4];
   const size_t base = (size_t)blockIdx.x * head_dim;
   const U* const xu = reinterpret_cast<const U*>(x + base);
   const U* const gu = reinterpret_cast<const U*>(MODE == 2 ? gate + base : x + base);
@@ -185,12 +195,22 @@ __global__ __launch_bounds__(1024) void rms_norm_kernel(const float* __restrict_
 
 bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0u; }
 
+// Rows that give each thread at most one or two units take the kernel with as
+// many loads unrolled: the code of eight alone costs such a launch 0.1-1.4 us
+// (64 x 24 3.06 us with eight, 2.64 with one; 20000 x 128 5.17, 3.77; 6600 x 512
+// 3.70 with eight, 3.42 with two).
 template <typename U, int WPR>
 void launch_matvec_as(const float* w, const float* x, float* y, uint32_t rows, uint32_t cols,
                       hipStream_t s) {
   constexpr uint32_t kRows = WPR > 4 ? 1u : 4u / WPR;
-  hipLaunchKernelGGL((f32_matvec_kernel<U, WPR>), dim3((rows + kRows - 1u) / kRows),
-                     dim3(WPR > 4 ? 64 * WPR : 256), 0, s, w, x, y, rows, cols);
+  const dim3 grid((rows + kRows - 1u) / kRows), block(WPR > 4 ? 64 * WPR : 256);
+  const uint32_t n = cols / (uint32_t)(sizeof(U) / sizeof(float));
+  if (n <= 64u * WPR)
+    hipLaunchKernelGGL((f32_matvec_kernel<U, WPR, 1>), grid, block, 0, s, w, x, y, rows, cols);
+  else if (n <= 128u * WPR)
+    hipLaunchKernelGGL((f32_matvec_kernel<U, WPR, 2>), grid, block, 0, s, w, x, y, rows, cols);
+  else
+    hipLaunchKernelGGL((f32_matvec_kernel<U, WPR, 8>), grid, block, 0, s, w, x, y, rows, cols);
 }
 // Waves per row: as many (up to 16) as give the row's waves a unit each while
 // all rows' waves stay within eight a CU (2048), else one.

@@ -341,6 +341,9 @@ def test_rms_norm_device_and_extremes(hip_ctx):
     (512, 1028), (256, 2052),      # four and eight waves a row
     (128, 4100), (129, 4097),      # sixteen; eight, in single floats
     (5, 64 * 16 * 8 * 4 + 4),      # a second pass of eight loads, one unit long
+    (3000, 64), (3000, 65), (3000, 127), (3000, 129),  # one, two and eight loads, in floats
+    (2049, 256), (2049, 260), (2049, 512), (2049, 516),  # and in float4s
+    (7, 1), (7, 4),
 ])
 def test_f32_matvec_wave_splits(hip_ctx, rows, cols):
     rng = np.random.default_rng(rows * 7 + cols)
