@@ -560,8 +560,8 @@ __device__ __forceinline__ float stage_rowsum(const StageRegs<QB, SB>& v, uint32
   const uint32_t counts = live_counts(__builtin_amdgcn_readfirstlane(cnt), nlive);
   const uint32_t rmask = rounded_mask(counts);
   if (rmask != 0u) {
-    const uint32_t list = sbase + L.expo + L.side_off + (uint32_t)SB * kSideBytes * ls;
-    const float err = rounded_bound<SB>(list, rmask, grp, [&](auto b) {
+    const uint32_t list = sbase + L.expo + L.side_off + (uint32_t)SB * kSideCountBytes * ls;
+    const float err = rounded_bound<SB>(list, rmask, grp, ex, [&](auto b) {
       return k4_bound<QB == 5 ? 31 : 15>(
           v.decode(decltype(b)::value, hi_units, bsh, rot_lo, rot_hi));
     });

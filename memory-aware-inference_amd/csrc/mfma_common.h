@@ -9,9 +9,9 @@
 // A block with smaller non-zero elements ("side" elements) is a "rounded"
 // block (side count kSideRounded), so that the dot stays within its bar of
 // 2e-5 * sum|w x| for any weights: the side elements stay in the fixed point,
-// rounded like the rest, and the block keeps, per 16-element chunk, a bound on
-// the sum of their rounding errors (half a unit 2^(e_b - 30) each).  The kernel
-// bounds a row's error from those blocks by (largest |w| the block header
+// rounded like the rest, and the block keeps, per 16-element chunk, their
+// number (each is off by at most half a unit 2^(e_b - 30)) or the bound that
+// gives.  The kernel bounds a row's error from those blocks by (largest |w| the block header
 // allows) x (that bound), and compares it with the sum of |partial dot| over the row's
 // stage, which is at most sum|w x| over the stage.  A row whose bound exceeds
 // kRoundedTol of it recomputes its rounded blocks exactly.  (The kernels of
@@ -55,12 +55,17 @@ constexpr int kBufferWord3 = 0x00020000;  // raw dword access (CDNA buffer descr
 constexpr int kFixBits = 30;
 constexpr uint32_t kLdsBytes = 163840u;
 constexpr int kBadBlock = 0x40000000;  // exponent slot of a block taking the exact path
-// Side elements: non-zero |x| below 2^(e_b - kSideShift).  Each block has
-// kSideBytes of LDS: for a rounded block, 16 f32 error bounds, that of chunk c
-// at position 4 p + t for the chunk in MFMA t of lane group p (the four of a
-// lane group side by side).
+// Side elements: non-zero |x| below 2^(e_b - kSideShift).  A rounded block has
+// 16 bounds on the rounding of its chunks, that of chunk c at position 4 p + t
+// for the chunk in MFMA t of lane group p (the four of a lane group side by
+// side): f32 in kSideBytes of LDS or, in layouts with unit sums (Q4_K, Q5_K),
+// the chunk's count of side elements in a byte, kSideCountBytes.  (With f32
+// bounds beside the f64 unit sums rows of 72 blocks had no room for eight waves
+// of Q4_K: a group of 800 + 96 + 143 rows 22.5 us, 11.7 with bytes; Q5_K 8192 x
+// 24832 142 us, 45.  In the Q6_K kernel, which has no unit sums, bytes cost 1 %
+// at twelve waves: 24000 x 16384 69.2 us, 70.0.)
 constexpr int kSideShift = 14;
-constexpr uint32_t kSideBytes = 64;
+constexpr uint32_t kSideBytes = 64, kSideCountBytes = 16;
 constexpr uint32_t kSideRounded = 0xffu;  // side count of a rounded block
 // A row's stage passes when (error bound) * 1.01 <= kRoundedTol *
 // (sum |partial| - error bound); 1.01 covers the f32 rounding of both sums.
@@ -82,7 +87,7 @@ constexpr int waitcnt_vm(int n) { return (n & 0xf) | ((n >> 4) << 14) | (0x7 << 
 // Block metadata (at expo): the exponents
 // [block] (4 bytes each, at most kMaxMetaBlocks blocks), at +kCountOff the
 // side counts, one byte per block, and at +side_off the side areas
-// [block][kSideBytes].  The counts of the bps blocks of a stage sit at
+// [block][side bytes].  The counts of the bps blocks of a stage sit at
 // kCountOff + 4 bps s, exactly kCountOff past the stage's exponents, so a
 // kernel reads both from one address register (bytes of blocks past the
 // matrix are not written; readers mask them).
@@ -93,6 +98,9 @@ struct Layout {
   uint32_t side_off, bps;  // side areas in the metadata; blocks per stage
   bool sums;               // unit sums are kept
 };
+__host__ __device__ constexpr uint32_t side_bytes(const Layout& l) {
+  return l.sums ? kSideCountBytes : kSideBytes;
+}
 __host__ __device__ constexpr Layout make_layout(uint32_t stage_bytes, uint32_t stage_blocks,
                                                  uint32_t xsum_per_block, uint32_t waves,
                                                  uint32_t depth, uint32_t nb, uint32_t slots,
@@ -106,7 +114,7 @@ __host__ __device__ constexpr Layout make_layout(uint32_t stage_bytes, uint32_t 
   l.img = waves * depth * stage_bytes;
   l.xsum = l.img + nb * 1024u + 4096u;
   l.expo = l.xsum + (xsum_per_block ? nb * xsum_per_block + 256u : 0u);
-  l.part = l.expo + l.side_off + nb * kSideBytes + 16u;
+  l.part = l.expo + l.side_off + nb * side_bytes(l) + 16u;
   l.cnt = l.part + slots * partials * 64u;
   l.owner = l.cnt + slots * 4u;
   l.ready = l.owner + slots * 4u;  // count of image builders done (16 bytes)
@@ -362,7 +370,7 @@ __device__ __forceinline__ void build_images(uint32_t sbase, const Layout& L, ui
     lds_read4<16>(sbase + img + 1024u * pbc + 64u * n, xq);
     const ChunkDigits cd = chunk_digits([&](int k) { return xq[k >> 2][k & 3]; });
     const bool store = pb < nb;
-    const uint32_t list = sbase + sdb + kSideBytes * pb;
+    const uint32_t list = sbase + sdb + side_bytes(L) * pb;
     const bool rounded =
         !cd.bad && ((__builtin_amdgcn_ballot_w64(cd.nside != 0u) >> (16u * grp)) & 0xffffull);
     const auto& dg = cd.dg;
@@ -373,9 +381,14 @@ __device__ __forceinline__ void build_images(uint32_t sbase, const Layout& L, ui
 #pragma unroll
       for (int d = 0; d < 4; ++d)
         lds_write_b128(ib + 16u * d, u32x4{dg[0][d], dg[1][d], dg[2][d], dg[3][d]});
-      if (rounded)  // position 4 p + t
-        lds_write_b32(list + 4u * (4u * ((slot >> 6) & 3u) + (slot >> 8)),
-                      __float_as_uint(__builtin_amdgcn_ldexpf((float)cd.nside, cd.e - kFixBits - 1)));
+      if (rounded) {
+        const uint32_t at = 4u * ((slot >> 6) & 3u) + (slot >> 8);  // position 4 p + t
+        if (L.sums)
+          lds_write_b8(list + at, cd.nside);
+        else
+          lds_write_b32(list + 4u * at, __float_as_uint(__builtin_amdgcn_ldexpf(
+                                            (float)cd.nside, cd.e - kFixBits - 1)));
+      }
     }
     if (L.sums) {
       // unit n / 2, whose two chunks meet in the odd lane: exact
@@ -403,12 +416,18 @@ __device__ __forceinline__ bool rounded_ok(float err, float abs_part) {
   const float e = sum_lane_groups(err), a = sum_lane_groups(abs_part);
   return e * 1.01f <= kRoundedTol * (a - e);
 }
-// Sum of a rounded block's error sums over the four chunks of lane group p.
+// The bound on the rounding of a rounded block's side elements over the four
+// chunks of lane group p: the sum of their f32 bounds, or half a unit for each
+// counted (eb: the block's exponent e_b - 30).
 __device__ __forceinline__ float rounded_err(uint32_t list, uint32_t p) {
   u32x4 v;
   asm volatile("ds_read_b128 %0, %1\ns_waitcnt lgkmcnt(0)" : "=&v"(v) : "v"(list + 16u * p) : "memory");
   return (__uint_as_float(v[0]) + __uint_as_float(v[1])) +
          (__uint_as_float(v[2]) + __uint_as_float(v[3]));
+}
+__device__ __forceinline__ float counted_err(uint32_t list, uint32_t p, int eb) {
+  const uint32_t n = lds_read_b32(list + 4u * p);
+  return __builtin_amdgcn_ldexpf((float)__builtin_amdgcn_sdot4((int)n, 0x01010101, 0, false), eb - 1);
 }
 
 // f(integral_constant<int, I>) for I = 0 .. N-1, so that register arrays are
@@ -451,15 +470,17 @@ __device__ __forceinline__ uint32_t rounded_redo(uint32_t list, uint32_t counts,
 }
 
 // The lane's error bound from the rounded blocks of a stage (rmask: bit b
-// for a rounded block b): the largest |w| of its share of the block times
-// that share's rounding-error sum.
+// for a rounded block b) whose side elements are counted: the largest |w| of its
+// share of the block times the bound on that share's rounding (ex[b]: the
+// block's exponent).
 template <int NB, typename Bound>
 __device__ __forceinline__ float rounded_bound(uint32_t list, uint32_t rmask, uint32_t grp,
-                                               Bound bound) {
+                                               const i32x4& ex, Bound bound) {
   float err = 0.0f;
   static_for<NB>([&](auto bc) {
     constexpr int b = decltype(bc)::value;
-    if ((rmask >> b) & 1u) err = fmaf(bound(bc), rounded_err(list + kSideBytes * b, grp), err);
+    if ((rmask >> b) & 1u)
+      err = fmaf(bound(bc), counted_err(list + kSideCountBytes * b, grp, ex[b]), err);
   });
   return err;
 }

@@ -140,3 +140,27 @@ def test_dot_on_small_activations(hip_ctx, t, rows, cols):
         assert_dot_close(y, y64, ab, 4e-6 + 34 * 2.0 ** -24, f"type {t} {rows}x{cols}")
     finally:
         W.free()
+
+
+@pytest.mark.parametrize("t,nb", [(12, 70), (12, 72), (12, 74), (12, 98), (13, 72), (13, 96),
+                                  (13, 98), (13, 128)])
+@pytest.mark.parametrize("case", ["tiny", "many"])
+def test_crafted_rows_that_fill_the_lds(hip_ctx, case, t, nb):
+    """Rows about as long as eight and four waves' launches hold: blocks that pass
+    on their counted side elements and blocks that are redone, alone and in a
+    group."""
+    rows, cols = [64, 1000], 256 * nb
+    log(f"crafted long rows {case} t={t} {rows} x {cols}")
+    ws = [crafted.zero_weight_matrix(t, r, cols, seed=nb + k) for k, r in enumerate(rows)]
+    x = crafted.crafted_x(cols, case, seed=nb)
+    x[-256:] = si_hip.synth_normal(nb, 256)
+    Ws = [hip_ctx.upload_quant_weight_private(w, t) for w in ws]
+    try:
+        outs = hip_ctx.gguf_quant_matvec_many_weights(Ws, rows, cols, x)
+        for w, W, r, y in zip(ws, Ws, rows, outs):
+            _, y64, ab = O.matvec(t, w, r, cols, x, threads=8)
+            assert_dot_close(y, y64, ab, what=f"grouped, {r} rows")
+            assert_dot_close(hip_ctx.gguf_quant_matvec_weight(W, r, cols, x), y64, ab, what=f"{r}")
+    finally:
+        for W in Ws:
+            W.free()
