@@ -517,8 +517,8 @@ __device__ __forceinline__ float k4_bound(const BlockQ4& w) {
 // that fails it), and the exact path for blocks that need it, summed over the
 // lane groups
 // (every lane of a row gets the row's sum).
-template <int QB, int SB>
-__device__ __forceinline__ float stage_rowsum(const StageRegs<QB, SB>& v, uint32_t sbase,
+template <int QB, int SB, typename Sum = float>
+__device__ __forceinline__ Sum stage_rowsum(const StageRegs<QB, SB>& v, uint32_t sbase,
                                               const Layout& L, uint32_t ls, uint32_t s,
                                               uint32_t nlive, uint32_t grp, uint32_t n,
                                               i32x4 (&A)[8], bool hi_units, int bsh,
@@ -570,10 +570,10 @@ __device__ __forceinline__ float stage_rowsum(const StageRegs<QB, SB>& v, uint32
     for (int b = 0; b < SB; ++b) apart += fabsf(part[b]);
     redo |= !rounded_ok(err, apart);
   }
-  float sum = (float)acc;
+  Sum sum = (Sum)acc;
   if (bad_any || __builtin_amdgcn_ballot_w64(redo) != 0u) {
     if (bad_any || redo) {
-      sum = 0.0f;
+      sum = Sum(0);
 #pragma unroll
       for (int b = 0; b < SB; ++b) {
         if ((uint32_t)b < nlive &&
@@ -598,8 +598,11 @@ __device__ __forceinline__ float stage_rowsum(const StageRegs<QB, SB>& v, uint32
 // workgroups have few pairs per wave (finer pairs, a shorter last one).
 // LINES (Q4_K, one vector, four-block stages of whole rows, nb a multiple of
 // 4, every matrix 128-byte aligned): full-line copies (kLineCopies above).
+// VECS = 2 (one matrix, whole rows): two vectors, one after the other in x, in
+// one pass over the weights: the LDS holds both vectors' images, the second
+// vector's from a whole stage on (hand_off_two).
 template <int WAVES, int DEPTH, int MATS, int QB, bool GROUPED, bool SLICED = false,
-          int SB = 4, bool LINES = false>
+          int SB = 4, bool LINES = false, int VECS = 1>
 __global__ __launch_bounds__(WAVES * 64) void q4k_matvec_mfma(const uint8_t* __restrict__ w,
                                                               const uint8_t* __restrict__ w2,
                                                               const float* __restrict__ x,
@@ -613,6 +616,8 @@ __global__ __launch_bounds__(WAVES * 64) void q4k_matvec_mfma(const uint8_t* __r
   static_assert(SB == 4 || (SB == 2 && MATS == 1), "two-block stages: one matrix");
   static_assert(!LINES || (QB == 4 && SB == 4 && !SLICED && DEPTH <= 2),
                 "full-line stages: Q4_K, four blocks, whole rows");
+  static_assert(VECS == 1 || (VECS == 2 && MATS == 1 && !GROUPED && !SLICED && !LINES),
+                "two vectors with whole rows of one matrix");
   if constexpr (GROUPED) load_group_args_early(ga);
   const uint32_t slots = sa.packed & 0xffu;
   // copy instructions per stage
@@ -631,9 +636,10 @@ __global__ __launch_bounds__(WAVES * 64) void q4k_matvec_mfma(const uint8_t* __r
     sc = make_sched(ntiles, tstages, WAVES, sa);
   // the stages whose images the LDS holds: from st0, nbl blocks
   const uint32_t st0 = SLICED ? ss.r_lo : 0u;
-  const uint32_t nbl = SLICED ? min(SB * ss.ns, nb - SB * st0) : nb;
-  const Layout L =
-      layout(WAVES, DEPTH, SLICED ? SB * ss.pstride : nb, slots, MATS, QB, SB, LINES);
+  const uint32_t nbl = SLICED ? min(SB * ss.ns, nb - SB * st0) : VECS == 2 ? SB * nstages + nb : nb;
+  const Layout L = layout(WAVES, DEPTH,
+                          SLICED ? SB * ss.pstride : VECS == 2 ? 2u * SB * nstages : nb, slots,
+                          VECS == 2 ? 2u : MATS, QB, SB, LINES);
   const SplitWs ws = split_ws(wsp);
   const uint32_t wave = uniform(threadIdx.x >> 6);
   const uint32_t lane = threadIdx.x & 63u;
@@ -643,7 +649,10 @@ __global__ __launch_bounds__(WAVES * 64) void q4k_matvec_mfma(const uint8_t* __r
   uint8_t* const wstage = smem + wave * DEPTH * kStage;
 
   // 1. x into the image area, natural order (block b at img + 1024 b)
-  copy_x<WAVES>(smem, L.img, x + (size_t)SB * st0 * kBlockElems, nbl, wave, lane);
+  if constexpr (VECS == 2)
+    copy_two_x<WAVES>(smem, L.img, x, nb, SB * nstages, wave, lane);
+  else
+    copy_x<WAVES>(smem, L.img, x + (size_t)SB * st0 * kBlockElems, nbl, wave, lane);
 
   // 2. this wave's pairs k = wave, wave + WAVES, ... of the workgroup's pairs
   //    (pair_at: a tile and its partial r, r being stage r % nstages of
@@ -860,6 +869,16 @@ __global__ __launch_bounds__(WAVES * 64) void q4k_matvec_mfma(const uint8_t* __r
       wait_images(sbase, L, builders, fail);
       images = true;
     }
+    if constexpr (VECS == 2) {
+      const double s0 = stage_rowsum<QB, SB, double>(v, sbase, L, s, s, nlive, grp, n, A, hi_units,
+                                                     bsh, rot_lo, rot_hi, x);
+      const double s1 = stage_rowsum<QB, SB, double>(v, sbase, L, s + nstages, s, nlive, grp, n, A,
+                                                     hi_units, bsh, rot_lo, rot_hi,
+                                                     x + (size_t)nb * kBlockElems);
+      issue_next();
+      hand_off_two(sbase, L, slots, sc, pr, nstages, s0, s1, lane, rows, y, fail);
+      continue;
+    }
     float rowsum = stage_rowsum(v, sbase, L, s - st0, s, nlive, grp, n, A, hi_units, bsh,
                                 rot_lo, rot_hi, x);
     // LINES: in odd stages lane n summed row n ^ 1; swap adjacent lanes back
@@ -875,26 +894,28 @@ __global__ __launch_bounds__(WAVES * 64) void q4k_matvec_mfma(const uint8_t* __r
   if (fail != 0u) report_device_error(wsp, fail);
 }
 
-template <int W, int D, int M, int QB = 4, bool G = false, int SB = 4, bool LN = false>
+template <int W, int D, int M, int QB = 4, bool G = false, int SB = 4, bool LN = false, int V = 1>
 bool launch_wd(const uint8_t* w, const uint8_t* w2, const float* x, float* y, uint32_t rows,
                uint32_t nb, const Workspace& ws, hipStream_t s, hipError_t* err,
                const GroupArgs& ga = GroupArgs{}) {
   const uint32_t ntiles = (rows + 15u) / 16u;
   const uint32_t tstages = (nb + SB - 1u) / SB * M;
-  const LaunchShape ls = launch_shape(ntiles, tstages, W, ws.bytes, M);
+  // (two vectors: whole tiles, as without a workspace)
+  const LaunchShape ls = launch_shape(ntiles, tstages, W, V == 2 ? 0u : ws.bytes, M);
   const uint32_t grid = ls.groups;
-  const uint32_t slots = ring_slots(W, D, ls.tiles_per_group, tstages);
-  const uint32_t lds = layout(W, D, nb, slots, M, QB, SB, LN).total;
+  const uint32_t slots = ring_slots(W, D, ls.tiles_per_group, V == 2 ? 4u * tstages : tstages);
+  const uint32_t lds =
+      layout(W, D, V == 2 ? 2u * SB * tstages : nb, slots, V == 2 ? 2 : M, QB, SB, LN).total;
   SchedArgs sa;
   if (lds > kLdsBytes || !make_sched_args(ntiles, tstages, slots, ls, &sa)) return false;
   static const hipError_t attr = hipFuncSetAttribute(
-      reinterpret_cast<const void*>(&q4k_matvec_mfma<W, D, M, QB, G, false, SB, LN>),
+      reinterpret_cast<const void*>(&q4k_matvec_mfma<W, D, M, QB, G, false, SB, LN, V>),
       hipFuncAttributeMaxDynamicSharedMemorySize, (int)kLdsBytes);
   if (attr != hipSuccess) {
     *err = attr;
     return true;
   }
-  hipLaunchKernelGGL((q4k_matvec_mfma<W, D, M, QB, G, false, SB, LN>), dim3(grid),
+  hipLaunchKernelGGL((q4k_matvec_mfma<W, D, M, QB, G, false, SB, LN, V>), dim3(grid),
                      dim3(W * 64), lds, s, w, w2, x, y, rows, nb, ws.ptr, sa, ga, SliceArgs{});
   *err = hipGetLastError();
   return true;
@@ -1245,14 +1266,22 @@ bool launch_q4k_matmul_mfma(const uint8_t* w, const float* x, float* y, uint32_t
                             uint32_t cols, uint32_t batch, const Workspace& ws, hipStream_t s,
                             hipError_t* err) {
   if (batch < 2 || batch > 16 || !shape_ok(rows, cols, 1u, 4)) return false;
-  return launch_q45_tokens(4, w, x, y, rows, cols / kBlockElems, batch, ws, s, err);
+  const uint32_t nb = cols / kBlockElems;
+  if (batch == 2u && two_vectors(kTypeQ4K, rows, nb) && shape_ok(rows, cols, 1u, 4, 2u) &&
+      launch_wd<12, 1, 1, 4, false, 2, false, 2>(w, nullptr, x, y, rows, nb, ws, s, err))
+    return true;
+  return launch_q45_tokens(4, w, x, y, rows, nb, batch, ws, s, err);
 }
 
 bool launch_q5k_matmul_mfma(const uint8_t* w, const float* x, float* y, uint32_t rows,
                             uint32_t cols, uint32_t batch, const Workspace& ws, hipStream_t s,
                             hipError_t* err) {
   if (batch < 2 || batch > 16 || !shape_ok(rows, cols, 1u, 5)) return false;
-  return launch_q45_tokens(5, w, x, y, rows, cols / kBlockElems, batch, ws, s, err);
+  const uint32_t nb = cols / kBlockElems;
+  if (batch == 2u && two_vectors(kTypeQ5K, rows, nb) && shape_ok(rows, cols, 1u, 5, 2u) &&
+      launch_wd<12, 1, 1, 5, false, 2, false, 2>(w, nullptr, x, y, rows, nb, ws, s, err))
+    return true;
+  return launch_q45_tokens(5, w, x, y, rows, nb, batch, ws, s, err);
 }
 
 bool launch_q4k_gate_up_mfma(const uint8_t* gate, const uint8_t* up, const float* x, float* h,

@@ -168,8 +168,10 @@ __device__ __forceinline__ void q6_sets(const u32x4& a, const u32x4& b, const u3
   }
 }
 
-// Fast-path dot of one block for one lane.
-__device__ __forceinline__ float block_terms(const i32x4 (&q)[4], const int (&sc)[4], float d,
+// Fast-path dot of one block for one lane, its digit sums combined in f32 or (two
+// vectors, as in the kernel of more) f64.
+template <typename Real = float>
+__device__ __forceinline__ Real block_terms(const i32x4 (&q)[4], const int (&sc)[4], float d,
                                              const i32x4& a0, const i32x4& a1, const i32x4& a2,
                                              const i32x4& a3, int eb) {
   const i32x4 zero = {0, 0, 0, 0};
@@ -188,9 +190,16 @@ __device__ __forceinline__ float block_terms(const i32x4 (&q)[4], const int (&sc
   for (int k = 0; k < 4; ++k)
     t[k] = mad_i24(sc[3], c3[k],
                    mad_i24(sc[2], c2[k], mad_i24(sc[1], c1[k], __mul24(sc[0], c0[k]))));
-  const float tc =
-      fmaf(fmaf(fmaf((float)t[3], 256.0f, (float)t[2]), 256.0f, (float)t[1]), 256.0f, (float)t[0]);
-  return __builtin_amdgcn_ldexpf(d * tc, eb);
+  if constexpr (std::is_same_v<Real, double>) {
+    double tc = (double)t[3];
+#pragma unroll
+    for (int k = 2; k >= 0; --k) tc = fma(tc, 256.0, (double)t[k]);
+    return __builtin_amdgcn_ldexp((double)d * tc, eb);
+  } else {
+    const float tc =
+        fmaf(fmaf(fmaf((float)t[3], 256.0f, (float)t[2]), 256.0f, (float)t[1]), 256.0f, (float)t[0]);
+    return __builtin_amdgcn_ldexpf(d * tc, eb);
+  }
 }
 
 // Exact per-weight path of one block: xs = x of the block + 128 h + 16 s.
@@ -227,6 +236,9 @@ __device__ __forceinline__ float q6_bound(const int (&sc)[4], float d) {
 // SLICED (one matrix): a K-sliced launch (SliceArgs,
 // mfma_common.h); the LDS holds the images and metadata of the workgroup's
 // slice only, stage r of the matrix at local stage r - r_lo.
+//
+// VECS = 2 (one matrix, whole rows): two vectors, one after the other in x, in
+// one pass over the weights: the LDS holds both vectors' images (hand_off_two).
 //
 // PAIRED (one matrix of an odd block count nr): the launch sees
 // rows / 2 rows of nb = 2 nr blocks, row r being rows 2 r and 2 r + 1 of the
@@ -270,7 +282,7 @@ struct ArgmaxArgs {
   uint32_t rule;
 };
 template <int WAVES, int DEPTH, bool GROUPED, bool ARGMAX = false, bool SLICED = false,
-          bool PAIRED = false>
+          bool PAIRED = false, int VECS = 1>
 __global__ __launch_bounds__(WAVES * 64) void q6k_matvec_mfma(const uint8_t* __restrict__ w,
                                                               const float* __restrict__ x,
                                                               float* __restrict__ y, uint32_t rows,
@@ -282,6 +294,8 @@ __global__ __launch_bounds__(WAVES * 64) void q6k_matvec_mfma(const uint8_t* __r
   static_assert(!SLICED || (!GROUPED && !ARGMAX), "slices of one matrix");
   static_assert(!PAIRED || !GROUPED, "row pairs of one matrix");
   static_assert(!(PAIRED && SLICED && ARGMAX), "sliced row pairs: no argmax");
+  static_assert(VECS == 1 || (VECS == 2 && !GROUPED && !ARGMAX && !SLICED && !PAIRED),
+                "two vectors with whole rows of one matrix");
   extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
   if constexpr (GROUPED) load_group_args_early(ga);
   if constexpr (PAIRED && !ARGMAX) {
@@ -303,8 +317,9 @@ __global__ __launch_bounds__(WAVES * 64) void q6k_matvec_mfma(const uint8_t* __r
     sc = make_sched(ntiles, nstages, WAVES, sa);
   // the stages whose images the LDS holds: [st0, st0 + nst), local index st - st0
   const uint32_t st0 = SLICED ? ss.r_lo : 0u;
-  const uint32_t nbl = SLICED ? 2u * ss.ns : nb;
-  const Layout L = layout(WAVES, DEPTH, SLICED ? 2u * ss.pstride : nb, slots, PAIRED ? 2u : 1u);
+  const uint32_t nbl = SLICED ? 2u * ss.ns : VECS * nb;
+  const Layout L = layout(WAVES, DEPTH, SLICED ? 2u * ss.pstride : VECS * nb, slots,
+                          PAIRED || VECS == 2 ? 2u : 1u);
   const uint32_t nr = nb / 2u;  // PAIRED: blocks of one matrix row
   const SplitWs ws = split_ws(wsp);
   const uint32_t wave = uniform(threadIdx.x >> 6);
@@ -463,13 +478,12 @@ __global__ __launch_bounds__(WAVES * 64) void q6k_matvec_mfma(const uint8_t* __r
     u32x4 v[13];
     lds_read_stage(qa0 + buf, qh0 + buf, sc0 + buf, v);
     if (j + DEPTH < my_pairs) issue(j + DEPTH);  // the buffer just read is free again
-    lds_read_images(sbase + L.img + 2048u * ls + 16u * n, kActiveLanes, A);
     u32x2 ex;
     uint32_t cnt;
-    lds_read_expo(sbase + L.expo + 8u * ls, ex, cnt);
-    const int e0 = __builtin_amdgcn_readfirstlane(ex[0]);
-    const int e1 = __builtin_amdgcn_readfirstlane(ex[1]);
-
+    if constexpr (VECS == 1) {
+      lds_read_images(sbase + L.img + 2048u * ls + 16u * n, kActiveLanes, A);
+      lds_read_expo(sbase + L.expo + 8u * ls, ex, cnt);
+    }
     // block 0: scales[8h + s + 2t] = bytes s, s + 2 of words 2h, 2h + 1 of v3
     i32x4 q0[4];
     q6_sets(v[0], v[1], v[2], q0);
@@ -487,7 +501,47 @@ __global__ __launch_bounds__(WAVES * 64) void q6k_matvec_mfma(const uint8_t* __r
                          scale_at(u2, sb_lo)};
     const float d1 = half_bits_to_float(v[12][3] >> 16);
 
-
+    if constexpr (VECS == 2) {
+      // one vector after the other, the second one's images a row's stages on (a
+      // loop kept as one, with the exact path's decode kept inside it: both
+      // vectors' unrolled, or 128 decoded weights held for them, spill)
+      auto exact = [&](const i32x4 (&q)[4], const int (&sc)[4], float d, const float* xs) {
+        i32x4 own[4] = {q[0], q[1], q[2], q[3]};
+        asm volatile("" : "+v"(own[0]), "+v"(own[1]), "+v"(own[2]), "+v"(own[3]));
+        return block_exact(own, sc, d, xs);
+      };
+      double sum1 = 0.0, sum2 = 0.0;
+#pragma unroll 1
+      for (uint32_t vec = 0; vec < 2u; ++vec) {
+        const uint32_t at = ls + vec * nstages;
+        lds_read_images(sbase + L.img + 2048u * at + 16u * n, kActiveLanes, A);
+        lds_read_expo(sbase + L.expo + 8u * at, ex, cnt);
+        const int e0 = __builtin_amdgcn_readfirstlane(ex[0]);
+        const int e1 = __builtin_amdgcn_readfirstlane(ex[1]);
+        const double c0 = block_terms<double>(q0, sc_0, d0, A[0], A[1], A[2], A[3], e0);
+        const double c1 = block_terms<double>(q1, sc_1, d1, A[4], A[5], A[6], A[7], e1);
+        double s0 = e0 != kBadBlock ? c0 : 0.0, s1 = e1 != kBadBlock ? c1 : 0.0;
+        const uint32_t counts = __builtin_amdgcn_readfirstlane(cnt);
+        uint32_t redo = 0u;
+        if (counts != 0u) {
+          const float pp[2] = {(float)s0, (float)s1};
+          redo = rounded_redo<2>(sbase + L.expo + L.side_off + 2u * kSideBytes * at, counts, grp,
+                                 pp, [&](auto b) {
+                                   return decltype(b)::value == 0 ? q6_bound(sc_0, d0)
+                                                                  : q6_bound(sc_1, d1);
+                                 });
+        }
+        const float* const xs = x + 256u * (size_t)(vec * nb) + 512u * st + 128u * half + 16u * sub;
+        if (e0 == kBadBlock || (redo & 1u)) s0 = exact(q0, sc_0, d0, xs);
+        if (e1 == kBadBlock || (redo & 2u)) s1 = exact(q1, sc_1, d1, xs + 256);
+        sum1 = sum2;
+        sum2 = sum_lane_groups(s0 + s1);
+      }
+      hand_off_two(sbase, L, slots, sc, pr, nstages, sum1, sum2, lane, rows, y, fail);
+      continue;
+    }
+    const int e0 = __builtin_amdgcn_readfirstlane(ex[0]);
+    const int e1 = __builtin_amdgcn_readfirstlane(ex[1]);
     const float c0 = block_terms(q0, sc_0, d0, A[0], A[1], A[2], A[3], e0);
     const float c1 = block_terms(q1, sc_1, d1, A[4], A[5], A[6], A[7], e1);
     float pp[2] = {e0 != kBadBlock ? c0 : 0.0f, e1 != kBadBlock ? c1 : 0.0f};
@@ -799,23 +853,24 @@ __global__ __launch_bounds__(WAVES * 64) void q6k_tokens_mfma(const uint8_t* __r
   }
 }
 
-template <int W, int D, bool G = false, bool AM = false, bool P = false>
+template <int W, int D, bool G = false, bool AM = false, bool P = false, int V = 1>
 bool launch_wd(const uint8_t* w, const float* x, float* y, uint32_t rows, uint32_t nb,
                const Workspace& ws, hipStream_t s, hipError_t* err,
                const GroupArgs& ga = GroupArgs{}, const ArgmaxArgs& aa = ArgmaxArgs{},
                bool last_row = false) {
   const uint32_t ntiles = (rows + 15u) / 16u;
   const uint32_t nstages = (nb + 1u) / 2u;
-  const LaunchShape ls = launch_shape(ntiles, nstages, W, ws.bytes, P ? 2u : 1u,
+  // (two vectors: whole tiles, as without a workspace)
+  const LaunchShape ls = launch_shape(ntiles, nstages, W, V == 2 ? 0u : ws.bytes, P ? 2u : 1u,
                                       (uint32_t)cu_count() - (last_row ? 1u : 0u));
   const uint32_t grid = ls.groups;
-  const uint32_t slots = ring_slots(W, D, ls.tiles_per_group, P ? 2u * nstages : nstages);
+  const uint32_t slots = ring_slots(W, D, ls.tiles_per_group, (V == 2 ? 4u : P ? 2u : 1u) * nstages);
   // One pair touched ahead pays where the image build is long (the 68-block
   // down projection: 1 us of 22); with 20 blocks (the output head) it costs.
   static const int pf_env = env_int("SI_HIP_Q6K_PREFETCH", -1);
   const uint32_t prefetch = pf_env >= 0 ? (uint32_t)pf_env : (nb >= 48u ? 1u : 0u);
   const uint32_t lds =
-      layout(W, D, nb, slots, P ? 2u : 1u).total + (D == 1 && prefetch ? 256u : 0u);
+      layout(W, D, V * nb, slots, P || V == 2 ? 2u : 1u).total + (D == 1 && prefetch ? 256u : 0u);
   SchedArgs sa;
   if (lds > kLdsBytes || !make_sched_args(ntiles, nstages, slots, ls, &sa)) return false;
   // the argmax: an entry per workgroup, the waves' candidates at the LDS start
@@ -823,13 +878,13 @@ bool launch_wd(const uint8_t* w, const float* x, float* y, uint32_t rows, uint32
              ws.bytes < kWorkspaceBytes))
     return false;
   static const hipError_t attr = hipFuncSetAttribute(
-      reinterpret_cast<const void*>(&q6k_matvec_mfma<W, D, G, AM, false, P>),
+      reinterpret_cast<const void*>(&q6k_matvec_mfma<W, D, G, AM, false, P, V>),
       hipFuncAttributeMaxDynamicSharedMemorySize, (int)kLdsBytes);
   if (attr != hipSuccess) {
     *err = attr;
     return true;
   }
-  hipLaunchKernelGGL((q6k_matvec_mfma<W, D, G, AM, false, P>),
+  hipLaunchKernelGGL((q6k_matvec_mfma<W, D, G, AM, false, P, V>),
                      dim3(grid + (last_row ? 1u : 0u)), dim3(W * 64), lds, s, w, x, y, rows, nb,
                      ws.ptr, sa, D == 1 ? prefetch : 0u, ga, aa, SliceArgs{});
   *err = hipGetLastError();
@@ -1105,6 +1160,11 @@ bool launch_q6k_matmul_mfma(const uint8_t* w, const float* x, float* y, uint32_t
       rows * batch < 12288u &&
       (rows < 16u ? batch * nb < 64u : batch < 8u && batch * nb < 33u))
     return false;
+  // Two vectors over short rows: whole rows in one launch, no reduce behind it
+  // (two_vectors, mfma_common.h).
+  if (batch == 2u && two_vectors(kTypeQ6K, rows, nb) && q6_shape_ok(rows, nb) &&
+      launch_wd<12, 1, false, false, false, 2>(w, x, y, rows, nb, ws, s, err))
+    return true;
   return (nb & 1u) != 0u ? launch_tok6_any<true>(w, x, y, rows, nb, batch, ws, s, err)
                          : launch_tok6_any<false>(w, x, y, rows, nb, batch, ws, s, err);
 }

@@ -259,18 +259,31 @@ __device__ __forceinline__ float sum_lane_groups(float v) {
   return __uint_as_float(b[0]) + __uint_as_float(b[1]);
 }
 
+__device__ __forceinline__ double sum_lane_groups(double v) {
+  auto halves = [](double d) { return __builtin_bit_cast(u32x2, d); };
+  auto whole = [](uint32_t lo, uint32_t hi) { return __builtin_bit_cast(double, u32x2{lo, hi}); };
+  const u32x2 w = halves(v);
+  auto al = __builtin_amdgcn_permlane16_swap(w[0], w[0], false, false);
+  auto ah = __builtin_amdgcn_permlane16_swap(w[1], w[1], false, false);
+  const u32x2 t = halves(whole(al[0], ah[0]) + whole(al[1], ah[1]));
+  auto bl = __builtin_amdgcn_permlane32_swap(t[0], t[0], false, false);
+  auto bh = __builtin_amdgcn_permlane32_swap(t[1], t[1], false, false);
+  return whole(bl[0], bh[0]) + whole(bl[1], bh[1]);
+}
+
 // Copy of x (nb blocks of 256 f32) into the image area in natural order
 // (block b at img + 1024 b): pass j of wave v copies blocks 4 (v + WAVES j)
 // .. +3, one 64-lane 16-byte copy each -- the blocks build_images has the
 // same wave convert, so that a wave's own wait covers what it converts.
 // src_nb != 0: the image holds blocks first .. first + nb - 1 of x twice
 // over (first + nb <= 2 src_nb), image block b being x block
-// (first + b) mod src_nb.
-template <int WAVES>
-__device__ __forceinline__ void copy_x(uint8_t* smem, uint32_t img, const float* x, uint32_t nb,
-                                       uint32_t wave, uint32_t lane, uint32_t src_nb = 0u,
-                                       uint32_t first = 0u) {
-  const uint32_t xn = src_nb != 0u ? src_nb : nb;
+// (first + b) mod src_nb.  copy_two_x: two vectors of src_nb blocks each, one
+// after the other in x, the second at image block `second` (the image blocks
+// between them are not used).
+template <int WAVES, typename Source>
+__device__ __forceinline__ void copy_x_from(uint8_t* smem, uint32_t img, const float* x,
+                                            uint32_t nb, uint32_t wave, uint32_t lane, uint32_t xn,
+                                            Source source) {
   const uint32_t npass = (nb + 4u * WAVES - 1u) / (4u * WAVES);
   const __amdgpu_buffer_rsrc_t xr = __builtin_amdgcn_make_buffer_rsrc(
       const_cast<float*>(x), 0, (int)(xn * 1024u), kBufferWord3);
@@ -278,13 +291,29 @@ __device__ __forceinline__ void copy_x(uint8_t* smem, uint32_t img, const float*
     const uint32_t b0 = 4u * (wave + WAVES * j);
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-      const uint32_t b = b0 + i, v = first + b;
-      const uint32_t sb = v >= xn ? v - xn : v;
+      const uint32_t b = b0 + i;
       if (b < nb)
         __builtin_amdgcn_raw_ptr_buffer_load_lds(xr, (lds_void*)(smem + img + 1024u * b), 16,
-                                                  1024u * sb + 16u * lane, 0, 0, 0);
+                                                  1024u * source(b) + 16u * lane, 0, 0, 0);
     }
   }
+}
+template <int WAVES>
+__device__ __forceinline__ void copy_x(uint8_t* smem, uint32_t img, const float* x, uint32_t nb,
+                                       uint32_t wave, uint32_t lane, uint32_t src_nb = 0u,
+                                       uint32_t first = 0u) {
+  const uint32_t xn = src_nb != 0u ? src_nb : nb;
+  copy_x_from<WAVES>(smem, img, x, nb, wave, lane, xn, [=](uint32_t b) {
+    const uint32_t v = first + b;
+    return v >= xn ? v - xn : v;
+  });
+}
+template <int WAVES>
+__device__ __forceinline__ void copy_two_x(uint8_t* smem, uint32_t img, const float* x,
+                                           uint32_t src_nb, uint32_t second, uint32_t wave,
+                                           uint32_t lane) {
+  copy_x_from<WAVES>(smem, img, x, second + src_nb, wave, lane, 2u * src_nb,
+                     [=](uint32_t b) { return b < second ? b : b - second + src_nb; });
 }
 
 // Largest of a DPP row's 16 values, in every lane.
@@ -894,6 +923,34 @@ __device__ __forceinline__ void hand_off(uint32_t sbase, const Layout& L, uint32
   }
 }
 
+// hand_off for two vectors (whole tiles only, no exchange between workgroups):
+// s0 and s1, the row's sums of the pair's stage with either vector, go to the
+// tile's slot as f64, and the wave that completes the tile adds them in stage
+// order, lane groups 0 and 1 a vector each, and rounds y[row] and y[rows + row]
+// once.
+__device__ __forceinline__ void hand_off_two(uint32_t sbase, const Layout& L, uint32_t slots,
+                                             const Sched& sc, const Pair& pr, uint32_t nparts,
+                                             double s0, double s1, uint32_t lane, uint32_t rows,
+                                             float* __restrict__ y, uint32_t& fail) {
+  const uint32_t vec = lane >> 4, n = lane & 15u;
+  const uint32_t slot = pr.lt - quo(pr.lt, sc.by_slots) * slots;
+  const uint32_t part = sbase + L.part + 256u * slot * nparts + 128u * (vec & 1u) + 8u * n;
+  wait_slot(sbase + L.owner + 4u * slot, pr.lt, fail);
+  if (vec < 2u) lds_write_b64(part + 256u * pr.r, __builtin_bit_cast(u32x2, vec ? s1 : s0));
+  uint32_t old = 0u;
+  if (lane == 0u) old = lds_add_rtn(sbase + L.cnt + 4u * slot, 1u);
+  if (__builtin_amdgcn_readlane(old, 0) != nparts - 1u) return;
+  double sum = 0.0;
+  for (uint32_t st = 0; st < nparts; ++st)
+    sum += __builtin_bit_cast(double, lds_read_b64(part + 256u * st));
+  const uint32_t row = pr.tile * 16u + n;
+  if (vec < 2u && row < rows) y[(size_t)vec * rows + row] = (float)sum;
+  if (lane == 0u) {
+    lds_write_b32(sbase + L.cnt + 4u * slot, 0u);
+    lds_write_b32(sbase + L.owner + 4u * slot, pr.lt + slots);
+  }
+}
+
 // K-sliced launches, for matrices of few tiles and long rows (a down
 // projection): the stages of every tile are cut into S slices as even as the
 // stage count allows, and workgroup g = S tg + s works on slice s of the tiles
@@ -1179,6 +1236,29 @@ inline uint32_t ring_slots(uint32_t waves, uint32_t depth, uint32_t tiles_per_wg
   uint32_t slots = min(tiles_per_wg, max(4u, (2u * waves * depth + tparts - 1u) / tparts + 2u));
   while (slots > 2u && slots * tparts * 64u > 8192u) --slots;
   return slots;
+}
+
+// Whether two vectors of a matrix (Q6_K: of an even block count) go through the one-vector kernel's two-vector form, whole rows
+// in one launch, instead of the vectors-in-rows kernel and its reduce.  The
+// launch of the reduce is what this saves: the form is ahead up to 16 blocks a
+// row, whose images of two vectors cost little, and up to 20 (Q6_K 24) where its
+// whole tiles leave at most a fifth of the workgroups without one; far larger
+// launches the vectors-in-rows kernel streams faster.  Us, this form / that kernel:
+// Q6_K 4096 x 2560 7.0 / 9.3, 16384 x 1536 8.8 / 11.9, 28000 x 3584 25.4 / 27.0,
+// 64 x 4608 8.2 / 7.5, 4096 x 6144 10.1 / 12.0, 5120 x 6144 13.4 / 12.5, 28000 x
+// 6144 41.1 / 36.9; Q5_K 4096 x 2048 6.5 / 8.9, 28000 x 3072 19.3 / 20.7, 20000 x
+// 4096 18.5 / 17.9, 16384 x 5120 20.0 / 20.3, 28000 x 5120 31.7 / 29.1; Q4_K 1024 x 1024 5.7 / 7.1, 16384 x 3584 11.8 / 12.5, 28000 x
+// 3584 19.3 / 17.5, 8192 x 5120 11.1 / 11.7, 12000 x 5120 13.6 / 13.0.
+inline bool two_vectors(uint32_t type, uint32_t rows, uint32_t nb) {
+  const uint64_t blocks = (uint64_t)rows * nb;
+  const bool longer = nb > 12u && nb <= 16u;
+  const uint64_t most = type == kTypeQ6K   ? 400000u
+                        : type == kTypeQ5K ? (longer ? 256000u : 340000u)
+                                           : (nb <= 16u ? 256000u : 200000u);
+  if (nb <= 16u) return blocks < most;
+  const uint64_t tiles = (rows + 15u) / 16u, cus = (uint64_t)cu_count();
+  return nb <= (type == kTypeQ6K ? 24u : 20u) && blocks < most &&
+         4u * ((tiles + cus - 1u) / cus) * cus <= 5u * tiles;
 }
 
 // kernels_q45_tokens.hip: Q4_K (qb 4) or Q5_K (qb 5), ntok = 2..16 vectors
