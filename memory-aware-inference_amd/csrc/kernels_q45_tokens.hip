@@ -37,7 +37,7 @@
 // largest weight that d and dmin allow) could be off by more than they may be
 // (kFewTol, tokens_common.h).
 //
-// Work split.  A launch cuts K into slices of four blocks: workgroup g works
+// Work split.  A launch cuts K into slices of four blocks (slice_first): workgroup g works
 // on slice g / GS for tiles g % GS, g % GS + GS, ..., keeping that slice's
 // images in LDS; each wave takes (tile, slice) pairs, their two-block stages
 // one after another through one stage buffer (buffer->LDS copies, row by row;
@@ -63,7 +63,7 @@ namespace {
 
 using namespace mfma;
 
-constexpr uint32_t kSliceBlocks = 4u;
+constexpr uint32_t kSliceBlocks = kStageBlocks;  // (slice_first)
 
 template <int QB>
 struct Format {
@@ -244,7 +244,7 @@ __global__ __launch_bounds__(WAVES * 64) void q45_tokens_mfma(const uint8_t* __r
   const FastDiv by_gps{ta.groups_per_slice, ta.m_gps};
   const uint32_t k = quo(blockIdx.x, by_gps);
   const uint32_t tg = blockIdx.x - k * ta.groups_per_slice;
-  const uint32_t blk0 = kSliceBlocks * k, nbl = min(kSliceBlocks, nb - blk0);
+  const uint32_t blk0 = slice_first(k, nb), nbl = min(slice_first(k + 1u, nb), nb) - blk0;
   const uint32_t nst = (nbl + 1u) / 2u;
   const uint32_t ntw = tg < ntiles ? quo(ntiles - 1u - tg, by_gps) + 1u : 0u;
 
@@ -401,8 +401,7 @@ bool launch_tok45(const uint8_t* w, const float* x, float* y, uint32_t rows, uin
                        dim3(W * 64), kLds, s, wr, x, nr, nb, ntok, ws.scratch, ta);
     *err = hipGetLastError();
     if (*err != hipSuccess) break;
-    launch_tok_reduce<F::kType>(ws.scratch, y + r0, nr, rows, slices, 4u * NG, ntok, wr, x, nb,
-                                kSliceBlocks, s);
+    launch_tok_reduce<F::kType>(ws.scratch, y + r0, nr, rows, slices, 4u * NG, ntok, wr, x, nb, s);
     *err = hipGetLastError();
   }
   return true;

@@ -643,7 +643,7 @@ __global__ __launch_bounds__(WAVES * 64) void q6k_matvec_mfma(const uint8_t* __r
 // rows', the next `slices` the odd rows', and a "row" here is a pair.
 // 4096 x 11008, M = 2 / 4 / 8 / 16: 28.3 / 55.3 / 108.5 / 215.6 us one vector
 // at a time, 15.3 / 15.5 / 17.4 / 20.5 so.
-constexpr uint32_t kTokBlocks = 4u;
+constexpr uint32_t kTokBlocks = kStageBlocks;
 
 struct Q6TokArgs {
   uint32_t groups_per_slice, m_gps;
@@ -713,8 +713,12 @@ __global__ __launch_bounds__(WAVES * 64) void q6k_tokens_mfma(const uint8_t* __r
   const uint32_t k = quo(blockIdx.x, by_gps);
   const uint32_t tg = blockIdx.x - k * ta.groups_per_slice;
   const uint32_t odd = PAIRED && k >= ta.slices ? 1u : 0u;
-  const uint32_t blk0 = kTokBlocks * (PAIRED ? k - odd * ta.slices : k);
-  const uint32_t nbl = min(kTokBlocks, nb + (PAIRED ? 1u : 0u) - blk0), nst = nbl / 2u;
+  const uint32_t ks = PAIRED ? k - odd * ta.slices : k;
+  auto first = [&](uint32_t i) {
+    return PAIRED ? paired_slice_first(i, nb, odd) : kTokBlocks * i;
+  };
+  const uint32_t blk0 = first(ks);
+  const uint32_t nbl = min(first(ks + 1u), nb + (PAIRED ? 1u : 0u)) - blk0, nst = nbl / 2u;
   const uint32_t places = PAIRED ? (rows + 1u) / 2u : rows;  // of the partials
   const uint32_t trows = odd ? rows / 2u : places;           // the slice's rows
   const uint32_t ntiles = (trows + 15u) / 16u;
@@ -1075,8 +1079,7 @@ bool launch_tok6(const uint8_t* w, const float* x, float* y, uint32_t rows, uint
                        dim3(W * 64), kLds, s, wr, x, nr, nb, ntok, ws.scratch, ta);
     *err = hipGetLastError();
     if (*err != hipSuccess) break;
-    launch_tok_reduce<kTypeQ6K, P>(ws.scratch, y + r0, nr, rows, slices, 4u * NG, ntok, wr, x, nb,
-                                   kTokBlocks, s);
+    launch_tok_reduce<kTypeQ6K, P>(ws.scratch, y + r0, nr, rows, slices, 4u * NG, ntok, wr, x, nb, s);
     *err = hipGetLastError();
   }
   return true;

@@ -129,4 +129,45 @@ __device__ __forceinline__ void decode_unit_exact(const uint8_t* __restrict__ bl
   }
 }
 
+// A little-endian word at any alignment.
+__device__ __forceinline__ uint32_t load_word(const uint8_t* p) {
+  uint32_t v;
+  __builtin_memcpy(&v, p, 4);
+  return v;
+}
+
+// The exact values of elements i .. i + 3 (i a multiple of 4) of a block, as
+// decode_unit_exact gives them (quant.rs order).
+template <uint32_t T>
+__device__ __forceinline__ float4 decode_four_exact(const uint8_t* __restrict__ blk, uint32_t i) {
+  float v[4];
+  const uint32_t l = i & 31u;
+  if constexpr (T == kTypeQ4K || T == kTypeQ5K) {
+    const uint32_t unit = i >> 5, s = unit & 3u, dd = load_word(blk);
+    const uint32_t w0 = load_word(blk + 4) >> (8u * s), w1 = load_word(blk + 8) >> (8u * s);
+    const uint32_t w2 = load_word(blk + 12) >> (8u * s);
+    // scale_min_k4 on byte s of the three words
+    const uint32_t sc = unit < 4u ? w0 & 63u : (w2 & 0x0fu) | ((w0 >> 2) & 0x30u);
+    const uint32_t mn = unit < 4u ? w1 & 63u : ((w2 >> 4) & 0x0fu) | ((w1 >> 2) & 0x30u);
+    const float d1 = __fmul_rn(half_bits_to_float_exact(dd & 0xffffu), (float)sc);
+    const float m1 = __fmul_rn(half_bits_to_float_exact(dd >> 16), (float)mn);
+    uint32_t q = (load_word(blk + (T == kTypeQ4K ? 16 : 48) + 32u * (unit >> 1) + l) >>
+                  (4u * (unit & 1u))) & 0x0f0f0f0fu;
+    if constexpr (T == kTypeQ5K) q |= ((load_word(blk + 16 + l) >> unit) & 0x01010101u) << 4;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) v[k] = k4_value_exact(d1, m1, (q >> (8 * k)) & 0xffu);
+  } else {
+    const uint32_t half = i >> 7, quartet = (i >> 5) & 3u;
+    const float d = half_bits_to_float_exact(blk[208] | (blk[209] << 8));
+    const int sc = (int8_t)blk[192 + (i >> 4)];
+    const uint32_t q =
+        ((load_word(blk + 64u * half + 32u * (quartet & 1u) + l) >> (4u * (quartet >> 1))) &
+         0x0f0f0f0fu) |
+        (((load_word(blk + 128u + 32u * half + l) >> (2u * quartet)) & 0x03030303u) << 4);
+#pragma unroll
+    for (int k = 0; k < 4; ++k) v[k] = k6_value_exact(d, sc, (int)((q >> (8 * k)) & 0xffu) - 32);
+  }
+  return make_float4(v[0], v[1], v[2], v[3]);
+}
+
 }  // namespace sihip

@@ -38,15 +38,31 @@ __device__ __forceinline__ void lds_write_b16(uint32_t addr, uint32_t v) {
 constexpr int kBadTok = -(1 << 20);
 
 // What a vector's side elements (mfma_common.h) may cost its dot with a row
-// over a slice: 2^-22 of the row's sum |block term| where no block has more
-// than eight of them, which is what the f32 rounding of such sums would be
-// (the terms here are f64), and kRoundedTol of it for the blocks that have
+// over a slice: 2^-21 of the row's sum |block term| where no block has more
+// than eight of them, which is what the f32 rounding of such terms was bounded
+// by (they are f64 here), and kRoundedTol of it for the blocks that have
 // more.  A (vector, row) past that takes the slice's exact dot.  (Up to eight
 // per block used to be listed and added from the exact weights; held to
 // kRoundedTol like the rest, a dot that rides on them was up to 7.6e-6 off.)
 // Slices of ordinary activations reach 1e-8 of the sum.
 constexpr uint32_t kFewSide = 8;
-constexpr float kFewTol = 0x1p-22f;
+constexpr float kFewTol = 0x1p-21f;
+
+// First block of K slice k of rows of nb blocks: slices of four, the last of what
+// is left; where that is one block, it takes another from the slice before it.
+// One block's |term| is often enough small against what its side elements could
+// cost that most launches had a row to redo: with slices of three and two at the
+// end 4096 x 2304 M = 16 takes 14.3 -> 12.6 us (Q4_K), 15.3 -> 13.2 (Q5_K).
+__host__ __device__ constexpr uint32_t slice_first(uint32_t k, uint32_t nb) {
+  return 4u * k - (k != 0u && 4u * k + 1u == nb ? 1u : 0u);
+}
+// The same in a paired launch (Q6_K, odd nb), whose rows are nb + 1 blocks wide:
+// an even row's own nb blocks and the next, an odd row's after the one before it.
+// Where slices of four leave two blocks the even rows' first slice is the short
+// one, the odd rows' the last, so that both have two blocks of the row itself.
+__host__ __device__ constexpr uint32_t paired_slice_first(uint32_t k, uint32_t nb, uint32_t odd) {
+  return 4u * k - (k != 0u && odd == 0u && (nb & 3u) == 1u ? 2u : 0u);
+}
 
 // LDS map of a launch whose workgroups keep up to stride = 4 blocks of ng
 // groups (group g's block b is group-block gb = stride g + b): the
@@ -205,22 +221,21 @@ __device__ __forceinline__ float slice_err(const uint8_t* rerr, uint32_t nbl) {
 
 // y[t * yrows + row] = sum over the stages s of part[(s * nv + t) * rows + row],
 // in stage order (the sliced launch's second kernel; a "stage" here is the
-// first kernel's unit of partial sums, bps blocks).  A partial that holds
+// first kernel's unit of partial sums, a K slice).  A partial that holds
 // kPartRedo (its lane failed a check in the first kernel) is the stage's
-// exact dot instead: quant.rs's per-weight values of blocks bps s ..
-// bps s + bps - 1 of the row (decode_unit_exact) times vector t of the
-// batch-major x, summed in f64 and rounded once.  The workgroup's 256
-// threads take such stages together from a queue in LDS, eight at a time,
-// 32 threads (half a wave) per stage and 32-weight units l, l + 32, ... per
-// thread, their f64 sums added with shuffles; a stage past the queue's room
-// is taken by its own thread.  A thread with such a stage sums its rows'
+// exact dot instead: quant.rs's per-weight values of the stage's blocks of the
+// row times vector t of the batch-major x, summed in f64 and rounded once.  The
+// workgroup's waves take such stages together from a queue in LDS, four at a
+// time; a stage past the queue's room is taken by its own thread.  (With 32
+// threads a stage, a 32-weight unit each, its bytes loaded one by one, one such
+// stage cost a launch 1-2 us.)  A thread with such a stage sums its rows'
 // partials again in stage order, the first eight stages kept in registers.
 // R rows per thread: 1, or 4 with 16-byte loads and stores (launch_tok_reduce
 // takes 4 when the rows, y and the grid allow it); each row's sum is the same.
 // PAIRED: rows 2 r and 2 r + 1 share place r of the partials, of ceil(rows / 2);
 // the first nstages stages are the even rows' and the next nstages the odd
-// rows', whose stage s starts a block earlier (the block before the row is no
-// part of it).
+// rows' (paired_slice_first; the block before the row is no part of it).
+constexpr uint32_t kStageBlocks = 4u;  // at most, in a stage
 constexpr uint32_t kRedoQueue = 64;
 template <uint32_t T>
 __device__ __noinline__ float stage_exact(const uint8_t* __restrict__ w, uint32_t row,
@@ -246,8 +261,7 @@ __global__ __launch_bounds__(256) void tok_reduce(const float* __restrict__ part
                                                   float* __restrict__ y, uint32_t rows,
                                                   uint32_t yrows, uint32_t nstages, uint32_t nv,
                                                   const uint8_t* __restrict__ w,
-                                                  const float* __restrict__ x, uint32_t nb,
-                                                  uint32_t bps) {
+                                                  const float* __restrict__ x, uint32_t nb) {
   static_assert(R == 1 || (R == 4 && !PAIRED), "one or four rows per thread");
   constexpr uint32_t kBytes = BlockBytes<T>::value;
   __shared__ uint32_t queue[kRedoQueue];  // (row in the workgroup) << 16 | stage
@@ -263,6 +277,11 @@ __global__ __launch_bounds__(256) void tok_reduce(const float* __restrict__ part
   const float* const xt = x + (size_t)t * nb * kBlockElems;
   if (tid == 0u) queued = 0u;
   __syncthreads();
+  // the first block of stage st of row r, and the block past its last
+  auto first_block = [&](uint32_t st, uint32_t r) {
+    return PAIRED ? paired_slice_first(st, nb, r & 1u) - (r & 1u) : slice_first(st, nb);
+  };
+  auto end_block = [&](uint32_t st, uint32_t r) { return min(first_block(st + 1u, r), nb); };
   // stages base .. base + 7 of the thread's rows, eight loads in flight
   auto load8 = [&](uint32_t base, float (&v)[8][R]) {
 #pragma unroll
@@ -312,36 +331,38 @@ __global__ __launch_bounds__(256) void tok_reduce(const float* __restrict__ part
     }
   }
   if (__syncthreads_or(mine)) {
-    // queued stages eight at a time, one per 32 threads (half a wave), which
-    // sum their units' f64 dots with shuffles inside the half wave
+    // queued stages four at a time, one a wave: lane l takes elements 4 l .. 4 l + 3
+    // of each block, all their loads in flight, and the lanes' f64 dots are summed
     const uint32_t nq = min(queued, kRedoQueue);
-    const uint32_t e = tid >> 5, l = tid & 31u;  // stage e of a batch; its units l, l + 32, ...
-    for (uint32_t k0 = 0; k0 < nq; k0 += 8u) {
+    const uint32_t e = tid >> 6, l = tid & 63u;
+    for (uint32_t k0 = 0; k0 < nq; k0 += 4u) {
       const uint32_t k = k0 + e;
       double acc = 0.0;
       if (k < nq) {
         const uint32_t r = blockIdx.x * (256u * R) + (queue[k] >> 16), st = queue[k] & 0xffffu;
-        const uint32_t early = PAIRED ? r & 1u : 0u;
-        for (uint32_t uu = l; uu < 8u * bps; uu += 32u) {
-          const uint32_t b = bps * st + (uu >> 3) - early, u = uu & 7u;  // unit u of block b
-          if (b < nb) {
-            float wv[32];
-            decode_unit_exact<T>(w + ((size_t)r * nb + b) * kBytes, u, wv);
-            const float* const xu = xt + (size_t)b * kBlockElems + 32u * u;
+        const uint32_t b0 = first_block(st, r), b1 = end_block(st, r);
 #pragma unroll
-            for (int i = 0; i < 32; ++i) acc = fma((double)wv[i], (double)xu[i], acc);
+        for (uint32_t i = 0; i < kStageBlocks; ++i) {
+          const uint32_t b = b0 + i;
+          if (b < b1) {  // (the block before an odd row's first is no part of it)
+            const float4 wv = decode_four_exact<T>(w + ((size_t)r * nb + b) * kBytes, 4u * l);
+            const float4 xv =
+                *reinterpret_cast<const float4*>(xt + (size_t)b * kBlockElems + 4u * l);
+            acc = fma((double)wv.x, (double)xv.x, acc);
+            acc = fma((double)wv.y, (double)xv.y, acc);
+            acc = fma((double)wv.z, (double)xv.z, acc);
+            acc = fma((double)wv.w, (double)xv.w, acc);
           }
         }
       }
 #pragma unroll
-      for (int h = 16; h > 0; h >>= 1) acc += __shfl_xor(acc, h, 32);
+      for (int h = 32; h > 0; h >>= 1) acc += __shfl_xor(acc, h, 64);
       if (l == 0u && k < nq) value[k] = (float)acc;
     }
     __syncthreads();
   }
   if (row >= rows) return;
   if (mine) {  // the sums again, with the recomputed stages (unchanged for rows without one)
-    const uint32_t early = PAIRED ? row & 1u : 0u;
     const uint32_t nq = min(queued, kRedoQueue);
 #pragma unroll
     for (int c = 0; c < R; ++c) sum[c] = 0.0f;
@@ -366,10 +387,9 @@ __global__ __launch_bounds__(256) void tok_reduce(const float* __restrict__ part
             const uint32_t key = ((rw + (uint32_t)c) << 16) | st;
             uint32_t k = 0;
             while (k < nq && queue[k] != key) ++k;
+            const uint32_t r = row + (uint32_t)c, b0 = first_block(st, r);
             vc = k < nq ? value[k]
-                        : stage_exact<T>(w, row + (uint32_t)c, nb,
-                                         bps * st - (early != 0u && st != 0u ? 1u : 0u),
-                                         min(bps * st + bps - early, nb), xt);
+                        : stage_exact<T>(w, r, nb, b0 < nb ? b0 : 0u, end_block(st, r), xt);
           }
           sum[c] += vc;
         }
@@ -393,15 +413,15 @@ __global__ __launch_bounds__(256) void tok_reduce(const float* __restrict__ part
 template <uint32_t T, bool PAIRED = false>
 void launch_tok_reduce(const float* part, float* y, uint32_t rows, uint32_t yrows,
                        uint32_t nstages, uint32_t nv, uint32_t ntok, const uint8_t* w,
-                       const float* x, uint32_t nb, uint32_t bps, hipStream_t s) {
+                       const float* x, uint32_t nb, hipStream_t s) {
   const uint32_t g4 = (rows + 1023u) / 1024u;
   if (!PAIRED && rows % 4u == 0u && yrows % 4u == 0u && ((uintptr_t)y & 15u) == 0u &&
       (uint64_t)g4 * ntok >= 2u * (uint64_t)cu_count())
     hipLaunchKernelGGL((tok_reduce<T, 4, false>), dim3(g4, ntok), dim3(256), 0, s, part, y, rows, yrows,
-                       nstages, nv, w, x, nb, bps);
+                       nstages, nv, w, x, nb);
   else
     hipLaunchKernelGGL((tok_reduce<T, 1, PAIRED>), dim3((rows + 255u) / 256u, ntok), dim3(256), 0, s, part,
-                       y, rows, yrows, nstages, nv, w, x, nb, bps);
+                       y, rows, yrows, nstages, nv, w, x, nb);
 }
 
 }  // namespace
