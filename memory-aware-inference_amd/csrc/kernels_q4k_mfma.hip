@@ -987,12 +987,9 @@ bool launch_sliced(const uint8_t* w, const float* x, float* y, uint32_t rows, ui
 // images leave room for fewer than eight waves (or exceed the LDS
 // metadata), in four slices, else two, when that adds no pairs.  Rows
 // longer than the unsliced kernels take must slice.
-// The (tile, stage) pairs of an unsliced launch's busiest workgroup, on
-// launch_shape's grid at the given wave count.
+// The (tile, stage) pairs of an unsliced launch's busiest workgroup.
 uint64_t busiest_pairs(uint32_t ntiles, uint32_t tparts, uint32_t waves, size_t ws_bytes) {
-  const LaunchShape ls = launch_shape(ntiles, tparts, waves, ws_bytes, 1u);
-  const uint64_t g = ls.groups, q = ntiles / g, lp = (ntiles - q * g) * (uint64_t)tparts;
-  return ls.width != 0u ? q * tparts + (lp + g - 1u) / g : (ntiles + g - 1u) / g * tparts;
+  return launch_shape(ntiles, tparts, waves, ws_bytes, 1u).busiest;
 }
 
 // Whether an unsliced one-vector launch of W waves and SB-block stages fits

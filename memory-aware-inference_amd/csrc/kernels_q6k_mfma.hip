@@ -979,10 +979,7 @@ uint32_t q6_slices(uint32_t ntiles, uint32_t nb, size_t ws_bytes, bool pairs = f
     return S == 4u && cus >= 4u && (nst + 2u) / 3u <= 32u && most(3u) < most(4u) ? 3u : S;
   }
   // the unsliced launch's busiest workgroup (launch_shape's choice at 12 waves)
-  const LaunchShape ls = launch_shape(ntiles, nst, 12u, ws_bytes, 1u, (uint32_t)cus);
-  const uint64_t g1 = ls.groups;
-  const uint64_t q = ntiles / g1, lp = (ntiles - q * g1) * nst;
-  const uint64_t most0 = ls.width != 0u ? q * nst + (lp + g1 - 1u) / g1 : (ntiles + g1 - 1u) / g1 * nst;
+  const uint64_t most0 = launch_shape(ntiles, nst, 12u, ws_bytes, 1u, (uint32_t)cus).busiest;
   if (cus < 4u) return 0u;
   if (most0 <= 24u) {
     const uint32_t S = most(3u) < most(4u) ? 3u : 4u;

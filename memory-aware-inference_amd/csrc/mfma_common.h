@@ -1169,6 +1169,7 @@ struct LaunchShape {
   uint32_t groups;
   uint32_t width;  // pairs in a leftover range, 0: no tile is split
   uint32_t tiles_per_group;
+  uint64_t busiest;  // the most pairs of a workgroup
 };
 // Pair and tile indices divided with FastDiv stay below ntiles * tparts and
 // the ring's tile count below ntiles; the kernels need those times their
@@ -1211,6 +1212,8 @@ inline LaunchShape launch_shape(uint32_t ntiles, uint32_t tparts, uint32_t waves
   ls.tiles_per_group =
       split ? q + min(ntiles - q * g1, (uint32_t)((width + tparts - 2u) / tparts) + 1u)
             : (ntiles + g0 - 1u) / g0;
+  ls.busiest = split ? (uint64_t)q * tparts + min(width, lpairs)
+                     : (uint64_t)((ntiles + g0 - 1u) / g0) * tparts;
   return ls;
 }
 
