@@ -1074,8 +1074,9 @@ SliceChoice q4_slices(uint32_t ntiles, uint32_t nb, size_t ws_bytes, int qb) {
 //   Q5_K  1024 x 8192       -       7.9      8.3
 // So Q4_K takes two-block stages when the four-block launch leaves waves
 // idle (fewer pairs per workgroup than waves) and the two-block one needs at
-// most two rounds, or when 12 waves of four-block stages do not fit (three
-// rounds); Q5_K, whose four-block stages leave registers for only 8 waves,
+// most two rounds, or (three rounds) in rows of more than 40 blocks, which
+// leave 12 waves of four-block stages room for a few ring slots only, or none
+// (a group of 3200 + 512 + 512 x 10496 13.7 us, 12.1 in two-block stages); Q5_K, whose four-block stages leave registers for only 8 waves,
 // whenever 12 waves fit.  Slices stay where every unsliced workgroup would
 // build the whole row's activation images for a small share of the work:
 // at most a quarter as many tiles as CUs, rows of 64 blocks or more over
@@ -1093,7 +1094,7 @@ bool two_block_stages(uint32_t ntiles, uint32_t nb, size_t ws_bytes, int qb,
   if (nb > 56u) return false;
   const uint64_t rounds2 = (busiest_pairs(ntiles, (nb + 1u) / 2u, kWaves, ws_bytes) + kWaves - 1u) /
                            kWaves;
-  if (!unsliced_fits(ntiles, nb, kWaves, qb, 4, ws_bytes)) return rounds2 <= 3u;
+  if (nb > 40u) return rounds2 <= 3u;
   return rounds2 <= 2u && busiest_pairs(ntiles, (nb + 3u) / 4u, kWaves, ws_bytes) < kWaves;
 }
 
