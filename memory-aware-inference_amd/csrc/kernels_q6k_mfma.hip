@@ -954,12 +954,24 @@ bool launch_sliced(const uint8_t* w, const float* x, float* y, uint32_t rows, ui
 // unsliced): 4096 x 11008 13.8 / 16.0 / 14.6, 2047 x 11008 12.1 / 9.9 / 12.6,
 // 8192 x 11008 22.4 / 26.0 / 22.1 (unsliced 64), 4097 x 17152 - / 21.9 / 23.6;
 // 2560 x 17408 S = 3 / 4 14.4 / 14.9, 1360 x 17408 9.4 / 10.1.
+// and, with more pairs in rows whose images leave room for four waves at most
+// (unsliced / S = 2 / 3 / 4; - : not even those):
+//   3000 x 23552   24.9 / 22.1 / 23.1 / 21.7    5120 x 23552   35.9 / 32.4 / 31.2 / 33.5
+//   7000 x 24064   43.3 / 40.0 / 43.8 / 44.3   15062 x 25088   79.5 / 78.5 / 81.3 / 85.7
+//  24000 x 24064  110.8 / 115 / 120 / 131      30000 x 25088  140.1 / 144 / 149 / 164
+//   8192 x 32768      - / 51.5 / 59.1 / 57.2   10000 x 14080      - / 38.0 / 36.2 / 37.0
+//  24000 x 11520   66.9 / 60.2 / 62.1 / 67.0 (row pairs)
+//  10000 x 11008      - /    - / 31.0 / 29.5   10000 x 11520   38.4 / 33.3 / 31.4 / 33.1
+// A pair costs 3 % more in three slices than in two and 22 % more in four (12 %
+// with row pairs).
 // So: four slices, or three where that leaves the busiest workgroup fewer
 // pairs, when the unsliced launch's busiest workgroup has at most two rounds
 // of pairs (24; its build is then exposed) and slicing adds it none or the
 // rows are long (48 blocks or more); with more pairs, only when the unsliced
 // images leave room for fewer than eight waves (very long rows), in the
-// number of two to four that gives the busiest workgroup the fewest.
+// number of two to four whose busiest workgroup takes the least time, except
+// that whole rows stay where four waves fit and more than 250 pairs hide their
+// build.
 uint32_t q6_slices(uint32_t ntiles, uint32_t nb, size_t ws_bytes, bool pairs = false,
                    uint64_t cus = (uint64_t)cu_count()) {
   static const int env = env_int("SI_HIP_Q6K_SLICES", -1);
@@ -989,9 +1001,12 @@ uint32_t q6_slices(uint32_t ntiles, uint32_t nb, size_t ws_bytes, bool pairs = f
       ring_slots(8u, 1u, launch_shape(ntiles, nst, 8u, ws_bytes, 1u, (uint32_t)cus).tiles_per_group,
                  pairs ? 2u * nst : nst);
   if (layout(8u, 1u, nb, slots, pairs ? 2u : 1u).total <= kLdsBytes) return 0u;
+  if (!pairs && most0 > 250u && layout(4u, 1u, nb, 4u).total <= kLdsBytes) return 0u;
+  const uint32_t four = pairs ? 112u : 122u;
+  auto cost = [&](uint32_t S) { return most(S) * (S == 2u ? 100u : S == 3u ? 103u : four); };
   uint32_t best = 2u;
   for (uint32_t S : {3u, 4u})
-    if (most(S) < most(best)) best = S;
+    if (cost(S) < cost(best)) best = S;
   return best;
 }
 

@@ -40,7 +40,9 @@ def log(msg):
 # blocks, which must slice (136 blocks: four slices of 17 stages; 256
 # blocks: four of 32; 548 blocks: sixteen of 18)
 SHAPES = [(16, 12288), (1000, 12800), (2560, 17408), (640, 17408), (2048, 32768), (3, 27648),
-          (100, 34816), (2560, 34816), (40, 65536), (17, 140288)]
+          (100, 34816), (2560, 34816), (40, 65536), (17, 140288),
+          # more than two rounds of pairs: four, three and two slices, and whole rows
+          (3000, 23552), (5120, 23552), (7000, 24064), (24000, 23552)]
 
 
 @pytest.mark.parametrize("rows,cols", SHAPES)
