@@ -15,6 +15,7 @@ import pytest
 
 import crafted
 import oracle_lib as O
+import quantize
 import si_hip
 from test_gpu_parity import _category, assert_dot_close, log, same_bits
 
@@ -107,18 +108,37 @@ def test_verify_special_blocks(hip_ctx, t, rows, cols):
 
 
 @pytest.mark.parametrize("t", [12, 13])
-@pytest.mark.parametrize("rows,cols", [(48, 512), (80, 5120), (33, 2816)])
-def test_matvec_cancelling_terms(hip_ctx, t, rows, cols):
-    """One vector: a constant vector against weights of nearly zero mean in
-    every block, so that the scale and the minimum terms cancel: the row's
-    error stays far under its terms' size."""
-    w = si_hip.synth_matrix(t, seed=rows + 9 * cols + t, rows=rows, cols=cols, threads=8)
-    dq = O.dequantize(t, w, rows * cols).reshape(rows, cols).astype(np.float64)
-    x = (np.ones(cols) + 1e-3 * si_hip.synth_normal(cols, cols)).astype(np.float32)
-    W = hip_ctx.upload_quant_weight_private(w, t)
+@pytest.mark.parametrize("rows,cols,batch", [(480, 512, 1), (400, 5120, 1), (17408, 5120, 1),
+                                             (330, 2816, 2), (400, 8192, 2), (400, 5120, 4),
+                                             (330, 2816, 5), (400, 5120, 16)])
+def test_cancelling_terms(hip_ctx, t, rows, cols, batch):
+    """A nearly constant vector against weights quantised from zero-mean ones, so
+    that a block's scale and minimum terms are some seventy times its dot: the error
+    stays what the f32 rounding of the partial sums makes it, at most 2^-25 of a sum
+    and of either sign, under 2^-24 of the blocks' |dots| over the rows.  (With the
+    terms in f32 it is their size that counts.)"""
+    log(f"cancelling terms t={t} {rows}x{cols} M={batch}")
+    rng = np.random.default_rng(rows + 9 * cols + t)
+    base = min(rows, 480)
+    w = quantize.quantize(t, 0.02 * rng.standard_normal((base, cols)))
+    scales, mins = quantize.terms(t, w)
+    assert np.median(np.abs(scales - mins) / (scales + mins)) < 0.02
+    X = (1.0 + 1e-3 * rng.standard_normal((batch, cols))).astype(np.float32)
+    dq = O.dequantize(t, w, base * cols).reshape(base, cols // 256, 256).astype(np.float64)
+    X64 = X.astype(np.float64).reshape(batch, cols // 256, 256)
+    reps = -(-rows // base)
+    W = hip_ctx.upload_quant_weight_private(
+        np.tile(w.reshape(base, -1), (reps, 1))[:rows].reshape(-1), t)
     try:
-        y = hip_ctx.gguf_quant_matvec_weight(W, rows, cols, x)
-        assert_dot_close(y, dq @ x.astype(np.float64), np.abs(dq) @ np.abs(x.astype(np.float64)))
+        if batch == 1:
+            outs = [hip_ctx.gguf_quant_matvec_weight(W, rows, cols, X[0])]
+        else:
+            outs = hip_ctx.gguf_quant_matmul_many_weight(W, rows, cols, batch, X)
+        for b in range(batch):
+            dots = (dq * X64[b]).sum(2)
+            err = outs[b][:base].astype(np.float64) - dots.sum(1)
+            rms = np.sqrt(np.mean(err ** 2)) / np.sqrt(np.mean(np.abs(dots).sum(1) ** 2))
+            assert rms <= 2.0 ** -24, f"vector {b}: {rms:.2e}"
     finally:
         W.free()
 
@@ -193,4 +213,33 @@ def test_verify_redone_slices(hip_ctx, t, nb, batch):
             _, y64, ab = O.matvec(t, w, rows, cols, X[b], threads=8)
             assert_dot_close(outs[b], y64, ab, 1e-6, f"vector {b}")
     finally:
+        W.free()
+
+
+@pytest.mark.parametrize("t,rows,nb", [(12, 65573, 128), (13, 65573, 128), (14, 65573, 128),
+                                       (14, 65573, 127), (14, 65574, 127)])
+def test_verify_in_several_row_ranges(hip_ctx, t, rows, nb):
+    """Sixteen vectors whose partial sums fill the scratch three times over: the
+    ranges are 32768 rows and a ragged rest (an odd and an even one where the rows
+    run in pairs).  The matrix is 64 rows over and over, so every row is, bit for
+    bit, that of a matrix of those alone, one range."""
+    cols, period, batch = 256 * nb, 64, 16
+    log(f"verify in ranges t={t} {rows}x{cols}")
+    small = si_hip.synth_matrix(t, seed=nb + t, rows=period, cols=cols, threads=8)
+    row_bytes = small.size // period
+    big = np.tile(small, -(-rows // period))[:rows * row_bytes]
+    X = si_hip.synth_normal(nb, batch * cols).reshape(batch, cols).copy()
+    X[3, 300:600] *= np.float32(1e-6)
+    X[5, cols - 1] = np.inf
+    S, W = (hip_ctx.upload_quant_weight_private(m, t) for m in (small, big))
+    del big
+    try:
+        want = [o.copy() for o in hip_ctx.gguf_quant_matmul_many_weight(S, period, cols, batch, X)]
+        outs = hip_ctx.gguf_quant_matmul_many_weight(W, rows, cols, batch, X)
+        for b in range(batch):
+            assert same_bits(outs[b], np.tile(want[b], -(-rows // period))[:rows]), f"vector {b}"
+        _, y64, ab = O.matvec(t, small, period, cols, X[0], threads=8)
+        assert_dot_close(want[0], y64, ab, what="the repeated rows")
+    finally:
+        S.free()
         W.free()
