@@ -9,12 +9,13 @@ and small activations everywhere else, which then carry the whole dot:
 
   "tiny"  x = +-1 on the zero weights, +-(0.5..2)e-7 elsewhere
   "side"  x = +-1 on the zero weights, 1..8 elements of +-(0.5..2)e-6 per
-          block (as many as a block's side list holds), the rest 0
+          block (few enough to be held to f32 rounding with several vectors),
+          the rest 0
   "edge"  x = +-1 on the zero weights, +-2^-13 (1..1.5) elsewhere: just above
           the side threshold 2^(e - 14) of a block whose maximum is 1 (e = 1)
   "many"  x = +-1 next to the zero weights (element 16 c + 1), 9..16 elements
-          of +-(0.5..2)e-6 per block, the rest 0: more side elements than a
-          block lists, on a dot that the large activations carry
+          of +-(0.5..2)e-6 per block, the rest 0: more side elements than that,
+          on a dot that the large activations carry
 
 Zero weights: Q4_K q = 0 with every min 0; Q5_K q = 0 (qh bit clear) with
 every min 0; Q6_K q = 32 (quant.rs:36-63, 90-122, 145-171).

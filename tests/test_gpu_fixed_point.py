@@ -1,7 +1,7 @@
 """GPU: the matrix-core kernels' fixed-point activations against the oracle on
 inputs built to defeat them (tests/crafted.py): small activations carrying the
-whole dot next to large ones on zero weights, side lists of 1..5 entries per
-block, and activations just above the side threshold.  Every dot must stay
+whole dot next to large ones on zero weights, 1..16 side elements per block,
+and activations just above the side threshold.  Every dot must stay
 within 2e-5 * sum|w*x| of the f64 value of the exact products (quant.rs
 weights), through every kernel that builds digit images: Q4_K/Q5_K/Q6_K at
 M = 1 (including the 17408-column down projection), fused gate/up, the fused
