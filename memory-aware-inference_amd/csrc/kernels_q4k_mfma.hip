@@ -234,21 +234,6 @@ __device__ __forceinline__ i32x4 high_nibbles(const u32x4& q) {
                (int)((q[2] >> 4) & 0x0f0f0f0fu), (int)((q[3] >> 4) & 0x0f0f0f0fu)};
 }
 
-// Exact value of a Q4_K/Q5_K weight with quant q of unit u (uniform) from
-// the block's 16-byte header (d, dmin, the 12 scale bytes; quant.rs:176-185).
-__device__ __forceinline__ float k4_weight(const u32x4& h, uint32_t u, uint32_t q) {
-  const uint32_t sc03 = h[1] & 0x3f3f3f3fu;
-  const uint32_t mn03 = h[2] & 0x3f3f3f3fu;
-  const uint32_t sc47 = (h[3] & 0x0f0f0f0fu) | ((h[1] >> 2) & 0x30303030u);
-  const uint32_t mn47 = ((h[3] >> 4) & 0x0f0f0f0fu) | ((h[2] >> 2) & 0x30303030u);
-  const uint32_t sh = 8u * (u & 3u);
-  const uint32_t sc = ((u < 4u ? sc03 : sc47) >> sh) & 0xffu;
-  const uint32_t mn = ((u < 4u ? mn03 : mn47) >> sh) & 0xffu;
-  const float d = half_bits_to_float(h[0] & 0xffffu);
-  const float dmin = half_bits_to_float(h[0] >> 16);
-  return k4_value_exact(__fmul_rn(d, (float)sc), __fmul_rn(dmin, (float)mn), q);
-}
-
 // Exact per-weight f32 dot of 16 nibbles (low or high half of each byte of q)
 // with 16 activations.
 __device__ __forceinline__ float exact_dot16(const u32x4& q, int shift, float d1, float m1,

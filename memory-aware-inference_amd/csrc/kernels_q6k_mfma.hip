@@ -24,15 +24,14 @@
 // Data path.  Blocks are 210 bytes, so they are not 16-byte aligned; with an
 // even block count nb every row and every stage of two blocks (420 bytes)
 // starts on a 4-byte boundary, which the 16-byte buffer->LDS copies need (odd
-// nb runs as row pairs, PAIRED below).  Each row's 420 bytes of a stage arrive
-// with 27 copies in piece-major order, piece q of row r at LDS byte
-// 16 (16 q + r), so every read is a conflict-free 16-lane sweep.  Pieces 0..25
-// are bytes 16 q .. 16 q + 15; piece 26 is bytes 404..419, so no copy runs
-// past the stage (a copy that crosses the end of its buffer descriptor reads
-// as zero in full).  The second block of a stage starts 2 bytes into piece
-// 13: its chunks are read as two pieces and realigned with v_alignbyte.
-// Scheduling, the LDS slot ring and the finishing wave are the Q4_K
-// kernel's (mfma_common.h).
+// nb runs as row pairs, PAIRED below; a matrix that starts off a word, on the
+// generic kernels).  A stage is copied row by row (copy_offsets): piece q of row
+// r at LDS byte 432 r + 16 q, 27 pieces a row, an odd pitch.  Pieces 0..25 are
+// bytes 16 q .. 16 q + 15; piece 26 is bytes 404..419, so no copy runs past the
+// stage.  A copy's words past the end of its buffer descriptor read as zero, each
+// word by itself.  The second block of a stage starts 2 bytes into piece 13: its
+// chunks are read as two pieces and realigned with v_alignbyte.  Scheduling, the
+// LDS slot ring and the finishing wave are the Q4_K kernel's (mfma_common.h).
 #include "argmax_device.h"
 #include "mfma_common.h"
 #include "si_hip_tuned.h"
@@ -340,10 +339,8 @@ __global__ __launch_bounds__(WAVES * 64) void q6k_matvec_mfma(const uint8_t* __r
 
   // 2. this wave's pairs k = wave, wave + WAVES, ... of the workgroup's pairs
   //    (pair_at: a tile and its stage) and the copies of its first DEPTH, pair
-  //    j into buffer j % DEPTH.  Copy i, lane l moves
-  //    piece 4 i + l / 16 of row l % 16; the 16 lanes whose piece would be the
-  //    28th re-read the 27th (same addresses, no extra traffic).  All copies
-  //    lie inside the stage's 420 bytes of their row.
+  //    j into buffer j % DEPTH (copy_offsets).  All copies lie inside the stage's
+  //    420 bytes of their row.
   auto pair_of = [&](uint32_t k) -> Pair {
     if constexpr (SLICED)
       return pair_at(ss, k);
@@ -739,7 +736,8 @@ __global__ __launch_bounds__(WAVES * 64) void q6k_tokens_mfma(const uint8_t* __r
     uint32_t size = nrows * row_bytes;
     if constexpr (PAIRED) {
       // the last pair of an odd row count is one row, its last 2 bytes the
-      // lower half of a word
+      // lower half of a word: the size is rounded up to that word, which the last
+      // block's d lies in (the words of its piece past it read as zero)
       if (2u * (row0 + nrows) > rows) size = (size - nb * kQ6Bytes + 3u) & ~3u;
     }
     const __amdgpu_buffer_rsrc_t rsrc = __builtin_amdgcn_make_buffer_rsrc(

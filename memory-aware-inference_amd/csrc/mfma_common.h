@@ -153,15 +153,6 @@ constexpr int kRowShr1 = 0x111, kRowShr2 = 0x112, kRowShr4 = 0x114, kRowShr8 = 0
 constexpr int kQuadSwap = 0xb1;  // quad_perm [1, 0, 3, 2]: lanes 2 k and 2 k + 1 trade
 constexpr int kRowBcast15 = 0x15f;
 
-// Word k (uniform, 0..3) of a 16-byte piece.
-__device__ __forceinline__ uint32_t word_of(const u32x4& p, uint32_t k) {
-  return k == 0u ? p[0] : k == 1u ? p[1] : k == 2u ? p[2] : p[3];
-}
-// Byte k (uniform, 0..15) of a 16-byte piece.
-__device__ __forceinline__ uint32_t byte_of(const u32x4& p, uint32_t k) {
-  return (word_of(p, k >> 2) >> (8u * (k & 3u))) & 0xffu;
-}
-
 // The stage's side counts, one byte per block, with the bytes of blocks at
 // or past `nlive` cleared.
 __device__ __forceinline__ uint32_t live_counts(uint32_t word, uint32_t nlive) {
@@ -209,11 +200,6 @@ __device__ __forceinline__ uint32_t lds_claim(uint32_t addr) {
 __device__ __forceinline__ uint32_t lds_read_b32(uint32_t addr) {
   uint32_t v;
   asm volatile("ds_read_b32 %0, %1\ns_waitcnt lgkmcnt(0)" : "=&v"(v) : "v"(addr) : "memory");
-  return v;
-}
-__device__ __forceinline__ uint32_t lds_read_u16(uint32_t addr) {
-  uint32_t v;
-  asm volatile("ds_read_u16 %0, %1\ns_waitcnt lgkmcnt(0)" : "=&v"(v) : "v"(addr) : "memory");
   return v;
 }
 __device__ __forceinline__ u32x2 lds_read_b64(uint32_t addr) {

@@ -16,18 +16,15 @@ namespace sihip {
 namespace mfma {
 namespace {
 
-// Plain LDS reads: the compiler places their waits, so that a block's reads
-// overlap.  (For kernels without buffer->LDS copies, which the compiler would
-// wait for at the first such read.)
 typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
 typedef _Float16 f16x4 __attribute__((ext_vector_type(4)));
 typedef uint16_t u16x2 __attribute__((ext_vector_type(2)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
+// A plain LDS read, its wait placed by the compiler, which also waits there for
+// the buffer->LDS copies in flight: only for reads before the stage loop
+// (slice_err, once a launch and group).
 __device__ __forceinline__ u32x4 lds_u32x4(const uint8_t* p) {
   return *(const __attribute__((address_space(3))) u32x4*)p;
-}
-__device__ __forceinline__ uint32_t lds_u32(const uint8_t* p) {
-  return *(const __attribute__((address_space(3))) uint32_t*)p;
 }
 __device__ __forceinline__ void lds_write_b16(uint32_t addr, uint32_t v) {
   asm volatile("ds_write_b16 %0, %1" : : "v"(addr), "v"(v) : "memory");
