@@ -949,22 +949,23 @@ bool launch_sliced(const uint8_t* w, const float* x, float* y, uint32_t rows, ui
 }
 
 // Slices for a one-vector Q4_K / Q5_K launch, or 0.  The same rule as the
-// Q6_K kernel's (q6_slices), measured on this kernel (MI355X, us):
+// Q6_K kernel's (q6_slices), measured on this kernel (MI355X, us, weights
+// quantised from zero-mean ones, 600 MB of them in turn):
 //   type  rows x cols    unsliced  S = 2   S = 4   S = 8
-//   Q4_K  5120 x 17408     18.3     18.3    16.5    21.5
-//   Q4_K  2048 x 16384     12.4     10.0     9.0    10.2
-//   Q4_K  640 x 17408      11.5      9.3     8.0     8.5
-//   Q4_K  8192 x 28672    140.0     38.1    34.9    41.1   (unsliced: 4 waves)
-//   Q4_K  2560 x 34816     75.7     22.8    18.8    18.2   (unsliced: generic kernel)
-//   Q4_K  2560 x 9728       8.6      9.1     8.6     9.7
-//   Q4_K  17408 x 5120     13.6     17.7    22.7
-//   Q4_K  5120 x 5120       7.7      8.1     8.8
-//   Q4_K  8192 x 8192      11.5              15.6
-//   Q4_K  12288 x 8192     15.0              18.5
-//   Q4_K  4096 x 8192       8.9               9.4
-//   Q4_K  4096 x 12288     10.3              10.5            (unsliced: 8 waves)
-//   Q5_K  5120 x 17408     25.6     23.9    22.1    27.0
-//   Q5_K  5120 x 5120       9.2     11.2    11.7
+//   Q4_K  5120 x 17408     20.0     18.3    16.7    22.0   (unsliced: 8 waves)
+//   Q4_K  2048 x 16384     13.4     10.5     9.5    12.4
+//   Q4_K  640 x 17408      11.2     10.5     7.7     8.4
+//   Q4_K  8192 x 28672              38.6    35.5    41.3
+//   Q4_K  2560 x 34816     66.0     24.7    18.8    18.4   (unsliced: generic kernel)
+//   Q4_K  2560 x 9728      10.1              9.0           (two-block stages 8.9)
+//   Q4_K  17408 x 5120     12.3             23.6
+//   Q4_K  5120 x 5120       7.8             10.4
+//   Q4_K  8192 x 8192      11.9     13.0    14.0
+//   Q4_K  12288 x 8192     15.9             19.1
+//   Q4_K  4096 x 8192       9.1             10.7
+//   Q4_K  4096 x 12288     12.5     11.0    10.9           (unsliced: 8 waves)
+//   Q5_K  5120 x 17408     21.5     24.0    22.0    27.8   (unsliced: two-block)
+//   Q5_K  5120 x 5120       9.7             11.0
 // So: rows of fewer than 8 stages (K < 8192) stay whole; four slices when
 // the unsliced launch's busiest workgroup has at most two rounds of pairs
 // (24) and slicing takes some of them (a tie keeps the whole rows) or the
@@ -1035,34 +1036,34 @@ SliceChoice q4_slices(uint32_t ntiles, uint32_t nb, size_t ws_bytes, int qb) {
 // Whether one Q4_K / Q5_K vector runs as two-block stages (12 waves,
 // unsliced) rather than the slices of `sc` or four-block stages.  A stage of
 // two blocks halves each pair, so more waves share a short launch; it costs
-// more per block (twice the pairs, hand-offs and waits).  Measured on MI355X
+// more per block (twice the pairs, hand-offs and waits).  Measured as above
 // (us; the four-block kernel unsliced at 12 waves, or at 8 where 12 do not
 // fit):
 //   type  rows x cols    4-block  sliced  2-block
-//   Q4_K  4096 x 4096       5.6      -       5.2
-//   Q4_K  8192 x 5120       8.0      -       7.5
-//   Q4_K  5120 x 5120       7.6      -       7.1
-//   Q4_K  1024 x 5120       6.1      -       5.6
-//   Q4_K  4096 x 8192       8.9     9.4      8.1
-//   Q4_K  8192 x 6144       8.6      -       9.1   (12 pairs per workgroup)
-//   Q4_K  8192 x 8192      11.5    15.6     12.4   (16)
-//   Q4_K  17408 x 5120     13.8      -      14.8   (22)
-//   Q4_K  4096 x 14336     11.8    13.6     11.4   (12 waves do not fit)
-//   Q4_K  2048 x 11008      -       8.4      8.9
-//   Q4_K  1024 x 17408     11.2     8.1     10.7
-//   Q5_K  5120 x 5120       9.1      -       7.9
-//   Q5_K  8192 x 8192      16.0    16.6     14.6
-//   Q5_K  17408 x 5120     18.0      -      18.1
-//   Q5_K  5120 x 17408     22.2    22.2     20.3
-//   Q5_K  2560 x 17408      -      15.0     15.7
-//   Q5_K  640 x 17408       -       8.7     11.4
-//   Q5_K  1024 x 8192       -       7.9      8.3
+//   Q4_K  4096 x 4096       6.1      -       5.8
+//   Q4_K  8192 x 5120       8.3      -       8.3
+//   Q4_K  5120 x 5120       7.9      -       7.8
+//   Q4_K  1024 x 5120       6.5      -       6.0
+//   Q4_K  4096 x 8192       9.1    10.7      9.0
+//   Q4_K  8192 x 6144       9.2      -       9.7   (12 pairs per workgroup)
+//   Q4_K  8192 x 8192      11.9    14.0     12.3   (16)
+//   Q4_K  17408 x 5120     12.3      -      14.8   (22)
+//   Q4_K  4096 x 14336     14.1    13.0     13.7   (12 waves do not fit)
+//   Q4_K  2048 x 11008       -      8.1     10.0
+//   Q4_K  1024 x 17408     11.9     8.1     11.6
+//   Q5_K  5120 x 5120       9.7      -       8.4
+//   Q5_K  8192 x 8192      15.1    15.9     14.2
+//   Q5_K  17408 x 5120     17.2      -      16.7
+//   Q5_K  5120 x 17408       -     22.0     21.5
+//   Q5_K  2560 x 17408       -     14.5     15.3
+//   Q5_K  640 x 17408        -      8.1     11.2
+//   Q5_K  1024 x 8192        -      7.4      8.7
 // So Q4_K takes two-block stages when the four-block launch leaves waves
 // idle (fewer pairs per workgroup than waves) and the two-block one needs at
 // most two rounds, or (three rounds) in rows of more than 40 blocks, which
 // leave 12 waves of four-block stages room for a few ring slots only, or none
-// (a group of 3200 + 512 + 512 x 10496 13.7 us, 12.1 in two-block stages); Q5_K, whose four-block stages leave registers for only 8 waves,
-// whenever 12 waves fit.  Slices stay where every unsliced workgroup would
+// (a group of 3200 + 512 + 512 x 10496 13.7 us, 12.1 in two-block stages); Q5_K,
+// whose four-block stages leave registers for only 8 waves, whenever 12 waves fit.  Slices stay where every unsliced workgroup would
 // build the whole row's activation images for a small share of the work:
 // at most a quarter as many tiles as CUs, rows of 64 blocks or more over
 // fewer tiles than CUs, and rows past 32 blocks whose busiest workgroup the
@@ -1096,11 +1097,11 @@ bool shape_ok(uint32_t rows, uint32_t cols, uint32_t mats, int qb, uint32_t sb =
 
 // Whether a sliced launch takes two-block stages: when the busiest sliced
 // workgroup of four-block stages has fewer pairs than 12 waves, so that
-// waves would idle.  Measured on MI355X (us, S = 4, four- / two-block):
-// Q4_K 1024 x 17408 7.62 / 7.17, 640 x 17408 7.27 / 6.99, 2048 x 16384 8.39 /
-// 8.14, 1000 x 12800 7.07 / 6.69, 2048 x 11008 7.53 / 7.37; Q5_K 1024 x 17408
-// 8.48 / 7.77, 2048 x 16384 9.40 / 8.85; with more pairs four-block stages
-// win: Q4_K 2560 x 17408 9.94 / 11.95, 5120 x 17408 16.2 / 19.9.
+// waves would idle.  Measured as above (us, S = 4, four- / two-block): Q4_K
+// 1024 x 17408 9.0 / 8.0, 640 x 17408 8.6 / 7.7, 2048 x 16384 9.4 / 9.5,
+// 1000 x 12800 7.9 / 7.7, 2048 x 11008 8.6 / 8.1; Q5_K 1024 x 17408 9.9 / 8.5,
+// 2048 x 16384 10.4 / 10.0; with more pairs four-block stages win: Q4_K
+// 2560 x 17408 10.9 / 12.0, 5120 x 17408 16.9 / 20.7.
 // SI_HIP_Q4K_SLICE_SB (2 or 4) fixes the choice.
 bool sliced_two_block(uint32_t ntiles, uint32_t nb, uint32_t S, size_t ws_bytes) {
   static const int env = env_int("SI_HIP_Q4K_SLICE_SB", 0);
@@ -1177,11 +1178,12 @@ bool launch_q4k_matvec_mfma(const uint8_t* w, const float* x, float* y, uint32_t
              launch_wd<8, 1, 1, 4, false, 4, true>(w, nullptr, x, y, rows, nb, ws, s, err);
     default: break;
   }
-  // full-line copies where the shape allows them, measured on MI355X
-  // (17408 x 5120, us, back to back over 8 resident copies): 12 waves 13.1,
-  // 8 waves 13.5, 6 waves with two stages in flight 15.9 (the stage
-  // arithmetic needs three waves per SIMD to hide its latency); the
-  // half-line copies at 12 waves 13.6
+  // full-line copies where the shape allows them (17408 x 5120, us, 600 MB of
+  // copies in turn): 12 waves 12.3, 8 waves 14.1, 6 waves with two stages in
+  // flight 16.4 (the stage arithmetic needs three waves per SIMD to hide its
+  // latency); the half-line copies at 12 waves 13.0.  (Out of the 256 MB Infinity
+  // Cache, which the nontemporal lines pass by, the half-line copies are up to 3 %
+  // ahead; a model's weights come from HBM.)
   if (lines_fit(nb, w) &&
       launch_wd<12, 1, 1, 4, false, 4, true>(w, nullptr, x, y, rows, nb, ws, s, err))
     return true;
@@ -1285,14 +1287,13 @@ bool launch_q4k_gate_up_mfma(const uint8_t* gate, const uint8_t* up, const float
              launch_wd<12, 1, 2, 4, false, 4, true>(gate, up, x, h, rows, nb, ws, s, err);
     default: break;
   }
-  // full-line copies at 12 waves: 17408 x 5120 22.9 us against 23.5 (27.7
-  // with 6 waves and two stages in flight)
+  // full-line copies at 12 waves: 17408 x 5120 21.3 us against 22.1
   if (lines_fit(nb, gate, up) &&
       launch_wd<12, 1, 2, 4, false, 4, true>(gate, up, x, h, rows, nb, ws, s, err))
     return true;
-  // 12 waves (161 VGPRs, no spills): measured on MI355X against 8, us:
-  // 17408 x 5120 23.1 / 24.0, 14336 x 4096 15.5 / 16.6, 11008 x 4096
-  // 12.8 / 13.5, 8192 x 2048 6.9 / 7.1-7.4, 4096 x 4096 7.0 / 7.1-7.4
+  // 12 waves (163 VGPRs, no spills) against 8, half-line copies, us: 17408 x 5120
+  // 22.1 / 23.9, 14336 x 4096 16.8 / 17.4, 11008 x 4096 14.1 / 14.6, 8192 x 2048
+  // and 4096 x 4096 level at 7.8
   return launch_wd<12, 1, 2>(gate, up, x, h, rows, nb, ws, s, err) ||
          launch_wd<8, 1, 2>(gate, up, x, h, rows, nb, ws, s, err) ||
          launch_wd<4, 1, 2>(gate, up, x, h, rows, nb, ws, s, err);

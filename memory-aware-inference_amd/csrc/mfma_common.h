@@ -27,8 +27,8 @@
 // Which chunk goes to which (MFMA, lane group) slot depends on how a format
 // lays its weights out; build_images takes that map as a template argument.
 //
-// Workgroup protocol.  One persistent workgroup per CU walks a contiguous
-// range of (tile, stage) pairs; a wave leaves each stage's 16 row partials in
+// Workgroup protocol.  One persistent workgroup per CU works through its share
+// of the (tile, stage) pairs (Sched below); a wave leaves each stage's 16 row partials in
 // an LDS slot of its tile and counts them with an LDS atomic; the wave that
 // completes the workgroup's share of a tile sums the partials in stage order
 // (results do not depend on timing).  LDS is
