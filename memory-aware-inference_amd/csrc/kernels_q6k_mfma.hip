@@ -938,20 +938,19 @@ bool launch_sliced(const uint8_t* w, const float* x, float* y, uint32_t rows, ui
 // and only its first stages (one per wave, plus a pair touched into L2) are
 // in flight meanwhile; slicing shrinks the build S-fold but rounds each
 // slice's stages and each workgroup's tiles up.  Measured (MI355X, us):
-//   rows x cols      unsliced  S = 2   S = 4
-//   640 x 17408        12.1     11.0     8.3
-//   2560 x 17408       18.4     19.1    15.2
-//   2048 x 16384       13.3     10.8    10.0
-//   512 x 12288        10.9      8.3     7.3
-//   4096 x 14336       16.2     17.0    16.3
-//   5120 x 17408       24.5     27.2    25.7
-//   8192 x 28672       57.0     52.4    56.0
-//   2048 x 32768       50.4     20.2
-//   2560 x 9728         9.5              9.7
-// and, rows of odd block counts taken as pairs (S = 2 / 3 / 4, four waves
-// unsliced): 4096 x 11008 13.8 / 16.0 / 14.6, 2047 x 11008 12.1 / 9.9 / 12.6,
-// 8192 x 11008 22.4 / 26.0 / 22.1 (unsliced 64), 4097 x 17152 - / 21.9 / 23.6;
-// 2560 x 17408 S = 3 / 4 14.4 / 14.9, 1360 x 17408 9.4 / 10.1.
+//   rows x cols      unsliced  S = 2   S = 3   S = 4
+//   640 x 17408        10.4     10.2     8.6     8.4
+//   2560 x 17408       15.6     17.6    14.7    15.3
+//   2048 x 16384       12.3     10.6    13.7    11.1
+//   512 x 12288        10.1      8.1     7.3     7.2
+//   4096 x 14336       15.3     16.7    19.4    16.1
+//   5120 x 17408       21.9     24.2    24.7    24.3
+//   8192 x 28672       49.9     48.2    55.8    54.6
+//   2048 x 32768       51.2     17.7    20.3    18.1
+//   2560 x 9728         9.7     10.3     9.6     9.9
+// and, rows of odd block counts taken as pairs (four waves unsliced): 4096 x
+// 11008 - / 14.5 / 16.1 / 14.8, 2047 x 11008 - / 12.3 / 9.9 / 12.4, 8192 x 11008
+// 21.9 / 23.1 / 26.3 / 22.2, 1360 x 17408 11.2 / 10.8 / 9.6 / 10.2.
 // and, with more pairs in rows whose images leave room for four waves at most
 // (unsliced / S = 2 / 3 / 4; - : not even those):
 //   3000 x 23552   24.9 / 22.1 / 23.1 / 21.7    5120 x 23552   35.9 / 32.4 / 31.2 / 33.5
@@ -1164,14 +1163,19 @@ bool launch_q6k_matmul_mfma(const uint8_t* w, const float* x, float* y, uint32_t
                             hipError_t* err) {
   if (batch < 2u || batch > 16u) return false;
   const uint32_t nb = cols / kBlockElems;
-  // Odd row and block counts: the generic kernel, which takes any, where it is
-  // faster, short rows and few vectors (us, generic / here: 129 x 2816 M = 2 / 3
-  // 6.5 / 7.2, 8.0 / 7.2; 1025 x 1280 M = 5 / 8 7.8 / 9.0, 10.9 / 9.0; 4097 x 256
-  // M = 2 / 4 6.0 / 6.8, 8.8 / 7.0; 33 x 5376 M = 2 9.0 / 7.2; 2049 x 2816 M = 2
-  // 10.2 / 8.6; a single row of 2816 M = 5 / 8 7.7 / 8.0, 10.6 / 8.2).
-  if ((nb & 1u) != 0u && (rows & 1u) != 0u && nb < 16u && (uint64_t)rows * nb < 16384u &&
-      rows * batch < 12288u &&
-      (rows < 16u ? batch * nb < 64u : batch < 8u && batch * nb < 33u))
+  // Odd row and block counts: the generic kernel, a wave a row, where it is faster.
+  // Its latency is that of one row, some 0.7 us a vector for each eight blocks,
+  // against the 7 to 8 us of the pass and the reduce here: five or six vectors in
+  // rows of up to eight blocks and two of up to sixteen, or eleven and five over a
+  // single row, whose loads meet nobody else's; and it does every weight's products one by
+  // one, which many rows, or many of their sums, make the larger part.  Us, generic
+  // / here: 257 x 768 M = 6 / 8 6.8 / 8.1, 8.1 / 8.0; 513 x 2304 M = 2 / 3 7.7 /
+  // 8.0, 9.3 / 8.1; one row of 1792 M = 8 / 16 6.9 / 8.0, 12.0 / 10.0; 2049 x 1280
+  // M = 3 / 4 7.8 / 8.1, 9.4 / 8.1; 4097 x 256 M = 2 / 3 6.2 / 6.7, 7.5 / 6.9;
+  // 4097 x 1280 M = 2 9.2 / 8.5.
+  const uint32_t most = rows == 1u ? (nb < 8u ? 11u : 5u) : nb < 6u ? 6u : nb < 8u ? 5u : 2u;
+  if ((nb & 1u) != 0u && (rows & 1u) != 0u && nb < 16u && batch <= most &&
+      (uint64_t)rows * batch <= 10300u && (uint64_t)rows * batch * nb <= 32768u)
     return false;
   // Two vectors over short rows: whole rows in one launch, no reduce behind it
   // (two_vectors, mfma_common.h).

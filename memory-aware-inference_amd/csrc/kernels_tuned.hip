@@ -32,9 +32,9 @@ bool launch_matvec_tuned(uint32_t type, const uint8_t* w, const float* x, float*
   if (type == kTypeQ6K && batch > 1 &&
       launch_q6k_matmul_mfma(w, x, y, rows, cols, batch, ws, s, err))
     return true;
-  // Odd row and block counts that launch left: the generic kernel reads the
-  // weights once for all the vectors, up to the size where one vector at a time
-  // is faster.
+  // Odd row and block counts that launch left, for the generic kernel (which reads
+  // the weights once for all the vectors) or, rows of more than 500 blocks, as not
+  // its own: those go one vector at a time unless they are few.
   if (type == kTypeQ6K && batch > 1 && (rows & 1u) != 0u && ((cols / kBlockElems) & 1u) != 0u &&
       (uint64_t)rows * (cols / kBlockElems) < 65536u)
     return false;
