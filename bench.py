@@ -706,8 +706,9 @@ def main() -> int:
         "vs_baseline": None,
         "dtype": ("q4_k weights (u8 packed; 4-bit quants, 6-bit scales) x activations as "
                   "block fixed point (per 256-element block: an exponent and 30-bit integers "
-                  "in four int8 digits; tiny or non-finite elements exact in f32), int8 MFMA "
-                  "with int32 accumulate, f32 combine of block sums"),
+                  "in four int8 digits; rows that small elements could put off and blocks of "
+                  "non-finite ones exact per weight), int8 MFMA with int32 accumulate, f64 "
+                  "block terms, f32 sums of them"),
         "data": "synthetic (seeded generator, BASELINE.json config 2)",
         "config": {"workload": "Q4_K matvec N=17408 x K=5120, batch 1", "rows": rows,
                    "cols": cols, "batch": 1, "weight_copies": NCOPIES,

@@ -1058,16 +1058,16 @@ SliceChoice q4_slices(uint32_t ntiles, uint32_t nb, size_t ws_bytes, int qb) {
 //   Q5_K  2560 x 17408       -     14.5     15.3
 //   Q5_K  640 x 17408        -      8.1     11.2
 //   Q5_K  1024 x 8192        -      7.4      8.7
-// So Q4_K takes two-block stages when the four-block launch leaves waves
-// idle (fewer pairs per workgroup than waves) and the two-block one needs at
-// most two rounds, or (three rounds) in rows of more than 40 blocks, which
-// leave 12 waves of four-block stages room for a few ring slots only, or none
-// (a group of 3200 + 512 + 512 x 10496 13.7 us, 12.1 in two-block stages); Q5_K,
-// whose four-block stages leave registers for only 8 waves, whenever 12 waves fit.  Slices stay where every unsliced workgroup would
-// build the whole row's activation images for a small share of the work:
-// at most a quarter as many tiles as CUs, rows of 64 blocks or more over
-// fewer tiles than CUs, and rows past 32 blocks whose busiest workgroup the
-// slices shorten.
+// So Q4_K takes two-block stages when the four-block launch leaves waves idle
+// (fewer pairs per workgroup than waves) and the two-block one needs at most two
+// rounds, or (three rounds) in rows of more than 40 blocks, which leave 12 waves
+// of four-block stages room for a few ring slots only, or none (a group of 3200 +
+// 512 + 512 x 10496 13.7 us, 12.1 in two-block stages); Q5_K, whose four-block
+// stages leave registers for only 8 waves, whenever 12 waves fit.  Slices stay
+// where every unsliced workgroup would build the whole row's activation images for
+// a small share of the work: at most a quarter as many tiles as CUs, rows of 64
+// blocks or more over fewer tiles than CUs, and rows past 32 blocks whose busiest
+// workgroup the slices shorten.
 bool two_block_stages(uint32_t ntiles, uint32_t nb, size_t ws_bytes, int qb,
                       const SliceChoice& sc) {
   constexpr uint32_t kWaves = 12u;
@@ -1214,7 +1214,8 @@ bool launch_matvec_group(uint32_t type, const uint8_t* const* w, const uint32_t*
   const uint32_t nb = cols / kBlockElems, trows = (uint32_t)total;
   // two-block stages where one matrix of the group's rows would take them
   static const int group_two_block = env_int("SI_HIP_GROUP_TWO_BLOCK", 1);
-  if (group_two_block != 0 && (type == kTypeQ4K || type == kTypeQ5K) && shape_ok(trows, cols, 1u, type == kTypeQ4K ? 4 : 5, 2u) &&
+  if (group_two_block != 0 && (type == kTypeQ4K || type == kTypeQ5K) &&
+      shape_ok(trows, cols, 1u, type == kTypeQ4K ? 4 : 5, 2u) &&
       two_block_stages((uint32_t)tiles, nb, ws.bytes, type == kTypeQ4K ? 4 : 5, SliceChoice{})) {
     if (type == kTypeQ4K &&
         launch_wd<12, 1, 1, 4, true, 2>(w[0], nullptr, x, y, trows, nb, ws, s, err, ga))

@@ -927,8 +927,8 @@ bool launch_sliced(const uint8_t* w, const float* x, float* y, uint32_t rows, ui
     return true;
   }
   hipLaunchKernelGGL((q6k_matvec_mfma<W, D, false, false, true, P>),
-                     dim3(sh.groups + (last_row ? 1u : 0u)), dim3(W * 64), lds, s, w, x, y, rows, nb, ws.ptr, sa, prefetch, GroupArgs{}, ArgmaxArgs{},
-                     sh.args);
+                     dim3(sh.groups + (last_row ? 1u : 0u)), dim3(W * 64), lds, s, w, x, y, rows,
+                     nb, ws.ptr, sa, prefetch, GroupArgs{}, ArgmaxArgs{}, sh.args);
   *err = hipGetLastError();
   return true;
 }

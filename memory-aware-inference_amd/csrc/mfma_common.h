@@ -11,11 +11,11 @@
 // 2e-5 * sum|w x| for any weights: the side elements stay in the fixed point,
 // rounded like the rest, and the block keeps, per 16-element chunk, their
 // number (each is off by at most half a unit 2^(e_b - 30)) or the bound that
-// gives.  The kernel bounds a row's error from those blocks by (largest |w| the block header
-// allows) x (that bound), and compares it with the sum of |partial dot| over the row's
-// stage, which is at most sum|w x| over the stage.  A row whose bound exceeds
-// kRoundedTol of it recomputes its rounded blocks exactly.  (The kernels of
-// several vectors build their own images, tokens_common.h.)
+// gives.  The kernel bounds a row's error from those blocks by (largest |w| the
+// block header allows) x (that bound), and compares it with the sum of |partial
+// dot| over the row's stage, which is at most sum|w x| over the stage.  A row
+// whose bound exceeds kRoundedTol of it recomputes its rounded blocks exactly.
+// (The kernels of several vectors build their own images, tokens_common.h.)
 //
 // A block with an activation that is not finite or reaches 2^100 takes the
 // exact per-weight path whole.  For every
@@ -28,8 +28,8 @@
 // lays its weights out; build_images takes that map as a template argument.
 //
 // Workgroup protocol.  One persistent workgroup per CU works through its share
-// of the (tile, stage) pairs (Sched below); a wave leaves each stage's 16 row partials in
-// an LDS slot of its tile and counts them with an LDS atomic; the wave that
+// of the (tile, stage) pairs (Sched below); a wave leaves each stage's 16 row
+// partials in an LDS slot of its tile and counts them with an LDS atomic; the wave that
 // completes the workgroup's share of a tile sums the partials in stage order
 // (results do not depend on timing).  LDS is
 // touched only through inline asm and the one barrier is a bare s_barrier:
@@ -1227,17 +1227,19 @@ inline uint32_t ring_slots(uint32_t waves, uint32_t depth, uint32_t tiles_per_wg
   return slots;
 }
 
-// Whether two vectors of a matrix (Q6_K: of an even block count) go through the one-vector kernel's two-vector form, whole rows
-// in one launch, instead of the vectors-in-rows kernel and its reduce.  The
-// launch of the reduce is what this saves: the form is ahead up to 16 blocks a
-// row, whose images of two vectors cost little, and up to 20 (Q6_K 24) where its
-// whole tiles leave at most a fifth of the workgroups without one; far larger
-// launches the vectors-in-rows kernel streams faster.  Us, this form / that kernel:
-// Q6_K 4096 x 2560 7.0 / 9.3, 16384 x 1536 8.8 / 11.9, 28000 x 3584 25.4 / 27.0,
-// 64 x 4608 8.2 / 7.5, 4096 x 6144 10.1 / 12.0, 5120 x 6144 13.4 / 12.5, 28000 x
-// 6144 41.1 / 36.9; Q5_K 4096 x 2048 6.5 / 8.9, 28000 x 3072 19.3 / 20.7, 20000 x
-// 4096 18.5 / 17.9, 16384 x 5120 20.0 / 20.3, 28000 x 5120 31.7 / 29.1; Q4_K 1024 x 1024 5.7 / 7.1, 16384 x 3584 11.8 / 12.5, 28000 x
-// 3584 19.3 / 17.5, 8192 x 5120 11.1 / 11.7, 12000 x 5120 13.6 / 13.0.
+// Whether two vectors of a matrix (Q6_K: of an even block count) go through the
+// one-vector kernel's two-vector form, whole rows in one launch, instead of the
+// vectors-in-rows kernel and its reduce.  The launch of the reduce is what this
+// saves: the form is ahead up to 16 blocks a row, whose images of two vectors cost
+// little, and up to 20 (Q6_K 24) where its whole tiles leave at most a fifth of
+// the workgroups without one; far larger launches the vectors-in-rows kernel
+// streams faster.  Us, this form / that kernel: Q6_K 4096 x 2560 7.0 / 9.3, 16384
+// x 1536 8.8 / 11.9, 28000 x 3584 25.4 / 27.0, 64 x 4608 8.2 / 7.5, 4096 x 6144
+// 10.1 / 12.0, 5120 x 6144 13.4 / 12.5, 28000 x 6144 41.1 / 36.9; Q5_K 4096 x 2048
+// 6.5 / 8.9, 28000 x 3072 19.3 / 20.7, 20000 x 4096 18.5 / 17.9, 16384 x 5120 20.0
+// / 20.3, 28000 x 5120 31.7 / 29.1; Q4_K 1024 x 1024 5.7 / 7.1, 16384 x 3584 11.8
+// / 12.5, 28000 x 3584 19.3 / 17.5, 8192 x 5120 11.1 / 11.7, 12000 x 5120 13.6 /
+// 13.0.
 inline bool two_vectors(uint32_t type, uint32_t rows, uint32_t nb) {
   const uint64_t blocks = (uint64_t)rows * nb;
   const bool longer = nb > 12u && nb <= 16u;
