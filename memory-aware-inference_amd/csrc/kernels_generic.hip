@@ -106,8 +106,9 @@ __global__ __launch_bounds__(256) void fused_gate_up_generic_kernel(
 }
 
 // Exact dequantisation of whole blocks, four elements a thread, so that a
-// wave's loads are a block's consecutive words and its stores whole lines;
-// workgroup (c, r) takes 1024 consecutive elements (chunk c) of output row r.
+// wave's loads are a block's consecutive words and its stores whole lines; the
+// four waves of workgroup (c, g) take blocks P c .. P c + P - 1 of the 4 / P
+// output rows from 4 g / P on, P = 2^lp.
 // (One 32-weight unit a thread, its bytes loaded one by one and 64-bit divisions
 // per thread: 64 rows of 5120 4.1 us by kernel trace, of which an empty launch
 // is 1.7; so 2.7.)
@@ -118,11 +119,14 @@ __global__ __launch_bounds__(256) void fused_gate_up_generic_kernel(
 template <uint32_t T>
 __global__ __launch_bounds__(256) void dequant_kernel(const uint8_t* __restrict__ w,
                                                       const uint32_t* __restrict__ row_index,
-                                                      float* __restrict__ out, uint32_t nb,
+                                                      float* __restrict__ out, uint32_t rows,
+                                                      uint32_t nb, uint32_t lp,
                                                       uint32_t table_rows, void* ws) {
   constexpr uint32_t BB = BlockBytes<T>::value;
-  const uint32_t r = blockIdx.y, blk = 4u * blockIdx.x + (threadIdx.x >> 6);
-  if (blk >= nb) return;
+  const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  const uint32_t r = (blockIdx.y << (2u - lp)) + (wave >> lp);
+  const uint32_t blk = (blockIdx.x << lp) + (wave & ((1u << lp) - 1u));
+  if (r >= rows || blk >= nb) return;
   const uint64_t src_row = row_index ? row_index[r] : r;
   const uint32_t i = 4u * (threadIdx.x & 63u);
   float4 v;
@@ -182,28 +186,35 @@ hipError_t launch_dequant(uint32_t type, const uint8_t* w, const uint32_t* row_i
   const uint64_t nb = row_index ? row_blocks : row_blocks * out_rows;
   const uint64_t nrows = row_index ? out_rows : 1u;
   if (!row_index) table_rows = 1u;
-  // A launch takes less than 2^32 threads and 2^16 workgroups in y; more rows
+  // The blocks of a row that a workgroup takes: four, or so many that no wave is
+  // left without one where the row count allows it.  (With four always, a workgroup
+  // of 256 columns had one live wave: 20,000 ids 13.7 us, 8.7 so; 400,000 233 us,
+  // 123; of 1280 columns 20,000 ids 42.8 us, 38.1.)
+  const uint32_t lp = nrows < 4u || nb % 4u == 0u ? 2u : nb % 2u == 0u ? 1u : 0u;
+  // A launch takes less than 2^32 threads in x and 2^16 workgroups in y; more rows
   // (or blocks of the one row) run as several.
-  constexpr uint64_t kRows = 32768u, kBlocks = 1u << 24;
-  for (uint64_t r0 = 0; r0 < nrows; r0 += kRows) {
+  const uint64_t most = 32768u << (2u - lp);
+  constexpr uint64_t kBlocks = 1u << 24;
+  for (uint64_t r0 = 0; r0 < nrows; r0 += most) {
     for (uint64_t b0 = 0; b0 < nb; b0 += row_index ? nb : kBlocks) {
       // (an indexed row's blocks, less than 2^24, are one launch's)
       const uint32_t n = (uint32_t)(row_index ? nb : min(nb - b0, kBlocks));
       const uint32_t* const ids = row_index ? row_index + r0 : nullptr;
       float* const o = out + (r0 * nb + b0) * kBlockElems;
-      const dim3 grid((n + 3u) / 4u, (uint32_t)min(nrows - r0, kRows));
+      const uint32_t m = (uint32_t)min(nrows - r0, most);
+      const dim3 grid((n + (1u << lp) - 1u) >> lp, (m + (4u >> lp) - 1u) >> (2u - lp));
       switch (type) {
         case kTypeQ4K:
           hipLaunchKernelGGL(dequant_kernel<kTypeQ4K>, grid, dim3(256), 0, s, w + b0 * kQ4Bytes,
-                             ids, o, n, table_rows, ws);
+                             ids, o, m, n, lp, table_rows, ws);
           break;
         case kTypeQ5K:
           hipLaunchKernelGGL(dequant_kernel<kTypeQ5K>, grid, dim3(256), 0, s, w + b0 * kQ5Bytes,
-                             ids, o, n, table_rows, ws);
+                             ids, o, m, n, lp, table_rows, ws);
           break;
         case kTypeQ6K:
           hipLaunchKernelGGL(dequant_kernel<kTypeQ6K>, grid, dim3(256), 0, s, w + b0 * kQ6Bytes,
-                             ids, o, n, table_rows, ws);
+                             ids, o, m, n, lp, table_rows, ws);
           break;
         default:
           return hipErrorInvalidValue;

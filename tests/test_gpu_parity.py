@@ -1109,10 +1109,12 @@ def test_graph_capture_state_errors(hip_ctx):
     g.free()
 
 
-@pytest.mark.parametrize("tokens,cols", [(32769, 512), (70001, 256), ((1 << 24) + 3, 256)])
+@pytest.mark.parametrize("tokens,cols", [(4, 256), (5, 512), (7, 768), (1001, 1280), (65541, 512),
+                                         (32773, 1024), (131077, 256), ((1 << 24) + 3, 256)])
 def test_embedding_many_tokens(hip_ctx, tokens, cols):
-    """More tokens than one launch's workgroups reach: the rows at both ends, at
-    the edges of a launch's share and at the most that 2^32 threads would cover."""
+    """Rows of one to five blocks, one, two or four of them in a workgroup, and more
+    than one launch's workgroups reach: the rows at both ends, at the edges of a
+    launch's share and at the most that 2^32 threads would cover."""
     log(f"embedding {tokens} x {cols}")
     vocab = 5
     table = si_hip.synth_matrix(12, seed=tokens, rows=vocab, cols=cols)
@@ -1128,7 +1130,7 @@ def test_embedding_many_tokens(hip_ctx, tokens, cols):
                                                   ctypes.c_void_p(d_out))
         assert rc == 0, si_hip.last_error()
         hip_ctx.synchronize()
-        for at in (0, 32766, 65534, (1 << 24) - 2, tokens - 4):
+        for at in (0, 32766, 65534, 131070, (1 << 24) - 2, tokens - 4):
             if at + 4 <= tokens:
                 got = hip_ctx.from_device(d_out + 4 * at * cols, 4 * cols).view(np.uint32)
                 assert np.array_equal(got.reshape(4, cols), exp[ids[at:at + 4]]), at
