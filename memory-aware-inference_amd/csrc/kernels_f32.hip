@@ -229,6 +229,8 @@ void launch_matvec_units(const float* w, const float* x, float* y, uint32_t rows
   }
 }
 
+constexpr uint64_t kManyThreads = 256u * 1024u;
+
 template <int MODE, typename U>
 void launch_norm_units(const float* x, const float* gate, const float* w, float* y,
                        uint32_t heads, uint32_t head_dim, float eps, hipStream_t s) {
@@ -246,9 +248,18 @@ void launch_norm_units(const float* x, const float* gate, const float* w, float*
                          gate ? gate + at : nullptr, w, y + at, head_dim, eps);
     }
   };
-  if (n <= 1024u)
+  uint32_t upt = n <= 1024u ? 1u : n <= 2048u ? 2u : 4u;
+  // More where single floats would take more threads than 1024 a CU of 256: a
+  // workgroup's waves cost more than the loads they hide (4000 x 1001 13.6 us with
+  // one, 7.0 with four; 4000 x 2001 17.1 with two, 12.0 with four; 256 x 1001 2.84
+  // with one, 2.72 with four).  Of float4s the first choice stays ahead to 20000 x
+  // 1000.
+  if (sizeof(U) == sizeof(float))
+    while (upt < 4u && threads(upt) > 64u && (uint64_t)heads * threads(upt) > kManyThreads)
+      upt *= 2u;
+  if (upt == 1u)
     launch(1u, &rms_norm_kernel<MODE, U, 1>);
-  else if (n <= 2048u)
+  else if (upt == 2u)
     launch(2u, &rms_norm_kernel<MODE, U, 2>);
   else
     launch(4u, &rms_norm_kernel<MODE, U, 4>);
@@ -257,8 +268,14 @@ void launch_norm_units(const float* x, const float* gate, const float* w, float*
 template <int MODE>
 void launch_norm_mode(const float* x, const float* gate, const float* w, float* y, uint32_t heads,
                       uint32_t head_dim, float eps, hipStream_t s) {
-  const bool vec = head_dim % 4u == 0u && aligned16(x) && aligned16(w) && aligned16(y) &&
-                   (MODE != 2 || aligned16(gate));
+  // Short heads in a float a thread while the card holds all of them at once: a
+  // thread's four outputs, above all their four gates, cost more than its wider
+  // loads save (48 x 128 gated 2.54 us in float4s, 2.34 in floats, 256 x 64 2.59, 2.33,
+  // 256 x 512 the same; 4000 x 256 3.87, 4.63; 48 x 128 without a gate 2.36, 2.29).
+  const bool narrow = head_dim <= (MODE == 2 ? 512u : 128u) &&
+                      (uint64_t)heads * head_dim <= kManyThreads;
+  const bool vec = !narrow && head_dim % 4u == 0u && aligned16(x) && aligned16(w) &&
+                   aligned16(y) && (MODE != 2 || aligned16(gate));
   if (vec)
     launch_norm_units<MODE, float4>(x, gate, w, y, heads, head_dim, eps, s);
   else

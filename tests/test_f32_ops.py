@@ -375,6 +375,23 @@ def test_rms_norm_register_passes(hip_ctx, mode, heads, hd):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("mode,heads,hd", [(1, 2048, 128), (1, 2049, 128), (1, 7, 132), (2, 512, 512),
+                                           (2, 513, 512), (2, 5, 516), (2, 4100, 64),
+                                           (1, 257, 1001), (1, 700, 1001), (1, 300, 2001),
+                                           (2, 5000, 129), (1, 5000, 63)])
+def test_rms_norm_units(hip_ctx, mode, heads, hd):
+    """Head counts and lengths on both sides of where short heads leave a float a thread for
+    float4s, and where many odd ones take two or four floats a thread."""
+    rng = np.random.default_rng(heads + hd)
+    x = rng.standard_normal(heads * hd).astype(np.float32)
+    w = (rng.standard_normal(hd) * 0.5).astype(np.float32)
+    g = (rng.standard_normal(heads * hd) * 3).astype(np.float32)
+    y = (hip_ctx.rms_norm_heads(x, w, heads, hd, 1e-6) if mode == 1
+         else hip_ctx.rms_norm_gated(x, g, w, heads, hd, 1e-6))
+    assert_rms_close(y, f64_rms(mode, x, w, heads, hd, 1e-6, g), f"mode {mode}")
+
+
+@pytest.mark.gpu
 def test_rms_norm_many_heads(hip_ctx):
     """More heads than 2^32 threads cover at 832 a head: the first, the last and
     those at the edge of a launch's share."""
